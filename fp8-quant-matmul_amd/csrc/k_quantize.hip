@@ -17,43 +17,41 @@
 // (/root/reference/check.cu:164-167):  q at row + k*rows, the 1 x 128 scales at row + kb*rows,
 // the 128 x 128 scales at nb + kb*ceil(rows/128).
 //
-// One workgroup owns a 128-row x 128-k tile (one scale block, or 128 scale groups).  Sixteen
-// lanes read one row's 128 elements as 16- or 32-byte pieces (whole cache lines per row); the
-// fp8 bytes go through LDS transposed, and leave as 16-byte pieces of 128-byte row segments.
-// The kernel moves 2 (or 4) bytes in and 1 byte out per element: it is bound by HBM.
+// One workgroup owns QTILE rows x 128 k (QTILE / 128 scale blocks, or QTILE scale groups).  A thread reads 8 k of
+// four adjacent rows at a time (16 lanes take a row's 128 elements: whole cache lines) and converts pairs of ROWS, so
+// that the four bytes of one k leave the conversion as the dword the transposed layout wants: the transposition costs
+// eight dword writes into the LDS per 32 elements and no byte shuffling.  From there the tile leaves as 16-byte
+// pieces of QTILE-byte row segments.  The kernel moves 2 (or 4) bytes in and 1 byte out per element: bound by HBM.
 #include "device_common.h"
 #include "launchers.h"
+
+#include <type_traits>
 
 namespace fp8gemm {
 
 namespace {
 
-// LDS bytes per k-row of the transposed tile of 128 (64) rows.  33 (17) dwords: the byte stores of a wave (16
-// k-rows 8 apart, 4 adjacent rows of the source) fall into 8 banks two deep, the dword reads into distinct banks.
-constexpr int q_stride(int rows) { return rows + 4; }
-
-__device__ __forceinline__ void load8(const uint16_t* p, float (&v)[8])
+// eight consecutive k of one row as they lie in memory: four words of bf16 pairs, or eight of fp32
+__device__ __forceinline__ void load_raw(const uint16_t* p, uint32_t (&w)[4])
 {
-    const uint4 w = *reinterpret_cast<const uint4*>(p);
-    const uint32_t u[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        v[2 * i] = __uint_as_float(u[i] << 16);
-        v[2 * i + 1] = __uint_as_float(u[i] & 0xFFFF0000u);
-    }
+    const uint4 v = *reinterpret_cast<const uint4*>(p);
+    w[0] = v.x; w[1] = v.y; w[2] = v.z; w[3] = v.w;
 }
-
-__device__ __forceinline__ void load8(const float* p, float (&v)[8])
+__device__ __forceinline__ void load_raw(const float* p, uint32_t (&w)[8])
 {
-    const float4 lo = reinterpret_cast<const float4*>(p)[0];
-    const float4 hi = reinterpret_cast<const float4*>(p)[1];
-    v[0] = lo.x; v[1] = lo.y; v[2] = lo.z; v[3] = lo.w;
-    v[4] = hi.x; v[5] = hi.y; v[6] = hi.z; v[7] = hi.w;
+    const uint4 lo = reinterpret_cast<const uint4*>(p)[0], hi = reinterpret_cast<const uint4*>(p)[1];
+    w[0] = lo.x; w[1] = lo.y; w[2] = lo.z; w[3] = lo.w;
+    w[4] = hi.x; w[5] = hi.y; w[6] = hi.z; w[7] = hi.w;
 }
-
-__device__ __forceinline__ float clamp_pm448(float v)
+template <int J>
+__device__ __forceinline__ float value(const uint32_t (&w)[4])
 {
-    return fminf(fmaxf(v, -448.0f), 448.0f);
+    return __uint_as_float((J & 1) ? w[J >> 1] & 0xFFFF0000u : w[J >> 1] << 16);
+}
+template <int J>
+__device__ __forceinline__ float value(const uint32_t (&w)[8])
+{
+    return __uint_as_float(w[J]);
 }
 
 template <bool BF16MATH>
@@ -62,161 +60,243 @@ __device__ __forceinline__ float q_round(float v)
     return BF16MATH ? __uint_as_float(pack_bf16x2(v, 0.0f) << 16) : v;
 }
 
-template <bool BF16MATH>
-__device__ __forceinline__ float q_value(float x, float scale)
+// two scaled values (of two rows), rounded to bf16 first where the source's arithmetic does that, saturated (NaN
+// becomes -448, as min(max(v, -448), 448) has it), as two fp8 bytes in the half of `old` that HIGH names
+template <bool BF16MATH, bool HIGH>
+__device__ __forceinline__ int q_pair(float x, float y, int old)
 {
-    return clamp_pm448(q_round<BF16MATH>(x * scale));
+    if (BF16MATH) {
+        const uint32_t u = pack_bf16x2(x, y);
+        x = __uint_as_float(u << 16);
+        y = __uint_as_float(u & 0xFFFF0000u);
+    }
+    return __builtin_amdgcn_cvt_pk_fp8_f32(__builtin_amdgcn_fmed3f(x, -448.0f, 448.0f),
+                                           __builtin_amdgcn_fmed3f(y, -448.0f, 448.0f), old, HIGH);
 }
 
-// BLOCK = false: one scale per row and tile (1 x 128).  BLOCK = true: one per tile (128 x 128).
-// QTILE = rows of a workgroup's tile: 128, or 64 for the 1 x 128 quantiser on matrices of a few hundred to a few
-// thousand rows, whose 128-row tiles are too few workgroups to overlap one's loads with another's stores.
-template <typename TIn, bool BLOCK, bool BF16MATH, int QTILE = 128>
-__global__ void __launch_bounds__(256)
+// v of another lane of the same 16-lane row (rotation by N), or of lane J of the same group of four
+template <int N>
+__device__ __forceinline__ float row_rotate(float v)
+{
+    return __uint_as_float((uint32_t)__builtin_amdgcn_mov_dpp((int)__float_as_uint(v), 0x120 + N, 0xF, 0xF, true));
+}
+template <int J>
+__device__ __forceinline__ float quad_lane(float v)
+{
+    return __uint_as_float((uint32_t)__builtin_amdgcn_mov_dpp((int)__float_as_uint(v), J * 0x55, 0xF, 0xF, true));
+}
+
+__device__ __forceinline__ float row_max(float a)
+{
+    a = fmaxf(a, row_rotate<1>(a));
+    a = fmaxf(a, row_rotate<2>(a));
+    a = fmaxf(a, row_rotate<4>(a));
+    return fmaxf(a, row_rotate<8>(a));
+}
+template <int J>
+using Index = std::integral_constant<int, J>;
+
+template <bool BF16MATH>
+__device__ __forceinline__ float scale_of(float amax)
+{
+    const float recip = q_round<BF16MATH>(1.0f / fmaxf(amax, q_round<BF16MATH>(1e-12f)));
+    return q_round<BF16MATH>(recip * 448.0f);
+}
+
+// BLOCK = false: one scale per row and 128 k (1 x 128).  BLOCK = true: one per 128 x 128.
+// QTILE = rows of a workgroup's tile, 16 per wave (4 rows x 8 k per thread).
+template <typename TIn, bool BLOCK, bool BF16MATH, int QTILE>
+__global__ void __launch_bounds__(QTILE * 4)
 quantize_kernel(const TIn* __restrict__ x, uint8_t* __restrict__ q, float* __restrict__ scale_out,
                 int rows, int K, int vec_store)
 {
-    static_assert(QTILE == 128 || (QTILE == 64 && !BLOCK), "128 rows, or 64 for the row-wise scales");
-    constexpr int QSTRIDE = q_stride(QTILE);
-    constexpr int PASSES = QTILE / 16;  // rows per thread
-    __shared__ __attribute__((aligned(16))) uint8_t tile[128 * QSTRIDE];
-    __shared__ float s_inv[QTILE];
-    __shared__ float s_red[4];
+    constexpr int NT = QTILE * 4, NW = NT / 64;
+    static_assert(!BLOCK || QTILE % 128 == 0, "whole scale blocks");
+    // LDS: one row of QTILE bytes per k, its 16-byte chunks (four dwords: the rows of one wave) permuted by
+    // k so that the dword writes of a wave -- 16 k that are 8 apart, one chunk -- go to as many banks as there are
+    constexpr int CH = QTILE / 16;                        // chunks per k-row
+    constexpr int STRIDE = QTILE == 64 ? 80 : QTILE;
+    constexpr int KSH = QTILE == 64 ? 4 : 3;
+    __shared__ __attribute__((aligned(16))) uint8_t tile[128 * STRIDE];
+    __shared__ float s_red[NW];
 
     const int t = threadIdx.x;
-    const int c = t & 15;   // 8-element piece of the row's 128
-    const int r0 = t >> 4;  // row of the first pass; pass p handles row r0 + 16 p
+    const int lane = t & 63, wave = t >> 6;
+    const int c = lane & 15;   // 8-element piece of the row's 128
+    const int g = lane >> 4;   // four rows
     const int row0 = blockIdx.x * QTILE;
     const int kb = blockIdx.y;
+    // One tile holds all rows (a decode batch): the K block's output, [128][rows] bytes, is one contiguous piece of
+    // memory.  The tile is kept packed like it in the LDS and leaves as it lies.
+    const bool packed = QTILE <= 64 && rows <= QTILE && !vec_store && (reinterpret_cast<uintptr_t>(q) & 15) == 0;
 
-    float v[PASSES][8];
-    float amax[PASSES];
+    // rows past the last are read as the last one: no branch around a load, all of them are in flight together (they
+    // do not change the block's amax, and their bytes are not stored)
+    uint32_t raw[4][2 * sizeof(TIn)];
 #pragma unroll
-    for (int p = 0; p < PASSES; ++p) {
-        const int row = row0 + r0 + 16 * p;
-        if (row < rows) {
-            load8(x + (size_t)row * K + (size_t)kb * 128 + 8 * c, v[p]);
-        } else {
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-                v[p][j] = 0.0f;
-        }
-        float a = 0.0f;
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-            a = fmaxf(a, __builtin_fabsf(v[p][j]));
-        amax[p] = a;
+    for (int i = 0; i < 4; ++i) {
+        const int row = row0 + 16 * wave + 4 * g + i;
+        load_raw(x + (size_t)(row < rows ? row : rows - 1) * K + (size_t)kb * 128 + 8 * c, raw[i]);
     }
 
+    float amax[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        auto mag = [&](auto j) __attribute__((always_inline)) { return __builtin_fabsf(value<decltype(j)::value>(raw[i])); };
+        const float lo = fmaxf(fmaxf(mag(Index<0>{}), mag(Index<1>{})), fmaxf(mag(Index<2>{}), mag(Index<3>{})));
+        const float hi = fmaxf(fmaxf(mag(Index<4>{}), mag(Index<5>{})), fmaxf(mag(Index<6>{}), mag(Index<7>{})));
+        amax[i] = fmaxf(fmaxf(lo, hi), 0.0f);  // a group of NaNs has amax 0
+    }
+
+    float scale[4];
     if (BLOCK) {
-        float a = amax[0];
-#pragma unroll
-        for (int p = 1; p < PASSES; ++p)
-            a = fmaxf(a, amax[p]);
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1)
-            a = fmaxf(a, __shfl_xor(a, d));
-        if ((t & 63) == 0)
-            s_red[t >> 6] = a;
+        float a = fmaxf(fmaxf(amax[0], amax[1]), fmaxf(amax[2], amax[3]));
+        a = row_max(a);
+        a = fmaxf(a, __shfl_xor(a, 16));
+        a = fmaxf(a, __shfl_xor(a, 32));
+        if (lane == 0)
+            s_red[wave] = a;
         __syncthreads();
-        a = fmaxf(fmaxf(s_red[0], s_red[1]), fmaxf(s_red[2], s_red[3]));
+        const int first = wave & ~7;  // the eight waves of a scale block
+        a = s_red[first];
 #pragma unroll
-        for (int p = 0; p < PASSES; ++p)
-            amax[p] = a;
+        for (int w = 1; w < 8; ++w)
+            a = fmaxf(a, s_red[first + w]);
+        const float mine = scale_of<BF16MATH>(a);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            scale[i] = mine;
+        const int nb = blockIdx.x * (QTILE / 128) + (wave >> 3), nblocks = (rows + 127) >> 7;
+        if ((wave & 7) == 0 && lane == 0 && nb < nblocks)
+            scale_out[(size_t)kb * nblocks + nb] = 1.0f / mine;
     } else {
-#pragma unroll
-        for (int p = 0; p < PASSES; ++p)
-#pragma unroll
-            for (int d = 1; d < 16; d <<= 1)
-                amax[p] = fmaxf(amax[p], __shfl_xor(amax[p], d));
+        // lane c works out the scale of row c & 3 of its four, the others take it over from there
+        const float a0 = row_max(amax[0]), a1 = row_max(amax[1]), a2 = row_max(amax[2]), a3 = row_max(amax[3]);
+        const float lo = (c & 1) ? +a1 : +a0, hi = (c & 1) ? +a3 : +a2;
+        const float mine = scale_of<BF16MATH>((c & 2) ? +hi : +lo);
+        scale[0] = quad_lane<0>(mine);
+        scale[1] = quad_lane<1>(mine);
+        scale[2] = quad_lane<2>(mine);
+        scale[3] = quad_lane<3>(mine);
+        const int row = row0 + 16 * wave + 4 * g + c;
+        if (c < 4 && row < rows)
+            scale_out[(size_t)kb * rows + row] = 1.0f / mine;
     }
 
+    auto put = [&](auto jc) __attribute__((always_inline)) {
+        constexpr int j = decltype(jc)::value;
+        int w = q_pair<BF16MATH, false>(value<j>(raw[0]) * scale[0], value<j>(raw[1]) * scale[1], 0);
+        w = q_pair<BF16MATH, true>(value<j>(raw[2]) * scale[2], value<j>(raw[3]) * scale[3], w);
+        const int k = 8 * c + j;
+        if (packed) {
+            const int r = 16 * wave + 4 * g;
 #pragma unroll
-    for (int p = 0; p < PASSES; ++p) {
-        const int r = r0 + 16 * p;
-        const float recip = q_round<BF16MATH>(1.0f / fmaxf(amax[p], q_round<BF16MATH>(1e-12f)));
-        const float scale = q_round<BF16MATH>(recip * 448.0f);
-        int w0 = 0, w1 = 0;
-        w0 = __builtin_amdgcn_cvt_pk_fp8_f32(q_value<BF16MATH>(v[p][0], scale), q_value<BF16MATH>(v[p][1], scale), w0, false);
-        w0 = __builtin_amdgcn_cvt_pk_fp8_f32(q_value<BF16MATH>(v[p][2], scale), q_value<BF16MATH>(v[p][3], scale), w0, true);
-        w1 = __builtin_amdgcn_cvt_pk_fp8_f32(q_value<BF16MATH>(v[p][4], scale), q_value<BF16MATH>(v[p][5], scale), w1, false);
-        w1 = __builtin_amdgcn_cvt_pk_fp8_f32(q_value<BF16MATH>(v[p][6], scale), q_value<BF16MATH>(v[p][7], scale), w1, true);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            tile[(8 * c + j) * QSTRIDE + r] = (uint8_t)((uint32_t)w0 >> (8 * j));
-            tile[(8 * c + 4 + j) * QSTRIDE + r] = (uint8_t)((uint32_t)w1 >> (8 * j));
+            for (int i = 0; i < 4; ++i)
+                if (r + i < rows)
+                    tile[k * rows + r + i] = (uint8_t)((uint32_t)w >> (8 * i));
+        } else {
+            *reinterpret_cast<int*>(tile + k * STRIDE + ((wave ^ ((k >> KSH) & (CH - 1))) << 4) + 4 * g) = w;
         }
-        if (!BLOCK && c == 0)
-            s_inv[r] = 1.0f / scale;
-        if (BLOCK && t == 0 && p == 0)
-            scale_out[(size_t)kb * gridDim.x + blockIdx.x] = 1.0f / scale;
-    }
+    };
+    put(Index<0>{});
+    put(Index<1>{});
+    put(Index<2>{});
+    put(Index<3>{});
+    put(Index<4>{});
+    put(Index<5>{});
+    put(Index<6>{});
+    put(Index<7>{});
     __syncthreads();
 
-    if (!BLOCK && t < QTILE && row0 + t < rows)
-        scale_out[(size_t)kb * rows + row0 + t] = s_inv[t];
+    if (packed) {
+        for (int idx = t; idx < 8 * rows; idx += NT)
+            reinterpret_cast<uint4*>(q + (size_t)kb * 128 * rows)[idx] = reinterpret_cast<const uint4*>(tile)[idx];
+        return;
+    }
 
-    // k-row kk of the tile: QTILE bytes, one per source row; lane takes 16 of them
-    constexpr int LPR = QTILE / 16;  // lanes per k-row
-    const int dq = t % LPR;
+    // k-row kk of the tile: QTILE bytes, one per source row
+    if (vec_store) {  // every k-row starts on a 16-byte boundary: a lane takes 16 of its bytes
+        const int dq = t % CH, first = row0 + 16 * dq;
 #pragma unroll
-    for (int pass = 0; pass < 128 * LPR / 256; ++pass) {
-        const int kk = t / LPR + (256 / LPR) * pass;
-        const uint32_t* src = reinterpret_cast<const uint32_t*>(tile + kk * QSTRIDE + 16 * dq);
-        const uint32_t w[4] = {src[0], src[1], src[2], src[3]};
-        const int first = row0 + 16 * dq;
-        const size_t o = (size_t)(kb * 128 + kk) * rows + first;
-        if (vec_store && first + 16 <= rows) {
-            *reinterpret_cast<uint4*>(q + o) = make_uint4(w[0], w[1], w[2], w[3]);
-        } else if (first + 16 <= rows) {
-            // a row count off the 16-byte grid: the piece starts at any byte.  The bytes up to the next dword
-            // boundary one by one, three whole dwords shifted into place, the rest one by one
-            uint8_t* d = q + o;
-            const uint32_t head = (4u - (uint32_t)(reinterpret_cast<uintptr_t>(d) & 3)) & 3;  // 0 ... 3 bytes
-            if (head == 0) {
+        for (int pass = 0; pass < 128 * CH / NT; ++pass) {
+            const int kk = t / CH + (NT / CH) * pass;
+            const uint4 v = *reinterpret_cast<const uint4*>(tile + kk * STRIDE + ((dq ^ ((kk >> KSH) & (CH - 1))) << 4));
+            if (first < rows)
+                *reinterpret_cast<uint4*>(q + (size_t)(kb * 128 + kk) * rows + first) = v;
+        }
+        return;
+    }
+    // A row count off the 16-byte grid (a ragged token count): the segment starts at any byte.  The 16-byte pieces of
+    // MEMORY that lie inside it are shifted into place and leave as whole stores; the fewer than 16 bytes before the
+    // first and behind the last of them leave byte by byte, a lane each.
+    const int len = rows - row0 < QTILE ? rows - row0 : QTILE;
+    auto at = [&](int kk, int byte) __attribute__((always_inline)) {
+        return tile + kk * STRIDE + (((byte >> 4) ^ ((kk >> KSH) & (CH - 1))) << 4) + (byte & 15);
+    };
+#pragma unroll 2
+    for (int idx = t; idx < 128 * CH; idx += NT) {
+        const int kk = idx / CH, slot = idx % CH;
+        uint8_t* seg = q + (size_t)(kb * 128 + kk) * rows + row0;
+        const int o = 16 * slot + ((0 - (int)reinterpret_cast<uintptr_t>(seg)) & 15);  // the piece's first byte, in the segment
+        if (o + 16 <= len) {
+            uint32_t in[5], w[4];
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    reinterpret_cast<uint32_t*>(d)[i] = w[i];
-            } else {
+            for (int i = 0; i < 5; ++i)
+                in[i] = *reinterpret_cast<const uint32_t*>(at(kk, ((o & ~3) + 4 * i) & (QTILE - 1)));
 #pragma unroll
-                for (int j = 0; j < 3; ++j)
-                    if ((uint32_t)j < head)
-                        d[j] = (uint8_t)(w[0] >> (8 * j));
-#pragma unroll
-                for (int i = 0; i < 3; ++i)
-                    *reinterpret_cast<uint32_t*>(d + head + 4 * i) = __builtin_amdgcn_alignbyte(w[i + 1], w[i], head);
-#pragma unroll
-                for (int j = 1; j < 4; ++j)  // bytes head + 12 ... 15 are bytes head ... 3 of the last dword
-                    if ((uint32_t)j >= head)
-                        d[12 + j] = (uint8_t)(w[3] >> (8 * j));
-            }
-        } else {
-#pragma unroll
-            for (int j = 0; j < 16; ++j)
-                if (first + j < rows)
-                    q[o + j] = (uint8_t)(w[j >> 2] >> (8 * (j & 3)));
+            for (int i = 0; i < 4; ++i)
+                w[i] = __builtin_amdgcn_alignbyte(in[i + 1], in[i], (uint32_t)o & 3);
+            *reinterpret_cast<uint4*>(seg + o) = make_uint4(w[0], w[1], w[2], w[3]);
+        }
+    }
+#pragma unroll 4
+    for (int idx = t; idx < 128 * 32; idx += NT) {
+        const int kk = idx >> 5, e = idx & 31;
+        uint8_t* seg = q + (size_t)(kb * 128 + kk) * rows + row0;
+        int head = (0 - (int)reinterpret_cast<uintptr_t>(seg)) & 15;
+        head = head < len ? head : len;
+        const int tail = (len - head) & 15;
+        if (e < head + tail) {
+            const int byte = e < head ? e : len - tail + e - head;
+            seg[byte] = *at(kk, byte);
         }
     }
 }
 
-// 128-row tiles of the 1 x 128 quantiser between these counts run as 64-row tiles
-constexpr long HALF_TILE_LO = 1, HALF_TILE_HI = 2500;
-
-template <typename TIn, bool BF16MATH>
-void launch_quantize_typed(const TIn* x, uint8_t* q, float* scale_out, int rows, int k, bool block128,
-                           hipStream_t s)
+template <typename TIn, bool BLOCK, bool BF16MATH, int QTILE>
+void launch_quantize_tile(const TIn* x, uint8_t* q, float* scale_out, int rows, int k, hipStream_t s)
 {
-    const dim3 grid((rows + 127) / 128, k / 128);
     const int vec_store = (rows % 16 == 0) && (reinterpret_cast<uintptr_t>(q) % 16 == 0);
+    hipLaunchKernelGGL((quantize_kernel<TIn, BLOCK, BF16MATH, QTILE>), dim3((rows + QTILE - 1) / QTILE, k / 128),
+                       dim3(QTILE * 4), 0, s, x, q, scale_out, rows, k, vec_store);
+}
+
+// Tile sizes, measured with every operand from HBM (us, previous kernel -> this one):
+//   128 x 128 blocks: 128 rows, eight waves of 16, whatever the size (512 x 2048 6.5 -> 3.5, 4608 x 7168 28.8 -> 22.0 =
+//   4.5 TB/s; 256-row tiles 4.5 and 23.3).
+//   1 x 128 groups, up to 64 rows: a decode batch is launch and latency.  One wave per 16 rows up to 32 rows on the
+//   16-byte grid or 16 off it (16 rows 3.8 -> 2.5, 64-row tiles 3.1), else 64-row tiles (24 rows 3.9 -> 3.2, 64 rows
+//   4.5 -> 2.9).
+//   More rows: 256-row tiles once they make 256 workgroups, whose k-rows leave in pieces of 256 bytes (8192 x 7168
+//   46.3 -> 37.1 = 4.7 TB/s, 8191 x 7168 75 -> 48.6 against 54.1 with 128 rows).  Fewer than that, on the grid: 64 rows
+//   up to 1024 tiles (1024 x 2048 5.7 -> 3.8, with 128 rows 4.2), else 128; off the grid 128 rows, which have fewer
+//   ends of segments to store byte by byte (333 x 7168 8.1 -> 6.1, with 64 rows 7.5).
+template <typename TIn, bool BF16MATH>
+void launch_quantize_typed(const TIn* x, uint8_t* q, float* scale_out, int rows, int k, bool block128, hipStream_t s)
+{
+    const bool on_grid = rows % 16 == 0;
+    const long nkb = k / 128;
+    auto tiles = [&](int qtile) { return (rows + qtile - 1) / qtile * nkb; };
     if (block128)
-        hipLaunchKernelGGL((quantize_kernel<TIn, true, BF16MATH>), grid, dim3(256), 0, s, x, q, scale_out, rows,
-                           k, vec_store);
-    else if (HALF_TILE_LO <= (long)grid.x * grid.y && (long)grid.x * grid.y <= HALF_TILE_HI)
-        hipLaunchKernelGGL((quantize_kernel<TIn, false, BF16MATH, 64>), dim3((rows + 63) / 64, k / 128), dim3(256), 0, s, x,
-                           q, scale_out, rows, k, vec_store);
+        launch_quantize_tile<TIn, true, BF16MATH, 128>(x, q, scale_out, rows, k, s);
+    else if (rows <= (on_grid ? 32 : 16))
+        launch_quantize_tile<TIn, false, BF16MATH, 16>(x, q, scale_out, rows, k, s);
+    else if (rows <= 64 || (on_grid && tiles(64) <= 1024))
+        launch_quantize_tile<TIn, false, BF16MATH, 64>(x, q, scale_out, rows, k, s);
+    else if (tiles(256) < 256)
+        launch_quantize_tile<TIn, false, BF16MATH, 128>(x, q, scale_out, rows, k, s);
     else
-        hipLaunchKernelGGL((quantize_kernel<TIn, false, BF16MATH>), grid, dim3(256), 0, s, x, q, scale_out, rows,
-                           k, vec_store);
+        launch_quantize_tile<TIn, false, BF16MATH, 256>(x, q, scale_out, rows, k, s);
 }
 
 }  // namespace

@@ -148,3 +148,30 @@ def test_gemm_on_device_quantised_inputs_equals_gemm_on_oracle_inputs(pkg):
     ref = oracle.ref_gemm(a, b, sa, sb, m, n, k)
     r = oracle.compare_bf16(dc.cpu().numpy().view(np.uint16), ref, 1e-2, 1e-3)
     assert r["bad"] == 0, r
+
+
+@pytest.mark.parametrize("rows,k,offset", [
+    (15, 256, 0), (17, 256, 0), (31, 128, 0), (33, 384, 0), (64, 256, 0), (63, 256, 3),   # one tile, packed or not
+    (32, 256, 8), (65, 256, 0), (80, 128, 0), (255, 256, 1), (257, 128, 0),               # 64- and 128-row tiles
+    (16384, 512, 0), (16401, 512, 0), (16399, 512, 5),                                    # 256-row tiles
+])
+def test_quantize_tile_sizes_and_ends(pkg, rows, k, offset):
+    """every tile size of the quantisers at the row counts where one takes over from the next, with outputs that start
+    `offset` bytes off a 16-byte boundary: bytes and scales equal the oracle's, nothing around the output is written"""
+    import torch
+    x = oracle.gen_normal_bf16(rows, k, 7 + rows + k, 1.0, 50.0)
+    for which in ("a", "b"):
+        dx = torch.from_numpy(_bf16_bits(x).view(np.int16)).cuda()
+        buf = torch.full((64 + k * rows + 64,), 0x7F, dtype=torch.uint8, device="cuda")
+        dq = buf[64 + offset: 64 + offset + k * rows]
+        ncol = rows if which == "a" else (rows + 127) // 128
+        ds = torch.full((k // 128, ncol), float("nan"), dtype=torch.float32, device="cuda")
+        _say(f"[gpu case] quantize_{which} rows={rows} k={k} offset={offset}")
+        fn = pkg.quantize_a_1x128 if which == "a" else pkg.quantize_b_128x128
+        fn(dx, dq, ds, rows, k, pkg.DTYPE_BF16, torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        rq, rs = (oracle.quantize_a_1x128 if which == "a" else oracle.quantize_b_128x128)(x, bf16_arith=True)
+        assert np.array_equal(ds.cpu().numpy().view(np.uint32), rs.view(np.uint32)), which
+        assert np.array_equal(dq.cpu().numpy().reshape(k, rows), rq), which
+        guard = torch.cat([buf[:64 + offset], buf[64 + offset + k * rows:]])
+        assert (guard == 0x7F).all(), which
