@@ -23,7 +23,11 @@
 //     instruction would write 8-byte pieces of 32 different rows.
 //   * a_scale values of the tile travel through LDS with the stage (one extra 1 KiB copy), so
 //     the K loop holds no compiler-visible global load and every wait on the copies is the
-//     explicit one below.
+//     explicit one below.  b_scale is asked for by scalar loads one K block ahead: in the block that
+//     needs it its trip to the L2 would stand in front of the MFMAs (from the Infinity Cache, 128 x 128
+//     tiles, 336 x 4608 x 7168: 27.1 -> 22.6 us; 1024 x 1536 x 7168: 24.9 -> 21.6 us).  The smallest tile is
+//     done before that trip is: there a wave that does not multiply copies b_scale into the stage
+//     (48 x 4608 x 7168: 14.2 -> 10.9 us).
 //   * NS LDS stages form a ring: the copies of K blocks kb+1 .. kb+NS-1 are in flight while
 //     block kb is multiplied.  Large tiles fit two stages; smaller tiles get three or four,
 //     which is what hides the global latency when a K block is only a few MFMAs long.
@@ -57,6 +61,7 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
     static_assert(TN <= 128, "a wave's n range touches at most two 128-wide scale blocks");
     static_assert(BM <= 256 && BN <= 256, "LDS rows hold at most 256 bytes");
     constexpr int RSA = S::RSA, RSB = S::RSB, NA = S::NA, NB = S::NB, NCOPY = S::NCOPY;
+    constexpr int SCALE_WAVE = NCW == 4 ? 4 : 0;  // brings the a_scale slice: a wave that does not multiply, if there is one
 
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
     auto lds = LDS_PTR(uint8_t, smem);
@@ -118,6 +123,9 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
     // resources stay fixed; the K block's byte offset rides in the scalar offset operand.
     const v4i rsrc_a = make_rsrc_words(a, a_bytes), rsrc_b = make_rsrc_words(b, b_bytes);
     const v4i rsrc_s = make_rsrc_words(a_scale, as_bytes);
+    const int sn = (N + KBLOCK - 1) / KBLOCK;
+    const v4i rsrc_bs = make_rsrc_words(b_scale, (uint32_t)nkb * (uint32_t)sn * 4u);
+    const uint32_t voff_sb = lane == 0 ? (uint32_t)((n0 >> 7) * 4) : 0x80000000u;  // staged: the tile is at most 128 wide
     auto copy_step = [&](int slot, int kb, int q) __attribute__((always_inline)) {
         const uint32_t stage = lds_base + (uint32_t)(slot * S::STAGE);
         if (q < NA) {
@@ -127,8 +135,10 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
             lds_dma16(rsrc_b, voff_b[S::template voff_index<RSB>(q - NA)],
                       stage + S::MAT_A + (uint32_t)((NB * wave + (q - NA)) * 1024),
                       (uint32_t)(kb * KBLOCK + S::template extra_rows<RSB>(q - NA)) * (uint32_t)N);
-        } else if (wave == 0) {
+        } else if (wave == SCALE_WAVE) {
             lds_dma16(rsrc_s, voff_s, stage + S::SCALE_OFF, (uint32_t)kb * (uint32_t)lda * 4u);
+        } else if (S::SB_STAGED && wave == SCALE_WAVE + 1) {
+            lds_dma4(rsrc_bs, voff_sb, stage + S::SB_OFF, (uint32_t)kb * (uint32_t)sn * 4u);
         }
     };
 
@@ -161,7 +171,6 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
     // ---- scales.  One a_scale per lane and 32-row patch (the lane's m).  A wave's n range is at
     // most 128 wide, so it touches at most two 128-wide b_scale blocks (nb_lo, nb_hi); a 32-wide
     // patch never straddles a block boundary.
-    const int sn = (N + KBLOCK - 1) / KBLOCK;
     const int n_wave = n0 + wn * TN;
     int nb_lo = n_wave >> 7, nb_hi = (n_wave + TN - 1) >> 7;
     nb_lo = nb_lo < sn ? nb_lo : sn - 1;
@@ -193,6 +202,13 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
     int slot = 0;             // ring slot of block kb
     int slot_fill = NS - 1;   // ring slot that block kb + NS - 1 goes into (= slot of kb - 1)
 
+    // b_scale of the next block (wave-uniform addresses: scalar loads)
+    float next_lo = 0.f, next_hi = 0.f;
+    if (!S::SB_STAGED) {
+        next_lo = b_scale[__builtin_amdgcn_readfirstlane(kb0 * sn + nb_lo)];
+        next_hi = b_scale[__builtin_amdgcn_readfirstlane(kb0 * sn + nb_hi)];
+    }
+
     // One K block.  MORE = block kb+NS-1 exists and is copied here; two instantiations keep the
     // steady-state body free of branches.
     auto k_block = [&](auto more_tag, int kb) {
@@ -222,14 +238,17 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
             slot = (slot + 1 == NS) ? 0 : slot + 1;
             return;
         }
+        // b_scale of this block, asked for during the last one: waited for here, before any LDS read is in flight (behind
+        // a scalar load that is still out every wait for an LDS read is a wait for all of them)
+        const float sb_lo = next_lo, sb_hi = next_hi;
+        if (!S::SB_STAGED)
+            asm volatile("" ::"s"(sb_lo), "s"(sb_hi));
         const uint32_t so = (uint32_t)(slot * S::STAGE);
+        const float sb_stage = S::SB_STAGED ? *LDS_PTR(float, lds + so + S::SB_OFF) : 0.f;
         float sa[MI];
 #pragma unroll
         for (int i = 0; i < MI; ++i)
             sa[i] = *LDS_PTR(float, lds + so + addr_s + 128 * i);
-        // wave-uniform addresses: scalar loads
-        const float sb_lo = b_scale[__builtin_amdgcn_readfirstlane(kb * sn + nb_lo)];
-        const float sb_hi = b_scale[__builtin_amdgcn_readfirstlane(kb * sn + nb_hi)];
 
         v8i fa[MI][2];
 #pragma unroll
@@ -269,13 +288,21 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
                                                                           0, 0, 0);
                 copy_slot(PER_MFMA);
             }
+            if (j == NJ - 1 && !S::SB_STAGED) {
+                // the next block's b_scale, behind this block's last LDS read: its trip to the L2 (a block's values share
+                // no cache line with the next one's unless N is small) is covered by the fold and the barrier
+                int next = kb + 1 < kb1 ? kb + 1 : kb;
+                asm volatile("" : "+s"(next));
+                next_lo = b_scale[next * sn + nb_lo];
+                next_hi = b_scale[next * sn + nb_hi];
+            }
 #pragma unroll
             for (int i = 0; i < MI; ++i) {
                 // wave-uniform choice of the b_scale value on the scalar unit (bit select), then one
                 // product per patch
                 const float sbj = __uint_as_float((__float_as_uint(sb_hi) & hi_mask[j]) |
                                                   (__float_as_uint(sb_lo) & ~hi_mask[j]));
-                const float sc = sa[i] * sbj;
+                const float sc = sa[i] * (S::SB_STAGED ? sb_stage : sbj);
 #pragma unroll
                 for (int r = 0; r < 16; ++r)
                     acc[i][j][r] = fmaf(sc, blk[i][r], acc[i][j][r]);

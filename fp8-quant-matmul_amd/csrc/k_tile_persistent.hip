@@ -419,6 +419,9 @@ __device__ __forceinline__ void persistent_body(const Problem& one, const GroupT
                 for (int r = 0; r < 16; ++r)
                     acc[i][jj][r] = 0.f;
 
+        float next_lo = b_scale[__builtin_amdgcn_readfirstlane(nb_lo)];
+        float next_hi = b_scale[__builtin_amdgcn_readfirstlane(nb_hi)];
+
         // One K block.  MORE = the stream has a block left to copy (always, except for the last
         // NS-1 blocks of the last tile).
         auto k_block = [&](auto more_tag, int kb) __attribute__((always_inline)) {
@@ -441,14 +444,21 @@ __device__ __forceinline__ void persistent_body(const Problem& one, const GroupT
                 }
             }
             __syncthreads();  // block landed for everyone; slot_fill is no longer read
+            // b_scale of this block, asked for during the last one (k_tile.hip)
+            const float sb_lo = next_lo, sb_hi = next_hi;
+            asm volatile("" ::"s"(sb_lo), "s"(sb_hi));
             const uint32_t so = (uint32_t)(slot * S::STAGE);
             float sa[MI];
 #pragma unroll
             for (int i = 0; i < MI; ++i)
                 sa[i] = *LDS_PTR(float, lds + so + addr_s + 128 * i);
-            const float sb_lo = b_scale[__builtin_amdgcn_readfirstlane(kb * sn + nb_lo)];
-            const float sb_hi = b_scale[__builtin_amdgcn_readfirstlane(kb * sn + nb_hi)];
 
+            auto ask_next_scale = [&]() __attribute__((always_inline)) {
+                int next = __builtin_amdgcn_readfirstlane(kb + 1 < nkb ? kb + 1 : kb);
+                asm volatile("" : "+s"(next));
+                next_lo = b_scale[__builtin_amdgcn_readfirstlane(next * sn + nb_lo)];
+                next_hi = b_scale[__builtin_amdgcn_readfirstlane(next * sn + nb_hi)];
+            };
             v8i fa[MI][2];
 #pragma unroll
             for (int i = 0; i < MI; ++i) {
@@ -506,6 +516,8 @@ __device__ __forceinline__ void persistent_body(const Problem& one, const GroupT
                                                                                       0, 0, 0, 0);
                             copy_slot(PER_MFMA);
                         }
+                        if (jj == NJ - 1)
+                            ask_next_scale();
                         // wave-uniform choice of the b_scale value on the scalar unit (bit select),
                         // then one product per patch
                         const float sbj = __uint_as_float((__float_as_uint(sb_hi) & hi_mask[jj]) |
@@ -533,6 +545,8 @@ __device__ __forceinline__ void persistent_body(const Problem& one, const GroupT
                                                                                   0, 0, 0);
                         copy_slot(PER_MFMA);
                     }
+                    if (jj == NJ - 1)
+                        ask_next_scale();
 #pragma unroll
                     for (int i = 0; i < MI; ++i) {
                         // wave-uniform choice of the b_scale value on the scalar unit (bit select), then one

@@ -21,13 +21,15 @@ struct TileShape {
     static constexpr int MAT_A = KBLOCK * RSA;
     static constexpr int MAT_B = KBLOCK * RSB;
     static constexpr int SCALE_OFF = MAT_A + MAT_B;       // BM a_scale floats
-    static constexpr int SB_OFF = SCALE_OFF + 1024;       // four waves: 64 dwords, the first four = b_scale
-    static constexpr int STAGE = MAT_A + MAT_B + 1024 + (NW == 4 ? 256 : 0);
+    static constexpr int SB_OFF = SCALE_OFF + 1024;       // four waves per workgroup, or four multiplying ones: 64 dwords,
+                                                          // the first few = b_scale of the tile's columns
+    static constexpr bool SB_STAGED = NW == 4 || WM * WN == 4;
+    static constexpr int STAGE = MAT_A + MAT_B + 1024 + (SB_STAGED ? 256 : 0);
     static constexpr int LDS_BYTES = NS * STAGE;
     static constexpr int NA = RSA / (8 * NW);             // copy instructions per wave, A tile
     static constexpr int NB = RSB / (8 * NW);
-    static constexpr int NCOPY = NA + NB + 1;             // + the a_scale slice (wave 0 only; four
-                                                          // waves: wave 1 brings b_scale as well)
+    static constexpr int NCOPY = NA + NB + 1;             // + the a_scale slice (one wave); where it is staged,
+                                                          // another wave brings b_scale as well
     static_assert(NW == 4 || NW == 8, "four or eight waves");
     static_assert(NA * 8 * NW == RSA && NB * 8 * NW == RSB, "whole copy instructions per wave");
     // A wave's copy instructions of one matrix lie 4 (256-byte rows), 8 (128-byte rows) or 16
