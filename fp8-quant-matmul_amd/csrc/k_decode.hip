@@ -115,17 +115,20 @@ struct DecodeProblem {
     int lda;  // elements between consecutive k-rows of a and of a_scale (>= M; rows M .. lda-1 hold zeros)
 };
 
-// Work units = (problem, strip), numbered problem-major; `units` of them.  Linear workgroup ids that
-// agree modulo 8 share an XCD: the ksplit workgroups of unit u sit at ids xcd + 8 * (grp * ksplit + split)
-// with u = grp * 8 + xcd.
+// Work units = (problem, strip), numbered problem-major; `units` of them.  The workgroups of unit u are blockIdx.x = u,
+// blockIdx.y = split: gridDim.x is a multiple of 8, so their linear ids agree modulo 8 and they share an XCD.
 // TILES = the number of 16-row tiles when the launch knows it (a single problem: the count is then a constant
 // in the epilogue as well), 0 = read from the problem (grouped launches).
-template <int MT, bool GROUPED, int DS_NS, bool RAGGED, int TILES, int NB>
+template <int MT, bool GROUPED, int DS_NS, bool RAGGED, int TILES, int NB, int STEP>
 __device__ __forceinline__ void decode_body(const DecodeProblem& one, const GroupTable* tab, float* mailbox, int N, int K,
                                             int strips, int units, int ksplit, int kb_per_split)
 {
     using S = DecodeShape<MT, DS_NS, RAGGED, NB>;
     constexpr int BN = DS_BN * NB;  // columns of a strip
+    // Two stages to a barrier where the ring is deep enough.  A stage at a time, wait, barrier, LDS reads, MFMAs and fold
+    // are a chain of 700 - 800 clocks (1000 with slabs to spread) for 128 k-rows that arrive in 600: time stamps put
+    // the K loop, not the copies, in front (32 x 7168 x 2048 in four splits from the Infinity Cache).
+    static_assert(DS_NS % STEP == 0 && DS_NS >= 2 * STEP, "whole turns of stages, one being multiplied, one on its way");
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
     auto lds = LDS_PTR(uint8_t, smem);
     const uint32_t lds_base = (uint32_t)(uintptr_t)lds;
@@ -133,10 +136,7 @@ __device__ __forceinline__ void decode_body(const DecodeProblem& one, const Grou
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 
-    const int pid = blockIdx.x;
-    const int xcd = pid & 7, j = pid >> 3;
-    const int grp = j / ksplit, split = j - grp * ksplit;
-    const int unit = grp * 8 + xcd;
+    const int unit = blockIdx.x, split = blockIdx.y;
     if (unit >= units)
         return;
     DecodeProblem pr = one;
@@ -175,7 +175,7 @@ __device__ __forceinline__ void decode_body(const DecodeProblem& one, const Grou
             voff_b[h][q] = ok ? (uint32_t)((16 * wave + 8 * q + (lane >> 3)) * N + n0 + DS_BN * h + 16 * cc) : 0x80000000u;
         }
     const uint32_t voff_sa = lane < lda ? (uint32_t)(lane * 4) : 0x80000000u;
-    const uint32_t voff_sb = lane < NB ? (uint32_t)((strip * NB + lane) * 4) : 0x80000000u;  // past the last block: zeros
+    const uint32_t voff_sb = lane < NB && strip * NB + lane < sn ? (uint32_t)((strip * NB + lane) * 4) : 0x80000000u;
     uint32_t voff_a;
     if (RAGGED) {
         // the K block's slab of A, 128 * M contiguous bytes, in 16-byte pieces: piece 64 * wave + lane
@@ -189,33 +189,35 @@ __device__ __forceinline__ void decode_body(const DecodeProblem& one, const Grou
         voff_a = 16 * cc < lda ? (uint32_t)((16 * wave + (lane >> 2)) * lda + 16 * cc) : 0x80000000u;
     }
 
-    // Stage `slot` <- K block kb.  The resources of A and B start at the block's first k-row.
+    // Stage `slot` <- K block kb: the buffer resources stay fixed, the block's byte offset rides in the copies' scalar
+    // offset.  RAGGED: with it travels the slab of the K block STEP further on, into that block's slot: it has landed
+    // one turn of the loop before it is multiplied, which is when the threads spread it.
+    const v4i rsrc_b = make_rsrc_words(b, b_bytes), rsrc_a = make_rsrc_words(a, a_bytes);
+    const int scale_wave = MT == 2 ? wave - 4 : wave;  // 0: a_scale, 1..: b_scale, below 0: A (two row tiles)
+    const v4i rsrc_s = scale_wave == 0 ? make_rsrc_words(a_scale, (uint32_t)nkb * (uint32_t)lda * 4u)
+                                       : make_rsrc_words(b_scale, (uint32_t)nkb * (uint32_t)sn * 4u);
+    const uint32_t voff_s = scale_wave == 0 ? voff_sa : voff_sb;
+    const uint32_t step_s = (scale_wave == 0 ? (uint32_t)lda : (uint32_t)sn) * 4u;
+    const uint32_t dst_s = lds_base + (scale_wave == 0 ? S::SA_OFF : S::SB_OFF);
+    auto issue_slab = [&](int slot, int kb) __attribute__((always_inline)) {
+        if (MT == 4 || wave < 4)
+            lds_dma16(rsrc_a, kb < kb1 ? voff_a : 0x80000000u,
+                      lds_base + (uint32_t)(slot * S::STAGE + S::PACK_OFF + wave * 1024), (uint32_t)kb * KBLOCK * (uint32_t)lda);
+    };
     auto issue_stage = [&](int slot, int kb) __attribute__((always_inline)) {
         const uint32_t stage = lds_base + (uint32_t)(slot * S::STAGE);
         const uint32_t skip_b = (uint32_t)kb * KBLOCK * (uint32_t)N;
-        const uint32_t skip_a = (uint32_t)kb * KBLOCK * (uint32_t)lda;
-        const v4i rb = make_rsrc_words(b + skip_b, b_bytes - skip_b);
 #pragma unroll
         for (int h = 0; h < NB; ++h) {
-            lds_dma16(rb, voff_b[h][0], stage + (uint32_t)(h * S::HALF_B + (2 * wave) * 1024));
-            lds_dma16(rb, voff_b[h][1], stage + (uint32_t)(h * S::HALF_B + (2 * wave + 1) * 1024));
+            lds_dma16(rsrc_b, voff_b[h][0], stage + (uint32_t)(h * S::HALF_B + (2 * wave) * 1024), skip_b);
+            lds_dma16(rsrc_b, voff_b[h][1], stage + (uint32_t)(h * S::HALF_B + (2 * wave + 1) * 1024), skip_b);
         }
-        const int scale_wave = MT == 2 ? wave - 4 : wave;  // 0: a_scale, 1..: b_scale, below 0: A (two row tiles)
-        if (RAGGED) {
-            // the slab of the K block after this one, into the next slot: it has landed with this stage, one
-            // stage before it is multiplied, which is when the threads spread it
-            if (MT == 4 || wave < 4) {
-                const uint32_t next = lds_base + (uint32_t)((slot == DS_NS - 1 ? 0 : slot + 1) * S::STAGE);
-                const uint32_t skip_next = skip_a + KBLOCK * (uint32_t)lda;
-                lds_dma16(make_rsrc_words(a + skip_next, a_bytes - skip_next), kb + 1 < kb1 ? voff_a : 0x80000000u,
-                          next + S::PACK_OFF + (uint32_t)(wave * 1024));
-            }
-        } else if (MT == 4 || wave < 4)
-            lds_dma16(make_rsrc_words(a + skip_a, a_bytes - skip_a), voff_a, stage + S::MAT_B + (uint32_t)(wave * 1024));
-        if (scale_wave == 0)
-            lds_dma4(make_rsrc_words(a_scale + (size_t)kb * lda, (uint32_t)lda * 4u), voff_sa, stage + S::SA_OFF);
-        else if (scale_wave > 0)
-            lds_dma4(make_rsrc_words(b_scale + (size_t)kb * sn, (uint32_t)sn * 4u), voff_sb, stage + S::SB_OFF);
+        if (RAGGED)
+            issue_slab(slot + STEP >= DS_NS ? slot + STEP - DS_NS : slot + STEP, kb + STEP);
+        else if (MT == 4 || wave < 4)
+            lds_dma16(rsrc_a, voff_a, stage + S::MAT_B + (uint32_t)(wave * 1024), (uint32_t)kb * KBLOCK * (uint32_t)lda);
+        if (scale_wave >= 0)
+            lds_dma4(rsrc_s, voff_s, dst_s + (uint32_t)(slot * S::STAGE), (uint32_t)kb * step_s);
     };
     // RAGGED: thread 4 * r + j moves bytes 16 * j .. 16 * j + 15 of packed k-row r (they start at any byte:
     // five aligned words, shifted) to chunk j of the padded, swizzled row, zeros where the row has ended; only
@@ -236,18 +238,23 @@ __device__ __forceinline__ void decode_body(const DecodeProblem& one, const Grou
         const int valid = M - 16 * sp_j - 4 * i;  // bytes of word i inside the row
         sp_mask[i] = valid >= 4 ? 0xFFFFFFFFu : valid <= 0 ? 0u : (1u << (8 * valid)) - 1u;
     }
-    uint32_t sp_word[5];
-    auto slab_read = [&](int sl) __attribute__((always_inline)) {
+    uint32_t sp_word[STEP][5];
+    auto slab_read = [&](int sl) __attribute__((always_inline)) {  // the slabs of slots sl .. sl + STEP - 1
 #pragma unroll
-        for (int i = 0; i < 5; ++i)
-            sp_word[i] = *LDS_PTR(uint32_t, lds + sl * S::STAGE + sp_src + 4 * i);
+        for (int u = 0; u < STEP; ++u)
+#pragma unroll
+            for (int i = 0; i < 5; ++i)
+                sp_word[u][i] = *LDS_PTR(uint32_t, lds + (sl + u) * S::STAGE + sp_src + 4 * i);
     };
     auto slab_write = [&](int sl) __attribute__((always_inline)) {
-        v4i out;
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-            out[i] = (int)(__builtin_amdgcn_alignbyte(sp_word[i + 1], sp_word[i], sp_shift) & sp_mask[i]);
-        *LDS_PTR(v4i, lds + sl * S::STAGE + sp_dst) = out;
+        for (int u = 0; u < STEP; ++u) {
+            v4i out;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                out[i] = (int)(__builtin_amdgcn_alignbyte(sp_word[u][i + 1], sp_word[u][i], sp_shift) & sp_mask[i]);
+            *LDS_PTR(v4i, lds + (sl + u) * S::STAGE + sp_dst) = out;
+        }
     };
     // wait until at most the copies of `outstanding` stages are in flight (loads complete in order)
     auto wait_landed = [&](int outstanding) __attribute__((always_inline)) {
@@ -260,6 +267,7 @@ __device__ __forceinline__ void decode_body(const DecodeProblem& one, const Grou
         default: ds_wait_vmcnt<(DS_NS - 1) * S::COPIES>(); break;
         }
     };
+    static_assert(DS_NS <= 6, "the wait above knows up to five stages in flight besides the youngest");
 
     // ---- transposing reads.  Lane = 16*g + i; read t of a K block covers k-rows 32*t + 8*g + (i >> 1),
     // so (r >> 1) & 7 = (4*g + (i >> 2)) & 7, (r >> 3) & 1 = g & 1 and (r >> 2) & 3 = (2*g + (i >> 3)) & 3
@@ -284,72 +292,92 @@ __device__ __forceinline__ void decode_body(const DecodeProblem& one, const Grou
         for (int i = 0; i < MT; ++i)
             acc[h][i] = (v4f){0.f, 0.f, 0.f, 0.f};
 
+    // Stages are issued AHEAD of the turn that multiplies them: with a stage to a turn all slots but the one being
+    // multiplied are in flight, with two the ring less the pair.  (Before the first turn all slots are free; slabs,
+    // which go to the slot STEP further on, leave the last STEP of them for the first turn.)
+    constexpr int AHEAD = DS_NS - STEP;
+    constexpr int FIRST = STEP == 2 && !RAGGED ? DS_NS : AHEAD;  // stages issued before the first turn
     const int nstages = kb1 - kb0;
-    if (RAGGED && (MT == 4 || wave < 4)) {  // the first K block's slab, ahead of every stage
-        const uint32_t skip_a = (uint32_t)kb0 * KBLOCK * (uint32_t)lda;
-        lds_dma16(make_rsrc_words(a + skip_a, a_bytes - skip_a), voff_a, lds_base + S::PACK_OFF + (uint32_t)(wave * 1024));
+    if (RAGGED) {  // the first turn's slabs, ahead of every stage
+#pragma unroll
+        for (int u = 0; u < STEP; ++u)
+            issue_slab(u, kb0 + u);
     }
 #pragma unroll
-    for (int p = 0; p < DS_NS - 1; ++p)
+    for (int p = 0; p < FIRST; ++p)
         if (p < nstages)
             issue_stage(p, kb0 + p);
-    if (RAGGED) {  // the first slab has landed once only the stages' copies are in flight
-        wait_landed(nstages < DS_NS - 1 ? nstages : DS_NS - 1);
+    if (RAGGED) {  // the first slabs have landed once only the stages' copies are in flight
+        wait_landed(nstages < FIRST ? nstages : FIRST);
         __syncthreads();
         slab_read(0);
         slab_write(0);
     }
     // The K loop, one copy per number of 16-row tiles (chosen below, outside the loop): with the count fixed
-    // the loop has no branch around its LDS operations, every read of a stage is issued before the first MFMA,
+    // the loop has no branch around its LDS operations, every read of a turn is issued before the first MFMA,
     // and the compiler's wait counts name exactly the reads each MFMA needs (around a branch it waits for
     // everything in flight, which serialises read latency and MFMAs tile after tile).
     auto k_loop = [&](auto tile_count) __attribute__((always_inline)) {
-    constexpr int T = decltype(tile_count)::value;
-    int slot = 0;
-    for (int s = 0; s < nstages; ++s) {
-        // loads complete in order: this wave's copies of stage s have landed once at most those of the
-        // younger stages in flight are outstanding
-        wait_landed(nstages - 1 - s < DS_NS - 2 ? nstages - 1 - s : DS_NS - 2);
-        __syncthreads();  // everyone's copies landed and spreads are done; the slot of stage s - 1 is no longer read
-        if (s + DS_NS - 1 < nstages)
-            issue_stage(slot == 0 ? DS_NS - 1 : slot - 1, kb0 + s + DS_NS - 1);
-        const uint32_t so = (uint32_t)(slot * S::STAGE);
-        const int next_slot = slot == DS_NS - 1 ? 0 : slot + 1;
-        // RAGGED: the next stage's slab, also behind the last stage (nothing reads what that spreads)
-        if (RAGGED)
-            slab_read(next_slot);
-        v8i fb[NB];
-        float sb[NB];
+        constexpr int T = decltype(tile_count)::value;
+        int slot = 0;
+        // stages s .. s + CNT - 1
+        auto turn = [&](auto count, int s) __attribute__((always_inline)) {
+            constexpr int CNT = decltype(count)::value;
+            // loads complete in order: this wave's copies of these stages have landed once at most those of the
+            // younger stages in flight are outstanding
+            const int issued = s == 0 ? FIRST : s + AHEAD;
+            wait_landed((nstages < issued ? nstages : issued) - s - CNT);
+            __syncthreads();  // everyone's copies landed and spreads are done; the slots of the last turn are no longer read
+            if (STEP == 1 || RAGGED || s > 0) {
+                const int free_slot = slot == 0 ? DS_NS - STEP : slot - STEP;
 #pragma unroll
-        for (int h = 0; h < NB; ++h) {
-            fb[h] = read_frag(so + h * S::HALF_B + addr_b, 32 * 128);
-            sb[h] = *LDS_PTR(float, lds + so + S::SB_OFF + 4 * h);
-        }
-        auto multiply = [&](int h, int i, const v8i& fa, float sa) __attribute__((always_inline)) {
-            const v4f blk = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fb[h], fa, (v4f){0.f, 0.f, 0.f, 0.f}, 0, 0,
-                                                                             0, 0, 0, 0);
-            const float sc = sa * sb[h];
-            acc[h][i] = (v4f){fmaf(sc, blk[0], acc[h][i][0]), fmaf(sc, blk[1], acc[h][i][1]),
-                              fmaf(sc, blk[2], acc[h][i][2]), fmaf(sc, blk[3], acc[h][i][3])};
+                for (int u = 0; u < STEP; ++u)
+                    if (s + AHEAD + u < nstages)
+                        issue_stage(free_slot + u, kb0 + s + AHEAD + u);
+            }
+            const int next_slot = slot == DS_NS - STEP ? 0 : slot + STEP;
+            // RAGGED: the next turn's slabs, also behind the last turn (nothing reads what that spreads)
+            if (RAGGED)
+                slab_read(next_slot);
+            v8i fb[CNT][NB], fa[CNT][T];
+            float sb[CNT][NB], sa[CNT][T];
+#pragma unroll
+            for (int u = 0; u < CNT; ++u) {
+                const uint32_t so = (uint32_t)((slot + u) * S::STAGE);
+#pragma unroll
+                for (int h = 0; h < NB; ++h) {
+                    fb[u][h] = read_frag(so + h * S::HALF_B + addr_b, 32 * 128);
+                    sb[u][h] = *LDS_PTR(float, lds + so + S::SB_OFF + 4 * h);
+                }
+#pragma unroll
+                for (int i = 0; i < T; ++i) {
+                    sa[u][i] = *LDS_PTR(float, lds + so + S::SA_OFF + (16 * i + i16) * 4);
+                    fa[u][i] = read_frag(so + addr_a + (uint32_t)((i ^ swz_a) * 16), 32 * S::RSA);
+                }
+            }
+            // the spread words are written behind the turn's reads: the LDS works in order, a write among the
+            // reads would hold the later ones back
+            if (RAGGED)
+                slab_write(next_slot);
+#pragma unroll
+            for (int u = 0; u < CNT; ++u)
+#pragma unroll
+                for (int h = 0; h < NB; ++h)
+#pragma unroll
+                    for (int i = 0; i < T; ++i) {
+                        const v4f blk = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+                            fb[u][h], fa[u][i], (v4f){0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 0, 0, 0);
+                        const float sc = sa[u][i] * sb[u][h];
+                        acc[h][i] = (v4f){fmaf(sc, blk[0], acc[h][i][0]), fmaf(sc, blk[1], acc[h][i][1]),
+                                          fmaf(sc, blk[2], acc[h][i][2]), fmaf(sc, blk[3], acc[h][i][3])};
+                    }
+            slot = next_slot;
         };
-        // the spread words are written behind the stage's reads: the LDS works in order, a write among the
-        // reads would hold the later ones back
-        v8i fa[T];
-        float sa[T];
-#pragma unroll
-        for (int i = 0; i < T; ++i) {
-            sa[i] = *LDS_PTR(float, lds + so + S::SA_OFF + (16 * i + i16) * 4);
-            fa[i] = read_frag(so + addr_a + (uint32_t)((i ^ swz_a) * 16), 32 * S::RSA);
-        }
-        if (RAGGED)
-            slab_write(next_slot);
-#pragma unroll
-        for (int h = 0; h < NB; ++h)
-#pragma unroll
-            for (int i = 0; i < T; ++i)
-                multiply(h, i, fa[i], sa[i]);
-        slot = next_slot;
-    }
+        int s = 0;
+        for (; s + STEP <= nstages; s += STEP)
+            turn(std::integral_constant<int, STEP>{}, s);
+        if (STEP == 2 && s < nstages)
+            turn(std::integral_constant<int, 1>{}, s);
     };
     if (TILES > 0)
         k_loop(std::integral_constant<int, (TILES > 0 ? TILES : 1)>{});
@@ -394,13 +422,15 @@ __device__ __forceinline__ void decode_body(const DecodeProblem& one, const Grou
     constexpr int PER_SPLIT = 8 * PER_WAVE;  // patches of one split of one unit
     const int senders = ksplit - 1;
     const size_t patch = ((size_t)unit * senders * 8 + wave) * PER_WAVE;  // split 0
+    // lanes whose row exists take part: a CU takes in 64 bytes per clock, which is most of what the hand-over takes
+    auto row_exists = [&](int i) __attribute__((always_inline)) { return 16 * i + i16 < M; };
     if (split < senders) {
         v4i* mine = reinterpret_cast<v4i*>(mailbox) + (patch + (size_t)split * PER_SPLIT) * 64 + lane;
 #pragma unroll
         for (int h = 0; h < NB; ++h)
 #pragma unroll
             for (int i = 0; i < MT; ++i)
-                if (i < mtiles) {
+                if (row_exists(i)) {
                     v4i bits = __builtin_bit_cast(v4i, acc[h][i]);
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
@@ -420,11 +450,19 @@ __device__ __forceinline__ void decode_body(const DecodeProblem& one, const Grou
             sum[h][i] = (v4f){0.f, 0.f, 0.f, 0.f};
     bool gave_up = false;
     const unsigned long long t_first = __builtin_amdgcn_s_memrealtime();
+    // byte offset of a lane's 16 bytes of split 0, per pair of row tiles; outside the resource (which fetches and stores
+    // nothing, without a branch among the loads) where the lane's row does not exist
+    uint32_t off[MT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+        off[i] = row_exists(i) ? (uint32_t)(i * 64 + lane) * 16u : 0x80000000u;
     for (int z0 = 0; z0 < senders; z0 += 4) {
 #pragma unroll
         for (int hp = 0; hp < NB * (MT / 2); ++hp) {  // two row tiles of a half at a time
             const int hb = hp / (MT / 2), h = hp % (MT / 2);
             if (2 * h < mtiles) {
+                auto tile_here = [&](int i) __attribute__((always_inline)) { return TILES == 0 || 2 * h + i < TILES; };
+                auto place = [&](int z) __attribute__((always_inline)) { return (uint32_t)((z0 + z) * PER_SPLIT + hb * MT) * 1024u; };
                 v4i v[4][2];
                 for (;;) {
                     asm volatile("" ::: "memory");  // the loads belong to this round of the loop
@@ -433,15 +471,16 @@ __device__ __forceinline__ void decode_body(const DecodeProblem& one, const Grou
                     for (int z = 0; z < 4; ++z)
 #pragma unroll
                         for (int i = 0; i < 2; ++i)
-                            v[z][i] = __builtin_amdgcn_raw_buffer_load_b128(
-                                rp, (uint32_t)(((z0 + z) * PER_SPLIT + hb * MT + 2 * h + i) * 64 + lane) * 16u, 0, AUX_L1_MISS);
+                            if (tile_here(i))
+                                v[z][i] = __builtin_amdgcn_raw_buffer_load_b128(rp, off[2 * h + i] + place(z), 0, AUX_L1_MISS);
                     bool missing = false;
 #pragma unroll
                     for (int z = 0; z < 4; ++z)
 #pragma unroll
                         for (int i = 0; i < 2; ++i)
-                            if (z0 + z < senders && 2 * h + i < mtiles)
-                                missing = missing || v[z][i][0] == 0 || v[z][i][1] == 0 || v[z][i][2] == 0 || v[z][i][3] == 0;
+                            if (z0 + z < senders && tile_here(i))
+                                missing = missing | (row_exists(2 * h + i) & ((v[z][i][0] == 0) | (v[z][i][1] == 0) |
+                                                                              (v[z][i][2] == 0) | (v[z][i][3] == 0)));
                     if (__builtin_amdgcn_ballot_w64(missing) == 0)
                         break;
                     if (__builtin_amdgcn_s_memrealtime() - t_first > SPIN_LIMIT_TICKS) {
@@ -454,10 +493,9 @@ __device__ __forceinline__ void decode_body(const DecodeProblem& one, const Grou
                     if (z0 + z < senders) {
 #pragma unroll
                         for (int i = 0; i < 2; ++i) {
-                            if (2 * h + i < mtiles)
-                                __builtin_amdgcn_raw_buffer_store_b128(
-                                    (v4i){0, 0, 0, 0}, rp,
-                                    (uint32_t)(((z0 + z) * PER_SPLIT + hb * MT + 2 * h + i) * 64 + lane) * 16u, 0, 0);
+                            if (!tile_here(i))
+                                continue;
+                            __builtin_amdgcn_raw_buffer_store_b128((v4i){0, 0, 0, 0}, rp, off[2 * h + i] + place(z), 0, 0);
                             const v4f f = __builtin_bit_cast(v4f, v[z][i]);
                             sum[hb][2 * h + i] = z0 + z == 0 ? f : sum[hb][2 * h + i] + f;
                         }
@@ -476,22 +514,23 @@ __device__ __forceinline__ void decode_body(const DecodeProblem& one, const Grou
     store_c(sum);
 }
 
-template <int MT, int DS_NS, bool RAGGED, int TILES, int NB>
+template <int MT, int DS_NS, bool RAGGED, int TILES, int NB, int STEP>
 __global__ void __launch_bounds__(DS_THREADS)
-decode_strip_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b, const float* __restrict__ a_scale,
-                    const float* __restrict__ b_scale, uint16_t* __restrict__ c, float* mailbox, int M, int lda, int N,
-                    int K, int strips, int ksplit, int kb_per_split)
+decode_strip_kernel(const uint8_t* __restrict__ b, const uint8_t* __restrict__ a, int N, int K, int M, int lda,
+                    int kb_per_split, int strips, const float* __restrict__ a_scale, const float* __restrict__ b_scale,
+                    uint16_t* __restrict__ c, float* mailbox, int ksplit)
 {
+    // (the first 14 words of the arguments are in registers when a wave starts: what the copies need comes first)
     const DecodeProblem one{a, b, a_scale, b_scale, c, M, lda};
-    decode_body<MT, false, DS_NS, RAGGED, TILES, NB>(one, nullptr, mailbox, N, K, strips, strips, ksplit, kb_per_split);
+    decode_body<MT, false, DS_NS, RAGGED, TILES, NB, STEP>(one, nullptr, mailbox, N, K, strips, strips, ksplit, kb_per_split);
 }
 
-template <int MT, int DS_NS, bool RAGGED>
+template <int MT, int DS_NS, bool RAGGED, int STEP>
 __global__ void __launch_bounds__(DS_THREADS)
 decode_strip_grouped_kernel(const GroupTable tab, float* mailbox, int N, int K, int strips, int ksplit, int kb_per_split)
 {
     const DecodeProblem none{nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0};
-    decode_body<MT, true, DS_NS, RAGGED, 0, 1>(none, &tab, mailbox, N, K, strips, strips * tab.groups, ksplit, kb_per_split);
+    decode_body<MT, true, DS_NS, RAGGED, 0, 1, STEP>(none, &tab, mailbox, N, K, strips, strips * tab.groups, ksplit, kb_per_split);
 }
 
 // The streaming form, for a single problem without a K split whose strips outnumber the workgroups the
@@ -764,6 +803,18 @@ struct StreamShape {
 constexpr int STREAM_WORKGROUPS = 256;
 constexpr int SLAB_FORM_MIN_KBLOCKS = 28;  // K blocks per workgroup from which up to 32 rows on the grid take the slab-spreading instances too
 
+// Two stages to a barrier (STEP = 2 of decode_body): for launches of one round of workgroups with short K ranges, whose
+// time is the chain of one K block after the other -- from the Infinity Cache / from HBM, against one stage to a
+// barrier: 16 x 16384 x 1024 unsplit 4.8 / 7.0 against 5.6 / 7.5 us, 24 x 28672 x 2048 unsplit 12.5 / 14.7 against
+// 14.2 / 15.4 us, 16 x 7168 x 7168 in four splits 11.7 / 14.2 against 12.5 / 14.4 us.  Long K ranges and several rounds
+// live on the copies in flight, of which a pair of stages in hand leaves fewer: 16 x 28672 x 8192 47.7 against 45.4 us
+// from HBM, eight groups of 1 - 64 rows, 7168 x 2048 (448 workgroups) 35.2 against 31.4 us.  So does the ring of four
+// stages (33 - 64 rows off the grid) beyond a few blocks: 50 x 7168 x 7168 in four splits 19.1 against 17.2 us.
+inline bool stages_in_pairs(long workgroups, int kb_per_split, int ring)
+{
+    return workgroups <= 256 && kb_per_split < (ring >= 6 ? SLAB_FORM_MIN_KBLOCKS : 5);
+}
+
 // Two workgroups per CU with a three-stage ring instead of one with six: one streams while the other starts up.
 // Measured on grouped launches: 64 groups x 56 strips, 16 K blocks each: 221 against 236 us; with 768-1152
 // workgroups (1.5-2.25 rounds of 512 resident ones) 1-3 % slower than three to four and a half rounds of 256.
@@ -880,11 +931,11 @@ hipError_t launch_decode_strips(const GemmArgs& g, int ksplit, int halves, float
     const int kb_per_split = (nkb + ksplit - 1) / ksplit;
     if ((ksplit - 1) * kb_per_split >= nkb)  // every split owns at least one K block
         return hipErrorInvalidValue;
-    const dim3 grid(8 * ((strips + 7) / 8) * ksplit);
+    const dim3 grid(8 * ((strips + 7) / 8), ksplit);
     auto go = [&](auto kern, int lds) -> hipError_t {
         FP8GEMM_ALLOW_LDS(kern, lds);
-        hipLaunchKernelGGL(kern, grid, dim3(DS_THREADS), lds, s, g.a, g.b, g.a_scale, g.b_scale, g.c, mailbox, g.m,
-                           leading_dim(g), g.n, g.k, strips, ksplit, kb_per_split);
+        hipLaunchKernelGGL(kern, grid, dim3(DS_THREADS), lds, s, g.b, g.a, g.n, g.k, g.m, leading_dim(g), kb_per_split, strips,
+                           g.a_scale, g.b_scale, g.c, mailbox, ksplit);
         return hipGetLastError();
     };
     // more strips than resident workgroups, no K split: one copy stream per workgroup (the streaming form chooses
@@ -928,7 +979,7 @@ hipError_t launch_decode_strips(const GemmArgs& g, int ksplit, int halves, float
         auto wide = [&](auto mt_c, auto ragged_c, auto tiles_c) -> hipError_t {
             constexpr int MT = decltype(mt_c)::value, T = decltype(tiles_c)::value;
             constexpr bool RG = decltype(ragged_c)::value;
-            return go(decode_strip_kernel<MT, STREAM_NS_WIDE, RG, T, 2>, DecodeShape<MT, STREAM_NS_WIDE, RG, 2>::LDS);
+            return go(decode_strip_kernel<MT, STREAM_NS_WIDE, RG, T, 2, 1>, DecodeShape<MT, STREAM_NS_WIDE, RG, 2>::LDS);
         };
         auto by_tiles = [&](auto ragged_c) -> hipError_t {
             switch (tiles) {
@@ -946,24 +997,29 @@ hipError_t launch_decode_strips(const GemmArgs& g, int ksplit, int halves, float
     // 16384 x 7168 in two splits, 47 / 48 rows: 26.3 / 27.8 us), a short one 3 - 10 % slower (24576 x 2048 unsplit,
     // 31 / 32 rows: 14.4 / 13.9 us; 7168 x 2048 in four splits: 8.0 / 7.3 us).  With three or four row tiles the
     // two measure level (their slab form has a ring of four stages, not six).
-    if (leading_dim(g) % 16 != 0 || (kb_per_split >= SLAB_FORM_MIN_KBLOCKS && tiles <= 2)) {
-        constexpr int L2 = DecodeShape<2, 6, true>::LDS, L4 = DecodeShape<4, RAGGED4_NS, true>::LDS;
+    auto strips_of = [&](auto mt_c, auto ns_c, auto ragged_c, auto tiles_c) -> hipError_t {
+        constexpr int MT = decltype(mt_c)::value, NS = decltype(ns_c)::value, T = decltype(tiles_c)::value;
+        constexpr bool RG = decltype(ragged_c)::value;
+        constexpr int lds = DecodeShape<MT, NS, RG>::LDS;
+        if constexpr (NS % 2 == 0)
+            if (stages_in_pairs((long)strips * ksplit, kb_per_split, NS))
+                return go(decode_strip_kernel<MT, NS, RG, T, 1, 2>, lds);
+        return go(decode_strip_kernel<MT, NS, RG, T, 1, 1>, lds);
+    };
+    using std::integral_constant;
+    auto by_tiles = [&](auto ns2, auto ns4, auto ragged_c) -> hipError_t {
         switch (tiles) {
-        case 1: return go(decode_strip_kernel<2, 6, true, 1, 1>, L2);
-        case 2: return go(decode_strip_kernel<2, 6, true, 2, 1>, L2);
-        case 3: return go(decode_strip_kernel<4, RAGGED4_NS, true, 3, 1>, L4);
-        default: return go(decode_strip_kernel<4, RAGGED4_NS, true, 4, 1>, L4);
+        case 1: return strips_of(integral_constant<int, 2>{}, ns2, ragged_c, integral_constant<int, 1>{});
+        case 2: return strips_of(integral_constant<int, 2>{}, ns2, ragged_c, integral_constant<int, 2>{});
+        case 3: return strips_of(integral_constant<int, 4>{}, ns4, ragged_c, integral_constant<int, 3>{});
+        default: return strips_of(integral_constant<int, 4>{}, ns4, ragged_c, integral_constant<int, 4>{});
         }
-    }
-    const bool deep = !shallow_ring_pays((long)strips * ksplit, kb_per_split);
-    constexpr int D2 = DecodeShape<2, 6>::LDS, S2 = DecodeShape<2, 3>::LDS, D4 = DecodeShape<4, 6>::LDS,
-                  S4 = DecodeShape<4, 3>::LDS;
-    switch (tiles) {
-    case 1: return deep ? go(decode_strip_kernel<2, 6, false, 1, 1>, D2) : go(decode_strip_kernel<2, 3, false, 1, 1>, S2);
-    case 2: return deep ? go(decode_strip_kernel<2, 6, false, 2, 1>, D2) : go(decode_strip_kernel<2, 3, false, 2, 1>, S2);
-    case 3: return deep ? go(decode_strip_kernel<4, 6, false, 3, 1>, D4) : go(decode_strip_kernel<4, 3, false, 3, 1>, S4);
-    default: return deep ? go(decode_strip_kernel<4, 6, false, 4, 1>, D4) : go(decode_strip_kernel<4, 3, false, 4, 1>, S4);
-    }
+    };
+    if (leading_dim(g) % 16 != 0 || (kb_per_split >= SLAB_FORM_MIN_KBLOCKS && tiles <= 2))
+        return by_tiles(integral_constant<int, 6>{}, integral_constant<int, RAGGED4_NS>{}, std::true_type{});
+    if (!shallow_ring_pays((long)strips * ksplit, kb_per_split))
+        return by_tiles(integral_constant<int, 6>{}, integral_constant<int, 6>{}, std::false_type{});
+    return by_tiles(integral_constant<int, 3>{}, integral_constant<int, 3>{}, std::false_type{});
 }
 
 // every group: 1 <= m <= lda <= 64 (rows m .. lda-1 of a and a_scale readable), operands aligned like a
@@ -1066,22 +1122,32 @@ hipError_t launch_decode_grouped(const GroupTable& tab, int n, int k, int ksplit
         return staged ? stream(StreamShape<4, STREAM_NS_WIDE, 2>{}, std::true_type{})
                       : stream(StreamShape<4, STREAM_NS_WIDE, 2>{}, std::false_type{});
     }
-    const dim3 grid((unsigned)(8 * ((units + 7) / 8) * ksplit));
+    const dim3 grid((unsigned)(8 * ((units + 7) / 8)), (unsigned)ksplit);
     auto go = [&](auto kern, int lds) -> hipError_t {
         FP8GEMM_ALLOW_LDS(kern, lds);
         hipLaunchKernelGGL(kern, grid, dim3(DS_THREADS), lds, s, tab, mailbox, n, k, strips, ksplit, kb_per_split);
         return hipGetLastError();
     };
+    auto strips_of = [&](auto mt_c, auto ns_c, auto ragged_c) -> hipError_t {
+        constexpr int MT = decltype(mt_c)::value, NS = decltype(ns_c)::value;
+        constexpr bool RG = decltype(ragged_c)::value;
+        constexpr int lds = DecodeShape<MT, NS, RG>::LDS;
+        if constexpr (NS % 2 == 0)
+            if (stages_in_pairs(units * ksplit, kb_per_split, NS))
+                return go(decode_strip_grouped_kernel<MT, NS, RG, 2>, lds);
+        return go(decode_strip_grouped_kernel<MT, NS, RG, 1>, lds);
+    };
+    using std::integral_constant;
+    const integral_constant<int, 2> two{};
+    const integral_constant<int, 4> four{};
     if (ragged)
-        return row_tiles(mmax) == 2
-                   ? go(decode_strip_grouped_kernel<2, 6, true>, DecodeShape<2, 6, true>::LDS)
-                   : go(decode_strip_grouped_kernel<4, RAGGED4_NS, true>, DecodeShape<4, RAGGED4_NS, true>::LDS);
-    const bool deep = !shallow_ring_pays(units * ksplit, kb_per_split);
-    if (row_tiles(mmax) == 2)
-        return deep ? go(decode_strip_grouped_kernel<2, 6, false>, DecodeShape<2, 6>::LDS)
-                    : go(decode_strip_grouped_kernel<2, 3, false>, DecodeShape<2, 3>::LDS);
-    return deep ? go(decode_strip_grouped_kernel<4, 6, false>, DecodeShape<4, 6>::LDS)
-                : go(decode_strip_grouped_kernel<4, 3, false>, DecodeShape<4, 3>::LDS);
+        return row_tiles(mmax) == 2 ? strips_of(two, integral_constant<int, 6>{}, std::true_type{})
+                                    : strips_of(four, integral_constant<int, RAGGED4_NS>{}, std::true_type{});
+    if (!shallow_ring_pays(units * ksplit, kb_per_split))
+        return row_tiles(mmax) == 2 ? strips_of(two, integral_constant<int, 6>{}, std::false_type{})
+                                    : strips_of(four, integral_constant<int, 6>{}, std::false_type{});
+    return row_tiles(mmax) == 2 ? strips_of(two, integral_constant<int, 3>{}, std::false_type{})
+                                : strips_of(four, integral_constant<int, 3>{}, std::false_type{});
 }
 
 }  // namespace fp8gemm
