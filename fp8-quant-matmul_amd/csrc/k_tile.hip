@@ -325,17 +325,22 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
     // split but the last stores its accumulators there in register order (1 KiB per instruction) with
     // every +0.0 replaced by -0.0, so that no word it writes is zero, and is done.  The waves of the last
     // split -- the workgroup with the highest id of its tile, dispatched after the others -- load the other
-    // splits' patches past their L1 until no word is zero, store zeros back, add them in split order, their
-    // own registers last (the arithmetic of splitk_reduce_kernel: adding -0.0 changes nothing), and the
-    // workgroup leaves through the bf16 epilogue.  A wave that has polled for a second gives up and
+    // splits' patches past their L1 until no word is zero, add them in split order, their own registers last (the
+    // arithmetic of splitk_reduce_kernel: adding -0.0 changes nothing), the workgroup leaves through the bf16
+    // epilogue, and zeros go back into the mailbox behind it (in front of it, the epilogue's first barrier waits until
+    // they are acknowledged).  A wave that has polled for a second gives up and
     // writes NaN.
     bool as_partial = SPLIT;
+    constexpr int PATCHES = NCW * MI * NJ;  // 32x32 patches of a tile: 4 KiB of fp32 each
+    const int senders = (int)gridDim.y - 1;
+    const size_t first = ((size_t)pid * senders * PATCHES + (size_t)wave * (MI * NJ)) * 256;  // in 16-byte units
+    const uint32_t mail_span = (uint32_t)senders * PATCHES * 4096u;
+    auto mail_at = [&](int z, int patch, int q) __attribute__((always_inline)) {
+        return (uint32_t)(((z * PATCHES + patch) * 4 + q) * 64 + lane) * 16u;
+    };
     if constexpr (SPLIT) {
         if (mailbox != nullptr) {
             as_partial = false;
-            constexpr int PATCHES = NCW * MI * NJ;  // 32x32 patches of a tile: 4 KiB of fp32 each
-            const int senders = (int)gridDim.y - 1;
-            const size_t first = ((size_t)pid * senders * PATCHES + (size_t)wave * (MI * NJ)) * 256;  // in 16-byte units
             if ((int)blockIdx.y < senders) {
                 if (compute) {
                     v4i* mine = reinterpret_cast<v4i*>(mailbox) + first + (size_t)blockIdx.y * PATCHES * 256 + lane;
@@ -357,60 +362,73 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
                 return;
             }
             if (compute) {
-                constexpr int ZC = MI * NJ <= 2 ? 4 : 2;  // splits polled together (registers)
-                const uint32_t span = (uint32_t)senders * PATCHES * 4096u;
-                const __amdgpu_buffer_rsrc_t rp = make_rsrc(reinterpret_cast<const v4i*>(mailbox) + first, span);
+                // PG patches at a time (all of them when there are at most two: one trip to the L2 for everything that is
+                // there), ZB splits at a time
+                constexpr int PG = MI * NJ <= 2 ? MI * NJ : 1, ZB = MI * NJ == 1 ? 3 : 2;
+                const __amdgpu_buffer_rsrc_t rp = make_rsrc(reinterpret_cast<const v4i*>(mailbox) + first, mail_span);
                 const unsigned long long t_first = __builtin_amdgcn_s_memrealtime();
                 bool gave_up = false;
 #pragma unroll
-                for (int i = 0; i < MI; ++i)
-#pragma unroll
-                    for (int j = 0; j < NJ; ++j) {
-                        v4f sum[4];
-                        for (int z0 = 0; z0 < senders; z0 += ZC) {
-                            v4i v[ZC][4];
-                            for (;;) {
-                                asm volatile("" ::: "memory");  // the loads belong to this round of the loop
-#pragma unroll
-                                for (int z = 0; z < ZC; ++z)
-#pragma unroll
-                                    for (int q = 0; q < 4; ++q)  // a split past the last: outside the resource, zeros
-                                        v[z][q] = __builtin_amdgcn_raw_buffer_load_b128(
-                                            rp, (uint32_t)((((z0 + z) * PATCHES + i * NJ + j) * 4 + q) * 64 + lane) * 16u, 0, 16);
-                                bool missing = false;
-#pragma unroll
-                                for (int z = 0; z < ZC; ++z)
-#pragma unroll
-                                    for (int q = 0; q < 4; ++q)
-                                        if (z0 + z < senders)
-                                            missing = missing || v[z][q][0] == 0 || v[z][q][1] == 0 || v[z][q][2] == 0 ||
-                                                      v[z][q][3] == 0;
-                                if (__builtin_amdgcn_ballot_w64(missing) == 0)
-                                    break;
-                                if (__builtin_amdgcn_s_memrealtime() - t_first > 100000000ull) {  // one second at 100 MHz
-                                    gave_up = true;
-                                    break;
-                                }
-                            }
+                for (int pg = 0; pg < MI * NJ; pg += PG) {
+                    v4f sum[PG][4];
+                    auto gather = [&](auto count, int z0) __attribute__((always_inline)) {  // splits z0 .. z0 + ZC - 1
+                        constexpr int ZC = decltype(count)::value;
+                        v4i v[ZC][PG][4];
+                        for (;;) {
+                            asm volatile("" ::: "memory");  // the loads belong to this round of the loop
 #pragma unroll
                             for (int z = 0; z < ZC; ++z)
-                                if (z0 + z < senders) {
 #pragma unroll
-                                    for (int q = 0; q < 4; ++q) {
-                                        __builtin_amdgcn_raw_buffer_store_b128(
-                                            (v4i){0, 0, 0, 0}, rp,
-                                            (uint32_t)((((z0 + z) * PATCHES + i * NJ + j) * 4 + q) * 64 + lane) * 16u, 0, 0);
-                                        const v4f f = __builtin_bit_cast(v4f, v[z][q]);
-                                        sum[q] = z0 + z == 0 ? f : sum[q] + f;
-                                    }
-                                }
+                                for (int g = 0; g < PG; ++g)
+#pragma unroll
+                                    for (int q = 0; q < 4; ++q)
+                                        v[z][g][q] = __builtin_amdgcn_raw_buffer_load_b128(
+                                            rp, mail_at(z0 + z, pg + g, q), 0, 16);
+                            bool missing = false;
+#pragma unroll
+                            for (int z = 0; z < ZC; ++z)
+#pragma unroll
+                                for (int g = 0; g < PG; ++g)
+#pragma unroll
+                                    for (int q = 0; q < 4; ++q)
+                                        missing = missing | (v[z][g][q][0] == 0) | (v[z][g][q][1] == 0) |
+                                                  (v[z][g][q][2] == 0) | (v[z][g][q][3] == 0);
+                            if (__builtin_amdgcn_ballot_w64(missing) == 0)
+                                break;
+                            if (__builtin_amdgcn_s_memrealtime() - t_first > 100000000ull) {  // one second at 100 MHz
+                                gave_up = true;
+                                break;
+                            }
                         }
+#pragma unroll
+                        for (int z = 0; z < ZC; ++z)
+#pragma unroll
+                            for (int g = 0; g < PG; ++g)
+#pragma unroll
+                                for (int q = 0; q < 4; ++q) {
+                                    const v4f f = __builtin_bit_cast(v4f, v[z][g][q]);
+                                    sum[g][q] = z0 + z == 0 ? f : sum[g][q] + f;
+                                }
+                    };
+                    int z0 = 0;
+                    for (; z0 + ZB <= senders; z0 += ZB)
+                        gather(std::integral_constant<int, ZB>{}, z0);
+                    if (ZB > 2 && senders - z0 == 2) {
+                        gather(std::integral_constant<int, 2>{}, z0);
+                        z0 += 2;
+                    }
+                    if (z0 < senders)
+                        gather(std::integral_constant<int, 1>{}, z0);
+#pragma unroll
+                    for (int g = 0; g < PG; ++g)
 #pragma unroll
                         for (int q = 0; q < 4; ++q)
 #pragma unroll
-                            for (int e = 0; e < 4; ++e)
-                                acc[i][j][4 * q + e] = gave_up ? __builtin_nanf("") : sum[q][e] + acc[i][j][4 * q + e];
-                    }
+                            for (int e = 0; e < 4; ++e) {
+                                v16f& own = acc[(pg + g) / NJ][(pg + g) % NJ];
+                                own[4 * q + e] = gave_up ? __builtin_nanf("") : sum[g][q][e] + own[4 * q + e];
+                            }
+                }
             }
         }
     }
@@ -478,10 +496,20 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
         }
     };
     if constexpr (SPLIT) {
-        if (as_partial)
+        if (as_partial) {
             write_tile(std::true_type{});
-        else
+        } else {
             write_tile(std::false_type{});
+            if (compute) {  // zeros back into the mailbox, behind the tile
+                const __amdgpu_buffer_rsrc_t rp = make_rsrc(reinterpret_cast<const v4i*>(mailbox) + first, mail_span);
+                for (int z = 0; z < senders; ++z)
+#pragma unroll
+                    for (int patch = 0; patch < MI * NJ; ++patch)
+#pragma unroll
+                        for (int q = 0; q < 4; ++q)
+                            __builtin_amdgcn_raw_buffer_store_b128((v4i){0, 0, 0, 0}, rp, mail_at(z, patch, q), 0, 0);
+            }
+        }
     } else {
         write_tile(std::false_type{});
     }
