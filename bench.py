@@ -361,7 +361,7 @@ def main():
 
     def host_boundary_report():
         """fp8_gemm_host on the headline shape: host fp32 values in, bf16 out, device memory
-        allocated, filled over PCIe, converted, multiplied, read back and freed inside the call
+        allocated, values converted and uploaded, multiplied, read back and freed inside the call
         (pageable host memory, as the reference's harness uses).  Never `value`."""
         ha, hb, sa, sb = host
         af, bf = oracle.e4m3fn_decode(ha), oracle.e4m3fn_decode(hb)
@@ -377,7 +377,7 @@ def main():
                 return {"error": rc}
             best = dt if best is None else min(best, dt)
         moved = af.nbytes + bf.nbytes + sa.nbytes + sb.nbytes + ch.nbytes
-        return {"what": "fp8_gemm_host, best of 3: alloc + PCIe in (fp32 values) + convert + GEMM + PCIe out + free",
+        return {"what": "fp8_gemm_host, best of 3: alloc + fp32 values converted and uploaded + GEMM + download + free",
                 "ms": round(best * 1e3, 2), "tflops": round(flops / best * 1e-12, 2),
                 "host_bytes_moved": moved, "host_gbs": round(moved / best * 1e-9, 1)}
 

@@ -1403,13 +1403,14 @@ int fp8_block_gemm_set_workspace(void* device_ptr, size_t bytes)
 
 int fp8_block_gemm_release(void)
 {
+    const hipError_t staging = release_host_staging();
     std::lock_guard<std::mutex> lock(g_ws_mutex);
     if (!g_ws_own && g_ws_retired.empty())
-        return FP8GEMM_OK;
+        return (int)staging;
     hipError_t e = hipDeviceSynchronize();  // kernels of earlier calls may still use the buffers
     if (e != hipSuccess)
         return (int)e;
-    hipError_t first = hipSuccess;
+    hipError_t first = staging;
     for (Retired& r : g_ws_retired) {
         if (r.done)
             (void)hipEventDestroy(r.done);

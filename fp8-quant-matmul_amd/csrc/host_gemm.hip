@@ -1,10 +1,25 @@
 // Host-buffer launcher: the counterpart of gemmGPU (/root/reference/check.cu:51-130,
-// /root/reference/sgemm.cu:24-191).  Allocate, upload, convert fp32 -> fp8 on the device,
-// launch, download, free -- with every HIP return code checked instead of discarded.
+// /root/reference/sgemm.cu:24-191): fp32 values in host memory in, bf16 in host memory out, with every
+// HIP return code checked instead of discarded.
+//
+// What bounds it is the way from pageable memory to the device.  Uploaded as they are, the fp32 values cross the
+// link at four times the size that the GEMM reads, through the runtime's own staging of pageable memory.  Here a few
+// host threads round the values to e4m3fn (bit for bit what k_convert.hip does) on their way into a pinned staging
+// buffer, which the values would have to be copied into anyway, and the staged bytes are uploaded while later ones are
+// converted; device memory is one allocation, made meanwhile.  1024 x 1536 x 7168 (73 MB of fp32 values): 4460 us with
+// fp32 uploads and a buffer per operand, 1660 us with conversion into staging memory pinned by each call, 1208 us with the
+// staging buffer kept; of these, by time stamps, 130 start the threads, 640 convert and upload (the values are read
+// from memory at 110 GB/s), 210 are the GEMM and the way back.
 #include "../../include/fp8_block_gemm.h"
 #include "launchers.h"
 
+#include <algorithm>
+#include <atomic>
 #include <cstdint>
+#include <cstdlib>
+#include <cstring>
+#include <mutex>
+#include <thread>
 
 namespace {
 
@@ -18,7 +33,278 @@ struct DeviceBuf {
     hipError_t alloc(size_t bytes) { return hipMalloc(&p, bytes ? bytes : 1); }
 };
 
+constexpr size_t SCALES_STAGED = (size_t)1 << 20;  // bytes of scales that go through the staging buffer
+
+// Staging memory of a call.  Pinned if the system grants it, pageable otherwise: the copies below are right either way.
+// Pinning costs as much as converting into it (16 MiB: 0.5 to 1.2 ms), so one buffer of at most STAGING_MAX is kept
+// between calls, for whichever call asks first, and given back by fp8_block_gemm_release; calls that overlap with its
+// user pin their own.
+constexpr size_t STAGING_MAX = (size_t)32 << 20;
+std::mutex g_staging_mutex;
+void* g_staging = nullptr;  // the kept buffer while no call uses it
+size_t g_staging_bytes = 0;
+
+struct StagingBuf {
+    uint8_t* p = nullptr;
+    size_t bytes = 0;
+    bool pinned = false;
+    ~StagingBuf()
+    {
+        if (!pinned) {
+            std::free(p);
+            return;
+        }
+        void* drop = p;
+        if (bytes <= STAGING_MAX) {  // the larger of the two is kept
+            std::lock_guard<std::mutex> lock(g_staging_mutex);
+            if (bytes > g_staging_bytes) {
+                drop = g_staging;
+                g_staging = p;
+                g_staging_bytes = bytes;
+            }
+        }
+        if (drop)
+            (void)hipHostFree(drop);
+    }
+    bool alloc(size_t need)
+    {
+        {
+            std::lock_guard<std::mutex> lock(g_staging_mutex);
+            if (g_staging && g_staging_bytes >= need) {
+                p = static_cast<uint8_t*>(g_staging);
+                bytes = g_staging_bytes;
+                pinned = true;
+                g_staging = nullptr;
+                g_staging_bytes = 0;
+                return true;
+            }
+        }
+        void* q = nullptr;
+        if (hipHostMalloc(&q, need, hipHostMallocPortable) == hipSuccess) {
+            pinned = true;
+        } else {
+            (void)hipGetLastError();
+            q = std::malloc(need);
+        }
+        p = static_cast<uint8_t*>(q);
+        bytes = need;
+        return p != nullptr;
+    }
+};
+
+// fp32 -> e4m3fn, nearest even, beyond +-448 saturated, NaN kept.  Normal results: the upper bits of the fp32 word,
+// rounded by adding half a unit (less one, plus the bit that stays last), with the exponent's bias moved from 127 to 7.
+// Below 2^-6 the code counts steps of 2^-9: adding 2^14 rounds to that step in hardware.
+inline uint32_t e4m3fn_code(float x)
+{
+    uint32_t u;
+    std::memcpy(&u, &x, 4);
+    const uint32_t au = u & 0x7FFFFFFFu;
+    const uint32_t normal = ((au + 0x7FFFFu + ((au >> 20) & 1u)) >> 20) - (120u << 3);
+    float ax;
+    std::memcpy(&ax, &au, 4);
+    const float stepped = ax + 16384.0f;
+    uint32_t su;
+    std::memcpy(&su, &stepped, 4);
+    uint32_t code = au < 0x3C800000u ? (su & 0xFFu) : normal;  // 2^-6
+    code = au >= 0x43E00000u ? 0x7Eu : code;                   // 448
+    code = au > 0x7F800000u ? 0x7Fu : code;
+    return code | ((u >> 24) & 0x80u);
+}
+
+#if defined(__x86_64__)
+__attribute__((target("avx2"))) void convert_avx2(const float* __restrict__ in, uint8_t* __restrict__ out, size_t count)
+{
+    for (size_t i = 0; i < count; ++i)
+        out[i] = (uint8_t)e4m3fn_code(in[i]);
+}
+#endif
+
+void convert_plain(const float* __restrict__ in, uint8_t* __restrict__ out, size_t count)
+{
+    for (size_t i = 0; i < count; ++i)
+        out[i] = (uint8_t)e4m3fn_code(in[i]);
+}
+
+void convert_host(const float* in, uint8_t* out, size_t count)
+{
+#if defined(__x86_64__)
+    if (__builtin_cpu_supports("avx2"))
+        return convert_avx2(in, out, count);
+#endif
+    convert_plain(in, out, count);
+}
+
+// A and B as one run of pieces, a ring of SLOTS of which is staged at a time.  Workers take pieces in order, main
+// uploads them in order and hands slots back once their upload has completed.
+struct Pipeline {
+    static constexpr size_t PIECE = 128 * 1024;  // elements: 24 us of conversion, small enough to share out evenly
+    static constexpr size_t SLOTS = 248;         // 31 MiB: with the scales at most STAGING_MAX
+    static constexpr int MAX_WORKERS = 8;        // 4, 8, 16 threads convert 73 MB in 0.87, 0.54, 0.61 ms
+
+    const float* src[2];
+    size_t count[2], pieces[2];
+    size_t total;  // pieces of both
+    size_t slots;  // of the ring that this call needs
+    uint8_t* staging = nullptr;
+    std::atomic<size_t> next{0}, freed{0};
+    std::atomic<bool> abort{false};
+    std::atomic<size_t> ready[SLOTS];  // number of the last piece converted into the slot, plus one
+
+    Pipeline(const float* a, size_t na, const float* b, size_t nb)
+        : src{a, b}, count{na, nb}, pieces{(na + PIECE - 1) / PIECE, (nb + PIECE - 1) / PIECE}
+    {
+        total = pieces[0] + pieces[1];
+        slots = std::min(total, SLOTS);
+        for (auto& r : ready)
+            r.store(0, std::memory_order_relaxed);
+    }
+
+    // matrix, first element and number of elements of a piece
+    void piece(size_t p, int& which, size_t& first, size_t& n) const
+    {
+        which = p < pieces[0] ? 0 : 1;
+        first = (p - (which ? pieces[0] : 0)) * PIECE;
+        n = std::min(PIECE, count[which] - first);
+    }
+
+    void convert(size_t p)
+    {
+        int which;
+        size_t first, n;
+        piece(p, which, first, n);
+        convert_host(src[which] + first, staging + (p % slots) * PIECE, n);
+        ready[p % slots].store(p + 1, std::memory_order_release);
+    }
+
+    void work()
+    {
+        for (;;) {
+            const size_t p = next.fetch_add(1, std::memory_order_relaxed);
+            if (p >= total)
+                return;
+            while (p >= freed.load(std::memory_order_acquire) + slots) {
+                if (abort.load(std::memory_order_relaxed))
+                    return;
+                std::this_thread::yield();
+            }
+            convert(p);
+        }
+    }
+
+    bool is_ready(size_t p) const { return ready[p % slots].load(std::memory_order_acquire) == p + 1; }
+
+    // main: everything to dst[0] and dst[1] on the null stream; the last copies may be in flight on return
+    hipError_t upload(void* const dst[2], bool have_workers)
+    {
+        size_t p = 0;
+        while (p < total) {
+            // half of the ring back at a time: the other half is what the workers fill meanwhile
+            if (total > slots && p - freed.load(std::memory_order_relaxed) >= slots / 2) {
+                const hipError_t e = hipStreamSynchronize(nullptr);
+                if (e != hipSuccess)
+                    return e;
+                freed.store(p, std::memory_order_release);
+            }
+            if (!have_workers)
+                convert(p);
+            while (!is_ready(p))
+                std::this_thread::yield();
+            // as many pieces as lie behind one another, converted, in the same matrix: a copy costs about 9 us
+            int which;
+            size_t first, n;
+            piece(p, which, first, n);
+            size_t end = p + 1, bytes = n;
+            const size_t stop = std::min(which ? total : pieces[0], p + (slots - p % slots));
+            while (have_workers && end < stop && end - p < slots / 4 && is_ready(end)) {
+                int w;
+                size_t f, more;
+                piece(end, w, f, more);
+                bytes += more;
+                ++end;
+            }
+            const hipError_t e = hipMemcpyAsync(static_cast<uint8_t*>(dst[which]) + first, staging + (p % slots) * PIECE,
+                                                bytes, hipMemcpyHostToDevice, nullptr);
+            if (e != hipSuccess)
+                return e;
+            p = end;
+        }
+        return hipSuccess;
+    }
+};
+
+// The worker threads of one call: joined whatever way the call ends.
+struct Workers {
+    Pipeline& pipe;
+    std::thread thread[Pipeline::MAX_WORKERS];
+    int count = 0;
+
+    explicit Workers(Pipeline& p) : pipe(p) {}
+    ~Workers()
+    {
+        pipe.abort.store(true, std::memory_order_relaxed);
+        join();
+    }
+    void start()
+    {
+        const int cpus = (int)std::thread::hardware_concurrency();
+        const int want = std::min({Pipeline::MAX_WORKERS, cpus - 1, (int)std::min<size_t>(pipe.total / 4, 64)});
+        try {
+            for (; count < want; ++count)
+                thread[count] = std::thread([this] { pipe.work(); });
+        } catch (...) {  // no more threads to be had: those that run, or the caller alone, do it all
+        }
+    }
+    void join()
+    {
+        for (int i = 0; i < count; ++i)
+            if (thread[i].joinable())
+                thread[i].join();
+    }
+};
+
+// c through the staging buffer, in two halves that take turns: one is copied out of while the other fills
+hipError_t download(unsigned short* c, const void* d_c, size_t bytes, uint8_t* staging, size_t staging_bytes)
+{
+    const size_t half = std::min<size_t>(staging_bytes / 2, 1 << 20);
+    uint8_t* out = reinterpret_cast<uint8_t*>(c);
+    size_t done = 0, n = 0;
+    for (size_t at = 0, turn = 0; done < bytes; ++turn) {
+        const size_t coming = std::min(half, bytes - at);
+        if (coming) {
+            const hipError_t e = hipMemcpyAsync(staging + (turn & 1) * half, static_cast<const uint8_t*>(d_c) + at, coming,
+                                                hipMemcpyDeviceToHost, nullptr);
+            if (e != hipSuccess)
+                return e;
+        }
+        if (n)
+            std::memcpy(out + done, staging + ((turn & 1) ^ 1) * half, n);
+        done += n;
+        n = coming;
+        at += coming;
+        const hipError_t e = hipStreamSynchronize(nullptr);
+        if (e != hipSuccess)
+            return e;
+    }
+    return hipSuccess;
+}
+
+size_t padded(size_t bytes) { return (bytes + 255) / 256 * 256; }
+
 }  // namespace
+
+// the kept staging buffer back to the system (fp8_block_gemm_release)
+hipError_t fp8gemm::release_host_staging()
+{
+    void* drop;
+    {
+        std::lock_guard<std::mutex> lock(g_staging_mutex);
+        drop = g_staging;
+        g_staging = nullptr;
+        g_staging_bytes = 0;
+    }
+    return drop ? hipHostFree(drop) : hipSuccess;
+}
 
 extern "C" int fp8_gemm_host(unsigned short* c, const float* a, const float* b, const float* a_scale,
                              const float* b_scale, size_t m, size_t n, size_t k, int option)
@@ -29,34 +315,6 @@ extern "C" int fp8_gemm_host(unsigned short* c, const float* a, const float* b, 
         return FP8GEMM_E_SHAPE;
     if (m * k > 0x7FFFFFFFull || n * k > 0x7FFFFFFFull || m * n > 0x7FFFFFFFull)
         return FP8GEMM_E_TOOLARGE;
-    const size_t nkb = k / 128, sn = (n + 127) / 128;
-    DeviceBuf d_a32, d_b32, d_a8, d_b8, d_as, d_bs, d_c;
-    hipError_t e;
-#define TRY(x)                 \
-    do {                       \
-        e = (x);               \
-        if (e != hipSuccess)   \
-            return (int)e;     \
-    } while (0)
-    TRY(d_a32.alloc(m * k * sizeof(float)));
-    TRY(d_b32.alloc(n * k * sizeof(float)));
-    TRY(d_a8.alloc(m * k));
-    TRY(d_b8.alloc(n * k));
-    TRY(d_as.alloc(nkb * m * sizeof(float)));
-    TRY(d_bs.alloc(nkb * sn * sizeof(float)));
-    TRY(d_c.alloc(m * n * 2));
-    TRY(hipMemcpy(d_a32.p, a, m * k * sizeof(float), hipMemcpyHostToDevice));
-    TRY(hipMemcpy(d_b32.p, b, n * k * sizeof(float), hipMemcpyHostToDevice));
-    TRY(hipMemcpy(d_as.p, a_scale, nkb * m * sizeof(float), hipMemcpyHostToDevice));
-    TRY(hipMemcpy(d_bs.p, b_scale, nkb * sn * sizeof(float), hipMemcpyHostToDevice));
-    int rc = fp8_convert_f32_to_e4m3fn(static_cast<const float*>(d_a32.p), d_a8.p, m * k, nullptr);
-    if (rc != 0)
-        return rc;
-    rc = fp8_convert_f32_to_e4m3fn(static_cast<const float*>(d_b32.p), d_b8.p, n * k, nullptr);
-    if (rc != 0)
-        return rc;
-    const float* das = static_cast<const float*>(d_as.p);
-    const float* dbs = static_cast<const float*>(d_bs.p);
     // per-call options and a workspace of this call's own: no process-wide switch is touched
     fp8gemm_options opt{FP8GEMM_KERNEL_AUTO, -1, 0, -1, 0};
     if (option == 2)
@@ -65,15 +323,50 @@ extern "C" int fp8_gemm_host(unsigned short* c, const float* a, const float* b, 
         opt.kernel = option - 100;
     else if (option != 0 && option != 1)
         return FP8GEMM_E_KERNEL;
+    const size_t nkb = k / 128, sn = (n + 127) / 128;
     const size_t ws_bytes = fp8_block_gemm_workspace_bytes_ex((int)m, (int)n, (int)k, &opt, 0);
-    DeviceBuf d_ws;
-    if (ws_bytes)
-        TRY(d_ws.alloc(ws_bytes));
-    rc = fp8_block_gemm_ex(d_a8.p, d_b8.p, das, dbs, d_c.p, (int)m, (int)n, (int)k, &opt, d_ws.p, ws_bytes,
-                           nullptr);
-    if (rc != 0)
-        return rc;
-    TRY(hipMemcpy(c, d_c.p, m * n * 2, hipMemcpyDeviceToHost));  // blocking: also the sync
+    hipError_t e;
+#define TRY(x)                 \
+    do {                       \
+        e = (x);               \
+        if (e != hipSuccess)   \
+            return (int)e;     \
+    } while (0)
+    StagingBuf staging;
+    DeviceBuf device;
+    Pipeline pipe(a, m * k, b, n * k);
+    // behind the ring the scales, if they are small: a pageable copy of 200 KB takes up to 0.15 ms
+    const size_t ring_bytes = pipe.slots * Pipeline::PIECE;  // two pieces at least
+    const size_t scale_bytes = padded(nkb * m * 4) + nkb * sn * 4;
+    const bool stage_scales = scale_bytes <= SCALES_STAGED;
+    if (!staging.alloc(ring_bytes + (stage_scales ? scale_bytes : 0)))
+        return (int)hipErrorOutOfMemory;
+    pipe.staging = staging.p;
+    {
+        Workers workers(pipe);
+        workers.start();
+        const size_t o_b = padded(m * k), o_as = o_b + padded(n * k), o_bs = o_as + padded(nkb * m * 4),
+                     o_c = o_bs + padded(nkb * sn * 4), o_ws = o_c + padded(m * n * 2);
+        TRY(device.alloc(o_ws + ws_bytes));
+        uint8_t* const d = static_cast<uint8_t*>(device.p);
+        if (stage_scales) {  // laid out as on the device: one copy
+            std::memcpy(staging.p + ring_bytes, a_scale, nkb * m * 4);
+            std::memcpy(staging.p + ring_bytes + (o_bs - o_as), b_scale, nkb * sn * 4);
+            TRY(hipMemcpyAsync(d + o_as, staging.p + ring_bytes, scale_bytes, hipMemcpyHostToDevice, nullptr));
+        } else {
+            TRY(hipMemcpy(d + o_as, a_scale, nkb * m * 4, hipMemcpyHostToDevice));
+            TRY(hipMemcpy(d + o_bs, b_scale, nkb * sn * 4, hipMemcpyHostToDevice));
+        }
+        void* const dst[2] = {d, d + o_b};
+        TRY(pipe.upload(dst, workers.count > 0));
+        workers.join();
+        const int rc = fp8_block_gemm_ex(d, d + o_b, reinterpret_cast<const float*>(d + o_as),
+                                         reinterpret_cast<const float*>(d + o_bs), d + o_c, (int)m, (int)n, (int)k, &opt,
+                                         ws_bytes ? d + o_ws : nullptr, ws_bytes, nullptr);
+        if (rc != 0)
+            return rc;
+        TRY(download(c, d + o_c, m * n * 2, staging.p, ring_bytes));  // blocking: also the sync
+    }
 #undef TRY
     return FP8GEMM_OK;
 }

@@ -157,4 +157,7 @@ enum QuantSource { QUANT_SOURCE_BF16 = 0, QUANT_SOURCE_F32 = 1, QUANT_SOURCE_BF1
 hipError_t launch_quantize(const void* x, QuantSource source, uint8_t* q, float* scale_out, int rows,
                            int k, bool block128, hipStream_t s);
 
+// host_gemm.hip: the pinned staging buffer kept between calls of fp8_gemm_host, back to the system
+hipError_t release_host_staging();
+
 }  // namespace fp8gemm

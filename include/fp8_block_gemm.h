@@ -294,8 +294,10 @@ int fp8_block_gemm_abi_version(void);
 /* ---- host-buffer convenience layer: the reference's host launcher ----
  * Counterpart of gemmGPU (/root/reference/check.cu:51-130): takes HOST buffers with fp32
  * values for a and b (already in the column-major layouts above), allocates device
- * memory, uploads, converts fp32 -> fp8 on the device, runs the kernel selected by
- * `option`, downloads c (bf16 bits) and frees.  option: 2 = scalar definition kernel,
+ * memory, converts fp32 -> fp8 (fp8_convert_f32_to_e4m3fn's rounding, on a few host threads
+ * of this call's own) while it uploads, runs the kernel selected by `option`, downloads c
+ * (bf16 bits) and frees.  A pinned staging buffer of at most 32 MiB is kept between calls
+ * until fp8_block_gemm_release.  option: 2 = scalar definition kernel,
  * 0 = automatic dispatch, 1 = same as 0 (the reference's "reverse" grid has no meaning
  * here), or 100 + FP8GEMM_KERNEL_* to force a family.  Synchronous. */
 int fp8_gemm_host(unsigned short* c, const float* a, const float* b, const float* a_scale,

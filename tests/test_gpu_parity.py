@@ -723,6 +723,67 @@ def test_host_launcher_matches_device_path(pkg):
     assert L.fp8_gemm_host(c.ctypes.data, af.ctypes.data, bf.ctypes.data, sa.ctypes.data, sb.ctypes.data, m, n, k, 7) == -3
 
 
+@pytest.mark.parametrize("m,n,k", [
+    (1, 128, 128),        # no worker threads
+    (520, 128, 1024),     # a's last piece is a part of one
+    (2052, 2304, 8192),   # 272 pieces: the staging ring of 256 goes round, the last piece of a ragged
+    (4100, 2304, 256),    # c larger than both staging halves
+])
+def test_host_launcher_converts_like_the_device(pkg, m, n, k):
+    """fp8_gemm_host rounds on the host, in pieces: codes, and so c, bit for bit those of the device converter"""
+    import torch
+    rng = np.random.default_rng(m + n + k)
+    af = rng.integers(0, 2**32, m * k, dtype=np.uint32).view(np.float32)   # every exponent, ties rare
+    af = np.where(np.abs(af) < 2.0**9, af, rng.standard_normal(m * k).astype(np.float32))  # no NaN: it would hide its row
+    af[::7] = (rng.integers(-960, 961, af[::7].size) * np.float32(2.0**-10))   # ties and steps below 2^-6
+    af[3], af[5] = np.inf, -np.inf
+    af[m * k - 1] = np.nan
+    bf = (rng.standard_normal(n * k) * 100).astype(np.float32)
+    sa = rng.uniform(0.5, 2, (k // 128) * m).astype(np.float32)
+    sb = rng.uniform(0.5, 2, (k // 128) * ((n + 127) // 128)).astype(np.float32)
+    c = np.zeros((m, n), np.uint16)
+    _say(f"[gpu case] fp8_gemm_host {m}x{n}x{k} against the device converter")
+    rc = pkg.lib().fp8_gemm_host(c.ctypes.data, af.ctypes.data, bf.ctypes.data, sa.ctypes.data, sb.ctypes.data, m, n, k, 0)
+    assert rc == 0
+    da, db, dsa, dsb = (torch.from_numpy(x).cuda() for x in (af, bf, sa, sb))
+    a8 = torch.empty(m * k, dtype=torch.uint8, device="cuda")
+    b8 = torch.empty(n * k, dtype=torch.uint8, device="cuda")
+    pkg.convert_f32_to_e4m3fn(da, a8, m * k)
+    pkg.convert_f32_to_e4m3fn(db, b8, n * k)
+    opt = pkg.Options()
+    ws = torch.empty(max(256, pkg.workspace_bytes_ex(m, n, k, opt)), dtype=torch.uint8, device="cuda")
+    dc = torch.zeros((m, n), dtype=torch.int16, device="cuda")
+    pkg.gemm_ex(a8, b8, dsa, dsb, dc, m, n, k, opt, ws, ws.numel())
+    torch.cuda.synchronize()
+    assert np.array_equal(c, dc.cpu().numpy().view(np.uint16))
+
+def test_host_launcher_from_several_threads(pkg):
+    """calls that overlap (one uses the kept staging buffer, the others pin their own) and a release between them"""
+    import threading
+    m, n, k = 300, 256, 2048
+    a, b, sa, sb = oracle.make_inputs(m, n, k, 63)
+    af, bf = oracle.e4m3fn_decode(a), oracle.e4m3fn_decode(b)
+    out = [[np.zeros((m, n), np.uint16) for _ in range(4)] for _ in range(3)]
+    rcs = []
+
+    def work(mine):
+        for c in mine:
+            rcs.append(pkg.lib().fp8_gemm_host(c.ctypes.data, af.ctypes.data, bf.ctypes.data, sa.ctypes.data,
+                                               sb.ctypes.data, m, n, k, 0))
+            pkg.release()
+
+    _say("[gpu case] fp8_gemm_host from three threads")
+    threads = [threading.Thread(target=work, args=(mine,)) for mine in out]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert rcs == [0] * 12
+    for mine in out:
+        for c in mine:
+            assert np.array_equal(c, out[0][0])
+    _assert_close(out[0][0], oracle.ref_gemm(a, b, sa, sb, m, n, k), "host launcher, several threads")
+
 def test_caller_workspace(pkg):
     import torch
     m, n, k = 256, 256, 1024
