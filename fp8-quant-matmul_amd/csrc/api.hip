@@ -675,22 +675,21 @@ int run_padded(const GemmArgs& g, const Plan& p, const Workspace& w, hipStream_t
     uint8_t* base = reinterpret_cast<uint8_t*>(ws_data(w));
     const int nkb = g.k / 128;
     // every operand that needs a padded copy, in one launch
-    PadJobs jobs;
-    jobs.count = 0;
+    PadJobs<PAD_JOBS_SINGLE> jobs;
+    jobs.base = base;
     if (L.a) {
-        jobs.job[jobs.count++] = PadJob{g.a, base + L.off_a, g.k, g.m, m16, 0};
+        jobs.add(g.a, L.off_a, g.k, g.m, m16);
         gp.a = base + L.off_a;
     }
     if (L.as) {
-        float* as = reinterpret_cast<float*>(base + L.off_as);
-        jobs.job[jobs.count++] = PadJob{g.a_scale, as, nkb, g.m, m16, 1};
-        gp.a_scale = as;
+        jobs.add(g.a_scale, L.off_as, nkb, (size_t)g.m * 4, (size_t)m16 * 4);
+        gp.a_scale = reinterpret_cast<float*>(base + L.off_as);
     }
     if (L.b) {
-        jobs.job[jobs.count++] = PadJob{g.b, base + L.off_b, g.k, g.n, gp.n, 0};
+        jobs.add(g.b, L.off_b, g.k, g.n, gp.n);
         gp.b = base + L.off_b;
     }
-    hipError_t e = launch_pad_jobs(jobs, stream);
+    hipError_t e = launch_pad(jobs, stream);
     if (L.c)
         gp.c = reinterpret_cast<uint16_t*>(base + L.off_c);
     if (e == hipSuccess)
@@ -963,20 +962,23 @@ int run_grouped_table(const GroupTable& tab, int n, int k, bool decode, hipStrea
     if (wrc != FP8GEMM_OK)
         return wrc;
     uint8_t* base = reinterpret_cast<uint8_t*>(ws_data(w));
-    RepackTable ta, tas, tb, tc;
-    ta.groups = tas.groups = tb.groups = tc.groups = tab.groups;
+    PadJobs<PAD_JOBS_GROUPED> jobs;
+    CropTable tc;
+    jobs.base = base;
+    tc.groups = tab.groups, tc.n = n, tc.ld_src = n16;
     if (padded)
         for (int g = 0; g < tab.groups; ++g) {
             const int m = tab.m[g], m16 = (m + 15) & ~15;
-            pt.a[g] = base + off_a[g];
-            pt.a_scale[g] = reinterpret_cast<const float*>(base + off_as[g]);
+            // a group that lies on the grid by itself stays where it is
+            if (m16 != m || misaligned16(tab.a[g]) || misaligned16(tab.a_scale[g])) {
+                jobs.add(tab.a[g], off_a[g], k, m, m16);
+                jobs.add(tab.a_scale[g], off_as[g], nkb, (size_t)m * 4, (size_t)m16 * 4);
+                pt.a[g] = base + off_a[g];
+                pt.a_scale[g] = reinterpret_cast<const float*>(base + off_as[g]);
+            }
             pt.b[g] = pad_b ? base + off_b[g] : tab.b[g];
             pt.c[g] = pad_c ? reinterpret_cast<uint16_t*>(base + off_c[g]) : tab.c[g];
-            ta.src[g] = tab.a[g], ta.dst[g] = base + off_a[g], ta.rows[g] = k, ta.ld_src[g] = m, ta.ld_dst[g] = m16;
-            tas.src[g] = tab.a_scale[g], tas.dst[g] = base + off_as[g], tas.rows[g] = (int)nkb, tas.ld_src[g] = m,
-            tas.ld_dst[g] = m16;
-            tb.src[g] = tab.b[g], tb.dst[g] = base + off_b[g], tb.rows[g] = k, tb.ld_src[g] = n, tb.ld_dst[g] = n16;
-            tc.src[g] = base + off_c[g], tc.dst[g] = tab.c[g], tc.rows[g] = m, tc.ld_src[g] = n16, tc.ld_dst[g] = n;
+            tc.src[g] = base + off_c[g], tc.dst[g] = tab.c[g], tc.m[g] = m;
         }
     if (!decode) {
         variant = grouped_variant(pt, n16, k, cfg);
@@ -990,9 +992,13 @@ int run_grouped_table(const GroupTable& tab, int n, int k, bool decode, hipStrea
     }
     hipError_t e = hipSuccess;
     if (padded) {
-        e = launch_pad_pair_batched(ta, tas, s);
-        if (e == hipSuccess && pad_b)
-            e = launch_pad_bytes_batched(tb, s);
+        e = launch_pad(jobs, s);
+        if (e == hipSuccess && pad_b) {
+            jobs.count = 0;
+            for (int g = 0; g < tab.groups; ++g)
+                jobs.add(tab.b[g], off_b[g], k, n, n16);
+            e = launch_pad(jobs, s);
+        }
     }
     if (e == hipSuccess)
         e = decode ? launch_decode_grouped(pt, n16, k, ksplit, ws_mailbox(w), s)

@@ -14,53 +14,108 @@ namespace fp8gemm {
 
 namespace {
 
-// dst[r][0..ld_dst) = src[r][0..ld_src) followed by zeros; ld_dst is a multiple of 4 floats and
-// dst is 16-byte aligned.  One thread (number idx) writes one 16-byte piece.
-__device__ __forceinline__ void pad_piece_floats(const float* __restrict__ src, float* __restrict__ dst, int rows,
-                                                 int ld_src, int ld_dst, size_t idx)
-{
-    const int chunks = ld_dst / 4;
-    if (idx >= (size_t)rows * chunks)
-        return;
-    const int r = (int)(idx / chunks), ch = (int)(idx - (size_t)r * chunks);
-    float v[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int col = ch * 4 + j;
-        v[j] = col < ld_src ? src[(size_t)r * ld_src + col] : 0.0f;
+// 16 bytes of a padded row: dst[16 * ch ..] = src[16 * ch ..] of a row of ld_src bytes, zeros beyond it.  Whatever the
+// alignment of the row, the bytes lie in one or two aligned 16-byte pieces of memory, which are loaded whole and shifted
+// into place.  What such a piece holds beside the row is not used, and it lies on a page of the matrix.
+struct PadPiece {
+    v4i lo, hi;     // the aligned pieces
+    uint32_t sh;    // where the row's bytes start in them
+    int valid;      // bytes that belong to the row
+
+    __device__ __forceinline__ void load(const uint8_t* src, uint32_t row, uint32_t ch, uint32_t ld_src)
+    {
+        valid = (int)ld_src - 16 * (int)ch;
+        const uintptr_t ad = reinterpret_cast<uintptr_t>(src) + (size_t)row * ld_src + (size_t)ch * 16;
+        sh = (uint32_t)(ad & 15);
+        // no branch around a load: each would be waited for before the next is asked for.  A piece that holds none of the
+        // row's bytes is replaced by one that does (the other piece, or where the row starts: rows are not empty).
+        const uintptr_t p = valid > 0 ? ad - sh : (reinterpret_cast<uintptr_t>(src) + (size_t)row * ld_src) & ~(uintptr_t)15;
+        const bool both = (int)sh + (valid < 16 ? valid : 16) > 16;
+        lo = *reinterpret_cast<const __attribute__((address_space(1))) v4i*>(p);
+        hi = *reinterpret_cast<const __attribute__((address_space(1))) v4i*>(p + (both ? 16 : 0));
     }
-    *reinterpret_cast<float4*>(dst + (size_t)r * ld_dst + (size_t)ch * 4) = make_float4(v[0], v[1], v[2], v[3]);
+
+    __device__ __forceinline__ v4i bytes() const
+    {
+        const uint32_t w[8] = {(uint32_t)lo[0], (uint32_t)lo[1], (uint32_t)lo[2], (uint32_t)lo[3],
+                               (uint32_t)hi[0], (uint32_t)hi[1], (uint32_t)hi[2], (uint32_t)hi[3]};
+        // bit selects: a choice between two elements of an array becomes an indexed access, by way of the LDS
+        const uint32_t by2 = 0u - ((sh >> 3) & 1u), by1 = 0u - ((sh >> 2) & 1u);
+        uint32_t two[6], one[5];
+#pragma unroll
+        for (int i = 0; i < 6; ++i)
+            two[i] = (w[i + 2] & by2) | (w[i] & ~by2);
+#pragma unroll
+        for (int i = 0; i < 5; ++i)
+            one[i] = (two[i + 1] & by1) | (two[i] & ~by1);
+        v4i out;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t v = __builtin_amdgcn_alignbyte(one[i + 1], one[i], sh & 3);
+            const int left = valid - 4 * i;  // bytes of this dword that belong to the row
+            out[i] = (int)(left >= 4 ? v : (left <= 0 ? 0u : (v & ((1u << (8 * left)) - 1u))));
+        }
+        return out;
+    }
+};
+
+// All padding copies of a call in one launch: a workgroup moves PER_THREAD * 256 pieces of 16 bytes of one job.
+//
+// Bound by memory: 2 bytes move per byte of the operand.  All loads of a thread are out before the first is needed, indices
+// are 32 bits wide (an operand has less than 2^27 pieces), and the grid holds the pieces that there are.  Against one piece
+// per thread by five dword loads and a 64-bit division on a grid as large for every job as for the largest: 8191 x 7168
+// 25.0 -> 22.1 us (5.3 TB/s), eight groups of 250 ... 2051 rows x 2048 12.9 -> 9.6 us, thirty of 200 rows 8.6 -> 7.6 us;
+// a single operand of up to 3 MB, where the launch is what it takes, is level (333 x 7168: 5.0 us).
+template <int MAX, int PER_THREAD>
+__global__ void __launch_bounds__(256) pad_kernel(const PadJobs<MAX> jobs)
+{
+    const uint32_t block = blockIdx.x;
+    int job = 0;
+    if (MAX <= 4) {
+#pragma unroll
+        for (int j = 1; j < MAX; ++j)
+            job += j < jobs.count && block >= jobs.first_block[j];
+    } else {  // first_block ascends: how many jobs start at or before this workgroup, looked up by a lane each
+        const int lane = threadIdx.x & 63;
+        int upto = 0;
+#pragma unroll
+        for (int j = 0; j < MAX; j += 64)
+            upto += __builtin_popcountll(
+                __builtin_amdgcn_ballot_w64(j + lane < jobs.count && jobs.first_block[j + lane] <= block));
+        job = __builtin_amdgcn_readfirstlane(upto) - 1;
+    }
+    const uint8_t* const src = static_cast<const uint8_t*>(jobs.src[job]);
+    uint8_t* const dst = jobs.base + (size_t)jobs.dst256[job] * 256;
+    const uint32_t chunks = jobs.chunks[job], ld_src = jobs.ld_src[job], pieces = jobs.rows[job] * chunks;
+    const uint32_t at = (block - jobs.first_block[job]) * (256u * PER_THREAD) + threadIdx.x;
+    PadPiece piece[PER_THREAD];
+#pragma unroll
+    for (int u = 0; u < PER_THREAD; ++u) {
+        const uint32_t idx = min(at + 256u * u, pieces - 1), row = idx / chunks;
+        piece[u].load(src, row, idx - row * chunks, ld_src);
+    }
+#pragma unroll
+    for (int u = 0; u < PER_THREAD; ++u) {
+        const uint32_t idx = at + 256u * u;
+        if (idx < pieces)
+            *(__attribute__((address_space(1))) v4i*)(dst + (size_t)idx * 16) = piece[u].bytes();
+    }
 }
 
-// The same for bytes (ld_dst a multiple of 16), at dword speed whatever the alignment of a source
-// row: the (up to five) aligned dwords that hold the 16 source bytes are read and shifted into
-// place.  The first and the last dword may reach up to 3 bytes beyond the row: they stay inside
-// the aligned dwords that hold the matrix's first and last byte, so no access leaves its pages.
-__device__ __forceinline__ void pad_piece_bytes(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, int rows,
-                                                int ld_src, int ld_dst, size_t idx)
+// Four pieces to a thread from this many on (4 MB: four workgroups of 256 threads for every CU with one each): below, CUs
+// would be left without a workgroup.
+constexpr size_t PIECES_FOR_FOUR = (size_t)1 << 18;
+
+template <int MAX, int PER_THREAD>
+hipError_t launch_pad_typed(PadJobs<MAX>& jobs, hipStream_t s)
 {
-    const int chunks = ld_dst / 16;
-    if (idx >= (size_t)rows * chunks)
-        return;
-    const int r = (int)(idx / chunks), ch = (int)(idx - (size_t)r * chunks);
-    int valid = ld_src - 16 * ch;  // source bytes of this piece
-    valid = valid < 0 ? 0 : (valid > 16 ? 16 : valid);
-    const uintptr_t ad = reinterpret_cast<uintptr_t>(src) + (size_t)r * ld_src + (size_t)ch * 16;
-    const uint32_t sh = (uint32_t)(ad & 3);
-    const uint32_t* w = reinterpret_cast<const uint32_t*>(ad - sh);
-    const int need = valid > 0 ? ((int)sh + valid + 3) >> 2 : 0;
-    uint32_t in[5];
-#pragma unroll
-    for (int i = 0; i < 5; ++i)
-        in[i] = i < need ? w[i] : 0u;
-    uint32_t out[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const uint32_t v = __builtin_amdgcn_alignbyte(in[i + 1], in[i], sh);
-        const int left = valid - 4 * i;  // bytes of this dword that belong to the row
-        out[i] = left >= 4 ? v : (left <= 0 ? 0u : (v & ((1u << (8 * left)) - 1u)));
+    uint32_t blocks = 0;
+    for (int j = 0; j < jobs.count; ++j) {
+        jobs.first_block[j] = blocks;
+        blocks += (jobs.rows[j] * jobs.chunks[j] + 256 * PER_THREAD - 1) / (256 * PER_THREAD);
     }
-    *reinterpret_cast<uint4*>(dst + (size_t)r * ld_dst + (size_t)ch * 16) = make_uint4(out[0], out[1], out[2], out[3]);
+    hipLaunchKernelGGL((pad_kernel<MAX, PER_THREAD>), dim3(blocks), dim3(256), 0, s, jobs);
+    return hipGetLastError();
 }
 
 // dst[m][n] (dense) = src[m][0..n) of a matrix with ld_src elements per row (a multiple of 8, base
@@ -92,142 +147,60 @@ __device__ __forceinline__ void crop_piece(const uint16_t* __restrict__ src, uin
     }
 }
 
-enum RepackKind { REPACK_PAD_BYTES, REPACK_PAD_FLOATS, REPACK_CROP_BF16 };
-
-template <int KIND>
-__device__ __forceinline__ void repack_piece(const void* src, void* dst, int rows, int ld_src, int ld_dst, size_t idx)
+// a problem per blockIdx.y
+__global__ void __launch_bounds__(256) crop_batched_kernel(const CropTable tab)
 {
-    if (KIND == REPACK_PAD_BYTES)
-        pad_piece_bytes(static_cast<const uint8_t*>(src), static_cast<uint8_t*>(dst), rows, ld_src, ld_dst, idx);
-    else if (KIND == REPACK_PAD_FLOATS)
-        pad_piece_floats(static_cast<const float*>(src), static_cast<float*>(dst), rows, ld_src, ld_dst, idx);
-    else  // rows = m, ld_dst = n
-        crop_piece(static_cast<const uint16_t*>(src), static_cast<uint16_t*>(dst), rows, ld_dst, ld_src, idx);
+    const int g = blockIdx.y;
+    crop_piece(static_cast<const uint16_t*>(tab.src[g]), static_cast<uint16_t*>(tab.dst[g]), tab.m[g], tab.n, tab.ld_src,
+               (size_t)blockIdx.x * blockDim.x + threadIdx.x);
 }
 
-template <int KIND>
-__host__ __device__ inline size_t repack_pieces(int rows, int ld_dst)
-{
-    return (size_t)rows * (KIND == REPACK_PAD_BYTES ? ld_dst / 16 : KIND == REPACK_PAD_FLOATS ? ld_dst / 4
-                                                                                                : (ld_dst + 7) / 8);
-}
-
-template <int KIND>
 __global__ void __launch_bounds__(256)
-repack_kernel(const void* __restrict__ src, void* __restrict__ dst, int rows, int ld_src, int ld_dst)
+crop_kernel(const uint16_t* __restrict__ src, uint16_t* __restrict__ dst, int m, int n, int ld_src)
 {
-    repack_piece<KIND>(src, dst, rows, ld_src, ld_dst, (size_t)blockIdx.x * blockDim.x + threadIdx.x);
+    crop_piece(src, dst, m, n, ld_src, (size_t)blockIdx.x * blockDim.x + threadIdx.x);
 }
 
-// one matrix per blockIdx.y
-template <int KIND>
-__global__ void __launch_bounds__(256) repack_batched_kernel(const RepackTable tab)
-{
-    const int g = blockIdx.y;
-    repack_piece<KIND>(tab.src[g], tab.dst[g], tab.rows[g], tab.ld_src[g], tab.ld_dst[g],
-                       (size_t)blockIdx.x * blockDim.x + threadIdx.x);
-}
-
-// up to PadJobs::MAX padding copies of either kind in one launch, one per blockIdx.y
-__global__ void __launch_bounds__(256) pad_jobs_kernel(const PadJobs jobs)
-{
-    const PadJob& j = jobs.job[blockIdx.y];
-    const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (j.floats)
-        pad_piece_floats(static_cast<const float*>(j.src), static_cast<float*>(j.dst), j.rows, j.ld_src, j.ld_dst, idx);
-    else
-        pad_piece_bytes(static_cast<const uint8_t*>(j.src), static_cast<uint8_t*>(j.dst), j.rows, j.ld_src, j.ld_dst, idx);
-}
-
-// the byte copies (blockIdx.z = 0) and the fp32 copies (blockIdx.z = 1) of several problems in one launch
-__global__ void __launch_bounds__(256) pad_pair_batched_kernel(const RepackTable bytes, const RepackTable floats)
-{
-    const int g = blockIdx.y;
-    const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (blockIdx.z == 0)
-        repack_piece<REPACK_PAD_BYTES>(bytes.src[g], bytes.dst[g], bytes.rows[g], bytes.ld_src[g], bytes.ld_dst[g], idx);
-    else
-        repack_piece<REPACK_PAD_FLOATS>(floats.src[g], floats.dst[g], floats.rows[g], floats.ld_src[g], floats.ld_dst[g], idx);
-}
-
-template <int KIND>
-hipError_t launch_repack(const void* src, void* dst, int rows, int ld_src, int ld_dst, hipStream_t s)
-{
-    const size_t pieces = repack_pieces<KIND>(rows, ld_dst);
-    if (pieces == 0)
-        return hipSuccess;
-    hipLaunchKernelGGL((repack_kernel<KIND>), dim3((unsigned)((pieces + 255) / 256)), dim3(256), 0, s, src, dst,
-                       rows, ld_src, ld_dst);
-    return hipGetLastError();
-}
-
-template <int KIND>
-hipError_t launch_repack_batched(const RepackTable& tab, hipStream_t s)
-{
-    if (tab.groups < 1 || tab.groups > RepackTable::MAX_GROUPS)
-        return hipErrorInvalidValue;
-    size_t most = 0;
-    for (int g = 0; g < tab.groups; ++g) {
-        const size_t pieces = repack_pieces<KIND>(tab.rows[g], tab.ld_dst[g]);
-        most = pieces > most ? pieces : most;
-    }
-    if (most == 0)
-        return hipSuccess;
-    hipLaunchKernelGGL((repack_batched_kernel<KIND>), dim3((unsigned)((most + 255) / 256), (unsigned)tab.groups),
-                       dim3(256), 0, s, tab);
-    return hipGetLastError();
-}
+inline unsigned crop_blocks(int m, int n) { return (unsigned)(((size_t)m * ((n + 7) / 8) + 255) / 256); }
 
 }  // namespace
 
-hipError_t launch_pad_jobs(const PadJobs& jobs, hipStream_t s)
+template <int MAX>
+hipError_t launch_pad(PadJobs<MAX>& jobs, hipStream_t s)
 {
-    if (jobs.count < 0 || jobs.count > PadJobs::MAX)
+    if (jobs.count < 0 || jobs.count > MAX)
         return hipErrorInvalidValue;
-    size_t most = 0;
-    for (int i = 0; i < jobs.count; ++i) {
-        const PadJob& j = jobs.job[i];
-        const size_t pieces = j.floats ? repack_pieces<REPACK_PAD_FLOATS>(j.rows, j.ld_dst)
-                                       : repack_pieces<REPACK_PAD_BYTES>(j.rows, j.ld_dst);
-        most = pieces > most ? pieces : most;
-    }
-    if (most == 0)
+    size_t pieces = 0;
+    for (int j = 0; j < jobs.count; ++j)
+        pieces += (size_t)jobs.rows[j] * jobs.chunks[j];
+    if (pieces == 0)
         return hipSuccess;
-    hipLaunchKernelGGL(pad_jobs_kernel, dim3((unsigned)((most + 255) / 256), (unsigned)jobs.count), dim3(256), 0, s, jobs);
-    return hipGetLastError();
+    return pieces >= PIECES_FOR_FOUR ? launch_pad_typed<MAX, 4>(jobs, s) : launch_pad_typed<MAX, 1>(jobs, s);
 }
+template hipError_t launch_pad<PAD_JOBS_SINGLE>(PadJobs<PAD_JOBS_SINGLE>&, hipStream_t);
+template hipError_t launch_pad<PAD_JOBS_GROUPED>(PadJobs<PAD_JOBS_GROUPED>&, hipStream_t);
 
 hipError_t launch_crop_bf16(const uint16_t* src, uint16_t* dst, int m, int n, int ld_src, hipStream_t s)
 {
-    return launch_repack<REPACK_CROP_BF16>(src, dst, m, ld_src, n, s);
-}
-
-hipError_t launch_pad_pair_batched(const RepackTable& bytes, const RepackTable& floats, hipStream_t s)
-{
-    if (bytes.groups < 1 || bytes.groups > RepackTable::MAX_GROUPS || floats.groups != bytes.groups)
-        return hipErrorInvalidValue;
-    size_t most = 0;
-    for (int g = 0; g < bytes.groups; ++g) {
-        const size_t pb = repack_pieces<REPACK_PAD_BYTES>(bytes.rows[g], bytes.ld_dst[g]);
-        const size_t pf = repack_pieces<REPACK_PAD_FLOATS>(floats.rows[g], floats.ld_dst[g]);
-        most = pb > most ? pb : most;
-        most = pf > most ? pf : most;
-    }
-    if (most == 0)
+    if (m == 0 || n == 0)
         return hipSuccess;
-    hipLaunchKernelGGL(pad_pair_batched_kernel, dim3((unsigned)((most + 255) / 256), (unsigned)bytes.groups, 2), dim3(256), 0, s,
-                       bytes, floats);
+    hipLaunchKernelGGL(crop_kernel, dim3(crop_blocks(m, n)), dim3(256), 0, s, src, dst, m, n, ld_src);
     return hipGetLastError();
 }
 
-hipError_t launch_pad_bytes_batched(const RepackTable& tab, hipStream_t s)
+hipError_t launch_crop_bf16_batched(const CropTable& tab, hipStream_t s)
 {
-    return launch_repack_batched<REPACK_PAD_BYTES>(tab, s);
-}
-
-hipError_t launch_crop_bf16_batched(const RepackTable& tab, hipStream_t s)
-{
-    return launch_repack_batched<REPACK_CROP_BF16>(tab, s);
+    if (tab.groups < 1 || tab.groups > CropTable::MAX_GROUPS)
+        return hipErrorInvalidValue;
+    unsigned most = 0;
+    for (int g = 0; g < tab.groups; ++g) {
+        const unsigned blocks = crop_blocks(tab.m[g], tab.n);
+        most = blocks > most ? blocks : most;
+    }
+    if (most == 0)
+        return hipSuccess;
+    hipLaunchKernelGGL(crop_batched_kernel, dim3(most, (unsigned)tab.groups), dim3(256), 0, s, tab);
+    return hipGetLastError();
 }
 
 }  // namespace fp8gemm

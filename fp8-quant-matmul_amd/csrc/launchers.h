@@ -113,39 +113,43 @@ hipError_t launch_decode_grouped(const GroupTable& tab, int n, int k, int ksplit
 // 0 = they do not, or it could not be looked at; -1 = not looked at yet and may_probe is false
 int xcd_placement_confirmed(bool may_probe);
 
-// Padding: rows of ld_src elements copied into rows of ld_dst >= ld_src elements, the rest zero (dst
-// 16-byte aligned, ld_dst a multiple of 16 bytes).  Cropping: the m x n corner of a bf16 matrix with
-// ld_src elements per row copied into a dense one.
-hipError_t launch_crop_bf16(const uint16_t* src, uint16_t* dst, int m, int n, int ld_src, hipStream_t s);
-// the padding copies of one problem (bytes of a and b, fp32 values of a_scale) in one launch
-struct PadJob {
-    const void* src;
-    void* dst;
-    int rows, ld_src, ld_dst;
-    int floats;  // 0 = bytes (ld_dst a multiple of 16), 1 = fp32 values (ld_dst a multiple of 4)
-};
+// Padding copies of a call (bytes of a and b, fp32 values of a_scale taken as bytes), all in one launch: rows of ld_src
+// bytes copied into rows of 16 * chunks >= ld_src bytes, the rest zero.  The destinations are given as distances
+// from `base` (16-byte aligned) in steps of 256 bytes, which lets the jobs of a full grouped launch travel by value in the kernel arguments.
+constexpr int PAD_JOBS_SINGLE = 3, PAD_JOBS_GROUPED = 128;
+template <int MAX>
 struct PadJobs {
-    static constexpr int MAX = 4;
-    PadJob job[MAX];
-    int count;
+    const void* src[MAX];
+    uint8_t* base;
+    uint32_t dst256[MAX];  // distance of the destination from base in units of 256 bytes
+    uint32_t rows[MAX], ld_src[MAX], chunks[MAX];
+    uint32_t first_block[MAX];  // filled in by the launcher
+    int count = 0;
+    // offset (from base) is a multiple of 256
+    void add(const void* from, size_t offset, size_t n_rows, size_t row_bytes, size_t padded_bytes)
+    {
+        src[count] = from;
+        dst256[count] = (uint32_t)(offset / 256);
+        rows[count] = (uint32_t)n_rows;
+        ld_src[count] = (uint32_t)row_bytes;
+        chunks[count] = (uint32_t)(padded_bytes / 16);
+        ++count;
+    }
 };
-hipError_t launch_pad_jobs(const PadJobs& jobs, hipStream_t s);
-// one kind of copy for several matrices in one launch (the table travels by value in the kernel
-// arguments).  Padding: rows x ld_src -> rows x ld_dst.  Cropping: rows = m, ld_src = elements
-// per source row, ld_dst = n.
-struct RepackTable {
+template <int MAX>
+hipError_t launch_pad(PadJobs<MAX>& jobs, hipStream_t s);
+// Cropping: the m x n corner of a bf16 matrix with ld_src elements per row copied into a dense one; batched: for
+// several matrices in one launch
+hipError_t launch_crop_bf16(const uint16_t* src, uint16_t* dst, int m, int n, int ld_src, hipStream_t s);
+struct CropTable {
     static constexpr int MAX_GROUPS = 64;
     const void* src[MAX_GROUPS];
     void* dst[MAX_GROUPS];
-    int rows[MAX_GROUPS];
-    int ld_src[MAX_GROUPS];
-    int ld_dst[MAX_GROUPS];
+    int m[MAX_GROUPS];
+    int n, ld_src;
     int groups;
 };
-hipError_t launch_pad_bytes_batched(const RepackTable& tab, hipStream_t s);
-// byte copies (a of every group) and fp32 copies (a_scale of every group) in one launch; same group count
-hipError_t launch_pad_pair_batched(const RepackTable& bytes, const RepackTable& floats, hipStream_t s);
-hipError_t launch_crop_bf16_batched(const RepackTable& tab, hipStream_t s);
+hipError_t launch_crop_bf16_batched(const CropTable& tab, hipStream_t s);
 
 // fp32 -> e4m3fn (check.cu:17-22)
 hipError_t launch_convert(const float* in, uint8_t* out, size_t count, hipStream_t s);
