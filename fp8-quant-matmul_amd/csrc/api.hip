@@ -235,6 +235,22 @@ bool tile_plan_fused(const GemmArgs& g, int variant, int ksplit, const Config& c
     return cfg.fused_mode == 1 || tile_fused_pays(g, variant, ksplit);
 }
 
+// Row counts off the 16-byte grid: the tiles' form that takes them as they are against the copy launch and the plain
+// form.  A comes through registers in the former, 0.05 to 0.1 us more per K block, where the copies take 1.5 to 6 us: 101
+// random shapes of 65 ... 4000 rows 27 % faster on average with operands from the Infinity Cache, 25 % from HBM.  The lines
+// are where the two meet when a workgroup walks long (128x128: 333 x 4608 unsplit 18.9 / 23.6 / 37.6 us for 24 / 32 / 56
+// blocks against 19.4 / 23.8 / 36.0; 1501 x 1536, more to copy, 37.8 against 39.3 for 56; 128x192: 397 x 7168 25.1 /
+// 31.6 / 51.4 against 26.6 / 32.9 / 51.2).  256x128 tiles have no such form: no registers are left to hide a trip behind,
+// and it was level at four blocks and 20 % behind at 12.
+bool tile_ragged_pays(const GemmArgs& g, int variant, int ksplit)
+{
+    int bm, bn;
+    tile_variant_dims(variant, &bm, &bn);
+    const long items = (long)((g.m + bm - 1) / bm) * ((g.n + bn - 1) / bn) * ksplit;
+    const long rounds = (items + NUM_CU - 1) / NUM_CU, blocks = (g.k / 128 + ksplit - 1) / ksplit;
+    return rounds * blocks <= (variant == TILE_128x192 ? 40 : 56);
+}
+
 // Shapes whose best measured plan differs from the model's choice: {m, n, k, variant, ksplit}.
 struct TunedShape { int m, n, k, variant, ksplit; };
 constexpr TunedShape kTuned[] = {
@@ -423,6 +439,9 @@ Plan compute_plan(const GemmArgs& g, const Config& cfg)
         GemmArgs gp{al8, al8, reinterpret_cast<const float*>(uintptr_t(4096)), g.b_scale,
                     reinterpret_cast<uint16_t*>(uintptr_t(4096)), (int)m16, (int)n16, g.k};
         p = make_plan(gp, cfg);
+        const bool tiles = p.family == FP8GEMM_KERNEL_LARGE || p.family == FP8GEMM_KERNEL_SPLITK;
+        if (tiles && !p.persistent && tile_ragged_supports(g, p.variant) && tile_ragged_pays(g, p.variant, p.ksplit))
+            return p;  // rows off the 16-byte grid as they are
         p.padded = p.family != FP8GEMM_KERNEL_SCALAR && p.family >= 0;
         return p;
     }

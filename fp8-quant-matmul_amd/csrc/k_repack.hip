@@ -1,7 +1,8 @@
 // Padding copies for shapes the MFMA kernels cannot take as they are.
 //
 // The tile kernels move 16-byte pieces of A's and B's columns, which start at k*M and k*N:
-// they need M and N to be multiples of 16 (and 16-byte aligned bases).  The reference asks
+// they need M and N to be multiples of 16 (and 16-byte aligned bases; some tiles have a form that
+// takes any M).  The reference asks
 // for multiples of 64 or 32 and reads out of bounds otherwise (/root/reference/mn_large.hip:16).
 // For any other shape the operands are copied into buffers whose leading dimension is rounded
 // up to 16 (new rows zero), the GEMM runs on the padded problem into a padded C, and C's

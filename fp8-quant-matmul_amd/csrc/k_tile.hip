@@ -35,6 +35,14 @@
 //     of being issued in one burst after the barrier (a burst queues up in the address unit
 //     and holds every wave back from its LDS reads).
 //
+//   * RAGGED: M is no multiple of 16, so A's k-rows start anywhere and 16-byte copies straight to LDS are out.  Four of
+//     the eight waves load A's pieces into registers from where they lie (a load takes any address; measured: no slower
+//     off the grid than on it) and write them to the ring a step before they are multiplied, two or three register
+//     sets ahead; the other four copy B and the scales as ever.  Each kind has a loop of its own, so that the compiler's
+//     waits count the loads of A alone.  A K block takes 0.05 - 0.1 us more than with copies throughout (128 x 128, 336 x
+//     4608 from the Infinity Cache: 0.53 -> 0.59 us), and the launch that copied A into padded rows is gone: 121 x 7168
+//     x 256 5.6 -> 3.8 us, 244 x 3072 x 1536 9.2 -> 7.0, 1021 x 512 x 2048 11.4 -> 7.7, 2204 x 512 x 7168 26.9 -> 21.2.
+//
 // Work decomposition: grid.x = tiles (XCD-aware order), grid.y = K splits.
 #include "tile_common.h"
 
@@ -42,7 +50,15 @@ namespace fp8gemm {
 
 namespace {
 
-template <int BM, int BN, int WM, int WN, int NS, bool SPLIT>
+// v >> (8 * by) as one 128-bit number, by < 16
+__device__ __forceinline__ v4i shift_right_bytes(v4i v, uint32_t by)
+{
+    const unsigned __int128 x = __builtin_bit_cast(unsigned __int128, v);
+    return __builtin_bit_cast(v4i, x >> (8 * by));
+}
+
+// RAGGED: M is no multiple of 16 (see the head of this file)
+template <int BM, int BN, int WM, int WN, int NS, bool SPLIT, bool RAGGED>
 __global__ void __launch_bounds__(NTHREADS)
 tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
                  const float* __restrict__ a_scale, const float* __restrict__ b_scale,
@@ -61,6 +77,15 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
     static_assert(TN <= 128, "a wave's n range touches at most two 128-wide scale blocks");
     static_assert(BM <= 256 && BN <= 256, "LDS rows hold at most 256 bytes");
     constexpr int RSA = S::RSA, RSB = S::RSB, NA = S::NA, NB = S::NB, NCOPY = S::NCOPY;
+    static_assert(!RAGGED || NS >= 3, "A's registers are written a step ahead of the multiply");
+    // RAGGED: waves 0 - 3 copy B and the scales, waves 4 - 7 load A, twice as much per wave each
+    constexpr int A_WAVE = 4, NAW = 2 * NA, NBW = RAGGED ? 2 * NB : NB;
+    constexpr int SETS = NS - 1, LEAD = SETS + 1;  // register sets of A, and K blocks that they run ahead
+    // A's registers are emptied behind the first MFMA of a block; with two sets only behind its last one, a step is short
+    // for the loads' trip (128x192, per K block from the Infinity Cache: 0.83 us early, 0.76 us late; 128x128 with three
+    // sets 0.59 and 0.61 us)
+    constexpr bool A_EARLY = SETS >= 3;
+    static_assert(!RAGGED || BM <= 64 * A_WAVE, "a wave that copies for every 64 rows of a_scale");
     constexpr int SCALE_WAVE = NCW == 4 ? 4 : 0;  // brings the a_scale slice: a wave that does not multiply, if there is one
 
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
@@ -99,7 +124,7 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
     // NA*w .. NA*w+NA-1 of the A tile and likewise of B.  A lane writes chunk position p of
     // row r and therefore fetches column chunk p ^ swizzle(r).  Chunks outside the tile or the
     // matrix get an out-of-range offset: the buffer load then writes zeros and reads nothing.
-    uint32_t voff_a[S::NVA], voff_b[S::NVB];
+    uint32_t voff_a[S::NVA], voff_b[S::NVB];  // RAGGED: voff_a is not used, voff_b by the waves that copy
 #pragma unroll
     for (int q = 0; q < S::NVA; ++q) {
         const int r = (NA * wave + q) * (1024 / RSA) + S::template copy_row<RSA>(lane);
@@ -109,15 +134,53 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
     }
 #pragma unroll
     for (int q = 0; q < S::NVB; ++q) {
-        const int r = (NB * wave + q) * (1024 / RSB) + S::template copy_row<RSB>(lane);
+        const int r = (NBW * wave + q) * (1024 / RSB) + S::template copy_row<RSB>(lane);
         const int cc = S::template copy_pos<RSB>(lane) ^ row_swizzle<RSB>(r & 7);
         const bool ok = (16 * cc < BN) && (n0 + 16 * cc < N);
         voff_b[q] = ok ? (uint32_t)(r * N + n0 + 16 * cc) : 0x80000000u;
     }
     const uint32_t a_bytes = (uint32_t)lda * (uint32_t)K, b_bytes = (uint32_t)N * (uint32_t)K;
     const uint32_t as_bytes = (uint32_t)nkb * (uint32_t)lda * 4u;
-    const uint32_t voff_s =
-        (4 * lane < BM && m0 + 4 * lane < M) ? (uint32_t)((m0 + 4 * lane) * 4) : 0x80000000u;
+    // a_scale: 16 bytes per lane by one wave; rows that do not start on the 16-byte grid by 4 bytes per lane and a wave
+    // for every 64 of them
+    const int scale_m = RAGGED ? m0 + 64 * wave + lane : m0 + 4 * lane;
+    const uint32_t voff_s = (RAGGED ? 64 * wave < BM : 4 * lane < BM) && scale_m < M ? (uint32_t)(scale_m * 4) : 0x80000000u;
+
+    // RAGGED: the 16 bytes per lane that a copy instruction would bring, by a load from wherever they lie; pieces
+    // without a row of the matrix bring the tile's first one instead
+    uint32_t off_a[NAW];
+    v4i set_a[SETS][NAW];
+    const bool loads_a = wave >= A_WAVE;
+    const int a_first = NAW * (wave - A_WAVE);  // first KiB of the A tile that the wave brings
+    if constexpr (RAGGED) {
+#pragma unroll
+        for (int q = 0; q < NAW; ++q) {
+            const int r = (a_first + q) * (1024 / RSA) + S::template copy_row<RSA>(lane);
+            const int cc = S::template copy_pos<RSA>(lane) ^ row_swizzle<RSA>(r & 7);
+            const bool ok = (16 * cc < BM) && (m0 + 16 * cc < M);
+            off_a[q] = (uint32_t)r * (uint32_t)M + (uint32_t)(ok ? m0 + 16 * cc : m0);
+        }
+    }
+    // Nothing beyond the matrix is read: a piece of its last row that would reach there is its last 16 bytes instead,
+    // shifted into place behind the wait.
+    const uint32_t last_piece = (uint32_t)KBLOCK * (uint32_t)M - 16u;  // where they start in the last K block
+    auto load_a = [&](v4i(&set)[NAW], int kb) __attribute__((always_inline)) {
+        const uint8_t* const block = a + (size_t)kb * KBLOCK * (uint32_t)M;
+        const uint32_t last = kb == nkb - 1 ? last_piece : 0xFFFFFFFFu;
+#pragma unroll
+        for (int q = 0; q < NAW; ++q)
+            __builtin_memcpy(&set[q], block + min(off_a[q], last), 16);
+    };
+    auto write_a = [&](auto inner_tag, v4i(&set)[NAW], int slot, int kb) __attribute__((always_inline)) {
+        if (!decltype(inner_tag)::value && kb == nkb - 1) {
+#pragma unroll
+            for (int q = 0; q < NAW; ++q)
+                set[q] = shift_right_bytes(set[q], off_a[q] > last_piece ? off_a[q] - last_piece : 0u);
+        }
+#pragma unroll
+        for (int q = 0; q < NAW; ++q)
+            *LDS_PTR(v4i, lds + (uint32_t)(slot * S::STAGE + (a_first + q) * 1024 + lane * 16)) = set[q];
+    };
 
     // copy instruction q (0..NCOPY-1) of K block kb into ring slot `slot`.  The three buffer
     // resources stay fixed; the K block's byte offset rides in the scalar offset operand.
@@ -126,20 +189,33 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
     const int sn = (N + KBLOCK - 1) / KBLOCK;
     const v4i rsrc_bs = make_rsrc_words(b_scale, (uint32_t)nkb * (uint32_t)sn * 4u);
     const uint32_t voff_sb = lane == 0 ? (uint32_t)((n0 >> 7) * 4) : 0x80000000u;  // staged: the tile is at most 128 wide
+    auto copy_b = [&](uint32_t stage, int kb, int q) __attribute__((always_inline)) {
+        lds_dma16(rsrc_b, voff_b[S::template voff_index<RSB>(q)], stage + S::MAT_A + (uint32_t)((NBW * wave + q) * 1024),
+                  (uint32_t)(kb * KBLOCK + S::template extra_rows<RSB>(q)) * (uint32_t)N);
+    };
     auto copy_step = [&](int slot, int kb, int q) __attribute__((always_inline)) {
         const uint32_t stage = lds_base + (uint32_t)(slot * S::STAGE);
         if (q < NA) {
             lds_dma16(rsrc_a, voff_a[S::template voff_index<RSA>(q)], stage + (uint32_t)((NA * wave + q) * 1024),
                       (uint32_t)(kb * KBLOCK + S::template extra_rows<RSA>(q)) * (uint32_t)lda);
         } else if (q < NA + NB) {
-            lds_dma16(rsrc_b, voff_b[S::template voff_index<RSB>(q - NA)],
-                      stage + S::MAT_A + (uint32_t)((NB * wave + (q - NA)) * 1024),
-                      (uint32_t)(kb * KBLOCK + S::template extra_rows<RSB>(q - NA)) * (uint32_t)N);
+            copy_b(stage, kb, q - NA);
         } else if (wave == SCALE_WAVE) {
             lds_dma16(rsrc_s, voff_s, stage + S::SCALE_OFF, (uint32_t)kb * (uint32_t)lda * 4u);
         } else if (S::SB_STAGED && wave == SCALE_WAVE + 1) {
             lds_dma4(rsrc_bs, voff_sb, stage + S::SB_OFF, (uint32_t)kb * (uint32_t)sn * 4u);
         }
+    };
+    // RAGGED: all copies of a wave at once
+    auto copy_all = [&](int slot, int kb) __attribute__((always_inline)) {
+        const uint32_t stage = lds_base + (uint32_t)(slot * S::STAGE);
+#pragma unroll
+        for (int q = 0; q < NBW; ++q)
+            copy_b(stage, kb, q);
+        if (64 * wave < BM)
+            lds_dma4(rsrc_s, voff_s, stage + S::SCALE_OFF + (uint32_t)(256 * wave), (uint32_t)kb * (uint32_t)M * 4u);
+        else if (S::SB_STAGED && wave == A_WAVE - 1)
+            lds_dma4(rsrc_bs, voff_sb, stage + S::SB_OFF, (uint32_t)kb * (uint32_t)sn * 4u);
     };
 
     // ---- transposing LDS reads.  Lane l = 16*g + i feeds MFMA row/column (l & 31) and k half
@@ -194,11 +270,15 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
 #pragma unroll
     for (int p = 0; p < NS - 1; ++p)
         if (kb0 + p < kb1) {
+            if constexpr (RAGGED) {
+                if (!loads_a)
+                    copy_all(p, kb0 + p);
+            } else {
 #pragma unroll
-            for (int q = 0; q < NCOPY; ++q)
-                copy_step(p, kb0 + p, q);
+                for (int q = 0; q < NCOPY; ++q)
+                    copy_step(p, kb0 + p, q);
+            }
         }
-
     int slot = 0;             // ring slot of block kb
     int slot_fill = NS - 1;   // ring slot that block kb + NS - 1 goes into (= slot of kb - 1)
 
@@ -211,29 +291,50 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
 
     // One K block.  MORE = block kb+NS-1 exists and is copied here; two instantiations keep the
     // steady-state body free of branches.
-    auto k_block = [&](auto more_tag, int kb) {
-        constexpr bool more = decltype(more_tag)::value;
+    auto k_block = [&](auto more_tag, auto loads_tag, auto set_tag, int kb) __attribute__((always_inline)) {
+        constexpr bool loads_a = decltype(loads_tag)::value;
+        constexpr bool steady = decltype(more_tag)::value;
+        const bool more = steady || (RAGGED && kb + NS - 1 < kb1);
+        // RAGGED: A of the next block into its slot, and its registers filled again
+        auto next_a = [&]() __attribute__((always_inline)) {
+            if constexpr (loads_a) {
+                constexpr int set = (decltype(set_tag)::value + 1) % SETS;
+                if (steady || kb + 1 < kb1)
+                    write_a(more_tag, set_a[set], slot + 1 == NS ? 0 : slot + 1, kb + 1);  // steady: not the last block
+                if (steady || kb + LEAD < kb1)
+                    load_a(set_a[set], kb + LEAD);
+            }
+        };
         // Block kb has landed once at most the copies of the younger blocks in flight are
         // outstanding (loads complete in order).  NCOPY - 1 per block is exact for waves 1..7
         // and one short for wave 0, which then waits for one more copy than it must.
-        if (more) {
-            wait_vmcnt<(NS - 2) * (NCOPY - 1)>();
+        // RAGGED: the waves that load A have written it, the others' copies are B's, two of which bring one more.
+        constexpr int PER_BLOCK = RAGGED ? NBW : NCOPY - 1;
+        if (loads_a) {
+        } else if (steady) {
+            wait_vmcnt<(NS - 2) * PER_BLOCK>();
         } else {
             const int younger = (kb1 - 1 - kb < NS - 2) ? (kb1 - 1 - kb) : (NS - 2);
             if (NS >= 4 && younger >= 2)
-                wait_vmcnt<2 * (NCOPY - 1)>();
+                wait_vmcnt<2 * PER_BLOCK>();
             else if (NS >= 3 && younger >= 1)
-                wait_vmcnt<NCOPY - 1>();
+                wait_vmcnt<PER_BLOCK>();
             else
                 wait_vmcnt<0>();
         }
         __syncthreads();  // everyone's copies of block kb landed; slot_fill is no longer read
         if (!compute) {  // copy-only wave
             if (more) {
+                if constexpr (RAGGED) {
+                    if (!loads_a)
+                        copy_all(slot_fill, kb + NS - 1);
+                } else {
 #pragma unroll
-                for (int q = 0; q < NCOPY; ++q)
-                    copy_step(slot_fill, kb + NS - 1, q);
+                    for (int q = 0; q < NCOPY; ++q)
+                        copy_step(slot_fill, kb + NS - 1, q);
+                }
             }
+            next_a();
             slot_fill = slot;
             slot = (slot + 1 == NS) ? 0 : slot + 1;
             return;
@@ -262,6 +363,14 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
         constexpr int PER_MFMA = (NCOPY + N_MFMA - 1) / N_MFMA;  // copies behind each MFMA
         int cq = 0;
         auto copy_slot = [&](int n) {
+            if (RAGGED) {
+                if (cq == 0 && loads_a && A_EARLY)
+                    next_a();
+                if (cq == 0 && !loads_a && more)
+                    copy_all(slot_fill, kb + NS - 1);
+                cq = NCOPY;
+                return;
+            }
 #pragma unroll
             for (int u = 0; u < NCOPY; ++u)
                 if (u < n && cq < NCOPY) {
@@ -309,15 +418,51 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
             }
         }
         copy_slot(NCOPY);  // whatever is left (tiles with few MFMAs per K block)
+        if (!A_EARLY)
+            next_a();
 
         slot_fill = slot;
         slot = (slot + 1 == NS) ? 0 : slot + 1;
     };
     int kb = kb0;
-    for (; kb + NS - 1 < kb1; ++kb)
-        k_block(std::true_type{}, kb);
-    for (; kb < kb1; ++kb)
-        k_block(std::false_type{}, kb);
+    using Set0 = std::integral_constant<int, 0>;
+    if constexpr (RAGGED) {
+        // a loop for either kind of wave: with the loads of A in a branch of a common one, the compiler has to expect that
+        // an earlier block's were not followed by any, and waits for all of them
+        auto blocks = [&](auto loads_tag) __attribute__((always_inline)) {
+            if constexpr (decltype(loads_tag)::value) {  // A: block 0 into its slot, the next ones on their way
+#pragma unroll
+                for (int p = 0; p < SETS; ++p)
+                    if (kb0 + p < kb1)
+                        load_a(set_a[p], kb0 + p);
+                write_a(std::false_type{}, set_a[0], 0, kb0);
+                if (kb0 + SETS < kb1)
+                    load_a(set_a[0], kb0 + SETS);
+            }
+            auto round = [&](auto more_tag, int at) __attribute__((always_inline)) {  // the sets are numbered at compile time
+                constexpr bool steady = decltype(more_tag)::value;
+                k_block(more_tag, loads_tag, Set0{}, at);
+                if (steady || at + 1 < kb1)
+                    k_block(more_tag, loads_tag, std::integral_constant<int, 1>{}, at + 1);
+                if (SETS == 3 && (steady || at + 2 < kb1))
+                    k_block(more_tag, loads_tag, std::integral_constant<int, SETS - 1>{}, at + 2);
+            };
+            static_assert(SETS == 2 || SETS == 3, "unrolled above");
+            for (; kb + SETS - 1 + LEAD < kb1; kb += SETS)
+                round(std::true_type{}, kb);
+            for (; kb < kb1; kb += SETS)
+                round(std::false_type{}, kb);
+        };
+        if (loads_a)
+            blocks(std::true_type{});
+        else
+            blocks(std::false_type{});
+    } else {
+        for (; kb + NS - 1 < kb1; ++kb)
+            k_block(std::true_type{}, std::false_type{}, Set0{}, kb);
+        for (; kb < kb1; ++kb)
+            k_block(std::false_type{}, std::false_type{}, Set0{}, kb);
+    }
 
     // ---- K splits added inside the kernel (mailbox != nullptr).  grid.x is a multiple of 8, so the
     // workgroups of one tile (same blockIdx.x) have linear ids that agree modulo 8 and share an XCD: what
@@ -597,8 +742,11 @@ int choose_group_m(int tiles_m, int tiles_n, int bm, int bn)
     return best_g;
 }
 
-template <int BM, int BN, int WM, int WN, int NS>
-hipError_t launch_variant(const GemmArgs& g, int ksplit, float* partial, float* mailbox, hipStream_t s)
+// the tile shapes that have a form for row counts off the 16-byte grid
+constexpr bool tile_takes_ragged_rows(int bm, int ns) { return bm <= 128 && ns >= 3; }
+
+template <int BM, int BN, int WM, int WN, int NS, bool RAGGED>
+hipError_t launch_typed(const GemmArgs& g, int ksplit, float* partial, float* mailbox, hipStream_t s)
 {
     using S = TileShape<BM, BN, WM, WN, NS>;
     constexpr int LDS_TOTAL = S::LDS_BYTES;
@@ -612,18 +760,30 @@ hipError_t launch_variant(const GemmArgs& g, int ksplit, float* partial, float* 
         if (mailbox && (size_t)tiles * (ksplit - 1) * BM * BN * 4 > SPLIT_MAILBOX_BYTES)
             return hipErrorInvalidValue;
         dim3 grid(mailbox ? (tiles + 7) & ~7 : tiles, ksplit);
-        auto kern = tile_gemm_kernel<BM, BN, WM, WN, NS, true>;
+        auto kern = tile_gemm_kernel<BM, BN, WM, WN, NS, true, RAGGED>;
         FP8GEMM_ALLOW_LDS(kern, LDS_TOTAL);
         hipLaunchKernelGGL(kern, grid, dim3(NTHREADS), LDS_TOTAL, s, g.a, g.b, g.a_scale, g.b_scale, g.c, partial,
                            mailbox, g.m, leading_dim(g), g.n, g.k, tiles_m, tiles_n, kb_per_split, group_m);
     } else {
-        auto kern = tile_gemm_kernel<BM, BN, WM, WN, NS, false>;
+        auto kern = tile_gemm_kernel<BM, BN, WM, WN, NS, false, RAGGED>;
         FP8GEMM_ALLOW_LDS(kern, LDS_TOTAL);
         hipLaunchKernelGGL(kern, dim3(tiles, 1), dim3(NTHREADS), LDS_TOTAL, s, g.a, g.b, g.a_scale, g.b_scale, g.c,
                            partial, static_cast<float*>(nullptr), g.m, leading_dim(g), g.n, g.k, tiles_m,
                            tiles_n, kb_per_split, group_m);
     }
     return hipGetLastError();
+}
+
+template <int BM, int BN, int WM, int WN, int NS>
+hipError_t launch_variant(const GemmArgs& g, int ksplit, float* partial, float* mailbox, hipStream_t s)
+{
+    if (leading_dim(g) % 16 == 0)
+        return launch_typed<BM, BN, WM, WN, NS, false>(g, ksplit, partial, mailbox, s);
+    if constexpr (tile_takes_ragged_rows(BM, NS)) {
+        if (leading_dim(g) == g.m && g.m >= 16)
+            return launch_typed<BM, BN, WM, WN, NS, true>(g, ksplit, partial, mailbox, s);
+    }
+    return hipErrorInvalidValue;
 }
 
 }  // namespace
@@ -636,6 +796,14 @@ bool tile_supports(const GemmArgs& g)
            (reinterpret_cast<uintptr_t>(g.a) % 16 == 0) &&
            (reinterpret_cast<uintptr_t>(g.b) % 16 == 0) &&
            (reinterpret_cast<uintptr_t>(g.a_scale) % 16 == 0) &&
+           (reinterpret_cast<uintptr_t>(g.c) % 16 == 0);
+}
+
+bool tile_ragged_supports(const GemmArgs& g, int variant)
+{
+    return (variant == TILE_64x64 || variant == TILE_128x128 || variant == TILE_128x192) && g.m >= 16 && g.m % 16 != 0 &&
+           leading_dim(g) == g.m && g.n % 16 == 0 && (reinterpret_cast<uintptr_t>(g.a) % 16 == 0) &&
+           (reinterpret_cast<uintptr_t>(g.b) % 16 == 0) && (reinterpret_cast<uintptr_t>(g.a_scale) % 16 == 0) &&
            (reinterpret_cast<uintptr_t>(g.c) % 16 == 0);
 }
 

@@ -58,6 +58,8 @@ constexpr size_t SPLIT_MAILBOX_BYTES = (size_t)16 << 20;
 enum TileVariant { TILE_256x192 = 0, TILE_256x128 = 1, TILE_128x128 = 2, TILE_128x192 = 3,
                    TILE_64x64 = 4, TILE_256x192_W4 = 5, TILE_256x256 = 6, TILE_VARIANT_COUNT };
 bool tile_supports(const GemmArgs& g);
+// row counts off the 16-byte grid, taken as they are (launch_tile, plain form)
+bool tile_ragged_supports(const GemmArgs& g, int variant);
 const char* tile_variant_name(int variant);
 void tile_variant_dims(int variant, int* bm, int* bn);
 size_t tile_mailbox_bytes(const GemmArgs& g, int variant, int ksplit);

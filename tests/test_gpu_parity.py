@@ -212,6 +212,50 @@ def test_tile_kernel_split_k(pkg, variant, ksplit, m, n, k):
         assert np.array_equal(got, inside), f"{fname} run {rep}: differs from the reduction kernel's result"
 
 
+@pytest.mark.parametrize("variant,ksplit,m,n,k", [
+    # tiles that take them as they are: every number of K blocks around the register sets and the ring, one to fifteen
+    # rows beyond the grid, a last tile of one row, one tile and several, both ways of adding splits
+    (4, 1, 81, 64, 128), (4, 1, 65, 80, 256), (4, 1, 127, 576, 384), (4, 1, 66, 128, 512), (4, 1, 190, 64, 640),
+    (4, 3, 333, 208, 1920), (4, 2, 115, 64, 1664), (4, 5, 100, 128, 7168),
+    (2, 1, 131, 144, 128), (2, 1, 129, 128, 256), (2, 1, 255, 272, 384), (2, 1, 500, 128, 512), (2, 1, 77, 128, 896),
+    (2, 2, 333, 576, 1536), (2, 3, 389, 144, 2944), (2, 5, 257, 384, 3200),
+    (3, 1, 125, 208, 128), (3, 1, 129, 192, 256), (3, 1, 250, 400, 384), (3, 1, 136, 192, 640), (3, 2, 340, 592, 1792),
+    # padded copies: a few pieces, and from 2^18 pieces on four to a thread
+    (0, 1, 35, 192, 256), (0, 1, 2050, 192, 2048), (1, 2, 1031, 128, 4096),
+])
+def test_tile_kernel_with_rows_off_the_grid(pkg, variant, ksplit, m, n, k):
+    """bit for bit the same plan's result on operands padded with zeros, whatever lies behind a's last byte"""
+    import torch
+    a, b, sa, sb = oracle.make_inputs(m, n, k, 900 + m + k)
+    m16 = (m + 15) // 16 * 16
+    pa, psa = np.zeros((k, m16), a.dtype), np.zeros((k // 128, m16), sa.dtype)
+    pa[:, :m], psa[:, :m] = a.reshape(k, m), sa.reshape(k // 128, m)
+    da, dsa, dpa, dpsa, db, dsb = _dev(np.concatenate([a.reshape(-1), np.full(64, 0x7F, a.dtype)]), sa, pa, psa, b, sb)
+    got = torch.full((m + 1, n), 0x7FC1, dtype=torch.int32, device="cuda").to(torch.int16)  # one guard row
+    want = torch.zeros((m16, n), dtype=torch.int16, device="cuda")
+    st = torch.cuda.current_stream().cuda_stream
+    for fused in ([0, 1] if ksplit > 1 and variant in (2, 4) else [-1]):
+        _say(f"[gpu case] rows off the grid: variant={variant} ksplit={ksplit} {m}x{n}x{k} fused={fused}")
+        pkg.force_config(variant, ksplit)
+        pkg.set_persistent(0)
+        pkg.set_fused_reduction(fused)
+        try:
+            pkg.gemm(dpa, db, dpsa, dsb, want, m16, n, k, st)
+            aligned = pkg.last_kernel()
+            pkg.gemm(da, db, dsa, dsb, got, m, n, k, st)
+            torch.cuda.synchronize()
+            name = pkg.last_kernel()
+        finally:
+            pkg.force_config(-1, 0)
+            pkg.set_persistent(-1)
+            pkg.set_fused_reduction(-1)
+        assert name == ("" if variant in (2, 3, 4) else "padded_") + aligned, (name, aligned)
+        assert torch.equal(got[:m], want[:m]), name
+        assert (got[m].cpu().numpy().view(np.uint16) == 0x7FC1).all(), "rows beyond m written"
+    _assert_every_element(got[:m].cpu().numpy().view(np.uint16), a, b, sa, sb, m, n, k, name)
+    pkg.release()
+
+
 @pytest.mark.parametrize("m,n,k", [(32, 7168, 2048), (16, 96, 512), (32, 576, 7168), (32, 32, 128),
                                    (16, 1040, 384), (32, 4096, 256)])
 def test_skinny_kernel(pkg, m, n, k):
