@@ -330,6 +330,26 @@ Plan make_plan(const GemmArgs& g, const Config& cfg)
     return slot.plan;
 }
 
+// Rows without 16-byte alignment under automatic dispatch: the plan of the problem padded to the grid, on copies of the
+// operands that need one (their one or two extra launches cost about 5 us; the scalar kernel, one dependent load after the
+// other, takes 30 us for K = 128 already) or, where only m is off the grid, without any if the plan's tiles take that.  The
+// scalar kernel if padding pushes an operand past the size limit.
+Plan off_grid_plan(const GemmArgs& g, const Config& cfg)
+{
+    const long long m16 = (g.m + 15) & ~15, n16 = (g.n + 15) & ~15, lim = 0x7FFFFFFFll;
+    if (m16 * g.k > lim || n16 * g.k > lim || m16 * n16 > lim)
+        return Plan{FP8GEMM_KERNEL_SCALAR, 0, 1};
+    const uint8_t* const al8 = reinterpret_cast<const uint8_t*>(uintptr_t(4096));
+    GemmArgs gp{al8, al8, reinterpret_cast<const float*>(uintptr_t(4096)), g.b_scale,
+                reinterpret_cast<uint16_t*>(uintptr_t(4096)), (int)m16, (int)n16, g.k};
+    Plan p = make_plan(gp, cfg);
+    const bool tiles = p.family == FP8GEMM_KERNEL_LARGE || p.family == FP8GEMM_KERNEL_SPLITK;
+    if (tiles && !p.persistent && tile_ragged_supports(g, p.variant) && tile_ragged_pays(g, p.variant, p.ksplit))
+        return p;
+    p.padded = p.family != FP8GEMM_KERNEL_SCALAR && p.family >= 0;
+    return p;
+}
+
 Plan compute_plan(const GemmArgs& g, const Config& cfg)
 {
     const int selected = cfg.selected;
@@ -399,11 +419,21 @@ Plan compute_plan(const GemmArgs& g, const Config& cfg)
         // With more than 32 rows the 64x64 tile plans that add their K splits in the kernel are ahead of the wide
         // strips on 22 of 24 shapes (M = 48, 64; same N and K; from HBM 6.2-15 us against 7.5-16 us): the
         // four-row-tile form is there for grouped launches and runs single problems only when asked for by name.
-        // ... except where N x K is large (N = 7168, K >= 4096: 12.2 - 17.4 us against 13.7 - 20.4 us), and for row
-        // counts off the 16-byte grid, which the strips take as they are while the tiles need padded copies
-        // (M = 33 ... 63 on the same 12 shapes: 6.8 - 16.9 us against 10.8 - 23.8 us).
-        if (!by_name && g.m > 32 && g.m % 16 == 0 && !(g.n >= 6144 && (long long)g.n * g.k >= 28000000ll))
+        // ... except where N x K is large (N = 7168, K >= 4096: 12.2 - 17.4 us against 13.7 - 20.4 us).
+        const long long b_bytes = (long long)g.n * g.k;
+        if (!by_name && g.m > 32 && g.m % 16 == 0 && !(g.n >= 6144 && b_bytes >= 28000000ll))
             wide_us = 1e300;
+        // Row counts off the 16-byte grid, which the strips take as they are: tiles that do so too over a B of up to 16 MB
+        // (66 random shapes of 33 ... 63 rows, N = 288 ... 12912, K = 256 ... 7680: 19 % faster from the Infinity Cache, 13 %
+        // from HBM on average, worst -4 %).  Over 16.5 ... 23.5 MB (8 shapes) they are 7 - 35 % ahead with B in the
+        // Infinity Cache and behind from HBM, where such weights are, by 4 % on average and 21 % at worst.  No tiles that
+        // need padded copies (12 shapes: 6.8 - 16.9 us against 10.8 - 23.8 us).
+        if (!by_name && g.m > 32 && g.m % 16 != 0 && b_bytes < 16000000ll && cfg.force_variant < 0 &&
+            cfg.force_ksplit <= 0 && cfg.fused_ok) {
+            const Plan tiles = off_grid_plan(g, cfg);
+            if (!tiles.padded && (tiles.family == FP8GEMM_KERNEL_LARGE || tiles.family == FP8GEMM_KERNEL_SPLITK))
+                return tiles;
+        }
 
         if (!by_name && cfg.force_variant < 0 && cfg.force_ksplit <= 0 && wide_us < 1e300 && cfg.fused_ok)
             return wide;
@@ -429,21 +459,7 @@ Plan compute_plan(const GemmArgs& g, const Config& cfg)
             p.family = -1;
             return p;
         }
-        // rows without 16-byte alignment: the padded problem (its one or two extra launches cost
-        // about 5 us; the scalar kernel, one dependent load after the other, takes 30 us for
-        // K = 128 already), unless padding pushes an operand past the size limit
-        const long long m16 = (g.m + 15) & ~15, n16 = (g.n + 15) & ~15, lim = 0x7FFFFFFFll;
-        if (m16 * g.k > lim || n16 * g.k > lim || m16 * n16 > lim)
-            return p;
-        const uint8_t* const al8 = reinterpret_cast<const uint8_t*>(uintptr_t(4096));
-        GemmArgs gp{al8, al8, reinterpret_cast<const float*>(uintptr_t(4096)), g.b_scale,
-                    reinterpret_cast<uint16_t*>(uintptr_t(4096)), (int)m16, (int)n16, g.k};
-        p = make_plan(gp, cfg);
-        const bool tiles = p.family == FP8GEMM_KERNEL_LARGE || p.family == FP8GEMM_KERNEL_SPLITK;
-        if (tiles && !p.persistent && tile_ragged_supports(g, p.variant) && tile_ragged_pays(g, p.variant, p.ksplit))
-            return p;  // rows off the 16-byte grid as they are
-        p.padded = p.family != FP8GEMM_KERNEL_SCALAR && p.family >= 0;
-        return p;
+        return off_grid_plan(g, cfg);
     }
     const int fv = cfg.force_variant, fk = cfg.force_ksplit;
     const int nkb = g.k / 128;

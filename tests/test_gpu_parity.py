@@ -216,7 +216,7 @@ def test_tile_kernel_split_k(pkg, variant, ksplit, m, n, k):
     # tiles that take them as they are: every number of K blocks around the register sets and the ring, one to fifteen
     # rows beyond the grid, a last tile of one row, one tile and several, both ways of adding splits
     (4, 1, 81, 64, 128), (4, 1, 65, 80, 256), (4, 1, 127, 576, 384), (4, 1, 66, 128, 512), (4, 1, 190, 64, 640),
-    (4, 3, 333, 208, 1920), (4, 2, 115, 64, 1664), (4, 5, 100, 128, 7168),
+    (4, 1, 33, 320, 512), (4, 7, 63, 576, 7168), (4, 3, 333, 208, 1920), (4, 2, 115, 64, 1664), (4, 5, 100, 128, 7168),
     (2, 1, 131, 144, 128), (2, 1, 129, 128, 256), (2, 1, 255, 272, 384), (2, 1, 500, 128, 512), (2, 1, 77, 128, 896),
     (2, 2, 333, 576, 1536), (2, 3, 389, 144, 2944), (2, 5, 257, 384, 3200),
     (3, 1, 125, 208, 128), (3, 1, 129, 192, 256), (3, 1, 250, 400, 384), (3, 1, 136, 192, 640), (3, 2, 340, 592, 1792),
