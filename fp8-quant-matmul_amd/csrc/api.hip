@@ -431,7 +431,8 @@ Plan compute_plan(const GemmArgs& g, const Config& cfg)
         if (!by_name && g.m > 32 && g.m % 16 != 0 && b_bytes < 16000000ll && cfg.force_variant < 0 &&
             cfg.force_ksplit <= 0 && cfg.fused_ok) {
             const Plan tiles = off_grid_plan(g, cfg);
-            if (!tiles.padded && (tiles.family == FP8GEMM_KERNEL_LARGE || tiles.family == FP8GEMM_KERNEL_SPLITK))
+            const bool header_only = tiles.ksplit == 1 || tiles.fused;  // as the strips: no partial sums in the workspace
+            if (!tiles.padded && header_only && (tiles.family == FP8GEMM_KERNEL_LARGE || tiles.family == FP8GEMM_KERNEL_SPLITK))
                 return tiles;
         }
 

@@ -71,7 +71,8 @@ extern "C" {
  * the library copies the operands concerned into zero-padded buffers in its workspace, runs
  * there and copies c's m x n corner out (plans named "padded_...": one extra launch for the copies and
  * one for c's corner, about 2 bytes of extra traffic per operand byte).  The decode kernel ("decode128_kN",
- * chosen for m <= 32) takes any m as it is: a decode batch of 1 ... 15 rows needs no copy.  The reference
+ * chosen for m <= 32) takes any m as it is: a decode batch of 1 ... 15 rows needs no copy; so do the
+ * 64x64, 128x128 and 128x192 tiles where a problem does not fill the persistent form.  The reference
  * requires M, N % 64 (32) == 0
  * and reads out of bounds otherwise (mn_large.hip:16). */
 int fp8_block_gemm(const void* a, const void* b, const float* a_scale, const float* b_scale,
