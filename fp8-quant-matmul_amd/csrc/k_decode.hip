@@ -39,7 +39,8 @@
 // decode step), whose strips form one list of work items.
 //
 // Variants of the same body (template arguments): a row count off the 16-byte grid (RAGGED: A's packed K-block
-// slabs are copied whole and spread into padded rows in the LDS); strips of 256 columns (NB = 2: two
+// slabs are copied whole and spread into padded rows in the LDS; PACKED, multiples of 8: copied whole and read as they
+// are); strips of 256 columns (NB = 2: two
 // 128-column halves per stage; 256 contiguous bytes of a k-row come 10 % faster from HBM than 128, at half
 // the workgroups per split); one copy of the K loop per number of row tiles, so that no branch surrounds its
 // LDS operations.  The streaming form (decode_stream_body) is for launches with more strips than the device
@@ -74,6 +75,11 @@ constexpr unsigned long long SPIN_LIMIT_TICKS = 100000000ull;  // one second of 
 // RAGGED = the row count is not a multiple of 16, so that k-rows of A do not start on 16-byte boundaries: a stage
 // then also holds the K block's slab of A as it lies in memory, [128][M] bytes packed -- which does start on a
 // 16-byte boundary, 128 * M * kb bytes into A -- and the threads spread it into the padded rows the reads expect.
+// PACKED (decode_body) = the row count is a multiple of 8 but not of 16: the slab is copied as it lies, to where A's
+// padded rows would be, and the transposing reads, which want 8-byte alignment, take it from there at M bytes a
+// k-row.  Nothing is spread: no second trip through the LDS, no slab to ask for a turn ahead, and the deep ring with
+// four row tiles too.  Bound as on the grid; against the spreading form, from HBM: 8 x 7168 x 2048 5.91 -> 5.28 us,
+// 24 x 7168 x 2048 6.99 -> 6.43, 8 x 1536 x 7168 6.92 -> 5.89, 56 x 7168 x 7168 16.9 -> 15.2, 56 x 28672 x 2304 17.1 -> 14.5.
 // NB = 128-column halves of a strip (1; 2 in the streaming form of wide problems: 256 contiguous bytes of every
 // k-row instead of 128, which the memory system serves 10 % faster, and A's fragments used twice).  Each half is a
 // [128][128] byte matrix of its own in the stage, laid out and swizzled alike.
@@ -104,6 +110,10 @@ __device__ __forceinline__ void ds_wait_vmcnt()
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
+// how the k-rows of A lie in a stage: padded, copied there row by row (rows on the 16-byte grid); padded, spread from
+// the packed slab by the threads; packed as in memory
+enum class ARows { GRID, SPREAD, PACKED };
+
 // one problem as the kernel sees it
 struct DecodeProblem {
     const uint8_t* a;
@@ -119,10 +129,12 @@ struct DecodeProblem {
 // blockIdx.y = split: gridDim.x is a multiple of 8, so their linear ids agree modulo 8 and they share an XCD.
 // TILES = the number of 16-row tiles when the launch knows it (a single problem: the count is then a constant
 // in the epilogue as well), 0 = read from the problem (grouped launches).
-template <int MT, bool GROUPED, int DS_NS, bool RAGGED, int TILES, int NB, int STEP>
+template <int MT, bool GROUPED, int DS_NS, ARows FORM, int TILES, int NB, int STEP>
 __device__ __forceinline__ void decode_body(const DecodeProblem& one, const GroupTable* tab, float* mailbox, int N, int K,
                                             int strips, int units, int ksplit, int kb_per_split)
 {
+    constexpr bool RAGGED = FORM == ARows::SPREAD, PACKED = FORM == ARows::PACKED;
+    static_assert(!(GROUPED && PACKED), "the groups of a launch have row counts of their own");
     using S = DecodeShape<MT, DS_NS, RAGGED, NB>;
     constexpr int BN = DS_BN * NB;  // columns of a strip
     // Two stages to a barrier where the ring is deep enough.  A stage at a time, wait, barrier, LDS reads, MFMAs and fold
@@ -177,7 +189,7 @@ __device__ __forceinline__ void decode_body(const DecodeProblem& one, const Grou
     const uint32_t voff_sa = lane < lda ? (uint32_t)(lane * 4) : 0x80000000u;
     const uint32_t voff_sb = lane < NB && strip * NB + lane < sn ? (uint32_t)((strip * NB + lane) * 4) : 0x80000000u;
     uint32_t voff_a;
-    if (RAGGED) {
+    if (RAGGED || PACKED) {
         // the K block's slab of A, 128 * M contiguous bytes, in 16-byte pieces: piece 64 * wave + lane
         const int piece = 64 * wave + lane;
         voff_a = 16 * piece < KBLOCK * lda ? (uint32_t)(16 * piece) : 0x80000000u;
@@ -275,8 +287,11 @@ __device__ __forceinline__ void decode_body(const DecodeProblem& one, const Grou
     const int g4 = lane >> 4, i16 = lane & 15;
     const uint32_t addr_b = (uint32_t)((8 * g4 + (i16 >> 1)) * 128 + ((wave ^ ((4 * g4 + (i16 >> 2)) & 7)) * 16) +
                                        (i16 & 1) * 8);
-    const uint32_t addr_a = (uint32_t)(S::MAT_B + (8 * g4 + (i16 >> 1)) * S::RSA + (i16 & 1) * 8);
-    const int swz_a = MT == 2 ? (g4 & 1) : ((2 * g4 + (i16 >> 3)) & 3);
+    // PACKED: k-rows of lda bytes without a swizzle; what a read of the last row tile takes from beyond a row (the next
+    // one's first 8 bytes, or 8 bytes behind the slab) belongs to rows of C that do not exist.
+    const int rsa = PACKED ? lda : S::RSA;
+    const uint32_t addr_a = (uint32_t)(S::MAT_B + (8 * g4 + (i16 >> 1)) * rsa + (i16 & 1) * 8);
+    const int swz_a = PACKED ? 0 : MT == 2 ? (g4 & 1) : ((2 * g4 + (i16 >> 3)) & 3);
     auto read_frag = [&](uint32_t addr, int step) __attribute__((always_inline)) -> v8i {
         v2i r0 = __builtin_amdgcn_ds_read_tr8_b64_v2i32(LDS_PTR(v2i, lds + addr));
         v2i r1 = __builtin_amdgcn_ds_read_tr8_b64_v2i32(LDS_PTR(v2i, lds + addr + step));
@@ -352,7 +367,7 @@ __device__ __forceinline__ void decode_body(const DecodeProblem& one, const Grou
 #pragma unroll
                 for (int i = 0; i < T; ++i) {
                     sa[u][i] = *LDS_PTR(float, lds + so + S::SA_OFF + (16 * i + i16) * 4);
-                    fa[u][i] = read_frag(so + addr_a + (uint32_t)((i ^ swz_a) * 16), 32 * S::RSA);
+                    fa[u][i] = read_frag(so + addr_a + (uint32_t)((i ^ swz_a) * 16), 32 * rsa);
                 }
             }
             // the spread words are written behind the turn's reads: the LDS works in order, a write among the
@@ -514,7 +529,7 @@ __device__ __forceinline__ void decode_body(const DecodeProblem& one, const Grou
     store_c(sum);
 }
 
-template <int MT, int DS_NS, bool RAGGED, int TILES, int NB, int STEP>
+template <int MT, int DS_NS, ARows FORM, int TILES, int NB, int STEP>
 __global__ void __launch_bounds__(DS_THREADS)
 decode_strip_kernel(const uint8_t* __restrict__ b, const uint8_t* __restrict__ a, int N, int K, int M, int lda,
                     int kb_per_split, int strips, const float* __restrict__ a_scale, const float* __restrict__ b_scale,
@@ -522,7 +537,7 @@ decode_strip_kernel(const uint8_t* __restrict__ b, const uint8_t* __restrict__ a
 {
     // (the first 14 words of the arguments are in registers when a wave starts: what the copies need comes first)
     const DecodeProblem one{a, b, a_scale, b_scale, c, M, lda};
-    decode_body<MT, false, DS_NS, RAGGED, TILES, NB, STEP>(one, nullptr, mailbox, N, K, strips, strips, ksplit, kb_per_split);
+    decode_body<MT, false, DS_NS, FORM, TILES, NB, STEP>(one, nullptr, mailbox, N, K, strips, strips, ksplit, kb_per_split);
 }
 
 template <int MT, int DS_NS, bool RAGGED, int STEP>
@@ -530,7 +545,8 @@ __global__ void __launch_bounds__(DS_THREADS)
 decode_strip_grouped_kernel(const GroupTable tab, float* mailbox, int N, int K, int strips, int ksplit, int kb_per_split)
 {
     const DecodeProblem none{nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0};
-    decode_body<MT, true, DS_NS, RAGGED, 0, 1, STEP>(none, &tab, mailbox, N, K, strips, strips * tab.groups, ksplit, kb_per_split);
+    constexpr ARows FORM = RAGGED ? ARows::SPREAD : ARows::GRID;
+    decode_body<MT, true, DS_NS, FORM, 0, 1, STEP>(none, &tab, mailbox, N, K, strips, strips * tab.groups, ksplit, kb_per_split);
 }
 
 // The streaming form, for a single problem without a K split whose strips outnumber the workgroups the
@@ -801,7 +817,7 @@ struct StreamShape {
     static constexpr int MT = MT_, NS = NS_, NB = NB_;
 };
 constexpr int STREAM_WORKGROUPS = 256;
-constexpr int SLAB_FORM_MIN_KBLOCKS = 28;  // K blocks per workgroup from which up to 32 rows on the grid take the slab-spreading instances too
+constexpr int SLAB_FORM_MIN_KBLOCKS = 28;  // K blocks per workgroup from which up to 32 rows on the grid, and all on an 8-byte grid, take the slab-spreading instances too
 
 // Two stages to a barrier (STEP = 2 of decode_body): for launches of one round of workgroups with short K ranges, whose
 // time is the chain of one K block after the other -- from the Infinity Cache / from HBM, against one stage to a
@@ -822,7 +838,8 @@ inline bool shallow_ring_pays(long workgroups, int kb_per_split) { return workgr
 
 }  // namespace
 
-// any 1 <= m <= 64: a row count off the 16-byte grid runs the kernels that spread A's packed slabs in the LDS;
+// any 1 <= m <= 64: a row count off the 16-byte grid runs the kernels that copy A's packed slabs and read them as they
+// are (multiples of 8) or spread them in the LDS;
 // a and a_scale may have more elements per k-row than c has rows (lda: a multiple of 16, at most 64 -- padded
 // copies whose c is written in place)
 bool decode_strip_supports(const GemmArgs& g)
@@ -974,22 +991,27 @@ hipError_t launch_decode_strips(const GemmArgs& g, int ksplit, int halves, float
         return wide ? by_tiles(StreamShape<2, STREAM_NS_WIDE, 2>{}, StreamShape<4, STREAM_NS_WIDE, 2>{})
                     : by_tiles(StreamShape<2, STREAM_NS, 1>{}, StreamShape<4, STREAM_NS4, 1>{});
     }
+    using Grid = std::integral_constant<ARows, ARows::GRID>;
+    using Spread = std::integral_constant<ARows, ARows::SPREAD>;
+    using Packed = std::integral_constant<ARows, ARows::PACKED>;
+    const bool on_grid = leading_dim(g) % 16 == 0, packed = leading_dim(g) % 16 == 8;
     if (halves == 2) {  // 256-column strips: three stages of 32 KB of B
         const int tiles = (g.m + 15) / 16;
-        auto wide = [&](auto mt_c, auto ragged_c, auto tiles_c) -> hipError_t {
+        auto wide = [&](auto mt_c, auto form_c, auto tiles_c) -> hipError_t {
             constexpr int MT = decltype(mt_c)::value, T = decltype(tiles_c)::value;
-            constexpr bool RG = decltype(ragged_c)::value;
-            return go(decode_strip_kernel<MT, STREAM_NS_WIDE, RG, T, 2, 1>, DecodeShape<MT, STREAM_NS_WIDE, RG, 2>::LDS);
+            constexpr ARows F = decltype(form_c)::value;
+            return go(decode_strip_kernel<MT, STREAM_NS_WIDE, F, T, 2, 1>,
+                      DecodeShape<MT, STREAM_NS_WIDE, F == ARows::SPREAD, 2>::LDS);
         };
-        auto by_tiles = [&](auto ragged_c) -> hipError_t {
+        auto by_tiles = [&](auto form_c) -> hipError_t {
             switch (tiles) {
-            case 1: return wide(std::integral_constant<int, 2>{}, ragged_c, std::integral_constant<int, 1>{});
-            case 2: return wide(std::integral_constant<int, 2>{}, ragged_c, std::integral_constant<int, 2>{});
-            case 3: return wide(std::integral_constant<int, 4>{}, ragged_c, std::integral_constant<int, 3>{});
-            default: return wide(std::integral_constant<int, 4>{}, ragged_c, std::integral_constant<int, 4>{});
+            case 1: return wide(std::integral_constant<int, 2>{}, form_c, std::integral_constant<int, 1>{});
+            case 2: return wide(std::integral_constant<int, 2>{}, form_c, std::integral_constant<int, 2>{});
+            case 3: return wide(std::integral_constant<int, 4>{}, form_c, std::integral_constant<int, 3>{});
+            default: return wide(std::integral_constant<int, 4>{}, form_c, std::integral_constant<int, 4>{});
             }
         };
-        return leading_dim(g) % 16 != 0 ? by_tiles(std::true_type{}) : by_tiles(std::false_type{});
+        return on_grid ? by_tiles(Grid{}) : packed ? by_tiles(Packed{}) : by_tiles(Spread{});
     }
     const int tiles = (g.m + 15) / 16;
     // The instances that spread A's packed slabs take rows on the grid as well, and a workgroup with a long K
@@ -997,29 +1019,35 @@ hipError_t launch_decode_strips(const GemmArgs& g, int ksplit, int halves, float
     // 16384 x 7168 in two splits, 47 / 48 rows: 26.3 / 27.8 us), a short one 3 - 10 % slower (24576 x 2048 unsplit,
     // 31 / 32 rows: 14.4 / 13.9 us; 7168 x 2048 in four splits: 8.0 / 7.3 us).  With three or four row tiles the
     // two measure level (their slab form has a ring of four stages, not six).
-    auto strips_of = [&](auto mt_c, auto ns_c, auto ragged_c, auto tiles_c) -> hipError_t {
+    // Rows on an 8-byte grid run in the PACKED instances (21 shapes of 8 ... 56 rows, N = 512 ... 57344, 2 ... 27 K blocks
+    // per workgroup: 0 - 24 % faster than spreading, one level within its noise) up to the same 28 blocks, there with
+    // any number of row tiles (40 x 16384 x 7168 in two splits: 27.5 us packed, 25.1 us spread).
+    auto strips_of = [&](auto mt_c, auto ns_c, auto form_c, auto tiles_c) -> hipError_t {
         constexpr int MT = decltype(mt_c)::value, NS = decltype(ns_c)::value, T = decltype(tiles_c)::value;
-        constexpr bool RG = decltype(ragged_c)::value;
-        constexpr int lds = DecodeShape<MT, NS, RG>::LDS;
+        constexpr ARows F = decltype(form_c)::value;
+        constexpr int lds = DecodeShape<MT, NS, F == ARows::SPREAD>::LDS;
         if constexpr (NS % 2 == 0)
             if (stages_in_pairs((long)strips * ksplit, kb_per_split, NS))
-                return go(decode_strip_kernel<MT, NS, RG, T, 1, 2>, lds);
-        return go(decode_strip_kernel<MT, NS, RG, T, 1, 1>, lds);
+                return go(decode_strip_kernel<MT, NS, F, T, 1, 2>, lds);
+        return go(decode_strip_kernel<MT, NS, F, T, 1, 1>, lds);
     };
     using std::integral_constant;
-    auto by_tiles = [&](auto ns2, auto ns4, auto ragged_c) -> hipError_t {
+    auto by_tiles = [&](auto ns2, auto ns4, auto form_c) -> hipError_t {
         switch (tiles) {
-        case 1: return strips_of(integral_constant<int, 2>{}, ns2, ragged_c, integral_constant<int, 1>{});
-        case 2: return strips_of(integral_constant<int, 2>{}, ns2, ragged_c, integral_constant<int, 2>{});
-        case 3: return strips_of(integral_constant<int, 4>{}, ns4, ragged_c, integral_constant<int, 3>{});
-        default: return strips_of(integral_constant<int, 4>{}, ns4, ragged_c, integral_constant<int, 4>{});
+        case 1: return strips_of(integral_constant<int, 2>{}, ns2, form_c, integral_constant<int, 1>{});
+        case 2: return strips_of(integral_constant<int, 2>{}, ns2, form_c, integral_constant<int, 2>{});
+        case 3: return strips_of(integral_constant<int, 4>{}, ns4, form_c, integral_constant<int, 3>{});
+        default: return strips_of(integral_constant<int, 4>{}, ns4, form_c, integral_constant<int, 4>{});
         }
     };
-    if (leading_dim(g) % 16 != 0 || (kb_per_split >= SLAB_FORM_MIN_KBLOCKS && tiles <= 2))
-        return by_tiles(integral_constant<int, 6>{}, integral_constant<int, RAGGED4_NS>{}, std::true_type{});
-    if (!shallow_ring_pays((long)strips * ksplit, kb_per_split))
-        return by_tiles(integral_constant<int, 6>{}, integral_constant<int, 6>{}, std::false_type{});
-    return by_tiles(integral_constant<int, 3>{}, integral_constant<int, 3>{}, std::false_type{});
+    if (!(on_grid || packed) || (kb_per_split >= SLAB_FORM_MIN_KBLOCKS && (tiles <= 2 || packed)))
+        return by_tiles(integral_constant<int, 6>{}, integral_constant<int, RAGGED4_NS>{}, Spread{});
+    const bool deep = !shallow_ring_pays((long)strips * ksplit, kb_per_split);
+    auto by_ring = [&](auto form_c) -> hipError_t {
+        return deep ? by_tiles(integral_constant<int, 6>{}, integral_constant<int, 6>{}, form_c)
+                    : by_tiles(integral_constant<int, 3>{}, integral_constant<int, 3>{}, form_c);
+    };
+    return on_grid ? by_ring(Grid{}) : by_ring(Packed{});
 }
 
 // every group: 1 <= m <= lda <= 64 (rows m .. lda-1 of a and a_scale readable), operands aligned like a

@@ -351,6 +351,43 @@ def test_decode_strip_kernel_with_rows_off_the_grid(pkg, m, n, k, ksplit):
     assert (out[m:] == 0x7FC1).all(), "rows past m were written"
 
 
+@pytest.mark.parametrize("m", [8, 24, 40, 56])
+@pytest.mark.parametrize("variant,ksplit,n,k", [
+    # one K block, an odd count of them, the ring of six (three) gone round, splits of unequal length, strips that end
+    # inside; 256-column strips
+    (1, 1, 128, 128), (1, 1, 176, 640), (1, 1, 256, 1792), (1, 4, 400, 1664), (1, 3, 4608, 7168),
+    (2, 1, 288, 128), (2, 1, 512, 896), (2, 2, 4112, 1920),
+])
+def test_decode_rows_on_an_8_byte_grid(pkg, m, variant, ksplit, n, k):
+    """A's slabs read as they lie: bit for bit the result on rows padded to the 16-byte grid, with NaN codes around A"""
+    import torch
+    a, b, sa, sb = oracle.make_inputs(m, n, k, 1300 + m + k)
+    m16 = m + 8
+    pa, psa = np.zeros((k, m16), a.dtype), np.zeros((k // 128, m16), sa.dtype)
+    pa[:, :m], psa[:, :m] = a.reshape(k, m), sa.reshape(k // 128, m)
+    da, dsa, dpa, dpsa, db, dsb = _dev(np.concatenate([a.reshape(-1), np.full(64, 0x7F, a.dtype)]), sa, pa, psa, b, sb)
+    got = torch.full((m + 1, n), 0x7FC1, dtype=torch.int32, device="cuda").to(torch.int16)  # one guard row
+    want = torch.zeros((m16, n), dtype=torch.int16, device="cuda")
+    st = torch.cuda.current_stream().cuda_stream
+    _say(f"[gpu case] decode rows on an 8-byte grid: {m}x{n}x{k} variant={variant} ksplit={ksplit}")
+    pkg.select(pkg.KERNEL_SKINNY)
+    pkg.force_config(variant, ksplit)
+    try:
+        pkg.gemm(dpa, db, dpsa, dsb, want, m16, n, k, st)
+        aligned = pkg.last_kernel()
+        pkg.gemm(da, db, dsa, dsb, got, m, n, k, st)
+        torch.cuda.synchronize()
+        name = pkg.last_kernel()
+    finally:
+        pkg.force_config(-1, 0)
+        pkg.select(0)
+    assert name == aligned == f"decode{128 * variant}_k{ksplit}", (name, aligned)
+    assert torch.equal(got[:m], want[:m]), name
+    assert (got[m].cpu().numpy().view(np.uint16) == 0x7FC1).all(), "rows beyond m written"
+    _assert_every_element(got[:m].cpu().numpy().view(np.uint16), a, b, sa, sb, m, n, k, name)
+    pkg.release()
+
+
 def test_decode_rows_off_the_grid_run_without_a_padded_copy(pkg):
     """automatic dispatch: a decode batch of seven rows takes the decode kernel directly; with A off a 16-byte
     boundary it takes the padded plan as before"""
