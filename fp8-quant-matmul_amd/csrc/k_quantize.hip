@@ -108,7 +108,7 @@ __device__ __forceinline__ float scale_of(float amax)
 template <typename TIn, bool BLOCK, bool BF16MATH, int QTILE>
 __global__ void __launch_bounds__(QTILE * 4)
 quantize_kernel(const TIn* __restrict__ x, uint8_t* __restrict__ q, float* __restrict__ scale_out,
-                int rows, int K, int vec_store)
+                int rows, int K, int grid)
 {
     constexpr int NT = QTILE * 4, NW = NT / 64;
     static_assert(!BLOCK || QTILE % 128 == 0, "whole scale blocks");
@@ -128,7 +128,7 @@ quantize_kernel(const TIn* __restrict__ x, uint8_t* __restrict__ q, float* __res
     const int kb = blockIdx.y;
     // One tile holds all rows (a decode batch): the K block's output, [128][rows] bytes, is one contiguous piece of
     // memory.  The tile is kept packed like it in the LDS and leaves as it lies.
-    const bool packed = QTILE <= 64 && rows <= QTILE && !vec_store && (reinterpret_cast<uintptr_t>(q) & 15) == 0;
+    const bool packed = QTILE <= 64 && rows <= QTILE && grid == 0 && (reinterpret_cast<uintptr_t>(q) & 15) == 0;
 
     // rows past the last are read as the last one: no branch around a load, all of them are in flight together (they
     // do not change the block's amax, and their bytes are not stored)
@@ -215,7 +215,7 @@ quantize_kernel(const TIn* __restrict__ x, uint8_t* __restrict__ q, float* __res
     }
 
     // k-row kk of the tile: QTILE bytes, one per source row
-    if (vec_store) {  // every k-row starts on a 16-byte boundary: a lane takes 16 of its bytes
+    if (grid == 16) {  // every k-row starts on a 16-byte boundary: a lane takes 16 of its bytes
         const int dq = t % CH, first = row0 + 16 * dq;
 #pragma unroll
         for (int pass = 0; pass < 128 * CH / NT; ++pass) {
@@ -223,6 +223,17 @@ quantize_kernel(const TIn* __restrict__ x, uint8_t* __restrict__ q, float* __res
             const uint4 v = *reinterpret_cast<const uint4*>(tile + kk * STRIDE + ((dq ^ ((kk >> KSH) & (CH - 1))) << 4));
             if (first < rows)
                 *reinterpret_cast<uint4*>(q + (size_t)(kb * 128 + kk) * rows + first) = v;
+        }
+        return;
+    }
+    if (grid == 8) {  // the same in pieces of 8 bytes
+#pragma unroll 4
+        for (int idx = t; idx < 128 * 2 * CH; idx += NT) {
+            const int kk = idx / (2 * CH), h = idx % (2 * CH), first = row0 + 8 * h;
+            const uint2 v = *reinterpret_cast<const uint2*>(tile + kk * STRIDE +
+                                                            (((h >> 1) ^ ((kk >> KSH) & (CH - 1))) << 4) + 8 * (h & 1));
+            if (first < rows)
+                *reinterpret_cast<uint2*>(q + (size_t)(kb * 128 + kk) * rows + first) = v;
         }
         return;
     }
@@ -263,28 +274,38 @@ quantize_kernel(const TIn* __restrict__ x, uint8_t* __restrict__ q, float* __res
     }
 }
 
+// the boundary that every k-row of the output starts on, if that is one of 16 or 8 bytes, else 0
+int output_grid(const uint8_t* q, int rows)
+{
+    const uintptr_t ends = reinterpret_cast<uintptr_t>(q) | (uintptr_t)rows;
+    return ends % 16 == 0 ? 16 : ends % 8 == 0 ? 8 : 0;
+}
+
 template <typename TIn, bool BLOCK, bool BF16MATH, int QTILE>
 void launch_quantize_tile(const TIn* x, uint8_t* q, float* scale_out, int rows, int k, hipStream_t s)
 {
-    const int vec_store = (rows % 16 == 0) && (reinterpret_cast<uintptr_t>(q) % 16 == 0);
+    const int grid = output_grid(q, rows);
     hipLaunchKernelGGL((quantize_kernel<TIn, BLOCK, BF16MATH, QTILE>), dim3((rows + QTILE - 1) / QTILE, k / 128),
-                       dim3(QTILE * 4), 0, s, x, q, scale_out, rows, k, vec_store);
+                       dim3(QTILE * 4), 0, s, x, q, scale_out, rows, k, grid);
 }
 
 // Tile sizes, measured with every operand from HBM (us, previous kernel -> this one):
 //   128 x 128 blocks: 128 rows, eight waves of 16, whatever the size (512 x 2048 6.5 -> 3.5, 4608 x 7168 28.8 -> 22.0 =
 //   4.5 TB/s; 256-row tiles 4.5 and 23.3).
-//   1 x 128 groups, up to 64 rows: a decode batch is launch and latency.  One wave per 16 rows up to 32 rows on the
-//   16-byte grid or 16 off it (16 rows 3.8 -> 2.5, 64-row tiles 3.1), else 64-row tiles (24 rows 3.9 -> 3.2, 64 rows
-//   4.5 -> 2.9).
+//   1 x 128 groups, up to 64 rows: a decode batch is launch and latency.  One wave per 16 rows up to 32 rows on a
+//   16- or 8-byte grid or 16 off them (16 rows 3.8 -> 2.5, 64-row tiles 3.1), else 64-row tiles (24 rows in
+//   one of them 3.9 -> 3.2, 64 rows 4.5 -> 2.9).
 //   More rows: 256-row tiles once they make 256 workgroups, whose k-rows leave in pieces of 256 bytes (8192 x 7168
 //   46.3 -> 37.1 = 4.7 TB/s, 8191 x 7168 75 -> 48.6 against 54.1 with 128 rows).  Fewer than that, on the grid: 64 rows
 //   up to 1024 tiles (1024 x 2048 5.7 -> 3.8, with 128 rows 4.2), else 128; off the grid 128 rows, which have fewer
 //   ends of segments to store byte by byte (333 x 7168 8.1 -> 6.1, with 64 rows 7.5).
+//   Multiples of 8 rows leave in 8-byte stores, without the shifting and the single bytes, and count as on the grid
+//   (with the GEMM behind it: 24 x 512 x 7168 10.43 -> 10.09, 200 x 512 x 7168 13.84 -> 13.25, 1032 x 512 x 7168 25.97 ->
+//   24.13, 8184 x 1536 x 2048 46.4 -> 45.3; 24 rows of fp32 10.52 -> 10.04).
 template <typename TIn, bool BF16MATH>
 void launch_quantize_typed(const TIn* x, uint8_t* q, float* scale_out, int rows, int k, bool block128, hipStream_t s)
 {
-    const bool on_grid = rows % 16 == 0;
+    const bool on_grid = rows % 16 == 0 || output_grid(q, rows) == 8;
     const long nkb = k / 128;
     auto tiles = [&](int qtile) { return (rows + qtile - 1) / qtile * nkb; };
     if (block128)

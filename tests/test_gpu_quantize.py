@@ -175,3 +175,11 @@ def test_quantize_tile_sizes_and_ends(pkg, rows, k, offset):
         assert np.array_equal(dq.cpu().numpy().reshape(k, rows), rq), which
         guard = torch.cat([buf[:64 + offset], buf[64 + offset + k * rows:]])
         assert (guard == 0x7F).all(), which
+
+
+@pytest.mark.parametrize("rows,k,offset", [
+    (8, 128, 0), (24, 256, 0), (24, 256, 8), (32, 128, 24), (40, 256, 0), (56, 128, 8), (72, 256, 0), (1000, 128, 0),
+    (136, 256, 8), (16392, 512, 0), (16, 128, 4), (24, 128, 4),   # the last two: 16-row tiles on a 4-byte boundary only
+])
+def test_quantize_rows_on_an_8_byte_grid(pkg, rows, k, offset):
+    test_quantize_tile_sizes_and_ends(pkg, rows, k, offset)
