@@ -157,6 +157,11 @@ __device__ __forceinline__ void decode_body(const DecodeProblem& one, const Grou
         const int g = unit / strips;
         strip = unit - g * strips;
         pr = DecodeProblem{tab->a[g], tab->b[g], tab->a_scale[g], tab->b_scale[g], tab->c[g], tab->m[g], tab->lda[g]};
+        // Everything in hand here: left to itself the compiler asks for each value where it is first used and waits for it,
+        // four trips to the table one after the other in front of the first copy (nine groups of 16 rows, 416 x 384, from
+        // the Infinity Cache 4.20 us, 3.85 this way; 2 % on average over 120 launches of 1 - 64 rows per group).
+        asm volatile("" ::"s"(pr.a), "s"(pr.b), "s"(pr.a_scale), "s"(pr.b_scale), "s"(pr.c), "s"(pr.M), "s"(pr.lda),
+                     "s"(kb_per_split));
     }
     const uint8_t* __restrict__ a = pr.a;
     const uint8_t* __restrict__ b = pr.b;
