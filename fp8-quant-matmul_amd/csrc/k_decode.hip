@@ -442,8 +442,12 @@ __device__ __forceinline__ void decode_body(const DecodeProblem& one, const Grou
     constexpr int PER_SPLIT = 8 * PER_WAVE;  // patches of one split of one unit
     const int senders = ksplit - 1;
     const size_t patch = ((size_t)unit * senders * 8 + wave) * PER_WAVE;  // split 0
-    // lanes whose row exists take part: a CU takes in 64 bytes per clock, which is most of what the hand-over takes
-    auto row_exists = [&](int i) __attribute__((always_inline)) { return 16 * i + i16 < M; };
+    // Lanes whose row exists take part: a CU takes in 64 bytes per clock, which is most of what the hand-over takes.  In
+    // a grouped launch, which learns its row count here only, whole row tiles do: the lane masks and the checks without
+    // branches cost more than the bytes there (40 launches of 2 - 8 groups of up to 64 rows, N = 256 ... 1008, in 4 - 10
+    // splits: 2 % slower than whole tiles on average, 5 % at worst; 50 of any number of rows 1.5 %).  Where the number of
+    // tiles is known, the checks without branches are 2 - 5 % ahead (79 single problems in splits).
+    auto row_exists = [&](int i) __attribute__((always_inline)) { return GROUPED ? i < mtiles : 16 * i + i16 < M; };
     if (split < senders) {
         v4i* mine = reinterpret_cast<v4i*>(mailbox) + (patch + (size_t)split * PER_SPLIT) * 64 + lane;
 #pragma unroll
@@ -471,11 +475,12 @@ __device__ __forceinline__ void decode_body(const DecodeProblem& one, const Grou
     bool gave_up = false;
     const unsigned long long t_first = __builtin_amdgcn_s_memrealtime();
     // byte offset of a lane's 16 bytes of split 0, per pair of row tiles; outside the resource (which fetches and stores
-    // nothing, without a branch among the loads) where the lane's row does not exist
+    // nothing, without a branch among the loads) where the lane's row does not exist.  Grouped: the loads of a row tile that
+    // does not exist bring the mailbox's zeros, which are added to rows that are not stored.
     uint32_t off[MT];
 #pragma unroll
     for (int i = 0; i < MT; ++i)
-        off[i] = row_exists(i) ? (uint32_t)(i * 64 + lane) * 16u : 0x80000000u;
+        off[i] = GROUPED || row_exists(i) ? (uint32_t)(i * 64 + lane) * 16u : 0x80000000u;
     for (int z0 = 0; z0 < senders; z0 += 4) {
 #pragma unroll
         for (int hp = 0; hp < NB * (MT / 2); ++hp) {  // two row tiles of a half at a time
@@ -498,9 +503,13 @@ __device__ __forceinline__ void decode_body(const DecodeProblem& one, const Grou
                     for (int z = 0; z < 4; ++z)
 #pragma unroll
                         for (int i = 0; i < 2; ++i)
-                            if (z0 + z < senders && tile_here(i))
-                                missing = missing | (row_exists(2 * h + i) & ((v[z][i][0] == 0) | (v[z][i][1] == 0) |
-                                                                              (v[z][i][2] == 0) | (v[z][i][3] == 0)));
+                            if (z0 + z < senders && tile_here(i)) {
+                                const v4i w = v[z][i];
+                                if (GROUPED)
+                                    missing = missing || (row_exists(2 * h + i) && (w[0] == 0 || w[1] == 0 || w[2] == 0 || w[3] == 0));
+                                else
+                                    missing = missing | (row_exists(2 * h + i) & ((w[0] == 0) | (w[1] == 0) | (w[2] == 0) | (w[3] == 0)));
+                            }
                     if (__builtin_amdgcn_ballot_w64(missing) == 0)
                         break;
                     if (__builtin_amdgcn_s_memrealtime() - t_first > SPIN_LIMIT_TICKS) {
@@ -515,7 +524,8 @@ __device__ __forceinline__ void decode_body(const DecodeProblem& one, const Grou
                         for (int i = 0; i < 2; ++i) {
                             if (!tile_here(i))
                                 continue;
-                            __builtin_amdgcn_raw_buffer_store_b128((v4i){0, 0, 0, 0}, rp, off[2 * h + i] + place(z), 0, 0);
+                            if (!GROUPED || row_exists(2 * h + i))
+                                __builtin_amdgcn_raw_buffer_store_b128((v4i){0, 0, 0, 0}, rp, off[2 * h + i] + place(z), 0, 0);
                             const v4f f = __builtin_bit_cast(v4f, v[z][i]);
                             sum[hb][2 * h + i] = z0 + z == 0 ? f : sum[hb][2 * h + i] + f;
                         }
