@@ -1171,12 +1171,17 @@ hipError_t launch_decode_grouped(const GroupTable& tab, int n, int k, int ksplit
         hipLaunchKernelGGL(kern, grid, dim3(DS_THREADS), lds, s, tab, mailbox, n, k, strips, ksplit, kb_per_split);
         return hipGetLastError();
     };
+    // One or three K blocks with slabs to spread are not taken in pairs, where the last turn handles a slab that does not
+    // exist (from the Infinity Cache / from L2, one block to a barrier against pairs: 14 groups of 5 - 60 rows, 1584 x 128,
+    // 4.72 / 3.58 against 5.04 / 3.92 us; 13 of 6 - 64 rows, 672 x 384, 5.91 / 5.02 against 6.10 / 5.35 us; 16 launches
+    // of 1 - 32 rows level to 5 % ahead).  From two blocks on, three excepted, pairs are ahead by up to 12 %.  Single problems,
+    // whose tile count is a constant, gain from pairs there too (12 shapes in splits of one or three blocks: 1.5 %).
     auto strips_of = [&](auto mt_c, auto ns_c, auto ragged_c) -> hipError_t {
         constexpr int MT = decltype(mt_c)::value, NS = decltype(ns_c)::value;
         constexpr bool RG = decltype(ragged_c)::value;
         constexpr int lds = DecodeShape<MT, NS, RG>::LDS;
         if constexpr (NS % 2 == 0)
-            if (stages_in_pairs(units * ksplit, kb_per_split, NS))
+            if (stages_in_pairs(units * ksplit, kb_per_split, NS) && !(RG && (kb_per_split == 1 || kb_per_split == 3)))
                 return go(decode_strip_grouped_kernel<MT, NS, RG, 2>, lds);
         return go(decode_strip_grouped_kernel<MT, NS, RG, 1>, lds);
     };
