@@ -63,16 +63,19 @@ struct PadPiece {
 // All padding copies of a call in one launch: a workgroup moves PER_THREAD * 256 pieces of 16 bytes of one job.
 //
 // Bound by memory: 2 bytes move per byte of the operand.  All loads of a thread are out before the first is needed, indices
-// are 32 bits wide (an operand has less than 2^27 pieces), and the grid holds the pieces that there are.  Against one piece
+// are 32 bits wide (an operand has less than 2^27 pieces), and a large grid holds the pieces that there are (a small one:
+// JOB_ROWS_MAX_WORKGROUPS below).  Against one piece
 // per thread by five dword loads and a 64-bit division on a grid as large for every job as for the largest: 8191 x 7168
 // 25.0 -> 22.1 us (5.3 TB/s), eight groups of 250 ... 2051 rows x 2048 12.9 -> 9.6 us, thirty of 200 rows 8.6 -> 7.6 us;
 // a single operand of up to 3 MB, where the launch is what it takes, is level (333 x 7168: 5.0 us).
-template <int MAX, int PER_THREAD>
+template <int MAX, int PER_THREAD, bool JOB_ROWS>
 __global__ void __launch_bounds__(256) pad_kernel(const PadJobs<MAX> jobs)
 {
     const uint32_t block = blockIdx.x;
     int job = 0;
-    if (MAX <= 4) {
+    if (JOB_ROWS) {
+        job = blockIdx.y;
+    } else if (MAX <= 4) {
 #pragma unroll
         for (int j = 1; j < MAX; ++j)
             job += j < jobs.count && block >= jobs.first_block[j];
@@ -88,7 +91,9 @@ __global__ void __launch_bounds__(256) pad_kernel(const PadJobs<MAX> jobs)
     const uint8_t* const src = static_cast<const uint8_t*>(jobs.src[job]);
     uint8_t* const dst = jobs.base + (size_t)jobs.dst256[job] * 256;
     const uint32_t chunks = jobs.chunks[job], ld_src = jobs.ld_src[job], pieces = jobs.rows[job] * chunks;
-    const uint32_t at = (block - jobs.first_block[job]) * (256u * PER_THREAD) + threadIdx.x;
+    const uint32_t first = (block - (JOB_ROWS ? 0u : jobs.first_block[job])) * (256u * PER_THREAD), at = first + threadIdx.x;
+    if (JOB_ROWS && first >= pieces)
+        return;
     PadPiece piece[PER_THREAD];
 #pragma unroll
     for (int u = 0; u < PER_THREAD; ++u) {
@@ -107,15 +112,30 @@ __global__ void __launch_bounds__(256) pad_kernel(const PadJobs<MAX> jobs)
 // would be left without a workgroup.
 constexpr size_t PIECES_FOR_FOUR = (size_t)1 << 18;
 
+// The copies of a grouped call: up to this many workgroups the grid has a row as long as the largest job's for every job
+// (JOB_ROWS), so that a workgroup knows its job without looking it up, a trip to the kernel arguments in front of the one
+// for the job itself; the surplus workgroups, at most 16 for a CU, leave at once.  39 grouped calls with 60 ... 4096 of
+// them, with the GEMM behind it: up to 13 % ahead of the looked-up form, 2 % behind at worst (eight groups of 87 - 166
+// rows, 2112 x 256, from HBM 11.84 -> 10.49 us; 59 of 2 - 16 rows, 3632 x 128, 15.54 -> 14.65); beyond, where the grid
+// would be mostly surplus, the two are level and the looked-up form 1 % ahead.
+constexpr uint32_t JOB_ROWS_MAX_WORKGROUPS = 4096;
+
 template <int MAX, int PER_THREAD>
 hipError_t launch_pad_typed(PadJobs<MAX>& jobs, hipStream_t s)
 {
-    uint32_t blocks = 0;
+    uint32_t blocks = 0, most = 0;
     for (int j = 0; j < jobs.count; ++j) {
+        const uint32_t mine = (jobs.rows[j] * jobs.chunks[j] + 256 * PER_THREAD - 1) / (256 * PER_THREAD);
         jobs.first_block[j] = blocks;
-        blocks += (jobs.rows[j] * jobs.chunks[j] + 256 * PER_THREAD - 1) / (256 * PER_THREAD);
+        blocks += mine;
+        most = mine > most ? mine : most;
     }
-    hipLaunchKernelGGL((pad_kernel<MAX, PER_THREAD>), dim3(blocks), dim3(256), 0, s, jobs);
+    if constexpr (MAX > 4)
+        if ((uint64_t)most * jobs.count <= JOB_ROWS_MAX_WORKGROUPS) {
+            hipLaunchKernelGGL((pad_kernel<MAX, PER_THREAD, true>), dim3(most, jobs.count), dim3(256), 0, s, jobs);
+            return hipGetLastError();
+        }
+    hipLaunchKernelGGL((pad_kernel<MAX, PER_THREAD, false>), dim3(blocks), dim3(256), 0, s, jobs);
     return hipGetLastError();
 }
 

@@ -975,7 +975,10 @@ def test_grouped_gemm_equals_the_problems_one_by_one(pkg, variant, ms, n, k):
 
 
 @pytest.mark.parametrize("ms,n,k", [([40, 256, 24], 256, 256), ([1, 0, 1000, 333, 16], 520, 384),
-                                    ([129] * 20, 100, 512), ([2049, 17], 1544, 1024)])
+                                    ([129] * 20, 100, 512), ([2049, 17], 1544, 1024),
+                                    # the copies: a grid row per group (above, and with four pieces to a thread),
+                                    # workgroups that look their group up (one piece, four pieces)
+                                    ([1100] * 6, 32, 640), ([2051] + [65] * 39, 64, 384), ([5001] + [129] * 20, 32, 640)])
 def test_grouped_gemm_pads_groups_off_the_16_byte_grid(pkg, ms, n, k):
     """ragged m (and n): one grouped launch on padded copies, C rows beyond m untouched"""
     import torch
