@@ -15,6 +15,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <cfenv>
 #include <cstdint>
 #include <cstdlib>
 #include <cstring>
@@ -94,7 +95,7 @@ struct StagingBuf {
 
 // fp32 -> e4m3fn, nearest even, beyond +-448 saturated, NaN kept.  Normal results: the upper bits of the fp32 word,
 // rounded by adding half a unit (less one, plus the bit that stays last), with the exponent's bias moved from 127 to 7.
-// Below 2^-6 the code counts steps of 2^-9: adding 2^14 rounds to that step in hardware.
+// Below 2^-6 the code counts steps of 2^-9: adding 2^14 rounds to that step in hardware (NearestEven below).
 inline uint32_t e4m3fn_code(float x)
 {
     uint32_t u;
@@ -112,11 +113,23 @@ inline uint32_t e4m3fn_code(float x)
     return code | ((u >> 24) & 0x80u);
 }
 
+// The arithmetic above rounds to nearest and raises no exception whatever the caller's floating-point environment (which
+// threads inherit) asks for, and leaves that environment as it was.
+struct NearestEven {
+    std::fenv_t caller;
+    NearestEven()
+    {
+        std::feholdexcept(&caller);
+        std::fesetround(FE_TONEAREST);
+    }
+    ~NearestEven() { std::fesetenv(&caller); }
+};
+
 #if defined(__x86_64__)
 // The values are read past the caches of the core that converts them: left there, they make the caller's next write to
 // that memory slower (new values into 73 MB, five page-sized temporaries and all: 31 ms, with the lines in other cores'
 // caches 50 ms, this way 31 to 35 ms).
-__attribute__((target("avx2"))) void convert_avx2(const float* __restrict__ in, uint8_t* __restrict__ out, size_t count)
+__attribute__((target("avx2"), noinline)) void convert_avx2(const float* __restrict__ in, uint8_t* __restrict__ out, size_t count)
 {
     constexpr size_t LINE = 16, AHEAD = 32 * LINE;
     size_t i = 0;
@@ -130,7 +143,7 @@ __attribute__((target("avx2"))) void convert_avx2(const float* __restrict__ in, 
 }
 #endif
 
-void convert_plain(const float* __restrict__ in, uint8_t* __restrict__ out, size_t count)
+__attribute__((noinline)) void convert_plain(const float* __restrict__ in, uint8_t* __restrict__ out, size_t count)
 {
     for (size_t i = 0; i < count; ++i)
         out[i] = (uint8_t)e4m3fn_code(in[i]);
@@ -138,6 +151,7 @@ void convert_plain(const float* __restrict__ in, uint8_t* __restrict__ out, size
 
 void convert_host(const float* in, uint8_t* out, size_t count)
 {
+    const NearestEven environment;  // (the converters are not inlined: nothing of theirs moves out of its span)
 #if defined(__x86_64__)
     if (__builtin_cpu_supports("avx2"))
         return convert_avx2(in, out, count);

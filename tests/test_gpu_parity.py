@@ -838,6 +838,28 @@ def test_host_launcher_converts_like_the_device(pkg, m, n, k):
     torch.cuda.synchronize()
     assert np.array_equal(c, dc.cpu().numpy().view(np.uint16))
 
+@pytest.mark.parametrize("m,n,k", [(3, 128, 128), (520, 128, 1024)])  # without and with worker threads
+def test_host_launcher_rounds_to_nearest_whatever_the_caller_rounds_to(pkg, m, n, k):
+    """the caller's floating-point environment neither changes the codes nor comes back changed"""
+    import ctypes
+    libm = ctypes.CDLL("libm.so.6")
+    upward = 0x800  # FE_UPWARD, x86
+    af = np.linspace(-2.0**-6, 2.0**-6, m * k, dtype=np.float32)  # down to a fraction of the smallest step
+    bf = np.linspace(-2.0**-6, 2.0**-6, n * k, dtype=np.float32)[::-1].copy()
+    sa, sb = np.full((k // 128) * m, 4096.0, np.float32), np.full((k // 128) * ((n + 127) // 128), 1.0, np.float32)
+    out = []
+    for mode in (0, upward):
+        c = np.zeros((m, n), np.uint16)
+        _say(f"[gpu case] fp8_gemm_host {m}x{n}x{k}, rounding mode {mode:#x}")
+        assert libm.fesetround(mode) == 0
+        rc = pkg.lib().fp8_gemm_host(c.ctypes.data, af.ctypes.data, bf.ctypes.data, sa.ctypes.data, sb.ctypes.data, m, n, k, 0)
+        after = libm.fegetround()
+        libm.fesetround(0)
+        assert (rc, after) == (0, mode)
+        out.append(c)
+    assert out[0].any() and np.array_equal(out[0], out[1])
+
+
 def test_host_launcher_from_several_threads(pkg):
     """calls that overlap (one uses the kept staging buffer, the others pin their own) and a release between them"""
     import threading
