@@ -21,6 +21,9 @@
 #include <cstring>
 #include <mutex>
 #include <thread>
+#if defined(__x86_64__)
+#include <cpuid.h>
+#endif
 
 namespace {
 
@@ -126,9 +129,8 @@ struct NearestEven {
 };
 
 #if defined(__x86_64__)
-// The values are read past the caches of the core that converts them: left there, they make the caller's next write to
-// that memory slower (new values into 73 MB, five page-sized temporaries and all: 31 ms, with the lines in other cores'
-// caches 50 ms, this way 31 to 35 ms).
+// The values are asked for past L2 and L3, which the caller's other data need: the call on 1024 x 1536 x 7168 takes 1.40 ms
+// instead of 1.65.
 __attribute__((target("avx2"), noinline)) void convert_avx2(const float* __restrict__ in, uint8_t* __restrict__ out, size_t count)
 {
     constexpr size_t LINE = 16, AHEAD = 32 * LINE;
@@ -140,6 +142,21 @@ __attribute__((target("avx2"), noinline)) void convert_avx2(const float* __restr
     }
     for (; i < count; ++i)
         out[i] = (uint8_t)e4m3fn_code(in[i]);
+}
+
+// (__builtin_cpu_supports answers from the compiler runtime's table, which does not hold this one everywhere)
+bool has_clflushopt()
+{
+    uint32_t a, b, c, d;
+    return __get_cpuid_count(7, 0, &a, &b, &c, &d) != 0 && ((b >> 23) & 1u) != 0;
+}
+
+// Every line of in[0 .. count) out of all caches, to memory if it is dirty.
+__attribute__((target("clflushopt"))) void evict_lines(const float* in, size_t count)
+{
+    const uintptr_t end = reinterpret_cast<uintptr_t>(in + count);
+    for (uintptr_t line = reinterpret_cast<uintptr_t>(in) & ~(uintptr_t)63; line < end; line += 64)
+        __builtin_ia32_clflushopt(reinterpret_cast<const void*>(line));
 }
 #endif
 
@@ -159,12 +176,36 @@ void convert_host(const float* in, uint8_t* out, size_t count)
     convert_plain(in, out, count);
 }
 
+// Values that a worker has read leave the caches.  Left in those of the core that converted them, they make the caller's
+// next write to that memory wait for that core, line by line, which can cost more than the workers save.  In ms, with the
+// values read and rewritten in place before each call, write / call / both: 300 x 2048 x 2048 without workers and with fp32
+// uploads 0.25 / 0.90 / 1.16, with workers 1.1 ... 1.7 / 0.52 / 1.6 ... 2.3, this way 0.48 / 0.57 / 1.1; 1024 x 1536 x 7168
+// 1.8 / 4.5 / 6.4, 2.3 ... 5.9 / 1.6 / 3.8 ... 7.6, 1.9 / 1.7 / 3.6.  Written by a plain copy or into new memory: 7.0 and 38,
+// 4.1 and 34, 3.9 and 34 for both.  From 117 MB of values on (2048 x 2048 x 7168 level) most have left the caches by
+// themselves, and the instructions cost more than they save (2048 x 3072 x 7168 6.6 without them, 7.0 with).  On a
+// processor without the instruction the lines stay.
+void give_back(const float* in, size_t count)
+{
+#if defined(__x86_64__)
+    static const bool can = has_clflushopt();
+    if (can)
+        evict_lines(in, count);
+#else
+    (void)in, (void)count;
+#endif
+}
+
 // A and B as one run of pieces, a ring of SLOTS of which is staged at a time.  Workers take pieces in order, main
 // uploads them in order and hands slots back once their upload has completed.
 struct Pipeline {
     static constexpr size_t PIECE = 128 * 1024;  // elements: 24 us of conversion, small enough to share out evenly
     static constexpr size_t SLOTS = 248;         // 31 MiB: with the scales at most STAGING_MAX
     static constexpr int MAX_WORKERS = 8;        // 4, 8, 16 threads convert 73 MB in 0.87, 0.54, 0.61 ms
+    // Fewer pieces than this the caller converts alone.  Call, and call with the values rewritten in place before it:
+    // 100 x 512 x 1024 (5 pieces) 0.19 and 0.22 ms against 0.27 and 0.32 with a worker, 128 x 1024 x 1024 (9) 0.30 and
+    // 0.36 against 0.27 and 0.40 with two, 300 x 2048 x 2048 (37) 1.07 and 1.32 against 0.59 and 1.15 with eight.
+    static constexpr size_t MIN_PIECES = 8;
+    static constexpr size_t GIVE_BACK_PIECES = 224;  // workers give lines back up to 117 MB of values
 
     const float* src[2];
     size_t count[2], pieces[2];
@@ -192,12 +233,14 @@ struct Pipeline {
         n = std::min(PIECE, count[which] - first);
     }
 
-    void convert(size_t p)
+    void convert(size_t p, bool in_worker)
     {
         int which;
         size_t first, n;
         piece(p, which, first, n);
         convert_host(src[which] + first, staging + (p % slots) * PIECE, n);
+        if (in_worker && total <= GIVE_BACK_PIECES)
+            give_back(src[which] + first, n);
         ready[p % slots].store(p + 1, std::memory_order_release);
     }
 
@@ -212,7 +255,7 @@ struct Pipeline {
                     return;
                 std::this_thread::yield();
             }
-            convert(p);
+            convert(p, true);
         }
     }
 
@@ -231,7 +274,7 @@ struct Pipeline {
                 freed.store(p, std::memory_order_release);
             }
             if (!have_workers)
-                convert(p);
+                convert(p, false);
             while (!is_ready(p))
                 std::this_thread::yield();
             // as many pieces as lie behind one another, converted, in the same matrix: a copy costs about 9 us
@@ -272,7 +315,9 @@ struct Workers {
     void start()
     {
         const int cpus = (int)std::thread::hardware_concurrency();
-        const int want = std::min({Pipeline::MAX_WORKERS, cpus - 1, (int)std::min<size_t>(pipe.total / 4, 64)});
+        const int want = pipe.total < Pipeline::MIN_PIECES
+                             ? 0
+                             : std::min({Pipeline::MAX_WORKERS, cpus - 1, (int)std::min<size_t>(pipe.total / 4, 64)});
         try {
             for (; count < want; ++count)
                 thread[count] = std::thread([this] { pipe.work(); });
