@@ -423,11 +423,15 @@ Plan compute_plan(const GemmArgs& g, const Config& cfg)
         const long long b_bytes = (long long)g.n * g.k;
         if (!by_name && g.m > 32 && g.m % 16 == 0 && !(g.n >= 6144 && b_bytes >= 28000000ll))
             wide_us = 1e300;
-        // Row counts off the 16-byte grid, which the strips take as they are: tiles that do so too over a B of up to 16 MB
-        // (66 random shapes of 33 ... 63 rows, N = 288 ... 12912, K = 256 ... 7680: 19 % faster from the Infinity Cache, 13 %
-        // from HBM on average, worst -4 %).  Over 16.5 ... 23.5 MB (8 shapes) they are 7 - 35 % ahead with B in the
-        // Infinity Cache and behind from HBM, where such weights are, by 4 % on average and 21 % at worst.  No tiles that
-        // need padded copies (12 shapes: 6.8 - 16.9 us against 10.8 - 23.8 us).
+        // Row counts off the 16-byte grid, which the strips take as they are: tiles that do so too over a B of up to 16 MB.
+        // 66 random shapes of 33 ... 63 rows, N = 288 ... 12912, K = 256 ... 7680: 19 % faster from the Infinity Cache, 13 %
+        // from HBM on average.  The line is where the gain with B in the cache and the loss from HBM, where such weights
+        // are, meet.  From 12 MB on and with N in whole 128-byte lines (strips of other columns straddle two), tiles of one
+        // or two splits are 15 and 7 % ahead from the cache and 7 and 8 % behind from HBM (77 and 43 shapes of 33 ... 47
+        // rows; 39 x 7168 x 2048 6.6 us either way and 9.5 against 8.3 us, the worst 47 x 9216 x 1536 6.6 against 6.7 and
+        // 11.1 against 8.3 us; with 49 rows and more 21 and 15 % ahead, 4 % behind and level); tiles of more splits 16 and
+        // 2 % ahead.  Over 16.5 ... 23.5 MB (8 shapes) tiles are 7 - 35 % ahead from the cache and behind from HBM by 4 % on
+        // average and 21 % at worst.  No tiles that need padded copies (12 shapes: 6.8 - 16.9 us against 10.8 - 23.8 us).
         if (!by_name && g.m > 32 && g.m % 16 != 0 && b_bytes < 16000000ll && cfg.force_variant < 0 &&
             cfg.force_ksplit <= 0 && cfg.fused_ok) {
             const Plan tiles = off_grid_plan(g, cfg);
