@@ -805,20 +805,22 @@ def test_host_launcher_matches_device_path(pkg):
 
 
 @pytest.mark.parametrize("m,n,k", [
-    (1, 128, 128),        # no worker threads
-    (520, 128, 1024),     # a's last piece is a part of one
-    (2052, 2304, 8192),   # 272 pieces: the staging ring of 256 goes round, the last piece of a ragged
-    (4100, 2304, 256),    # c larger than both staging halves
+    (1, 128, 128), (3, 128, 128),   # no worker threads
+    (520, 128, 1024),               # six pieces, none either, a's last one a part of a piece
+    (1100, 128, 1024),              # ten pieces: two workers
+    (2052, 2304, 8192),             # 273 pieces: the staging ring of 248 goes round, the last piece of a ragged
+    (4100, 2304, 256),              # c larger than both staging halves
 ])
 def test_host_launcher_converts_like_the_device(pkg, m, n, k):
     """fp8_gemm_host rounds on the host, in pieces: codes, and so c, bit for bit those of the device converter"""
     import torch
     rng = np.random.default_rng(m + n + k)
     af = rng.integers(0, 2**32, m * k, dtype=np.uint32).view(np.float32)   # every exponent, ties rare
-    af = np.where(np.abs(af) < 2.0**9, af, rng.standard_normal(m * k).astype(np.float32))  # no NaN: it would hide its row
+    af = np.where(np.abs(af) < 2.0**9, af, rng.standard_normal(m * k).astype(np.float32))  # no NaN: it hides its row
     af[::7] = (rng.integers(-960, 961, af[::7].size) * np.float32(2.0**-10))   # ties and steps below 2^-6
     af[3], af[5] = np.inf, -np.inf
-    af[m * k - 1] = np.nan
+    if m > 1:
+        af[m * k - 1] = np.nan  # column-major: in the last row
     bf = (rng.standard_normal(n * k) * 100).astype(np.float32)
     sa = rng.uniform(0.5, 2, (k // 128) * m).astype(np.float32)
     sb = rng.uniform(0.5, 2, (k // 128) * ((n + 127) // 128)).astype(np.float32)
@@ -837,8 +839,10 @@ def test_host_launcher_converts_like_the_device(pkg, m, n, k):
     pkg.gemm_ex(a8, b8, dsa, dsb, dc, m, n, k, opt, ws, ws.numel())
     torch.cuda.synchronize()
     assert np.array_equal(c, dc.cpu().numpy().view(np.uint16))
+    assert ((c[:max(1, m - 1)] & 0x7F80) != 0x7F80).all(), "a row that holds no NaN shows what was converted"
 
-@pytest.mark.parametrize("m,n,k", [(3, 128, 128), (520, 128, 1024)])  # without and with worker threads
+
+@pytest.mark.parametrize("m,n,k", [(3, 128, 128), (1100, 128, 1024)])  # without and with worker threads
 def test_host_launcher_rounds_to_nearest_whatever_the_caller_rounds_to(pkg, m, n, k):
     """the caller's floating-point environment neither changes the codes nor comes back changed"""
     import ctypes
@@ -886,6 +890,7 @@ def test_host_launcher_from_several_threads(pkg):
         for c in mine:
             assert np.array_equal(c, out[0][0])
     _assert_close(out[0][0], oracle.ref_gemm(a, b, sa, sb, m, n, k), "host launcher, several threads")
+
 
 def test_caller_workspace(pkg):
     import torch
