@@ -52,8 +52,8 @@ def _check(pkg, x, which, dtype):
     assert bad.size == 0, (which, x.shape, bad[:4], q[tuple(bad[0])], rq[tuple(bad[0])])
 
 
-# (row counts off the 16-byte grid leave through dword stores shifted into place: odd, 2 mod 4, 0 mod 4;
-# 20001 x 2048 is past the tile count up to which the 1 x 128 quantiser works in 64-row tiles)
+# (row counts off the 16- and 8-byte grids leave in 16-byte pieces shifted into place and single bytes at the ends: odd,
+# 2 mod 4, 4 mod 8; the last two of A in tiles of 256 rows)
 SHAPES_A = [(32, 2048), (1024, 2048), (2048, 7168), (16, 128), (1, 128), (130, 256), (77, 384),
             (200, 128), (1001, 512), (259, 256), (3, 256), (20001, 2048), (16384, 2560)]
 SHAPES_B = [(512, 2048), (576, 7168), (7168, 2048), (128, 128), (64, 128), (1, 256), (130, 256),
@@ -155,22 +155,30 @@ def test_gemm_on_device_quantised_inputs_equals_gemm_on_oracle_inputs(pkg):
     (32, 256, 8), (65, 256, 0), (80, 128, 0), (255, 256, 1), (257, 128, 0),               # 64- and 128-row tiles
     (16384, 512, 0), (16401, 512, 0), (16399, 512, 5),                                    # 256-row tiles
 ])
-def test_quantize_tile_sizes_and_ends(pkg, rows, k, offset):
+@pytest.mark.parametrize("source", ["bf16", "f32"])
+def test_quantize_tile_sizes_and_ends(pkg, rows, k, offset, source):
     """every tile size of the quantisers at the row counts where one takes over from the next, with outputs that start
     `offset` bytes off a 16-byte boundary: bytes and scales equal the oracle's, nothing around the output is written"""
     import torch
     x = oracle.gen_normal_bf16(rows, k, 7 + rows + k, 1.0, 50.0)
+    bf16 = source == "bf16"
+    if bf16:
+        src, dtype = _bf16_bits(x).view(np.int16), pkg.DTYPE_BF16
+    else:  # values that bf16 does not hold
+        x = (x * np.float32(1.0 + 2.0**-11)).astype(np.float32)
+        src, dtype = x, pkg.DTYPE_F32
+        assert (x.view(np.uint32) & 0xFFFF).any()
     for which in ("a", "b"):
-        dx = torch.from_numpy(_bf16_bits(x).view(np.int16)).cuda()
+        dx = torch.from_numpy(src).cuda()
         buf = torch.full((64 + k * rows + 64,), 0x7F, dtype=torch.uint8, device="cuda")
         dq = buf[64 + offset: 64 + offset + k * rows]
         ncol = rows if which == "a" else (rows + 127) // 128
         ds = torch.full((k // 128, ncol), float("nan"), dtype=torch.float32, device="cuda")
-        _say(f"[gpu case] quantize_{which} rows={rows} k={k} offset={offset}")
+        _say(f"[gpu case] quantize_{which} rows={rows} k={k} offset={offset} {source}")
         fn = pkg.quantize_a_1x128 if which == "a" else pkg.quantize_b_128x128
-        fn(dx, dq, ds, rows, k, pkg.DTYPE_BF16, torch.cuda.current_stream().cuda_stream)
+        fn(dx, dq, ds, rows, k, dtype, torch.cuda.current_stream().cuda_stream)
         torch.cuda.synchronize()
-        rq, rs = (oracle.quantize_a_1x128 if which == "a" else oracle.quantize_b_128x128)(x, bf16_arith=True)
+        rq, rs = (oracle.quantize_a_1x128 if which == "a" else oracle.quantize_b_128x128)(x, bf16_arith=bf16)
         assert np.array_equal(ds.cpu().numpy().view(np.uint32), rs.view(np.uint32)), which
         assert np.array_equal(dq.cpu().numpy().reshape(k, rows), rq), which
         guard = torch.cat([buf[:64 + offset], buf[64 + offset + k * rows:]])
@@ -181,5 +189,6 @@ def test_quantize_tile_sizes_and_ends(pkg, rows, k, offset):
     (8, 128, 0), (24, 256, 0), (24, 256, 8), (32, 128, 24), (40, 256, 0), (56, 128, 8), (72, 256, 0), (1000, 128, 0),
     (136, 256, 8), (16392, 512, 0), (16, 128, 4), (24, 128, 4),   # the last two: 16-row tiles on a 4-byte boundary only
 ])
-def test_quantize_rows_on_an_8_byte_grid(pkg, rows, k, offset):
-    test_quantize_tile_sizes_and_ends(pkg, rows, k, offset)
+@pytest.mark.parametrize("source", ["bf16", "f32"])
+def test_quantize_rows_on_an_8_byte_grid(pkg, rows, k, offset, source):
+    test_quantize_tile_sizes_and_ends(pkg, rows, k, offset, source)
