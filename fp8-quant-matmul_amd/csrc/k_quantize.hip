@@ -17,7 +17,7 @@
 // (/root/reference/check.cu:164-167):  q at row + k*rows, the 1 x 128 scales at row + kb*rows,
 // the 128 x 128 scales at nb + kb*ceil(rows/128).
 //
-// One workgroup owns QTILE rows x 128 k (QTILE / 128 scale blocks, or QTILE scale groups).  A thread reads 8 k of
+// One workgroup owns QTILE rows x 128 k (a 128 x 128 scale block, or QTILE scale groups).  A thread reads 8 k of
 // four adjacent rows at a time (16 lanes take a row's 128 elements: whole cache lines) and converts pairs of ROWS, so
 // that the four bytes of one k leave the conversion as the dword the transposed layout wants: the transposition costs
 // eight dword writes into the LDS per 32 elements and no byte shuffling.  From there the tile leaves as 16-byte
@@ -111,7 +111,7 @@ quantize_kernel(const TIn* __restrict__ x, uint8_t* __restrict__ q, float* __res
                 int rows, int K, int grid)
 {
     constexpr int NT = QTILE * 4, NW = NT / 64;
-    static_assert(!BLOCK || QTILE % 128 == 0, "whole scale blocks");
+    static_assert(!BLOCK || QTILE == 128, "one scale block");
     // LDS: one row of QTILE bytes per k, its 16-byte chunks (four dwords: the rows of one wave) permuted by
     // k so that the dword writes of a wave -- 16 k that are 8 apart, one chunk -- go to as many banks as there are
     constexpr int CH = QTILE / 16;                        // chunks per k-row
@@ -157,18 +157,16 @@ quantize_kernel(const TIn* __restrict__ x, uint8_t* __restrict__ q, float* __res
         if (lane == 0)
             s_red[wave] = a;
         __syncthreads();
-        const int first = wave & ~7;  // the eight waves of a scale block
-        a = s_red[first];
+        a = s_red[0];
 #pragma unroll
-        for (int w = 1; w < 8; ++w)
-            a = fmaxf(a, s_red[first + w]);
+        for (int w = 1; w < NW; ++w)
+            a = fmaxf(a, s_red[w]);
         const float mine = scale_of<BF16MATH>(a);
 #pragma unroll
         for (int i = 0; i < 4; ++i)
             scale[i] = mine;
-        const int nb = blockIdx.x * (QTILE / 128) + (wave >> 3), nblocks = (rows + 127) >> 7;
-        if ((wave & 7) == 0 && lane == 0 && nb < nblocks)
-            scale_out[(size_t)kb * nblocks + nb] = 1.0f / mine;
+        if (t == 0)
+            scale_out[(size_t)kb * gridDim.x + blockIdx.x] = 1.0f / mine;
     } else {
         // lane c works out the scale of row c & 3 of its four, the others take it over from there
         const float a0 = row_max(amax[0]), a1 = row_max(amax[1]), a2 = row_max(amax[2]), a3 = row_max(amax[3]);
