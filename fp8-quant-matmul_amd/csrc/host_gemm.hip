@@ -176,14 +176,15 @@ void convert_host(const float* in, uint8_t* out, size_t count)
     convert_plain(in, out, count);
 }
 
-// Values that a worker has read leave the caches.  Left in those of the core that converted them, they make the caller's
-// next write to that memory wait for that core, line by line, which can cost more than the workers save.  In ms, with the
-// values read and rewritten in place before each call, write / call / both: 300 x 2048 x 2048 without workers and with fp32
-// uploads 0.25 / 0.90 / 1.16, with workers 1.1 ... 1.7 / 0.52 / 1.6 ... 2.3, this way 0.48 / 0.57 / 1.1; 1024 x 1536 x 7168
-// 1.8 / 4.5 / 6.4, 2.3 ... 5.9 / 1.6 / 3.8 ... 7.6, 1.9 / 1.7 / 3.6.  Written by a plain copy or into new memory: 7.0 and 38,
-// 4.1 and 34, 3.9 and 34 for both.  From 117 MB of values on (2048 x 2048 x 7168 level) most have left the caches by
-// themselves, and the instructions cost more than they save (2048 x 3072 x 7168 6.6 without them, 7.0 with).  On a
-// processor without the instruction the lines stay.
+// Values that the workers have read leave the caches.  Left in those of the cores that converted them, they make the
+// caller's next write to that memory wait for those cores, line by line, which can cost more than the workers save.  In ms,
+// with the values read and rewritten in place before each call, write / call / both: 300 x 2048 x 2048 with fp32 uploads
+// 0.25 / 0.90 / 1.16, with workers 0.9 ... 1.7 / 0.48 / 1.4 ... 2.3, this way 0.46 / 0.53 / 1.0; 1024 x 1536 x 7168 1.8 / 4.5 /
+// 6.4, 2.3 ... 5.9 / 1.6 / 3.7 ... 7.6, 1.9 / 1.6 / 3.4; 4096 x 4608 x 7168 6.5 / 12.4 / 19, 7.5 ... 11.5 / 4.7 / 12.1 ... 16.7,
+// 6.5 / 5.3 / 11.9.  Written by a plain copy, which does not read, or into new memory, level with the workers alone (both
+// together 1.13, 4.0 and 12.8 against 1.12, 4.0 and 12.4; fp32 uploads 1.7, 7.0 and 21).  Each piece's lines right behind
+// its conversion instead of all of them behind the last one: 0.1 to 0.2 ms more on the first two.  On a processor without
+// the instruction the lines stay.
 void give_back(const float* in, size_t count)
 {
 #if defined(__x86_64__)
@@ -203,16 +204,15 @@ struct Pipeline {
     static constexpr int MAX_WORKERS = 8;        // 4, 8, 16 threads convert 73 MB in 0.87, 0.54, 0.61 ms
     // Fewer pieces than this the caller converts alone.  Call, and call with the values rewritten in place before it:
     // 100 x 512 x 1024 (5 pieces) 0.19 and 0.22 ms against 0.27 and 0.32 with a worker, 128 x 1024 x 1024 (9) 0.30 and
-    // 0.36 against 0.27 and 0.40 with two, 300 x 2048 x 2048 (37) 1.07 and 1.32 against 0.59 and 1.15 with eight.
+    // 0.36 against 0.23 and 0.36 with two, 300 x 2048 x 2048 (37) 1.07 and 1.32 against 0.53 and 1.0 with eight.
     static constexpr size_t MIN_PIECES = 8;
-    static constexpr size_t GIVE_BACK_PIECES = 224;  // workers give lines back up to 117 MB of values
 
     const float* src[2];
     size_t count[2], pieces[2];
     size_t total;  // pieces of both
     size_t slots;  // of the ring that this call needs
     uint8_t* staging = nullptr;
-    std::atomic<size_t> next{0}, freed{0};
+    std::atomic<size_t> next{0}, freed{0}, returned{0};
     std::atomic<bool> abort{false};
     std::atomic<size_t> ready[SLOTS];  // number of the last piece converted into the slot, plus one
 
@@ -233,14 +233,12 @@ struct Pipeline {
         n = std::min(PIECE, count[which] - first);
     }
 
-    void convert(size_t p, bool in_worker)
+    void convert(size_t p)
     {
         int which;
         size_t first, n;
         piece(p, which, first, n);
         convert_host(src[which] + first, staging + (p % slots) * PIECE, n);
-        if (in_worker && total <= GIVE_BACK_PIECES)
-            give_back(src[which] + first, n);
         ready[p % slots].store(p + 1, std::memory_order_release);
     }
 
@@ -249,13 +247,23 @@ struct Pipeline {
         for (;;) {
             const size_t p = next.fetch_add(1, std::memory_order_relaxed);
             if (p >= total)
-                return;
+                break;
             while (p >= freed.load(std::memory_order_acquire) + slots) {
                 if (abort.load(std::memory_order_relaxed))
                     return;
                 std::this_thread::yield();
             }
-            convert(p, true);
+            convert(p);
+        }
+        // the lines back to the caller, while main is busy with the last uploads, the GEMM and c
+        while (!abort.load(std::memory_order_relaxed)) {
+            const size_t p = returned.fetch_add(1, std::memory_order_relaxed);
+            if (p >= total)
+                return;
+            int which;
+            size_t first, n;
+            piece(p, which, first, n);
+            give_back(src[which] + first, n);
         }
     }
 
@@ -274,7 +282,7 @@ struct Pipeline {
                 freed.store(p, std::memory_order_release);
             }
             if (!have_workers)
-                convert(p, false);
+                convert(p);
             while (!is_ready(p))
                 std::this_thread::yield();
             // as many pieces as lie behind one another, converted, in the same matrix: a copy costs about 9 us
@@ -427,14 +435,14 @@ extern "C" int fp8_gemm_host(unsigned short* c, const float* a, const float* b, 
             TRY(hipMemcpy(d + o_bs, b_scale, nkb * sn * 4, hipMemcpyHostToDevice));
         }
         void* const dst[2] = {d, d + o_b};
-        TRY(pipe.upload(dst, workers.count > 0));
-        workers.join();
+        TRY(pipe.upload(dst, workers.count > 0));  // every value has been converted: the staging buffer is main's again
         const int rc = fp8_block_gemm_ex(d, d + o_b, reinterpret_cast<const float*>(d + o_as),
                                          reinterpret_cast<const float*>(d + o_bs), d + o_c, (int)m, (int)n, (int)k, &opt,
                                          ws_bytes ? d + o_ws : nullptr, ws_bytes, nullptr);
         if (rc != 0)
             return rc;
         TRY(download(c, d + o_c, m * n * 2, staging.p, ring_bytes));  // blocking: also the sync
+        workers.join();
     }
 #undef TRY
     return FP8GEMM_OK;
