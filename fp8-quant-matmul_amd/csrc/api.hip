@@ -920,7 +920,7 @@ int workspace_for(size_t need, hipStream_t stream, const Workspace* explicit_ws,
 // One grouped launch for the problems of `tab` (same n and k): the decode kernel when every group has at
 // most 64 rows (decode = true), else the persistent tile kernel.  Groups off the 16-byte grid (n, or for the
 // tile kernel m, not a multiple of 16; an operand off a 16-byte boundary) run on zero-padded copies in the
-// workspace made by one batched copy launch per operand kind.  Returns GROUPED_NOT_APPLICABLE when it cannot run (the caller
+// workspace: one launch for those of a and a_scale, one each for b and c where they need it.  Returns GROUPED_NOT_APPLICABLE when it cannot run (the caller
 // then takes the groups one by one).
 constexpr int GROUPED_NOT_APPLICABLE = -1000;
 int run_grouped_table(const GroupTable& tab, int n, int k, bool decode, hipStream_t s, const Config& cfg,

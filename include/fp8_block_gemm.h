@@ -130,8 +130,8 @@ int fp8_block_gemm_set_fused_reduction(int mode);
  * fp8_block_gemm_stream on that group.  Up to FP8GEMM_MAX_GROUPS problems
  * run as ONE launch of the persistent tile kernel (their tiles form one list that 256
  * workgroups walk through): as they are when every m[g] and n are multiples of 16 and the
- * operands 16-byte aligned, else on zero-padded copies in the workspace made by one batched copy
- * launch per operand kind ("padded_..._groupedN").  Groups of at most 64 rows (the experts of an MoE
+ * operands 16-byte aligned, else on zero-padded copies in the workspace ("padded_..._groupedN": one
+ * launch for those of a and a_scale, one each for b and c where they need it).  Groups of at most 64 rows (the experts of an MoE
  * layer in a decode step) do not go through 128-row tiles: they run as ONE launch of the decode kernel
  * ("decode128_kN_groupedG": 128-column strips of every group in one work list, every group's B read
  * once, the K range split and added inside the kernel as for a single problem; row counts off the 16-row
@@ -295,9 +295,10 @@ int fp8_block_gemm_abi_version(void);
 /* ---- host-buffer convenience layer: the reference's host launcher ----
  * Counterpart of gemmGPU (/root/reference/check.cu:51-130): takes HOST buffers with fp32
  * values for a and b (already in the column-major layouts above), allocates device
- * memory, converts fp32 -> fp8 (fp8_convert_f32_to_e4m3fn's rounding, on a few host threads
- * of this call's own) while it uploads, runs the kernel selected by `option`, downloads c
- * (bf16 bits) and frees.  A pinned staging buffer of at most 32 MiB is kept between calls
+ * memory, converts fp32 -> fp8 (fp8_convert_f32_to_e4m3fn's rounding) while it uploads, runs
+ * the kernel selected by `option`, downloads c (bf16 bits) and frees.  From 4 MB of values on up to
+ * eight threads of this call's own convert (fewer than the cores the process may use) and flush the
+ * cache lines of a and b that they have read.  A pinned staging buffer of at most 32 MiB is kept between calls
  * until fp8_block_gemm_release.  option: 2 = scalar definition kernel,
  * 0 = automatic dispatch, 1 = same as 0 (the reference's "reverse" grid has no meaning
  * here), or 100 + FP8GEMM_KERNEL_* to force a family.  Synchronous. */
