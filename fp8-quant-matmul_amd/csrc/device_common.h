@@ -79,6 +79,25 @@ __device__ __forceinline__ void lds_dma16(v4i rsrc, uint32_t voffset, uint32_t l
                  : "memory");
 }
 
+// The same where `skip` (wave-uniform) is zero.  The branch sits inside the statement: as one of the compiler's it would
+// end the block of instructions that LDS reads, MFMAs and folds are scheduled in.
+__device__ __forceinline__ void lds_dma16_unless(uint32_t skip, v4i rsrc, uint32_t voffset, uint32_t lds_addr, uint32_t soffset)
+{
+    asm volatile("s_cmp_lg_u32 %4, 0\n\ts_cbranch_scc1 .Lskip_dma_%=\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\t"
+                 "buffer_load_dwordx4 %0, %1, %3 offen lds\n.Lskip_dma_%=:"
+                 :
+                 : "v"(voffset), "s"(rsrc), "s"(lds_addr), "s"(soffset), "s"(skip)
+                 : "memory", "scc");
+}
+__device__ __forceinline__ void lds_dma4_unless(uint32_t skip, v4i rsrc, uint32_t voffset, uint32_t lds_addr, uint32_t soffset)
+{
+    asm volatile("s_cmp_lg_u32 %4, 0\n\ts_cbranch_scc1 .Lskip_dma_%=\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\t"
+                 "buffer_load_dword %0, %1, %3 offen lds\n.Lskip_dma_%=:"
+                 :
+                 : "v"(voffset), "s"(rsrc), "s"(lds_addr), "s"(soffset), "s"(skip)
+                 : "memory", "scc");
+}
+
 // The same with 4 bytes per lane: lane l's dword lands at lds_addr + 4*l (256 bytes per wave).
 __device__ __forceinline__ void lds_dma4(v4i rsrc, uint32_t voffset, uint32_t lds_addr, uint32_t soffset = 0)
 {

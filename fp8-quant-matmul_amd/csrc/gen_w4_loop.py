@@ -9,17 +9,19 @@ running sums wander between the two register files.  The text names physical reg
 preprocessor cannot compute, hence this script.   python3 gen_w4_loop.py > w4_loop.inc
 
 Register map of a wave
-    v[16q : 16q+15]   q = 0..11   running sums of patch q = jj * 4 + i  (i: 32 rows of m, jj: 32 columns of n)
+    v[16q : 16q+15]   q = 0..11   running sums of patch q = jj * 4 + i  (i: 32 rows of m, jj: 32 columns of n), four
+                                  registers for each of its four 16 x 16 quarters: 8 * (rows half) + 4 * (columns half)
     v192, v193                    LDS read addresses (A fragments, B fragments)
-    v[194:197]                    a_scale of the block, one value per patch row i
-    v198, v199                    the two b_scale values of the block (as read from LDS)
-    v200                          scale of the fold in progress (carried from block to block)
-    v[201:223]                    the compiler's (operands of the statement)
-    v[224:239], v[240:255]        block sums, set 0 / set 1 (patch p uses set p & 1)
-    a[8f : 8f+7]      f = 0..13   operand fragments: A(i, ks) = 2i + ks, B(jj, ks) = 8 + 2jj + ks
+    v[194:201]                    a_scale of the block, one value per 16 rows
+    v202, v203                    the two b_scale values of the block (as read from LDS)
+    v[204:205]                    scales of the fold in progress, per rows half (carried from block to block)
+    v[206:223]                    the compiler's (operands of the statement)
+    v[224:239], v[240:255]        block sums, set 0 / set 1 (patch p uses set p & 1), laid out like the running sums
+    a[8f : 8f+7]      f = 0..13   operand fragments, 16 rows x 128 k: A(i, h) = 2i + h, B(jj, h) = 8 + 2jj + h
     s[84:93]                      scratch scalars of the loop
 
-Schedule of one K block (MFMA g = 2p + ks; "gap g" = what is issued behind it)
+Schedule of one K block (two MFMAs g = 2p + h: rows half h of patch p against both columns halves; "gap g" = what is
+issued behind them)
     * patches column by column (jj outer); the fold of the patch before (16 FMAs: sums += scale *
       block sums) rides in this patch's two gaps, FOLD_EVEN of them in the first, after that gap's
       memory instructions (its block sums are only one MFMA old there);
@@ -31,7 +33,7 @@ Schedule of one K block (MFMA g = 2p + ks; "gap g" = what is issued behind it)
 LDS waits: reads return in order, so "at most N younger operations outstanding" (s_waitcnt lgkmcnt(N),
 N <= 15) is exact; N is derived below from the order of issue.  An MFMA's result may be read by an
 ordinary instruction MFMA_RESULT_SLOTS instructions later at the earliest (no interlock; the value is
-what the compiler pads a 16-pass MFMA with on this target): the FMAs of an even gap are padded with
+what the compiler pads a 16-pass MFMA with on this target, more than an 8-pass one needs): the FMAs of an even gap are padded with
 s_nop up to that distance, counted on the emitted text.
 """
 import sys
@@ -46,10 +48,10 @@ STAGE = 2 * MAT_A + 1024 + 256   # A rows, B rows, a_scale (1 KiB), b_scale (256
 NCOPY_AB = 8                # copy instructions per wave and matrix (128 rows * 256 B / 4 waves / 1 KiB)
 MFMA_RESULT_SLOTS = 20
 REFILL_SLOTS = 8             # instructions between an MFMA and a read that overwrites one of its operands
-FOLD_EVEN = 4               # FMAs of a fold placed in the even gap (the rest in the odd one)
-SCALE_OPS = 4
+FOLD_EVEN = 8               # FMAs of a fold placed in the even gap (the rest in the odd one)
+SCALE_OPS = 6
 BLK = (224, 240)
-V_ADDR_A, V_ADDR_B, V_SA, V_SB_LO, V_SB_HI, V_SC = 192, 193, 194, 198, 199, 200
+V_ADDR_A, V_ADDR_B, V_SA, V_SB_LO, V_SB_HI, V_SC = 192, 193, 194, 202, 203, 204
 S_SO, S_SO_NEXT, S_M0BASE, S_SOFF, S_SBLO, S_SBHI, S_SBJ, S_T0, S_T1 = 84, 85, 86, 88, 89, 90, 91, 92, 93
 
 
@@ -65,8 +67,8 @@ def piece_reg(f, t):
     return f"a[{8 * f + 2 * t}:{8 * f + 2 * t + 1}]"
 
 
-def piece_off(ks, t):
-    return (ks * 64 + 8 * t) * RS
+def piece_off(t):
+    return 8 * t * RS
 
 
 # ---- which LDS operations ride in which gap (program order inside the gap)
@@ -89,8 +91,8 @@ def gap_ops(g):
     if jj < NJ - 1:
         ops += [("B", jj + 1, u // 4, u % 4) for u in b_pieces_before_barrier(c)]
     else:
-        ops += [("A", c // 2, c % 2, t) for t in range(4)]
         ops += [("B", 0, u // 4, u % 4) for u in b0_pieces_behind_barrier(c)]
+        ops += [("A", c // 2, c % 2, t) for t in range(4)]
     return ops
 
 
@@ -114,7 +116,7 @@ def younger_ops(g, needed):
 def mfma_wait(g):
     p, ks = divmod(g, 2)
     jj, i = divmod(p, MI)
-    need = [("A", i, ks, t) for t in range(4)] + [("B", jj, ks, t) for t in range(4)]
+    need = [("A", i, ks, t) for t in range(4)] + [("B", jj, h, t) for h in range(2) for t in range(4)]
     return min(15, younger_ops(g, need))
 
 
@@ -186,29 +188,31 @@ def scale_copy(a):
 def fold_part(a, q, d, lo, hi):
     """elements lo .. hi-1 of: sums of patch q += scale * block sums in set d"""
     for r in range(lo, hi):
-        a(f"v_fmac_f32 v{16 * q + r}, v{V_SC}, v{BLK[d] + r}")
+        a(f"v_fmac_f32 v{16 * q + r}, v{V_SC + r // 8}, v{BLK[d] + r}")
 
 
 def lds_read_lines(op, jj):
     """instructions of one LDS operation of a gap in column jj"""
     if op[0] == "S":
         n = op[1]
-        if n == 0:
-            return [f"v_add_u32 v{V_SB_LO}, s{S_SO}, %[vaddr_s]",
-                    f"ds_read2_b32 v[{V_SA}:{V_SA + 1}], v{V_SB_LO} offset0:0 offset1:32"]
-        if n == 1:
-            return [f"ds_read2_b32 v[{V_SA + 2}:{V_SA + 3}], v{V_SB_LO} offset0:64 offset1:96"]
-        reg, name = (V_SB_LO, "sb_lo") if n == 2 else (V_SB_HI, "sb_hi")
+        if n < SCALE_OPS - 2:
+            pre = [f"v_add_u32 v{V_SB_LO}, s{S_SO}, %[vaddr_s]"] if n == 0 else []
+            return pre + [f"ds_read2_b32 v[{V_SA + 2 * n}:{V_SA + 2 * n + 1}], v{V_SB_LO} offset0:{32 * n} offset1:{32 * n + 16}"]
+        reg, name = (V_SB_LO, "sb_lo") if n == SCALE_OPS - 2 else (V_SB_HI, "sb_hi")
         return [f"s_add_u32 s{S_T0}, s{S_SO}, %[lds_{name}]", f"v_mov_b32 v{reg}, s{S_T0}",
                 f"ds_read_b32 v{reg}, v{reg}"]
     if op[0] == "B":
         _, bj, bks, bt = op
         src = S_SO_NEXT if jj == NJ - 1 else S_SO
-        pre = [f"v_add_u32 v{V_ADDR_B}, s{src}, %[vbase_b{bj}]"] if (bks, bt) == (0, 0) else []
-        return pre + [f"ds_read_b64_tr_b8 {piece_reg(frag_b(bj, bks), bt)}, v{V_ADDR_B} offset:{piece_off(bks, bt)}"]
+        pre = []
+        if bt == 0:  # the odd half's chunk is the even one's neighbour: bit 4 of the address
+            pre = [f"v_xor_b32 v{V_ADDR_B}, 16, v{V_ADDR_B}" if bks else f"v_add_u32 v{V_ADDR_B}, s{src}, %[vbase_b{bj}]"]
+        return pre + [f"ds_read_b64_tr_b8 {piece_reg(frag_b(bj, bks), bt)}, v{V_ADDR_B} offset:{piece_off(bt)}"]
     _, ai, aks, at = op
-    pre = [f"v_add_u32 v{V_ADDR_A}, s{S_SO_NEXT}, %[vbase_a{ai}]"] if (aks, at) == (0, 0) else []
-    return pre + [f"ds_read_b64_tr_b8 {piece_reg(frag_a(ai, aks), at)}, v{V_ADDR_A} offset:{piece_off(aks, at)}"]
+    pre = []
+    if at == 0:
+        pre = [f"v_xor_b32 v{V_ADDR_A}, 16, v{V_ADDR_A}" if aks else f"v_add_u32 v{V_ADDR_A}, s{S_SO_NEXT}, %[vbase_a{ai}]"]
+    return pre + [f"ds_read_b64_tr_b8 {piece_reg(frag_a(ai, aks), at)}, v{V_ADDR_A} offset:{piece_off(at)}"]
 
 
 def k_block(a, slots_before_first_fold):
@@ -234,7 +238,8 @@ def k_block(a, slots_before_first_fold):
             a(f"s_andn2_b32 s{S_T1}, s{S_SBLO}, %[hi_mask{pj}]")
             a(f"s_or_b32 s{S_SBJ}, s{S_T0}, s{S_T1}")
         if p >= 1:
-            a(f"v_mul_f32 v{V_SC}, s{S_SBJ}, v{V_SA + pq % MI}")
+            for h in range(2):
+                a(f"v_mul_f32 v{V_SC + h}, s{S_SBJ}, v{V_SA + 2 * (pq % MI) + h}")
         if jj == NJ - 1 and i == 0:
             a("s_waitcnt vmcnt(0) lgkmcnt(0)")
             a("s_barrier")
@@ -243,9 +248,11 @@ def k_block(a, slots_before_first_fold):
             c = g % GAPS_COL
             d = p & 1
             a(f"s_waitcnt lgkmcnt({mfma_wait(g)})")
-            last_mfma, this_mfma = this_mfma, len(a.lines)
-            a(f"v_mfma_f32_32x32x64_f8f6f4 v[{BLK[d]}:{BLK[d] + 15}], a[{8 * frag_b(jj, ks)}:{8 * frag_b(jj, ks) + 7}], "
-              f"a[{8 * frag_a(i, ks)}:{8 * frag_a(i, ks) + 7}], {'0' if ks == 0 else f'v[{BLK[d]}:{BLK[d] + 15}]'}")
+            last_mfma = this_mfma
+            for h in range(2):
+                this_mfma, reg = len(a.lines), BLK[d] + 8 * ks + 4 * h
+                a(f"v_mfma_f32_16x16x128_f8f6f4 v[{reg}:{reg + 3}], a[{8 * frag_b(jj, h)}:{8 * frag_b(jj, h) + 7}], "
+                  f"a[{8 * frag_a(i, ks)}:{8 * frag_a(i, ks) + 7}], 0")
             # ---- gap g.  Last column: the copies first (something must sit between the write of M0
             # and the load: a B read, else s_nop); the reads that refill the A fragment this MFMA is
             # reading come late in the gap (REFILL_SLOTS behind the MFMA at least, on top of the LDS
@@ -264,7 +271,7 @@ def k_block(a, slots_before_first_fold):
                         a(ln)
                     if b_reads:
                         a(b_reads.pop(0))
-                        if a.lines[-1].startswith("v_add_u32"):   # the add that feeds the read: take both
+                        if a.lines[-1].startswith(("v_add_u32", "v_xor_b32")):   # what feeds the read: take both
                             a(b_reads.pop(0))
                     else:
                         a("s_nop 0")
@@ -289,8 +296,9 @@ def k_block(a, slots_before_first_fold):
                 if spent < MFMA_RESULT_SLOTS:
                     a(f"s_nop {MFMA_RESULT_SLOTS - spent - 1}")
                 fold_part(a, pq, (p + 1) & 1, 0, FOLD_EVEN)
-    # scale of the last patch's fold, which rides on the next block's first MFMAs
-    a(f"v_mul_f32 v{V_SC}, s{S_SBJ}, v{V_SA + MI - 1}")
+    # scales of the last patch's fold, which rides on the next block's first MFMAs
+    for h in range(2):
+        a(f"v_mul_f32 v{V_SC + h}, s{S_SBJ}, v{V_SA + 2 * (MI - 1) + h}")
     for m in ("a", "b", "sc"):
         a(f"s_add_u32 %[off_{m}], %[off_{m}], %[str_{m}]")
     a(f"s_xor_b32 %[slot_off], %[slot_off], {STAGE}")
@@ -366,7 +374,7 @@ def emit_loop(out):
     w(f"// {STAGE}), toggled per block.  scale_kind: 0 = this wave copies a_scale, 1 = b_scale, else none.")
     w("__device__ __forceinline__ void w4_k_blocks(")
     w("    v32f& sums0, v32f& sums1, v32f& sums2, v32f& sums3, v32f& sums4, v32f& sums5, v32f& blk,")
-    w("    v32i& frag0, v32i& frag1, v32i& frag2, v16i& frag3, float& scale_carry,")
+    w("    v32i& frag0, v32i& frag1, v32i& frag2, v16i& frag3, v2f& scale_carry,")
     w("    uint32_t vbase_a0, uint32_t vbase_a1, uint32_t vbase_a2, uint32_t vbase_a3, uint32_t vbase_b0,")
     w("    uint32_t vbase_b1, uint32_t vbase_b2, uint32_t vaddr_s, uint32_t voff_a0, uint32_t voff_a1,")
     w("    uint32_t voff_b0, uint32_t voff_b1, uint32_t voff_sc, v4i rsrc_a, v4i rsrc_b, v4i rsrc_sc,")
@@ -379,7 +387,7 @@ def emit_loop(out):
     w(a.string(8))
     w('        : "+{v[0:31]}"(sums0), "+{v[32:63]}"(sums1), "+{v[64:95]}"(sums2), "+{v[96:127]}"(sums3),')
     w('          "+{v[128:159]}"(sums4), "+{v[160:191]}"(sums5), "+{v[224:255]}"(blk), "+{a[0:31]}"(frag0),')
-    w('          "+{a[32:63]}"(frag1), "+{a[64:95]}"(frag2), "+{a[96:111]}"(frag3), "+{v200}"(scale_carry),')
+    w('          "+{a[32:63]}"(frag1), "+{a[64:95]}"(frag2), "+{a[96:111]}"(frag3), "+{v[204:205]}"(scale_carry),')
     w('          [off_a] "+s"(off_a), [off_b] "+s"(off_b), [off_sc] "+s"(off_sc), [slot_off] "+s"(slot_off),')
     w('          [count] "+s"(count)')
     w('        : [vbase_a0] "v"(vbase_a0), [vbase_a1] "v"(vbase_a1), [vbase_a2] "v"(vbase_a2), [vbase_a3] "v"(vbase_a3),')
@@ -391,6 +399,7 @@ def emit_loop(out):
     w('          [lds_sb_lo] "s"(lds_sb_lo), [lds_sb_hi] "s"(lds_sb_hi), [hi_mask0] "s"(hi_mask0),')
     w('          [hi_mask1] "s"(hi_mask1), [hi_mask2] "s"(hi_mask2)')
     w('        : "memory", "scc", "v192", "v193", "v194", "v195", "v196", "v197", "v198", "v199",')
+    w('          "v200", "v201", "v202", "v203",')
     w('          "s84", "s85", "s86", "s87", "s88", "s89", "s90", "s91", "s92", "s93");')
     w("}")
 
@@ -401,10 +410,10 @@ def emit_first_reads(out):
         for op in gap_ops((NJ - 1) * GAPS_COL + c):
             if op[0] == "A":
                 _, ai, aks, at = op
-                a(f"ds_read_b64_tr_b8 {piece_reg(frag_a(ai, aks), at)}, %[vbase_a{ai}] offset:{piece_off(aks, at)}")
+                a(f"ds_read_b64_tr_b8 {piece_reg(frag_a(ai, aks), at)}, %[vbase_a{ai}{'x' * aks}] offset:{piece_off(at)}")
             else:
                 _, bj, bks, bt = op
-                a(f"ds_read_b64_tr_b8 {piece_reg(frag_b(bj, bks), bt)}, %[vbase_b0] offset:{piece_off(bks, bt)}")
+                a(f"ds_read_b64_tr_b8 {piece_reg(frag_b(bj, bks), bt)}, %[vbase_b0{'x' * bks}] offset:{piece_off(bt)}")
     w = out.append
     w("")
     w("// the fragments of the very first block, from ring slot 0, in the order the last column of a block")
@@ -417,7 +426,8 @@ def emit_first_reads(out):
     w(a.string(8))
     w('        : "+{a[0:31]}"(frag0), "+{a[32:63]}"(frag1), "+{a[64:95]}"(frag2), "+{a[96:111]}"(frag3)')
     w('        : [vbase_a0] "v"(vbase_a0), [vbase_a1] "v"(vbase_a1), [vbase_a2] "v"(vbase_a2), [vbase_a3] "v"(vbase_a3),')
-    w('          [vbase_b0] "v"(vbase_b0)')
+    w('          [vbase_b0] "v"(vbase_b0), [vbase_a0x] "v"(vbase_a0 ^ 16u), [vbase_a1x] "v"(vbase_a1 ^ 16u),')
+    w('          [vbase_a2x] "v"(vbase_a2 ^ 16u), [vbase_a3x] "v"(vbase_a3 ^ 16u), [vbase_b0x] "v"(vbase_b0 ^ 16u)')
     w('        : "memory");')
     w("}")
 
@@ -431,12 +441,12 @@ def emit_drain(out):
     w("")
     w("// the fold that a tile's last block leaves behind (its last patch, scale in scale_carry), behind")
     w("// the distance an MFMA result needs")
-    w("__device__ __forceinline__ void w4_last_fold(v32f& sums5, v32f& blk, float scale_carry)")
+    w("__device__ __forceinline__ void w4_last_fold(v32f& sums5, v32f& blk, v2f scale_carry)")
     w("{")
     w("    asm volatile(")
     w(a.string(8))
     w('        : "+{v[160:191]}"(sums5), "+{v[224:255]}"(blk)')
-    w('        : "{v200}"(scale_carry));')
+    w('        : "{v[204:205]}"(scale_carry));')
     w("}")
 
 

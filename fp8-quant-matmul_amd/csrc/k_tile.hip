@@ -9,13 +9,16 @@
 //     the transposing reads below bank-conflict free (measured: 0 conflicts).
 //   * Operands are fetched with ds_read_b64_tr_b8: 16 lanes read an 8(k) x 16(m|n) byte
 //     patch and receive it transposed, i.e. lane i holds 8 consecutive k of column i.  Four
-//     such reads give the 32 bytes per lane that v_mfma_f32_32x32x64_f8f6f4 consumes.
+//     such reads give the 32 bytes per lane that v_mfma_f32_16x16x128_f8f6f4 consumes.
 //     The k order inside the instruction is permuted identically for both operands, which
 //     leaves the dot product unchanged.
-//   * Two MFMAs (K = 64 each) cover a 128-wide scale block of one 32x32 patch; the block sum
-//     lives in 16 registers for a moment and is folded into the running result with
+//   * One MFMA covers a 128-wide scale block of one 16x16 patch; the block sum
+//     lives in 4 registers for a moment and is folded into the running result with
 //     a_scale[kb][m] * b_scale[kb][n/128] by one FMA per element (mn_large.hip:100-106,
-//     mn_small.hip:85-88 do the same with a second full-size accumulator).
+//     mn_small.hip:85-88 do the same with a second full-size accumulator).  Why this instruction and not two of
+//     32x32x64: with the fold beside them, on operands of quantised normal values, nothing else in the loop, it
+//     sustains 65.5 % of the peak against 58.2 % (78.6 against 74.2 % on constant operands: the rest is power), from as
+//     many LDS reads; its block sums are as far from the exact ones (2-norm 1.3e-5 and 2.3e-5 with outliers, both).
 //   * The MFMA computes the transposed patch (rows = n, columns = m) as mn_small.hip does,
 //     so that a lane owns one m (one a_scale value) and runs of 4 consecutive n.
 //   * The finished tile goes through the idle LDS ring (row-major, padded rows) and leaves as
@@ -72,8 +75,8 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
     constexpr int NCW = WM * WN;
     static_assert(NS >= 2 && NS <= 4, "two to four LDS stages");
     constexpr int TM = BM / WM, TN = BN / WN;      // wave tile
-    constexpr int MI = TM / 32, NJ = TN / 32;      // 32x32 patches per wave
-    static_assert(TM % 32 == 0 && TN % 32 == 0, "wave tile is made of 32x32 patches");
+    constexpr int MI = TM / 16, NJ = TN / 16;      // 16x16 patches per wave
+    static_assert(TM % 16 == 0 && TN % 32 == 0, "wave tile is made of 16x16 patches, pairs of them along n");
     static_assert(TN <= 128, "a wave's n range touches at most two 128-wide scale blocks");
     static_assert(BM <= 256 && BN <= 256, "LDS rows hold at most 256 bytes");
     constexpr int RSA = S::RSA, RSB = S::RSB, NA = S::NA, NB = S::NB, NCOPY = S::NCOPY;
@@ -128,14 +131,14 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
 #pragma unroll
     for (int q = 0; q < S::NVA; ++q) {
         const int r = (NA * wave + q) * (1024 / RSA) + S::template copy_row<RSA>(lane);
-        const int cc = S::template copy_pos<RSA>(lane) ^ row_swizzle<RSA>(r & 7);
+        const int cc = S::template copy_pos<RSA>(lane) ^ row_swizzle<RSA>(r);
         const bool ok = (16 * cc < BM) && (m0 + 16 * cc < M);
         voff_a[q] = ok ? (uint32_t)(r * lda + m0 + 16 * cc) : 0x80000000u;
     }
 #pragma unroll
     for (int q = 0; q < S::NVB; ++q) {
         const int r = (NBW * wave + q) * (1024 / RSB) + S::template copy_row<RSB>(lane);
-        const int cc = S::template copy_pos<RSB>(lane) ^ row_swizzle<RSB>(r & 7);
+        const int cc = S::template copy_pos<RSB>(lane) ^ row_swizzle<RSB>(r);
         const bool ok = (16 * cc < BN) && (n0 + 16 * cc < N);
         voff_b[q] = ok ? (uint32_t)(r * N + n0 + 16 * cc) : 0x80000000u;
     }
@@ -156,7 +159,7 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
 #pragma unroll
         for (int q = 0; q < NAW; ++q) {
             const int r = (a_first + q) * (1024 / RSA) + S::template copy_row<RSA>(lane);
-            const int cc = S::template copy_pos<RSA>(lane) ^ row_swizzle<RSA>(r & 7);
+            const int cc = S::template copy_pos<RSA>(lane) ^ row_swizzle<RSA>(r);
             const bool ok = (16 * cc < BM) && (m0 + 16 * cc < M);
             off_a[q] = (uint32_t)r * (uint32_t)M + (uint32_t)(ok ? m0 + 16 * cc : m0);
         }
@@ -200,6 +203,8 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
                       (uint32_t)(kb * KBLOCK + S::template extra_rows<RSA>(q)) * (uint32_t)lda);
         } else if (q < NA + NB) {
             copy_b(stage, kb, q - NA);
+        } else if (SCALE_WAVE == 0) {
+            lds_dma16_unless((uint32_t)wave, rsrc_s, voff_s, stage + S::SCALE_OFF, (uint32_t)kb * (uint32_t)lda * 4u);
         } else if (wave == SCALE_WAVE) {
             lds_dma16(rsrc_s, voff_s, stage + S::SCALE_OFF, (uint32_t)kb * (uint32_t)lda * 4u);
         } else if (S::SB_STAGED && wave == SCALE_WAVE + 1) {
@@ -218,53 +223,34 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
             lds_dma4(rsrc_bs, voff_sb, stage + S::SB_OFF, (uint32_t)kb * (uint32_t)sn * 4u);
     };
 
-    // ---- transposing LDS reads.  Lane l = 16*g + i feeds MFMA row/column (l & 31) and k half
-    // (l >> 5).  For K step ks (64 wide) read t of the lane covers k rows
-    // 64*ks + 32*(g>>1) + 8*t + (i>>1), 8-byte half (i & 1) of 16-byte chunk (patch chunk + (g&1)).
-    // (row & 7) = (i >> 1) does not depend on t or ks: one address per patch plus immediates.
-    const int g4 = lane >> 4, i16 = lane & 15;
+    // ---- transposing LDS reads: one address per patch row and column (frag_addr)
     uint32_t addr_a[MI], addr_b[NJ];
 #pragma unroll
     for (int i = 0; i < MI; ++i)
-        addr_a[i] = (uint32_t)((32 * (g4 >> 1) + (i16 >> 1)) * RSA + (i16 & 1) * 8 +
-                               ((((wm * TM) / 16 + 2 * i + (g4 & 1)) ^ row_swizzle<RSA>(i16 >> 1)) * 16));
+        addr_a[i] = frag_addr<RSA>(lane, (wm * TM) / 16 + i);
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
-        addr_b[j] = (uint32_t)(S::MAT_A + (32 * (g4 >> 1) + (i16 >> 1)) * RSB + (i16 & 1) * 8 +
-                               ((((wn * TN) / 16 + 2 * j + (g4 & 1)) ^ row_swizzle<RSB>(i16 >> 1)) * 16));
-    const uint32_t addr_s = S::SCALE_OFF + (uint32_t)((wm * TM + (lane & 31)) * 4);
+        addr_b[j] = S::MAT_A + frag_addr<RSB>(lane, (wn * TN) / 16 + j);
+    const uint32_t addr_s = S::SCALE_OFF + (uint32_t)((wm * TM + (lane & 15)) * 4);
 
-    // 32 bytes per lane of one operand for K step ks; rs = row stride of the matrix read
-    auto read_frag = [&](uint32_t addr, int ks, int rs) __attribute__((always_inline)) -> v8i {
-        const uint32_t base = addr + (uint32_t)(ks * 64 * rs);
-        v2i r0 = __builtin_amdgcn_ds_read_tr8_b64_v2i32(LDS_PTR(v2i, lds + base));
-        v2i r1 = __builtin_amdgcn_ds_read_tr8_b64_v2i32(LDS_PTR(v2i, lds + base + 8 * rs));
-        v2i r2 = __builtin_amdgcn_ds_read_tr8_b64_v2i32(LDS_PTR(v2i, lds + base + 16 * rs));
-        v2i r3 = __builtin_amdgcn_ds_read_tr8_b64_v2i32(LDS_PTR(v2i, lds + base + 24 * rs));
-        return (v8i){r0.x, r0.y, r1.x, r1.y, r2.x, r2.y, r3.x, r3.y};
-    };
-
-    // ---- scales.  One a_scale per lane and 32-row patch (the lane's m).  A wave's n range is at
-    // most 128 wide, so it touches at most two 128-wide b_scale blocks (nb_lo, nb_hi); a 32-wide
-    // patch never straddles a block boundary.
+    // ---- scales.  One a_scale per lane and 16-row patch (the lane's m).  A wave's n range is at
+    // most 128 wide, so it touches at most two 128-wide b_scale blocks (nb_lo, nb_hi); a pair of
+    // patch columns (32 wide) never straddles a block boundary.
     const int n_wave = n0 + wn * TN;
     int nb_lo = n_wave >> 7, nb_hi = (n_wave + TN - 1) >> 7;
     nb_lo = nb_lo < sn ? nb_lo : sn - 1;
     nb_hi = nb_hi < sn ? nb_hi : sn - 1;
-    uint32_t hi_mask[NJ];  // all ones when patch j lies in the wave's second b_scale block
+    uint32_t hi_mask[NJ / 2];  // all ones when patch columns 2 j and 2 j + 1 lie in the wave's second b_scale block
 #pragma unroll
-    for (int j = 0; j < NJ; ++j)
+    for (int j = 0; j < NJ / 2; ++j)
         hi_mask[j] = (uint32_t)-(int)(((n_wave + 32 * j) >> 7) > (n_wave >> 7));
 
-    v16f acc[MI][NJ];
+    v4f acc[MI][NJ];
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
         for (int j = 0; j < NJ; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r)
-                acc[i][j][r] = 0.f;
-    const v16f zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+            acc[i][j] = (v4f){0.f, 0.f, 0.f, 0.f};
 
     // ---- prologue: the first NS-1 K blocks go into ring slots 0 .. NS-2
 #pragma unroll
@@ -345,79 +331,78 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
         if (!S::SB_STAGED)
             asm volatile("" ::"s"(sb_lo), "s"(sb_hi));
         const uint32_t so = (uint32_t)(slot * S::STAGE);
-        const float sb_stage = S::SB_STAGED ? *LDS_PTR(float, lds + so + S::SB_OFF) : 0.f;
-        float sa[MI];
+        // The first column's fragments of B and all of A's, then the second column's; the later ones a column ahead.
+        v8i fa[MI], fb[NJ];
+        fb[0] = read_frag<RSB>(lds + (addr_b[0] + so));
 #pragma unroll
         for (int i = 0; i < MI; ++i)
-            sa[i] = *LDS_PTR(float, lds + so + addr_s + 128 * i);
-
-        v8i fa[MI][2];
+            fa[i] = read_frag<RSA>(lds + (addr_a[i] + so));
+        if (NJ > 1)
+            fb[1] = read_frag<RSB>(lds + (addr_b[1] + so));
+        const float sb_stage = S::SB_STAGED ? *LDS_PTR(float, lds + so + S::SB_OFF) : 0.f;
+        float sa[MI], sc[MI];
 #pragma unroll
-        for (int i = 0; i < MI; ++i) {
-            fa[i][0] = read_frag(addr_a[i] + so, 0, RSA);
-            fa[i][1] = read_frag(addr_a[i] + so, 1, RSA);
-        }
+        for (int i = 0; i < MI; ++i)
+            sa[i] = *LDS_PTR(float, lds + so + addr_s + 64 * i);
 
-        // the wave's NCOPY copy instructions of block kb+NS-1 ride on the first MFMAs
-        constexpr int N_MFMA = MI * NJ * 2;
-        constexpr int PER_MFMA = (NCOPY + N_MFMA - 1) / N_MFMA;  // copies behind each MFMA
-        int cq = 0;
-        auto copy_slot = [&](int n) {
-            if (RAGGED) {
-                if (cq == 0 && loads_a && A_EARLY)
-                    next_a();
-                if (cq == 0 && !loads_a && more)
-                    copy_all(slot_fill, kb + NS - 1);
-                cq = NCOPY;
-                return;
+        // MFMA number t multiplies patch (t % MI, t / MI).  Patches are folded LAG MFMAs behind their own, in the order that
+        // stands here (the next MFMA's operand passes through the fold's empty asm statement).  The wave's copy instructions
+        // of block kb + NS - 1 ride on the first MFMAs.
+        constexpr int T = MI * NJ, PER_MFMA = (NCOPY + T - 1) / T;
+        // two patch rows: six behind where there are that many (128x192: 300 x 12288 x 2048 17.16 -> 17.02 us, four behind 17.05)
+        constexpr int LAG = MI < 4 && T >= 12 ? 6 : MI;
+        v4f blk[LAG];
+        auto fold = [&](int t) __attribute__((always_inline)) {
+            if (t % MI == 0) {
+                // wave-uniform choice of the b_scale value on the scalar unit (bit select), then one product per patch
+                const float sbj = __uint_as_float((__float_as_uint(sb_hi) & hi_mask[t / MI / 2]) |
+                                                  (__float_as_uint(sb_lo) & ~hi_mask[t / MI / 2]));
+#pragma unroll
+                for (int i = 0; i < MI; ++i)
+                    sc[i] = sa[i] * (S::SB_STAGED ? sb_stage : sbj);
             }
 #pragma unroll
-            for (int u = 0; u < NCOPY; ++u)
-                if (u < n && cq < NCOPY) {
-                    if (more)
-                        copy_step(slot_fill, kb + NS - 1, cq);
-                    ++cq;
-                }
+            for (int e = 0; e < 4; ++e)
+                acc[t % MI][t / MI][e] = fmaf(sc[t % MI], blk[t % LAG][e], acc[t % MI][t / MI][e]);
         };
-
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-            const v8i fb0 = read_frag(addr_b[j] + so, 0, RSB);
-            const v8i fb1 = read_frag(addr_b[j] + so, 1, RSB);
-            v16f blk[MI];
-#pragma unroll
-            for (int i = 0; i < MI; ++i) {
-                blk[i] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fb0, fa[i][0], zero16, 0, 0, 0,
-                                                                          0, 0, 0);
-                copy_slot(PER_MFMA);
+        for (int t = 0; t < T; ++t) {
+            if (t % MI == 0 && t > 0 && t / MI + 1 < NJ)
+                fb[t / MI + 1] = read_frag<RSB>(lds + (addr_b[t / MI + 1] + so));
+            if (t >= LAG) {
+                fold(t - LAG);
+                if (t + 1 < T)
+                    asm volatile("" : "+v"(acc[(t - LAG) % MI][(t - LAG) / MI]), "+v"(fa[(t + 1) % MI]));
             }
+            blk[t % LAG] = block_sum(fb[t / MI], fa[t % MI]);
+            if (RAGGED) {
+                if (t == 0) {
+                    if (loads_a && A_EARLY)
+                        next_a();
+                    if (!loads_a && more)
+                        copy_all(slot_fill, kb + NS - 1);
+                }
+            } else if (more) {
 #pragma unroll
-            for (int i = 0; i < MI; ++i) {
-                blk[i] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fb1, fa[i][1], blk[i], 0, 0, 0,
-                                                                          0, 0, 0);
-                copy_slot(PER_MFMA);
+                for (int q = t * PER_MFMA; q < (t + 1) * PER_MFMA; ++q)
+                    if (q < NCOPY)
+                        copy_step(slot_fill, kb + NS - 1, q);
             }
-            if (j == NJ - 1 && !S::SB_STAGED) {
+            if (t == T - 1 && !S::SB_STAGED) {
                 // the next block's b_scale, behind this block's last LDS read: its trip to the L2 (a block's values share
-                // no cache line with the next one's unless N is small) is covered by the fold and the barrier
+                // no cache line with the next one's unless N is small) is covered by the folds and the barrier
                 int next = kb + 1 < kb1 ? kb + 1 : kb;
                 asm volatile("" : "+s"(next));
                 next_lo = b_scale[next * sn + nb_lo];
                 next_hi = b_scale[next * sn + nb_hi];
             }
-#pragma unroll
-            for (int i = 0; i < MI; ++i) {
-                // wave-uniform choice of the b_scale value on the scalar unit (bit select), then one
-                // product per patch
-                const float sbj = __uint_as_float((__float_as_uint(sb_hi) & hi_mask[j]) |
-                                                  (__float_as_uint(sb_lo) & ~hi_mask[j]));
-                const float sc = sa[i] * (S::SB_STAGED ? sb_stage : sbj);
-#pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    acc[i][j][r] = fmaf(sc, blk[i][r], acc[i][j][r]);
-            }
+            __builtin_amdgcn_sched_barrier(0);
         }
-        copy_slot(NCOPY);  // whatever is left (tiles with few MFMAs per K block)
+#pragma unroll
+        for (int t = T - LAG; t < T; ++t) {
+            fold(t);
+            asm volatile("" : "+v"(acc[t % MI][t / MI]));
+        }
         if (!A_EARLY)
             next_a();
 
@@ -476,68 +461,60 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
     // they are acknowledged).  A wave that has polled for a second gives up and
     // writes NaN.
     bool as_partial = SPLIT;
-    constexpr int PATCHES = NCW * MI * NJ;  // 32x32 patches of a tile: 4 KiB of fp32 each
+    constexpr int PATCHES = NCW * MI * NJ;  // 16x16 patches of a tile: 1 KiB of fp32 each
     const int senders = (int)gridDim.y - 1;
-    const size_t first = ((size_t)pid * senders * PATCHES + (size_t)wave * (MI * NJ)) * 256;  // in 16-byte units
-    const uint32_t mail_span = (uint32_t)senders * PATCHES * 4096u;
-    auto mail_at = [&](int z, int patch, int q) __attribute__((always_inline)) {
-        return (uint32_t)(((z * PATCHES + patch) * 4 + q) * 64 + lane) * 16u;
+    const size_t first = ((size_t)pid * senders * PATCHES + (size_t)wave * (MI * NJ)) * 64;  // in 16-byte units
+    const uint32_t mail_span = (uint32_t)senders * PATCHES * 1024u;
+    auto mail_at = [&](int z, int patch) __attribute__((always_inline)) {
+        return (uint32_t)((z * PATCHES + patch) * 64 + lane) * 16u;
     };
     if constexpr (SPLIT) {
         if (mailbox != nullptr) {
             as_partial = false;
             if ((int)blockIdx.y < senders) {
                 if (compute) {
-                    v4i* mine = reinterpret_cast<v4i*>(mailbox) + first + (size_t)blockIdx.y * PATCHES * 256 + lane;
+                    v4i* mine = reinterpret_cast<v4i*>(mailbox) + first + (size_t)blockIdx.y * PATCHES * 64 + lane;
 #pragma unroll
                     for (int i = 0; i < MI; ++i)
 #pragma unroll
-                        for (int j = 0; j < NJ; ++j)
+                        for (int j = 0; j < NJ; ++j) {
+                            v4i bits = __builtin_bit_cast(v4i, acc[i][j]);
 #pragma unroll
-                            for (int q = 0; q < 4; ++q) {
-                                v4i bits;
-#pragma unroll
-                                for (int e = 0; e < 4; ++e) {
-                                    const int w = (int)__float_as_uint(acc[i][j][4 * q + e]);
-                                    bits[e] = w == 0 ? (int)0x80000000 : w;
-                                }
-                                mine[((i * NJ + j) * 4 + q) * 64] = bits;
-                            }
+                            for (int e = 0; e < 4; ++e)
+                                bits[e] = bits[e] == 0 ? (int)0x80000000 : bits[e];
+                            mine[(i * NJ + j) * 64] = bits;
+                        }
                 }
                 return;
             }
             if (compute) {
-                // PG patches at a time (all of them when there are at most two: one trip to the L2 for everything that is
-                // there), ZB splits at a time
-                constexpr int PG = MI * NJ <= 2 ? MI * NJ : 1, ZB = MI * NJ == 1 ? 3 : 2;
+                // PG patches at a time (all of them when there are at most eight: one trip to the L2 for everything that
+                // is there), ZB splits at a time
+                constexpr int PG = MI * NJ <= 8 ? MI * NJ : 4, ZB = MI * NJ <= 4 ? 3 : 2;
+                static_assert(MI * NJ % PG == 0, "whole groups of patches");
                 const __amdgpu_buffer_rsrc_t rp = make_rsrc(reinterpret_cast<const v4i*>(mailbox) + first, mail_span);
                 const unsigned long long t_first = __builtin_amdgcn_s_memrealtime();
                 bool gave_up = false;
 #pragma unroll
                 for (int pg = 0; pg < MI * NJ; pg += PG) {
-                    v4f sum[PG][4];
+                    v4f sum[PG];
                     auto gather = [&](auto count, int z0) __attribute__((always_inline)) {  // splits z0 .. z0 + ZC - 1
                         constexpr int ZC = decltype(count)::value;
-                        v4i v[ZC][PG][4];
+                        v4i v[ZC][PG];
                         for (;;) {
                             asm volatile("" ::: "memory");  // the loads belong to this round of the loop
 #pragma unroll
                             for (int z = 0; z < ZC; ++z)
 #pragma unroll
                                 for (int g = 0; g < PG; ++g)
-#pragma unroll
-                                    for (int q = 0; q < 4; ++q)
-                                        v[z][g][q] = __builtin_amdgcn_raw_buffer_load_b128(
-                                            rp, mail_at(z0 + z, pg + g, q), 0, 16);
+                                    v[z][g] = __builtin_amdgcn_raw_buffer_load_b128(rp, mail_at(z0 + z, pg + g), 0, 16);
                             bool missing = false;
 #pragma unroll
                             for (int z = 0; z < ZC; ++z)
 #pragma unroll
                                 for (int g = 0; g < PG; ++g)
-#pragma unroll
-                                    for (int q = 0; q < 4; ++q)
-                                        missing = missing | (v[z][g][q][0] == 0) | (v[z][g][q][1] == 0) |
-                                                  (v[z][g][q][2] == 0) | (v[z][g][q][3] == 0);
+                                    missing = missing | (v[z][g][0] == 0) | (v[z][g][1] == 0) | (v[z][g][2] == 0) |
+                                              (v[z][g][3] == 0);
                             if (__builtin_amdgcn_ballot_w64(missing) == 0)
                                 break;
                             if (__builtin_amdgcn_s_memrealtime() - t_first > 100000000ull) {  // one second at 100 MHz
@@ -548,12 +525,10 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
 #pragma unroll
                         for (int z = 0; z < ZC; ++z)
 #pragma unroll
-                            for (int g = 0; g < PG; ++g)
-#pragma unroll
-                                for (int q = 0; q < 4; ++q) {
-                                    const v4f f = __builtin_bit_cast(v4f, v[z][g][q]);
-                                    sum[g][q] = z0 + z == 0 ? f : sum[g][q] + f;
-                                }
+                            for (int g = 0; g < PG; ++g) {
+                                const v4f f = __builtin_bit_cast(v4f, v[z][g]);
+                                sum[g] = z0 + z == 0 ? f : sum[g] + f;
+                            }
                     };
                     int z0 = 0;
                     for (; z0 + ZB <= senders; z0 += ZB)
@@ -565,34 +540,31 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
                     if (z0 < senders)
                         gather(std::integral_constant<int, 1>{}, z0);
 #pragma unroll
-                    for (int g = 0; g < PG; ++g)
+                    for (int g = 0; g < PG; ++g) {
+                        v4f& own = acc[(pg + g) / NJ][(pg + g) % NJ];
 #pragma unroll
-                        for (int q = 0; q < 4; ++q)
-#pragma unroll
-                            for (int e = 0; e < 4; ++e) {
-                                v16f& own = acc[(pg + g) / NJ][(pg + g) % NJ];
-                                own[4 * q + e] = gave_up ? __builtin_nanf("") : sum[g][q][e] + own[4 * q + e];
-                            }
+                        for (int e = 0; e < 4; ++e)
+                            own[e] = gave_up ? __builtin_nanf("") : sum[g][e] + own[e];
+                    }
                 }
             }
         }
     }
 
-    // ---- epilogue.  A lane owns row m = .. + (lane & 31) and, per patch, four runs of 4 columns
-    // (accumulator register 4*q + e is column 8*q + 4*(lane >> 5) + e of the patch): stored
-    // straight from the registers that would be 8- or 16-byte pieces of 32 different rows per
-    // instruction.  The tile therefore goes through the (now idle) LDS ring, row-major with a
+    // ---- epilogue.  A lane owns row m = .. + (lane & 15) and, per patch, a run of 4 columns, 4 * (lane >> 4)
+    // of the patch: stored straight from the registers that would be 8- or 16-byte pieces of 16 different
+    // rows per instruction.  The tile therefore goes through the (now idle) LDS ring, row-major with a
     // padded row stride that keeps the writes conflict free, and leaves as 16 bytes per lane
     // along whole rows of the tile.  A tile larger than the ring is written in two halves.
     // PARTIAL = fp32 into this split's partial tile (the reduction kernel follows), else bf16 into c.
     auto write_tile = [&](auto partial_tag) __attribute__((always_inline)) {
         constexpr bool PARTIAL = decltype(partial_tag)::value;
         constexpr int ESZ = PARTIAL ? 4 : 2;
-        constexpr int CROW = BN * ESZ + (PARTIAL ? 16 : 8);  // LDS bytes per tile row
+        constexpr int CROW = BN * ESZ + 16;                 // LDS bytes per tile row
         constexpr int HALVES = (BM * CROW <= S::LDS_BYTES) ? 1 : 2;
         constexpr int HROWS = BM / HALVES;
         static_assert(HROWS * CROW <= S::LDS_BYTES, "half a tile must fit the ring");
-        static_assert(HROWS % 32 == 0, "a 32-row patch lies in one half");
+        static_assert(HROWS % 16 == 0, "a patch lies in one half");
         constexpr int CPR = BN * ESZ / 16;                 // 16-byte chunks per tile row
         constexpr int CHUNKS = HROWS * CPR;
 #pragma unroll
@@ -600,23 +572,20 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
             __syncthreads();  // nobody reads the ring (or the previous half) any more
 #pragma unroll
             for (int i = 0; i < MI; ++i) {
-                const int prow = wm * TM + 32 * i;  // first tile row of the patch
+                const int prow = wm * TM + 16 * i;  // first tile row of the patch
                 if (compute && prow / HROWS == h) {
-                    const uint32_t rbase = (uint32_t)((prow - h * HROWS + (lane & 31)) * CROW);
+                    const uint32_t rbase = (uint32_t)((prow - h * HROWS + (lane & 15)) * CROW);
 #pragma unroll
-                    for (int j = 0; j < NJ; ++j)
-#pragma unroll
-                        for (int q = 0; q < 4; ++q) {
-                            const int col = wn * TN + 32 * j + 8 * q + 4 * (lane >> 5);
-                            const v4f v = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2],
-                                           acc[i][j][4 * q + 3]};
-                            if (PARTIAL) {
-                                *LDS_PTR(v4f, lds + rbase + col * 4) = v;
-                            } else {
-                                v2i pk = {(int)pack_bf16x2(v[0], v[1]), (int)pack_bf16x2(v[2], v[3])};
-                                *LDS_PTR(v2i, lds + rbase + col * 2) = pk;
-                            }
+                    for (int j = 0; j < NJ; ++j) {
+                        const int col = wn * TN + 16 * j + 4 * (lane >> 4);
+                        const v4f v = acc[i][j];
+                        if (PARTIAL) {
+                            *LDS_PTR(v4f, lds + rbase + col * 4) = v;
+                        } else {
+                            v2i pk = {(int)pack_bf16x2(v[0], v[1]), (int)pack_bf16x2(v[2], v[3])};
+                            *LDS_PTR(v2i, lds + rbase + col * 2) = pk;
                         }
+                    }
                 }
             }
             __syncthreads();
@@ -632,9 +601,7 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
                         const v4f v = *LDS_PTR(v4f, lds + row * CROW + ch * 16);
                         *reinterpret_cast<v4f*>(partial + (size_t)blockIdx.y * M * N + o) = v;
                     } else {
-                        const v2i lo = *LDS_PTR(v2i, lds + row * CROW + ch * 16);
-                        const v2i hi = *LDS_PTR(v2i, lds + row * CROW + ch * 16 + 8);
-                        *reinterpret_cast<v4i*>(c + o) = (v4i){lo.x, lo.y, hi.x, hi.y};
+                        *reinterpret_cast<v4i*>(c + o) = *LDS_PTR(v4i, lds + row * CROW + ch * 16);
                     }
                 }
             }
@@ -650,9 +617,7 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
                 for (int z = 0; z < senders; ++z)
 #pragma unroll
                     for (int patch = 0; patch < MI * NJ; ++patch)
-#pragma unroll
-                        for (int q = 0; q < 4; ++q)
-                            __builtin_amdgcn_raw_buffer_store_b128((v4i){0, 0, 0, 0}, rp, mail_at(z, patch, q), 0, 0);
+                        __builtin_amdgcn_raw_buffer_store_b128((v4i){0, 0, 0, 0}, rp, mail_at(z, patch), 0, 0);
             }
         }
     } else {

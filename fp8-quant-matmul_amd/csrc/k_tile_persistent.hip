@@ -24,21 +24,10 @@ namespace {
 
 #include "w4_loop.inc"
 
-// One problem of a grouped launch as the kernel sees it.
-struct Problem {
-    const uint8_t* a;
-    const uint8_t* b;
-    const float* a_scale;
-    const float* b_scale;
-    uint16_t* c;
-    int M;
-    int lda;  // elements between consecutive k-rows of a and of a_scale (>= M, a multiple of 16)
-};
-
 // GROUPED = false: one problem (`one`), tiles_m x tiles_n tiles.  GROUPED = true: the problems of
 // `tab` (same N and K, own M), whose tiles are numbered one group after the other.
 template <int BM, int BN, int WM, int WN, int NS, int PR, bool GROUPED>
-__device__ __forceinline__ void persistent_body(const Problem& one, const GroupTable* tab, int N, int K,
+__device__ __forceinline__ void persistent_body(const TileProblem& one, const GroupTable* tab, int N, int K,
                                                 int tiles_m, int tiles_n)
 {
     constexpr int NW = WM * WN;    // waves per workgroup; four = one wave per SIMD (k_block_w4)
@@ -47,19 +36,19 @@ __device__ __forceinline__ void persistent_body(const Problem& one, const GroupT
     static_assert(NW == 8 || NW == 4, "eight or four waves per workgroup");
     static_assert(NS >= 2 && NS <= 4, "two to four LDS stages");
     constexpr int TM = BM / WM, TN = BN / WN;
-    constexpr int MI = TM / 32, NJ = TN / 32;
+    constexpr int MI = TM / 16, NJ = TN / 16;  // 16x16 patches
     static_assert(TM % 32 == 0 && TN % 32 == 0 && TN <= 128 && BM <= 256 && BN <= 256, "wave tile");
     constexpr int RSA = S::RSA, RSB = S::RSB, NA = S::NA, NB = S::NB, NCOPY = S::NCOPY;
-    constexpr int CROW = BN * 2 + 8;          // staging bytes per tile row (conflict-free writes)
-    static_assert(PR % 32 == 0 && BM % PR == 0, "a piece is a whole number of 32-row patches");
+    // Staging bytes per tile row.  16 rows x two 8-byte pieces of one chunk are written together: the chunks of a row are
+    // permuted by the row (staged_chunk) so that they lie in different banks without any padding.
+    constexpr int CROW = BN * 2;
+    static_assert(BN % 128 == 0 || BN % 128 == 64, "rows that start on a multiple of half the banks");
+    static_assert(PR % 16 == 0 && BM % PR == 0, "a piece is a whole number of patches");
     static_assert(PR * CROW <= S::STAGE, "a piece must fit one ring slot");
     // four waves: the finished tile is staged beside the ring, which then never pauses
     constexpr int STAGING_W4 = NS * S::STAGE;
     static_assert(NW == 8 || STAGING_W4 + PR * CROW <= 160 * 1024, "ring and staging area exceed the LDS");
     constexpr int CPR = BN / 8;               // 16-byte chunks per tile row
-    // fold of a patch column under the next column's MFMAs: pays for the 2 x 3 patches of the
-    // 256 x 192 tile (4 % there), not for the smaller wave tiles (0 to -2 %)
-    constexpr bool PIPELINED_FOLD = MI * NJ >= 6;
     constexpr int CHUNKS = PR * CPR;
 
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
@@ -70,48 +59,17 @@ __device__ __forceinline__ void persistent_body(const Problem& one, const GroupT
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave % WM, wn = wave / WM;
 
-    // ---- this workgroup's tiles.  Workgroup ids go round the 8 XCDs (id % 8); each XCD owns
-    // a contiguous run of the tile order (groups of GROUP_M tile rows, as in k_tile.hip) and
-    // its workgroups take the run's tiles in turn, so that the tiles an XCD works on at any
-    // moment are neighbours and share A and B panels in its L2.
-    const int T = GROUPED ? tab->tile_start[tab->groups] : tiles_m * tiles_n;
-    const int pid = blockIdx.x, per_xcd = gridDim.x >> 3;  // gridDim.x is a multiple of 8
-    const int xcd = pid & 7, q8 = T >> 3, r8 = T & 7;
-    const int run0 = xcd * q8 + (xcd < r8 ? xcd : r8);
-    const int run_len = q8 + (xcd < r8 ? 1 : 0);
-    const int li = pid >> 3;
-    const int n_my = li < run_len ? (run_len - li + per_xcd - 1) / per_xcd : 0;
+    const TileWalk<BM, BN, GROUPED> walk(one, tab, tiles_m, tiles_n);
+    const int n_my = walk.count();
     if (n_my == 0)
         return;
-    const int per_group = GROUP_M * tiles_n;
-    // tile number j of this workgroup: its problem and its origin in that problem's C
-    auto tile_origin = [&](int j, Problem& pr, int& m0, int& n0) __attribute__((always_inline)) {
-        int logical = run0 + li + j * per_xcd;
-        int tm = tiles_m;
-        if (GROUPED) {
-            int g = 0;
-            while (g + 1 < tab->groups && logical >= tab->tile_start[g + 1])
-                ++g;
-            logical -= tab->tile_start[g];
-            pr = Problem{tab->a[g], tab->b[g], tab->a_scale[g], tab->b_scale[g], tab->c[g], tab->m[g], tab->lda[g]};
-            tm = (pr.M + BM - 1) / BM;
-        } else {
-            pr = one;
-        }
-        const int group = logical / per_group;
-        const int first_m = group * GROUP_M;
-        const int gsz = (tm - first_m < GROUP_M) ? (tm - first_m) : GROUP_M;
-        const int in_group = logical - group * per_group;
-        m0 = (first_m + in_group % gsz) * BM;
-        n0 = (in_group / gsz) * BN;
-    };
 
     const int nkb = K / KBLOCK;
     const int sn = (N + KBLOCK - 1) / KBLOCK;
     // buffer resources of the copy stream's current tile (fixed for a single problem)
     v4i rsrc_a, rsrc_b, rsrc_s, rsrc_bs;
     int f_lda = one.lda;  // leading dimension of the problem the copy stream is in
-    auto set_resources = [&](const Problem& pr) __attribute__((always_inline)) {
+    auto set_resources = [&](const TileProblem& pr) __attribute__((always_inline)) {
         rsrc_a = make_rsrc_words(pr.a, (uint32_t)pr.lda * (uint32_t)K);
         rsrc_b = make_rsrc_words(pr.b, (uint32_t)N * (uint32_t)K);
         rsrc_s = make_rsrc_words(pr.a_scale, (uint32_t)nkb * (uint32_t)pr.lda * 4u);
@@ -125,23 +83,23 @@ __device__ __forceinline__ void persistent_body(const Problem& one, const GroupT
     int f_tile = 0, f_kb = 0;
     int fill_left = n_my * nkb;  // blocks not yet copied
     auto fill_setup = [&](int j) __attribute__((always_inline)) {
-        Problem pr;
+        TileProblem pr;
         int m0, n0;
-        tile_origin(j, pr, m0, n0);
+        walk.origin(j, pr, m0, n0);
         if (GROUPED || j == 0)
             set_resources(pr);
         const int M = pr.M, lda = pr.lda;
 #pragma unroll
         for (int q = 0; q < S::NVA; ++q) {
             const int r = RSA == 256 ? (NA * wave + q) * 4 + (lane >> 4) : (NA * wave + q) * 8 + (lane >> 3);
-            const int cc = (RSA == 256 ? (lane & 15) : (lane & 7)) ^ row_swizzle<RSA>(r & 7);
+            const int cc = (RSA == 256 ? (lane & 15) : (lane & 7)) ^ row_swizzle<RSA>(r);
             const bool ok = (16 * cc < BM) && (m0 + 16 * cc < M);
             voff_a[q] = ok ? (uint32_t)(r * lda + m0 + 16 * cc) : 0x80000000u;
         }
 #pragma unroll
         for (int q = 0; q < S::NVB; ++q) {
             const int r = RSB == 256 ? (NB * wave + q) * 4 + (lane >> 4) : (NB * wave + q) * 8 + (lane >> 3);
-            const int cc = (RSB == 256 ? (lane & 15) : (lane & 7)) ^ row_swizzle<RSB>(r & 7);
+            const int cc = (RSB == 256 ? (lane & 15) : (lane & 7)) ^ row_swizzle<RSB>(r);
             const bool ok = (16 * cc < BN) && (n0 + 16 * cc < N);
             voff_b[q] = ok ? (uint32_t)(r * N + n0 + 16 * cc) : 0x80000000u;
         }
@@ -159,6 +117,8 @@ __device__ __forceinline__ void persistent_body(const Problem& one, const GroupT
             lds_dma16(rsrc_b, voff_b[S::template voff_index<RSB>(q - NA)],
                       stage + S::MAT_A + (uint32_t)((NB * wave + (q - NA)) * 1024),
                       (uint32_t)(f_kb * KBLOCK + S::template extra_rows<RSB>(q - NA)) * (uint32_t)N);
+        } else if (NW == 8) {
+            lds_dma16_unless((uint32_t)wave, rsrc_s, voff_s, stage + S::SCALE_OFF, (uint32_t)f_kb * (uint32_t)f_lda * 4u);
         } else if (wave == 0) {
             lds_dma16(rsrc_s, voff_s, stage + S::SCALE_OFF, (uint32_t)f_kb * (uint32_t)f_lda * 4u);
         } else if (NW == 4 && wave == 1) {
@@ -176,32 +136,23 @@ __device__ __forceinline__ void persistent_body(const Problem& one, const GroupT
     };
 
     // ---- LDS read addresses (k_tile.hip): they do not depend on the tile
-    const int g4 = lane >> 4, i16 = lane & 15;
     uint32_t addr_a[MI], addr_b[NJ];
 #pragma unroll
     for (int i = 0; i < MI; ++i)
-        addr_a[i] = (uint32_t)((32 * (g4 >> 1) + (i16 >> 1)) * RSA + (i16 & 1) * 8 +
-                               ((((wm * TM) / 16 + 2 * i + (g4 & 1)) ^ row_swizzle<RSA>(i16 >> 1)) * 16));
+        addr_a[i] = frag_addr<RSA>(lane, (wm * TM) / 16 + i);
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
-        addr_b[j] = (uint32_t)(S::MAT_A + (32 * (g4 >> 1) + (i16 >> 1)) * RSB + (i16 & 1) * 8 +
-                               ((((wn * TN) / 16 + 2 * j + (g4 & 1)) ^ row_swizzle<RSB>(i16 >> 1)) * 16));
-    const uint32_t addr_s = S::SCALE_OFF + (uint32_t)((wm * TM + (lane & 31)) * 4);
-    auto read_frag = [&](uint32_t addr, int ks, int rs) __attribute__((always_inline)) -> v8i {
-        const uint32_t base = addr + (uint32_t)(ks * 64 * rs);
-        v2i r0 = __builtin_amdgcn_ds_read_tr8_b64_v2i32(LDS_PTR(v2i, lds + base));
-        v2i r1 = __builtin_amdgcn_ds_read_tr8_b64_v2i32(LDS_PTR(v2i, lds + base + 8 * rs));
-        v2i r2 = __builtin_amdgcn_ds_read_tr8_b64_v2i32(LDS_PTR(v2i, lds + base + 16 * rs));
-        v2i r3 = __builtin_amdgcn_ds_read_tr8_b64_v2i32(LDS_PTR(v2i, lds + base + 24 * rs));
-        return (v8i){r0.x, r0.y, r1.x, r1.y, r2.x, r2.y, r3.x, r3.y};
-    };
-    const v16f zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        addr_b[j] = S::MAT_A + frag_addr<RSB>(lane, (wn * TN) / 16 + j);
+    const uint32_t addr_s = S::SCALE_OFF + (uint32_t)((wm * TM + (lane & 15)) * 4);
 
     // ---- a finished tile: bf16, in pieces of PR rows through `staging` (LDS bytes that nobody
     // else touches meanwhile), 16 bytes per lane along whole tile rows.  A lane owns row
-    // m = .. + (lane & 31) and, per patch, four runs of 4 columns: stored straight from the
-    // registers that would be 8-byte pieces of 32 different rows per instruction.
-    // sum(i, jj, r) = running sum r of patch (i, jj)
+    // m = .. + (lane & 15) and, per patch, a run of 4 columns: stored straight from the
+    // registers that would be 8-byte pieces of 16 different rows per instruction.
+    // sum(i, jj, e) = running sum e of patch (i, jj)
+    auto staged_chunk = [&](int row, int ch) __attribute__((always_inline)) {  // LDS offset of chunk ch of a piece's row
+        return (uint32_t)(row * CROW + ((ch ^ (BN % 128 == 0 ? row & 15 : (row >> 1) & 7)) << 4));
+    };
     auto store_tile = [&](auto sum, uint32_t staging, int m0, int n0, int M,
                           uint16_t* __restrict__ c) __attribute__((always_inline)) {
         // opaque copy of the thread id: keeps the address arithmetic below inside the tile loop
@@ -215,18 +166,16 @@ __device__ __forceinline__ void persistent_body(const Problem& one, const GroupT
                 __syncthreads();  // the previous piece has been read out
 #pragma unroll
             for (int i = 0; i < MI; ++i) {
-                const int prow = wm * TM + 32 * i;
+                const int prow = wm * TM + 16 * i;
                 if (prow / PR == p) {
-                    const uint32_t rbase = staging + (uint32_t)((prow - p * PR + (lane_e & 31)) * CROW);
+                    const int row = prow - p * PR + (lane_e & 15);
 #pragma unroll
-                    for (int jj = 0; jj < NJ; ++jj)
-#pragma unroll
-                        for (int q = 0; q < 4; ++q) {
-                            const int col = wn * TN + 32 * jj + 8 * q + 4 * (lane_e >> 5);
-                            v2i pk = {(int)pack_bf16x2(sum(i, jj, 4 * q), sum(i, jj, 4 * q + 1)),
-                                      (int)pack_bf16x2(sum(i, jj, 4 * q + 2), sum(i, jj, 4 * q + 3))};
-                            *LDS_PTR(v2i, lds + rbase + col * 2) = pk;
-                        }
+                    for (int jj = 0; jj < NJ; ++jj) {
+                        const int col = wn * TN + 16 * jj + 4 * (lane_e >> 4);
+                        v2i pk = {(int)pack_bf16x2(sum(i, jj, 0), sum(i, jj, 1)),
+                                  (int)pack_bf16x2(sum(i, jj, 2), sum(i, jj, 3))};
+                        *LDS_PTR(v2i, lds + staging + staged_chunk(row, col >> 3) + (col & 4) * 2) = pk;
+                    }
                 }
             }
             __syncthreads();
@@ -237,9 +186,7 @@ __device__ __forceinline__ void persistent_body(const Problem& one, const GroupT
                 const int mrow = m0 + p * PR + row;
                 const int ncol = n0 + ch * 8;
                 if (idx < CHUNKS && mrow < M && ncol < N) {
-                    const v2i lo = *LDS_PTR(v2i, lds + staging + row * CROW + ch * 16);
-                    const v2i hi = *LDS_PTR(v2i, lds + staging + row * CROW + ch * 16 + 8);
-                    *reinterpret_cast<v4i*>(c + (size_t)mrow * N + ncol) = (v4i){lo.x, lo.y, hi.x, hi.y};
+                    *reinterpret_cast<v4i*>(c + (size_t)mrow * N + ncol) = *LDS_PTR(v4i, lds + staging + staged_chunk(row, ch));
                 }
             }
         }
@@ -267,15 +214,16 @@ __device__ __forceinline__ void persistent_body(const Problem& one, const GroupT
         const uint32_t scale_kind = wave < 2 ? (uint32_t)wave : 2u;
         const uint32_t lds_wave = lds_base + (uint32_t)(NA * wave * 1024);
         const uint32_t lds_scale = lds_base + (wave == 0 ? S::SCALE_OFF : S::SB_OFF);
-        const uint32_t vbase_a0 = lds_base + addr_a[0], vbase_a1 = lds_base + addr_a[1];
-        const uint32_t vbase_a2 = lds_base + addr_a[2], vbase_a3 = lds_base + addr_a[3];
-        const uint32_t vbase_b0 = lds_base + addr_b[0], vbase_b1 = lds_base + addr_b[1], vbase_b2 = lds_base + addr_b[2];
+        // the even patch of each pair; the odd one's address differs in bit 4 (the pair's chunks are 2 i and 2 i + 1)
+        const uint32_t vbase_a0 = lds_base + addr_a[0], vbase_a1 = lds_base + addr_a[2];
+        const uint32_t vbase_a2 = lds_base + addr_a[4], vbase_a3 = lds_base + addr_a[6];
+        const uint32_t vbase_b0 = lds_base + addr_b[0], vbase_b1 = lds_base + addr_b[2], vbase_b2 = lds_base + addr_b[4];
         const uint32_t vaddr_s = lds_base + addr_s;
 
         v32f sums[6], blk;
         v32i frag0 = {}, frag1 = {}, frag2 = {};
         v16i frag3 = {};
-        float scale_carry = 0.f;
+        v2f scale_carry = {0.f, 0.f};
 #pragma unroll
         for (int r = 0; r < 32; ++r)
             blk[r] = 0.f;
@@ -312,16 +260,16 @@ __device__ __forceinline__ void persistent_body(const Problem& one, const GroupT
 
         uint32_t slot_off = 0;  // LDS offset of the ring slot of the block multiplied next
         for (int j = 0; j < n_my; ++j) {
-            Problem pr;
+            TileProblem pr;
             int m0, n0;
-            tile_origin(j, pr, m0, n0);
+            walk.origin(j, pr, m0, n0);
             const int n_wave = n0 + wn * TN;
             // the stage holds b_scale[kb][n0/128 + 0..3]; a wave's n range touches at most two of them
             const uint32_t lds_sb_lo = lds_base + S::SB_OFF + 4u * (uint32_t)((n_wave >> 7) - (n0 >> 7));
             const uint32_t lds_sb_hi = lds_base + S::SB_OFF + 4u * (uint32_t)(((n_wave + TN - 1) >> 7) - (n0 >> 7));
-            uint32_t hi_mask[NJ];  // all ones when patch column jj lies in the wave's second b_scale block
+            uint32_t hi_mask[NJ / 2];  // all ones when patch columns 2 jj and 2 jj + 1 lie in the wave's second b_scale block
 #pragma unroll
-            for (int jj = 0; jj < NJ; ++jj)
+            for (int jj = 0; jj < NJ / 2; ++jj)
                 hi_mask[jj] = (uint32_t)-(int)(((n_wave + 32 * jj) >> 7) > (n_wave >> 7));
 #pragma unroll
             for (int t = 0; t < 6; ++t)
@@ -368,13 +316,13 @@ __device__ __forceinline__ void persistent_body(const Problem& one, const GroupT
             }
             // the last patch's fold, then the tile leaves through the staging area
             w4_last_fold(sums[5], blk, scale_carry);
-            scale_carry = 0.f;
+            scale_carry = (v2f){0.f, 0.f};
 #pragma unroll
             for (int r = 16; r < 32; ++r)
                 blk[r] = 0.f;
             store_tile([&](int i, int jj, int r) __attribute__((always_inline)) {
-                           const int q = jj * MI + i;
-                           return sums[q / 2][(q % 2) * 16 + r];
+                           const int q = (jj / 2) * (MI / 2) + i / 2;  // pair of patch rows and columns
+                           return sums[q / 2][(q % 2) * 16 + 8 * (i % 2) + 4 * (jj % 2) + r];
                        },
                        (uint32_t)STAGING_W4, m0, n0, pr.M, pr.c);
         }
@@ -395,9 +343,9 @@ __device__ __forceinline__ void persistent_body(const Problem& one, const GroupT
     int slot_fill = NS - 1;  // ring slot the stream's next block goes into
 
     for (int j = 0; j < n_my; ++j) {
-        Problem pr;
+        TileProblem pr;
         int m0, n0;
-        tile_origin(j, pr, m0, n0);
+        walk.origin(j, pr, m0, n0);
         const float* __restrict__ b_scale = pr.b_scale;
         uint16_t* __restrict__ c = pr.c;
         const int M = pr.M;
@@ -405,19 +353,17 @@ __device__ __forceinline__ void persistent_body(const Problem& one, const GroupT
         int nb_lo = n_wave >> 7, nb_hi = (n_wave + TN - 1) >> 7;
         nb_lo = nb_lo < sn ? nb_lo : sn - 1;
         nb_hi = nb_hi < sn ? nb_hi : sn - 1;
-        uint32_t hi_mask[NJ];  // all ones when patch jj lies in the wave's second b_scale block
+        uint32_t hi_mask[NJ / 2];  // all ones when patch columns 2 jj and 2 jj + 1 lie in the wave's second b_scale block
 #pragma unroll
-        for (int jj = 0; jj < NJ; ++jj)
+        for (int jj = 0; jj < NJ / 2; ++jj)
             hi_mask[jj] = (uint32_t)-(int)(((n_wave + 32 * jj) >> 7) > (n_wave >> 7));
 
-        v16f acc[MI][NJ];
+        v4f acc[MI][NJ];
 #pragma unroll
         for (int i = 0; i < MI; ++i)
 #pragma unroll
             for (int jj = 0; jj < NJ; ++jj)
-#pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    acc[i][jj][r] = 0.f;
+                acc[i][jj] = (v4f){0.f, 0.f, 0.f, 0.f};
 
         float next_lo = b_scale[__builtin_amdgcn_readfirstlane(nb_lo)];
         float next_hi = b_scale[__builtin_amdgcn_readfirstlane(nb_hi)];
@@ -448,119 +394,64 @@ __device__ __forceinline__ void persistent_body(const Problem& one, const GroupT
             const float sb_lo = next_lo, sb_hi = next_hi;
             asm volatile("" ::"s"(sb_lo), "s"(sb_hi));
             const uint32_t so = (uint32_t)(slot * S::STAGE);
-            float sa[MI];
-#pragma unroll
-            for (int i = 0; i < MI; ++i)
-                sa[i] = *LDS_PTR(float, lds + so + addr_s + 128 * i);
-
             auto ask_next_scale = [&]() __attribute__((always_inline)) {
                 int next = __builtin_amdgcn_readfirstlane(kb + 1 < nkb ? kb + 1 : kb);
                 asm volatile("" : "+s"(next));
                 next_lo = b_scale[__builtin_amdgcn_readfirstlane(next * sn + nb_lo)];
                 next_hi = b_scale[__builtin_amdgcn_readfirstlane(next * sn + nb_hi)];
             };
-            v8i fa[MI][2];
+            // fragments, steps and folds as in k_tile.hip
+            v8i fa[MI], fb[NJ];
+            fb[0] = read_frag<RSB>(lds + (addr_b[0] + so));
 #pragma unroll
-            for (int i = 0; i < MI; ++i) {
-                fa[i][0] = read_frag(addr_a[i] + so, 0, RSA);
-                fa[i][1] = read_frag(addr_a[i] + so, 1, RSA);
-            }
-            constexpr int N_MFMA = MI * NJ * 2;
-            constexpr int PER_MFMA = (NCOPY + N_MFMA - 1) / N_MFMA;
-            int cq = 0;
-            auto copy_slot = [&](int n) __attribute__((always_inline)) {
+            for (int i = 0; i < MI; ++i)
+                fa[i] = read_frag<RSA>(lds + (addr_a[i] + so));
+            if (NJ > 1)
+                fb[1] = read_frag<RSB>(lds + (addr_b[1] + so));
+            float sa[MI], sc[MI];
 #pragma unroll
-                for (int u = 0; u < NCOPY; ++u)
-                    if (u < n && cq < NCOPY) {
-                        if (more)
-                            fill_copy(slot_fill, cq);
-                        ++cq;
-                    }
+            for (int i = 0; i < MI; ++i)
+                sa[i] = *LDS_PTR(float, lds + so + addr_s + 64 * i);
+            constexpr int T = MI * NJ, PER_MFMA = (NCOPY + T - 1) / T;
+            constexpr int LAG = MI < 4 && T >= 12 ? 6 : MI;
+            v4f blk[LAG];
+            auto fold = [&](int t) __attribute__((always_inline)) {
+                if (t % MI == 0) {
+                    // wave-uniform choice of the b_scale value on the scalar unit (bit select), then one product per patch
+                    const float sbj = __uint_as_float((__float_as_uint(sb_hi) & hi_mask[t / MI / 2]) |
+                                                      (__float_as_uint(sb_lo) & ~hi_mask[t / MI / 2]));
+#pragma unroll
+                    for (int i = 0; i < MI; ++i)
+                        sc[i] = sa[i] * sbj;
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    acc[t % MI][t / MI][e] = fmaf(sc[t % MI], blk[t % LAG][e], acc[t % MI][t / MI][e]);
             };
-            if (PIPELINED_FOLD) {
-                // Column jj's MFMAs write the block sums that column jj-1's fold has just read: the
-                // fold of patch (i, jj-1) sits in program order right before the first MFMA of
-                // patch (i, jj), pinned there (an empty asm statement that both the folded
-                // accumulator and the MFMA's B fragment pass through), so that its 16 FMAs issue
-                // while the MFMAs before it are still in the pipe.  Left alone, the compiler issues
-                // all MFMAs of a K block first and all folds after them, the matrix pipe idle
-                // meanwhile (both waves of a SIMD reach that phase together, after the barrier).
-                v16f blk[MI];
-                float sc_prev[MI];
 #pragma unroll
-                for (int jj = 0; jj <= NJ; ++jj) {
-                    v8i fb0, fb1;
-                    if (jj < NJ) {
-                        fb0 = read_frag(addr_b[jj] + so, 0, RSB);
-                        fb1 = read_frag(addr_b[jj] + so, 1, RSB);
-                    }
-#pragma unroll
-                    for (int i = 0; i < MI; ++i) {
-                        if (jj > 0) {
-#pragma unroll
-                            for (int r = 0; r < 16; ++r)
-                                acc[i][jj - 1][r] = fmaf(sc_prev[i], blk[i][r], acc[i][jj - 1][r]);
-                            if (jj < NJ)
-                                asm volatile("" : "+v"(acc[i][jj - 1]), "+v"(fb0));
-                        }
-                        if (jj < NJ) {
-                            blk[i] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fb0, fa[i][0], zero16, 0, 0,
-                                                                                      0, 0, 0, 0);
-                            copy_slot(PER_MFMA);
-                        }
-                    }
-                    if (jj < NJ) {
-#pragma unroll
-                        for (int i = 0; i < MI; ++i) {
-                            blk[i] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fb1, fa[i][1], blk[i], 0, 0,
-                                                                                      0, 0, 0, 0);
-                            copy_slot(PER_MFMA);
-                        }
-                        if (jj == NJ - 1)
-                            ask_next_scale();
-                        // wave-uniform choice of the b_scale value on the scalar unit (bit select),
-                        // then one product per patch
-                        const float sbj = __uint_as_float((__float_as_uint(sb_hi) & hi_mask[jj]) |
-                                                          (__float_as_uint(sb_lo) & ~hi_mask[jj]));
-#pragma unroll
-                        for (int i = 0; i < MI; ++i)
-                            sc_prev[i] = sa[i] * sbj;
-                    }
+            for (int t = 0; t < T; ++t) {
+                if (t % MI == 0 && t > 0 && t / MI + 1 < NJ)
+                    fb[t / MI + 1] = read_frag<RSB>(lds + (addr_b[t / MI + 1] + so));
+                if (t >= LAG) {
+                    fold(t - LAG);
+                    if (t + 1 < T)
+                        asm volatile("" : "+v"(acc[(t - LAG) % MI][(t - LAG) / MI]), "+v"(fa[(t + 1) % MI]));
                 }
-            } else {
+                blk[t % LAG] = block_sum(fb[t / MI], fa[t % MI]);
+                if (more)
 #pragma unroll
-                for (int jj = 0; jj < NJ; ++jj) {
-                    const v8i fb0 = read_frag(addr_b[jj] + so, 0, RSB);
-                    const v8i fb1 = read_frag(addr_b[jj] + so, 1, RSB);
-                    v16f blk[MI];
-#pragma unroll
-                    for (int i = 0; i < MI; ++i) {
-                        blk[i] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fb0, fa[i][0], zero16, 0, 0, 0,
-                                                                                  0, 0, 0);
-                        copy_slot(PER_MFMA);
-                    }
-#pragma unroll
-                    for (int i = 0; i < MI; ++i) {
-                        blk[i] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fb1, fa[i][1], blk[i], 0, 0, 0,
-                                                                                  0, 0, 0);
-                        copy_slot(PER_MFMA);
-                    }
-                    if (jj == NJ - 1)
-                        ask_next_scale();
-#pragma unroll
-                    for (int i = 0; i < MI; ++i) {
-                        // wave-uniform choice of the b_scale value on the scalar unit (bit select), then one
-                        // product per patch
-                        const float sbj = __uint_as_float((__float_as_uint(sb_hi) & hi_mask[jj]) |
-                                                          (__float_as_uint(sb_lo) & ~hi_mask[jj]));
-                        const float sc = sa[i] * sbj;
-#pragma unroll
-                        for (int r = 0; r < 16; ++r)
-                            acc[i][jj][r] = fmaf(sc, blk[i][r], acc[i][jj][r]);
-                    }
-                }
+                    for (int q = t * PER_MFMA; q < (t + 1) * PER_MFMA; ++q)
+                        if (q < NCOPY)
+                            fill_copy(slot_fill, q);
+                if (t == T - 1)
+                    ask_next_scale();
+                __builtin_amdgcn_sched_barrier(0);
             }
-            copy_slot(NCOPY);
+#pragma unroll
+            for (int t = T - LAG; t < T; ++t) {
+                fold(t);
+                asm volatile("" : "+v"(acc[t % MI][t / MI]));
+            }
             if (more)
                 fill_advance();
             slot_fill = slot;
@@ -596,18 +487,16 @@ __device__ __forceinline__ void persistent_body(const Problem& one, const GroupT
                     __syncthreads();  // the previous piece has been read out
 #pragma unroll
                 for (int i = 0; i < MI; ++i) {
-                    const int prow = wm * TM + 32 * i;
+                    const int prow = wm * TM + 16 * i;
                     if (prow / PR == p) {
-                        const uint32_t rbase = staging + (uint32_t)((prow - p * PR + (lane_e & 31)) * CROW);
+                        const int row = prow - p * PR + (lane_e & 15);
 #pragma unroll
-                        for (int jj = 0; jj < NJ; ++jj)
-#pragma unroll
-                            for (int q = 0; q < 4; ++q) {
-                                const int col = wn * TN + 32 * jj + 8 * q + 4 * (lane_e >> 5);
-                                v2i pk = {(int)pack_bf16x2(acc[i][jj][4 * q], acc[i][jj][4 * q + 1]),
-                                          (int)pack_bf16x2(acc[i][jj][4 * q + 2], acc[i][jj][4 * q + 3])};
-                                *LDS_PTR(v2i, lds + rbase + col * 2) = pk;
-                            }
+                        for (int jj = 0; jj < NJ; ++jj) {
+                            const int col = wn * TN + 16 * jj + 4 * (lane_e >> 4);
+                            v2i pk = {(int)pack_bf16x2(acc[i][jj][0], acc[i][jj][1]),
+                                      (int)pack_bf16x2(acc[i][jj][2], acc[i][jj][3])};
+                            *LDS_PTR(v2i, lds + staging + staged_chunk(row, col >> 3) + (col & 4) * 2) = pk;
+                        }
                     }
                 }
                 __syncthreads();
@@ -618,9 +507,7 @@ __device__ __forceinline__ void persistent_body(const Problem& one, const GroupT
                     const int mrow = m0 + p * PR + row;
                     const int ncol = n0 + ch * 8;
                     if (idx < CHUNKS && mrow < M && ncol < N) {
-                        const v2i lo = *LDS_PTR(v2i, lds + staging + row * CROW + ch * 16);
-                        const v2i hi = *LDS_PTR(v2i, lds + staging + row * CROW + ch * 16 + 8);
-                        *reinterpret_cast<v4i*>(c + (size_t)mrow * N + ncol) = (v4i){lo.x, lo.y, hi.x, hi.y};
+                        *reinterpret_cast<v4i*>(c + (size_t)mrow * N + ncol) = *LDS_PTR(v4i, lds + staging + staged_chunk(row, ch));
                     }
                 }
             }
@@ -636,7 +523,7 @@ tile_gemm_persistent_kernel(const uint8_t* __restrict__ a, const uint8_t* __rest
                             const float* __restrict__ a_scale, const float* __restrict__ b_scale,
                             uint16_t* __restrict__ c, int M, int lda, int N, int K, int tiles_m, int tiles_n)
 {
-    const Problem one{a, b, a_scale, b_scale, c, M, lda};
+    const TileProblem one{a, b, a_scale, b_scale, c, M, lda};
     persistent_body<BM, BN, WM, WN, NS, PR, false>(one, nullptr, N, K, tiles_m, tiles_n);
 }
 
@@ -644,7 +531,7 @@ template <int BM, int BN, int WM, int WN, int NS, int PR>
 __global__ void __launch_bounds__(64 * WM * WN)
 tile_gemm_grouped_kernel(const GroupTable tab, int N, int K, int tiles_n)
 {
-    const Problem none{nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0};
+    const TileProblem none{nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0};
     persistent_body<BM, BN, WM, WN, NS, PR, true>(none, &tab, N, K, 0, tiles_n);
 }
 
@@ -653,7 +540,7 @@ hipError_t launch_persistent_variant(const GemmArgs& g, int workgroups, hipStrea
 {
     using S = TileShape<BM, BN, WM, WN, NS, WM * WN>;
     // four waves stage the finished tile beside the ring
-    constexpr int LDS_TOTAL = S::LDS_BYTES + (WM * WN == 4 ? PR * (BN * 2 + 8) : 0);
+    constexpr int LDS_TOTAL = S::LDS_BYTES + (WM * WN == 4 ? PR * BN * 2 : 0);
     const int tiles_m = (g.m + BM - 1) / BM, tiles_n = (g.n + BN - 1) / BN;
     auto kern = tile_gemm_persistent_kernel<BM, BN, WM, WN, NS, PR>;
     FP8GEMM_ALLOW_LDS(kern, LDS_TOTAL);
@@ -703,12 +590,12 @@ hipError_t launch_tile_persistent(const GemmArgs& g, int variant, int workgroups
     if (workgroups <= 0 || workgroups % 8 != 0 || !tile_persistent_supports(g, variant))
         return hipErrorInvalidValue;
     switch (variant) {
-    case TILE_256x192: return launch_persistent_variant<256, 192, 4, 2, 2, 128>(g, workgroups, s);
+    case TILE_256x192:
+    case TILE_256x256: return launch_tile_large(g, variant, workgroups, s);
     case TILE_256x128: return launch_persistent_variant<256, 128, 4, 2, 3, 128>(g, workgroups, s);
     case TILE_128x192: return launch_persistent_variant<128, 192, 4, 2, 3, 128>(g, workgroups, s);
     case TILE_128x128: return launch_persistent_variant<128, 128, 2, 4, 4, 128>(g, workgroups, s);
     case TILE_256x192_W4: return launch_persistent_variant<256, 192, 2, 2, 2, 64>(g, workgroups, s);
-    case TILE_256x256: return launch_persistent_variant<256, 256, 4, 2, 2, 128>(g, workgroups, s);
     default: return hipErrorInvalidValue;
     }
 }
@@ -733,11 +620,11 @@ hipError_t launch_tile_grouped(GroupTable& tab, int n, int k, int variant, int w
     if (workgroups <= 0 || workgroups % 8 != 0 || !tile_grouped_supports(tab, n, k, variant))
         return hipErrorInvalidValue;
     switch (variant) {
-    case TILE_256x192: return launch_grouped_variant<256, 192, 4, 2, 2, 128>(tab, n, k, workgroups, s);
+    case TILE_256x192:
+    case TILE_256x256: return launch_tile_large_grouped(tab, n, k, variant, workgroups, s);
     case TILE_256x128: return launch_grouped_variant<256, 128, 4, 2, 3, 128>(tab, n, k, workgroups, s);
     case TILE_128x192: return launch_grouped_variant<128, 192, 4, 2, 3, 128>(tab, n, k, workgroups, s);
     case TILE_128x128: return launch_grouped_variant<128, 128, 2, 4, 4, 128>(tab, n, k, workgroups, s);
-    case TILE_256x256: return launch_grouped_variant<256, 256, 4, 2, 2, 128>(tab, n, k, workgroups, s);
     default: return hipErrorInvalidValue;
     }
 }

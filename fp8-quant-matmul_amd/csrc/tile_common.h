@@ -50,12 +50,103 @@ struct TileShape {
     static_assert(LDS_BYTES <= 160 * 1024, "stages exceed the 160 KiB of LDS");
 };
 
-// chunk swizzle of row r (0..7 within an 8-row group) for a row stride of RS bytes
+// chunk swizzle of k-row r (0 .. 127) for a row stride of RS bytes: the 16 rows whose pieces of one chunk are read
+// together (frag_row: eight adjacent rows and the eight 64 further on) lie in 16 different 16-byte bank groups.  The rows
+// that a wave copies agree in r >> 6.
 template <int RS>
 __device__ __forceinline__ int row_swizzle(int r)
 {
-    return RS == 256 ? 2 * (r & 7) : (RS == 128 ? 2 * ((r >> 1) & 3) : 2 * ((r >> 2) & 1));
+    return (RS == 256 ? 2 * (r & 7) : (RS == 128 ? 2 * ((r >> 1) & 3) : 2 * ((r >> 2) & 1))) + (r >> 6);
 }
+
+// ---- operand fragments of v_mfma_f32_16x16x128_f8f6f4 out of a stage: 16 rows of m or n (one 16-byte chunk) x 128 k in
+// four transposing reads.  In read t lane 16 * g + i supplies the half (i & 1) of the chunk in k-row frag_row + 8 * t and
+// receives 8 k of row i; the k order inside the instruction is permuted alike for both operands.
+__device__ __forceinline__ int frag_row(int lane)
+{
+    const int g = lane >> 4, i = lane & 15;
+    return 64 * (g & 1) + 32 * (g >> 1) + (i >> 1);
+}
+// LDS offset of a lane's first read of chunk `chunk` of a matrix with rows of RS bytes
+template <int RS>
+__device__ __forceinline__ uint32_t frag_addr(int lane, int chunk)
+{
+    const int r = frag_row(lane);
+    return (uint32_t)(r * RS + (lane & 1) * 8 + ((chunk ^ row_swizzle<RS>(r)) * 16));
+}
+template <int RS, typename Lds>
+__device__ __forceinline__ v8i read_frag(Lds first)  // the lane's first read
+{
+    const v2i r0 = __builtin_amdgcn_ds_read_tr8_b64_v2i32(LDS_PTR(v2i, first));
+    const v2i r1 = __builtin_amdgcn_ds_read_tr8_b64_v2i32(LDS_PTR(v2i, first + 8 * RS));
+    const v2i r2 = __builtin_amdgcn_ds_read_tr8_b64_v2i32(LDS_PTR(v2i, first + 16 * RS));
+    const v2i r3 = __builtin_amdgcn_ds_read_tr8_b64_v2i32(LDS_PTR(v2i, first + 24 * RS));
+    return (v8i){r0.x, r0.y, r1.x, r1.y, r2.x, r2.y, r3.x, r3.y};
+}
+// the block sum of a 16 x 16 patch: rows = n (4 * (lane >> 4) + register), columns = m (lane & 15)
+__device__ __forceinline__ v4f block_sum(v8i b, v8i a)
+{
+    return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(b, a, (v4f){0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 0, 0, 0);
+}
+
+// One problem of a launch as the persistent kernels see it.
+struct TileProblem {
+    const uint8_t* a;
+    const uint8_t* b;
+    const float* a_scale;
+    const float* b_scale;
+    uint16_t* c;
+    int M;
+    int lda;  // elements between consecutive k-rows of a and of a_scale (>= M, a multiple of 16)
+};
+
+// The tiles of one persistent workgroup.  Workgroup ids go round the 8 XCDs (id % 8); each XCD owns a contiguous run
+// of the tile order (groups of GROUP_M tile rows, as in k_tile.hip) and its workgroups take the run's tiles in turn, so that
+// the tiles an XCD works on at any moment are neighbours and share A and B panels in its L2.
+// GROUPED = false: one problem, tiles_m x tiles_n tiles.  GROUPED = true: the problems of `tab` (same N and K, own M),
+// whose tiles are numbered one group after the other.
+template <int BM, int BN, bool GROUPED>
+struct TileWalk {
+    const TileProblem& one;
+    const GroupTable* tab;
+    int tiles_m, tiles_n;
+    int per_xcd, run0, run_len, li;
+    __device__ __forceinline__ TileWalk(const TileProblem& p, const GroupTable* t, int tm, int tn)
+        : one(p), tab(t), tiles_m(tm), tiles_n(tn)
+    {
+        const int T = GROUPED ? tab->tile_start[tab->groups] : tiles_m * tiles_n;
+        const int pid = blockIdx.x;
+        per_xcd = gridDim.x >> 3;  // gridDim.x is a multiple of 8
+        const int xcd = pid & 7, q8 = T >> 3, r8 = T & 7;
+        run0 = xcd * q8 + (xcd < r8 ? xcd : r8);
+        run_len = q8 + (xcd < r8 ? 1 : 0);
+        li = pid >> 3;
+    }
+    __device__ __forceinline__ int count() const { return li < run_len ? (run_len - li + per_xcd - 1) / per_xcd : 0; }
+    // tile number j of this workgroup: its problem and its origin in that problem's C
+    __device__ __forceinline__ void origin(int j, TileProblem& pr, int& m0, int& n0) const
+    {
+        const int per_group = GROUP_M * tiles_n;
+        int logical = run0 + li + j * per_xcd;
+        int tm = tiles_m;
+        if (GROUPED) {
+            int g = 0;
+            while (g + 1 < tab->groups && logical >= tab->tile_start[g + 1])
+                ++g;
+            logical -= tab->tile_start[g];
+            pr = TileProblem{tab->a[g], tab->b[g], tab->a_scale[g], tab->b_scale[g], tab->c[g], tab->m[g], tab->lda[g]};
+            tm = (pr.M + BM - 1) / BM;
+        } else {
+            pr = one;
+        }
+        const int group = logical / per_group;
+        const int first_m = group * GROUP_M;
+        const int gsz = (tm - first_m < GROUP_M) ? (tm - first_m) : GROUP_M;
+        const int in_group = logical - group * per_group;
+        m0 = (first_m + in_group % gsz) * BM;
+        n0 = (in_group / gsz) * BN;
+    }
+};
 
 template <int N>
 __device__ __forceinline__ void wait_vmcnt()
