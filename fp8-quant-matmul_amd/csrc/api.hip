@@ -154,6 +154,25 @@ int validate(const void* a, const void* b, const float* as, const float* bs, con
     return FP8GEMM_OK;
 }
 
+// The 256x256 tile, in the units of the fit below (which was made on operands in the caches and at the clock of short
+// runs; 256x192 measures 1.39 us per K block where it says 1.10): full rounds and what is done with the tiles left over
+// (large_tile_tail).  Measured on 8192 x 4608, 8192 x 7168 and 4096 x 4608 with K = 512 ... 7168, operands in turn: a
+// round 4.0 us + 1.6 per K block, a round of halves 7.0 + 1.03, of quarters 3.7 + 0.57 (+ 2 with short K, where other
+// shapes are as fast: 4322 x 4096 x 512 24.8 us against 22.9 in 128x192 tiles).  30 random shapes whose plan changed with
+// this and the kernel: 26 faster, by up to 20 % (2192 x 8016 x 4864 113.2 -> 91.5 us, 6816 x 7312 x 3200 187.9 -> 156.5).
+double large_tile_cost(long tiles, int k, double per_kb)
+{
+    const int nkb = k / 128;
+    const Tail tail = large_tile_tail(tiles, k, NUM_CU);
+    const long rounds = tail == Tail::NONE ? (tiles + NUM_CU - 1) / NUM_CU : tiles / NUM_CU;
+    double cost = 1.79 + rounds * (4.5 + nkb * 1.335 * per_kb);
+    if (tail == Tail::HALVES)
+        cost += 6.0 + nkb * 0.86 * per_kb;
+    else if (tail == Tail::QUARTERS)
+        cost += 7.0 + nkb * 0.48 * per_kb;
+    return cost;
+}
+
 // Estimated run time of a tile plan in microseconds.  The form is launch + rounds of 256
 // workgroups x (pipeline fill + K blocks + store) + the split-K reduction; the constants are a
 // least-squares fit to a sweep of every tile variant x ksplit over the 18 shapes of the
@@ -164,11 +183,11 @@ double tile_cost(const GemmArgs& g, int variant, int ksplit, bool fused = false)
     int bm, bn;
     tile_variant_dims(variant, &bm, &bn);
     const long tiles = (long)((g.m + bm - 1) / bm) * ((g.n + bn - 1) / bn);
+    if (variant == TILE_256x256)
+        return large_tile_cost(tiles, g.k, 1.0);
     const int nkb = g.k / 128;
     const int kbs = (nkb + ksplit - 1) / ksplit;
     const double area = (double)bm * bn / 65536.0;
-    // (the 256x256 tile measures 3-5 % ahead of 256x192 per flop where both fill their rounds; the fitted
-    // line, extrapolated to its area, would put it 6 % ahead)
     // (a single row of tiles reads every byte of B once and from HBM -- decode weights do not fit the caches --,
     // where a K block takes a quarter longer than the fit to cached operands says: without this factor
     // 48 x 7168 x 1536 stays unsplit, 9.4 us from HBM against 8.1 us with two splits; the same for two rows of
@@ -186,8 +205,9 @@ double tile_cost(const GemmArgs& g, int variant, int ksplit, bool fused = false)
     // the splits inside the kernel starts 0.3 us earlier.  Problems of 96 ... 256 such tiles measure as the fit
     // says, or slower.)
     const bool light = variant == TILE_64x64 && !streams_b && tiles <= 64;
-    const double per_kb = (1.19 * area + 0.267) * (variant == TILE_256x256 ? 1.03 : 1.0) * (streams_b ? 1.25 : 1.0) *
-                          (light ? 0.8 : 1.0);
+    // (256x192 in the persistent form: the fit knows the kernel before its barrier moved, 5 % slower)
+    const double per_kb = (1.19 * area + 0.267) * (variant == TILE_256x192 && ksplit == 1 && tiles > NUM_CU ? 0.95 : 1.0) *
+                          (streams_b ? 1.25 : 1.0) * (light ? 0.8 : 1.0);
     // (unsplit 128x192 tiles in more than one round of workgroups: the fit has them 8 % too fast against the 256-row
     // tiles -- 36 random shapes of 512 ... 8192 rows where that margin decides, before / after: the 256x256 or
     // 256x128 plan +5.6 % with B cached, +10.3 % with B from HBM on average, worst -2.3 %)
@@ -256,8 +276,6 @@ struct TunedShape { int m, n, k, variant, ksplit; };
 constexpr TunedShape kTuned[] = {
     {1024, 512, 7168, TILE_64x64, 2},
     {1024, 576, 7168, TILE_128x128, 4},
-    {6144, 3072, 1536, TILE_256x192, 1},
-    {8192, 7168, 2048, TILE_256x192, 1},
 };
 
 // tile shapes that exist in the persistent form only (and run only when asked for by number)
@@ -860,7 +878,8 @@ long grouped_tiles(const GroupTable& tab, int n, int variant)
 // that come from HBM: every group brings its own B, and a tile row of a group reads all of it, so the launch
 // moves more bytes per flop than the single problems tile_cost was fitted on, the more the smaller the tile.
 // Factors on the K block from 25 launches (1 ... 64 groups of 65 ... 3000 rows, N = 1536 ... 7168, K = 2048 and
-// 7168, every tile shape pinned): 1.12 for 256x256, 1.5 for 256x192 and 256x128, 1.7 for 128x192 and 128x128 --
+// 7168, every tile shape pinned): 1.2 for 256x256, 1.43 for 256x192, 1.5 for 256x128, 1.7 for 128x192 and 128x128; the
+// first two have since got 5 % faster, which is in the factors and not in these figures --
 // e.g. 8 groups of 300 ... 3000 rows, 4608 x 7168: 498 / 610 / 680 / 775 / 893 us estimated for 256x256 / 256x192 /
 // 256x128 / 128x192 / 128x128, 515 / 615 / 727 / 875 / 1042 us measured; 4 groups of 65 ... 256 rows, 7168 x 2048:
 // 35 / 34 / 26 / 46 / 37 us estimated, 32 / 33 / 25 / 42 / 36 us measured.
@@ -869,8 +888,10 @@ double grouped_tile_cost(const GroupTable& tab, int n, int k, int variant)
     int bm, bn;
     tile_variant_dims(variant, &bm, &bn);
     const double area = (double)bm * bn / 65536.0;
-    const double from_hbm = variant == TILE_256x256 ? 1.12 : bm == 256 ? 1.5 : 1.7;
-    const double per_kb = (1.19 * area + 0.267) * (variant == TILE_256x256 ? 1.03 : 1.0) * from_hbm;
+    if (variant == TILE_256x256)
+        return large_tile_cost(grouped_tiles(tab, n, variant), k, 1.2);
+    const double from_hbm = variant == TILE_256x192 ? 1.43 : bm == 256 ? 1.5 : 1.7;
+    const double per_kb = (1.19 * area + 0.267) * from_hbm;
     const double per_item = 0.95 + 4.38 * area + (k / 128) * per_kb;
     const long rounds = (grouped_tiles(tab, n, variant) + NUM_CU - 1) / NUM_CU;
     return 1.79 + rounds * per_item;

@@ -349,8 +349,9 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
         // stands here (the next MFMA's operand passes through the fold's empty asm statement).  The wave's copy instructions
         // of block kb + NS - 1 ride on the first MFMAs.
         constexpr int T = MI * NJ, PER_MFMA = (NCOPY + T - 1) / T;
-        // two patch rows: six behind where there are that many (128x192: 300 x 12288 x 2048 17.16 -> 17.02 us, four behind 17.05)
-        constexpr int LAG = MI < 4 && T >= 12 ? 6 : MI;
+        // two patch rows: six behind where there are that many (128x192: 300 x 12288 x 2048 17.16 -> 17.02 us, four behind 17.05),
+        // four of four (64x64: 1024 x 512 x 2048 6.15 -> 6.03, 244 x 3072 x 1536 7.13 -> 7.00)
+        constexpr int LAG = T == 4 ? 4 : MI < 4 && T >= 12 ? 6 : MI;
         v4f blk[LAG];
         auto fold = [&](int t) __attribute__((always_inline)) {
             if (t % MI == 0) {
@@ -376,7 +377,7 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
             }
             blk[t % LAG] = block_sum(fb[t / MI], fa[t % MI]);
             if (RAGGED) {
-                if (t == 0) {
+                if (t == 1) {
                     if (loads_a && A_EARLY)
                         next_a();
                     if (!loads_a && more)

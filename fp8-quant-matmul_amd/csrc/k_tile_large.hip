@@ -24,7 +24,7 @@
 // 62 % busy; without its copies it takes 160 us.  Against 32x32x64 MFMAs with the barrier at the block's end and the
 // tile leaving through a slot: 8192 x 4096 x 7168 212.7 -> 189 us = 51 % of 5033 TFLOP/s; 8192 x 4608 x 7168 (256 x 192) 252.8 ->
 // 239; 8192 x 7168 x 2048 (256 x 192 and 256 x 256) 136.7 -> 129.5 and 123.8 -> 117; 8192 x 7168 x 256 32.8 -> 29.
-#include "tile_common.h"
+#include "tile_persistent_body.h"
 
 namespace fp8gemm {
 
@@ -53,13 +53,22 @@ struct LargeShape {
     static_assert(TILE_STORES < 64, "vmcnt is a 6-bit field");
 };
 
-template <int BN, bool GROUPED>
+// The lane number, found out anew: what is worked out from it once per tile, or behind the tiles, is not kept through the
+// K loop, which has no register left.
+__device__ __forceinline__ int lane_now()
+{
+    uint32_t zero;
+    asm volatile("v_mov_b32 %0, 0" : "=v"(zero));
+    return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, zero));
+}
+
+template <int BN, bool GROUPED, typename SHARE>
 __device__ __forceinline__ void large_tile_body(const TileProblem& one, const GroupTable* tab, int N, int K, int tiles_m,
                                                 int tiles_n)
 {
     using L = LargeShape<BN>;
     using S = typename L::S;
-    constexpr int BM = L::BM, TM = L::TM, TN = L::TN, MI = L::MI, NJ = L::NJ, NA = S::NA, NB = S::NB;
+    constexpr int TM = L::TM, TN = L::TN, MI = L::MI, NJ = L::NJ, NA = S::NA, NB = S::NB;
     constexpr int NCOPY = NA + NB + 1;  // copy instructions of a wave per K block; the last one brings the scales
     constexpr bool STRADDLES = TN == 96;  // a wave's columns may lie in two b_scale blocks
     // A block's MFMAs: column by column of its patches, the last two columns row by row of theirs.
@@ -83,15 +92,7 @@ __device__ __forceinline__ void large_tile_body(const TileProblem& one, const Gr
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave % L::WM, wn = wave / L::WM;
 
-    // The lane number, found out anew: what is worked out from it once per tile is not kept through the K loop, which has no
-    // register left.
-    auto lane_now = []() __attribute__((always_inline)) {
-        uint32_t zero;
-        asm volatile("v_mov_b32 %0, 0" : "=v"(zero));
-        return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, zero));
-    };
-
-    const TileWalk<BM, BN, GROUPED> walk(one, tab, tiles_m, tiles_n);
+    const TileWalk<SHARE, GROUPED> walk(one, tab, tiles_m, tiles_n);
     const int n_my = walk.count();
     if (n_my == 0)
         return;
@@ -383,58 +384,116 @@ __device__ __forceinline__ void large_tile_body(const TileProblem& one, const Gr
     wait_vmcnt<0>();  // no copy may land in LDS that has been given to somebody else
 }
 
-template <int BN>
+template <Tail TAIL>
+constexpr int tail_lds_bytes()
+{
+    return TAIL == Tail::NONE ? 0 : TAIL == Tail::HALVES ? TileShape<256, 128, 4, 2, 3>::LDS_BYTES : TileShape<128, 128, 2, 4, 4>::LDS_BYTES;
+}
+
+template <int BN, bool GROUPED, Tail TAIL>
+__device__ __forceinline__ void large_kernel_body(const TileProblem& one, const GroupTable* tab, int N, int K, int tiles_m,
+                                                  int tiles_n)
+{
+    if constexpr (TAIL == Tail::NONE) {
+        large_tile_body<BN, GROUPED, AllTiles<256, BN>>(one, tab, N, K, tiles_m, tiles_n);
+    } else {
+        static_assert(BN == 256, "halves and quarters of 256x256");
+        const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        large_tile_body<BN, GROUPED, FullRounds<256, BN>>(one, tab, N, K, tiles_m, tiles_n);
+        __syncthreads();  // nobody reads the slots any more
+        const int thread = 64 * wave + lane_now();
+        if constexpr (TAIL == Tail::HALVES)
+            persistent_body<256, 128, 4, 2, 3, 128, GROUPED, LeftOver<256, 256, 256, 128>>(one, tab, N, K, tiles_m,
+                                                                                                   tiles_n, thread);
+        else
+            persistent_body<128, 128, 2, 4, 4, 128, GROUPED, LeftOver<256, 256, 128, 128>>(one, tab, N, K, tiles_m,
+                                                                                                   tiles_n, thread);
+    }
+}
+
+template <int BN, Tail TAIL>
 __global__ void __launch_bounds__(NTHREADS)
 tile_gemm_large_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b, const float* __restrict__ a_scale,
                        const float* __restrict__ b_scale, uint16_t* __restrict__ c, int M, int lda, int N, int K, int tiles_m,
                        int tiles_n)
 {
     const TileProblem one{a, b, a_scale, b_scale, c, M, lda};
-    large_tile_body<BN, false>(one, nullptr, N, K, tiles_m, tiles_n);
+    large_kernel_body<BN, false, TAIL>(one, nullptr, N, K, tiles_m, tiles_n);
 }
 
-template <int BN>
+template <int BN, Tail TAIL>
 __global__ void __launch_bounds__(NTHREADS)
 tile_gemm_large_grouped_kernel(const GroupTable tab, int N, int K, int tiles_n)
 {
     const TileProblem none{nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0};
-    large_tile_body<BN, true>(none, &tab, N, K, 0, tiles_n);
+    large_kernel_body<BN, true, TAIL>(none, &tab, N, K, 0, tiles_n);
 }
 
-template <int BN>
+template <int BN, Tail TAIL>
 hipError_t launch_large(const GemmArgs& g, int workgroups, hipStream_t s)
 {
-    auto kern = tile_gemm_large_kernel<BN>;
-    FP8GEMM_ALLOW_LDS(kern, LargeShape<BN>::LDS_BYTES);
-    hipLaunchKernelGGL(kern, dim3(workgroups), dim3(NTHREADS), LargeShape<BN>::LDS_BYTES, s, g.a, g.b, g.a_scale, g.b_scale,
-                       g.c, g.m, leading_dim(g), g.n, g.k, (g.m + 255) / 256, (g.n + BN - 1) / BN);
+    constexpr int LDS = LargeShape<BN>::LDS_BYTES > tail_lds_bytes<TAIL>() ? LargeShape<BN>::LDS_BYTES : tail_lds_bytes<TAIL>();
+    auto kern = tile_gemm_large_kernel<BN, TAIL>;
+    FP8GEMM_ALLOW_LDS(kern, LDS);
+    hipLaunchKernelGGL(kern, dim3(workgroups), dim3(NTHREADS), LDS, s, g.a, g.b, g.a_scale, g.b_scale, g.c, g.m,
+                       leading_dim(g), g.n, g.k, (g.m + 255) / 256, (g.n + BN - 1) / BN);
     return hipGetLastError();
 }
 
-template <int BN>
-hipError_t launch_large_grouped(GroupTable& tab, int n, int k, int workgroups, hipStream_t s)
+template <int BN, Tail TAIL>
+hipError_t launch_large_grouped(const GroupTable& tab, int n, int k, int workgroups, hipStream_t s)
 {
-    const int tiles_n = (n + BN - 1) / BN;
-    tab.tile_start[0] = 0;
-    for (int g = 0; g < tab.groups; ++g)
-        tab.tile_start[g + 1] = tab.tile_start[g] + ((tab.m[g] + 255) / 256) * tiles_n;
-    auto kern = tile_gemm_large_grouped_kernel<BN>;
-    FP8GEMM_ALLOW_LDS(kern, LargeShape<BN>::LDS_BYTES);
-    hipLaunchKernelGGL(kern, dim3(workgroups), dim3(NTHREADS), LargeShape<BN>::LDS_BYTES, s, tab, n, k, tiles_n);
+    constexpr int LDS = LargeShape<BN>::LDS_BYTES > tail_lds_bytes<TAIL>() ? LargeShape<BN>::LDS_BYTES : tail_lds_bytes<TAIL>();
+    auto kern = tile_gemm_large_grouped_kernel<BN, TAIL>;
+    FP8GEMM_ALLOW_LDS(kern, LDS);
+    hipLaunchKernelGGL(kern, dim3(workgroups), dim3(NTHREADS), LDS, s, tab, n, k, (n + BN - 1) / BN);
     return hipGetLastError();
 }
 
 }  // namespace
 
+// An XCD's run of tiles, less the rounds in which each of its workgroups gets one, cut so that every workgroup gets at most
+// one piece.  Behind the full rounds a ring of stages starts anew, which halves need eight K blocks to make up for (full
+// tiles / halves, 8192 x 7168, half a round left over: K = 512 42.7 / 44.1 us, 1024 69.6 / 69.2, 1536 92.7 / 90.9, 2048
+// 118.0 / 114.0) and quarters none (8192 x 4608, a quarter left over: 512 29.8 / 29.2, 1024 45.2 / 43.4, 3072 115.1 /
+// 106.0, 7168 251.7 / 233.2; 4096 x 4608, an eighth on top of one round: 2048 49.4 / 42.0, 4096 90.4 / 74.5).
+Tail large_tile_tail(long tiles, int k, int workgroups)
+{
+    const int per_xcd = workgroups / 8, nkb = k / KBLOCK;
+    const long most = (tiles + 7) / 8;  // the XCDs' runs differ by one
+    const long left = most % per_xcd;
+    if (most < per_xcd || left == 0 || tiles / 8 / per_xcd != most / per_xcd)
+        return Tail::NONE;
+    if (4 * left <= per_xcd && nkb >= 3)  // the ring's depth
+        return Tail::QUARTERS;
+    return 2 * left <= per_xcd && nkb >= 8 ? Tail::HALVES : Tail::NONE;
+}
+
 hipError_t launch_tile_large(const GemmArgs& g, int variant, int workgroups, hipStream_t s)
 {
-    return variant == TILE_256x192 ? launch_large<192>(g, workgroups, s) : launch_large<256>(g, workgroups, s);
+    if (variant == TILE_256x192)
+        return launch_large<192, Tail::NONE>(g, workgroups, s);
+    const long tiles = (long)((g.m + 255) / 256) * ((g.n + 255) / 256);
+    switch (large_tile_tail(tiles, g.k, workgroups)) {
+    case Tail::QUARTERS: return launch_large<256, Tail::QUARTERS>(g, workgroups, s);
+    case Tail::HALVES: return launch_large<256, Tail::HALVES>(g, workgroups, s);
+    default: return launch_large<256, Tail::NONE>(g, workgroups, s);
+    }
 }
 
 hipError_t launch_tile_large_grouped(GroupTable& tab, int n, int k, int variant, int workgroups, hipStream_t s)
 {
-    return variant == TILE_256x192 ? launch_large_grouped<192>(tab, n, k, workgroups, s)
-                                   : launch_large_grouped<256>(tab, n, k, workgroups, s);
+    const int bn = variant == TILE_256x192 ? 192 : 256, tiles_n = (n + bn - 1) / bn;
+    tab.tile_start[0] = 0;
+    for (int g = 0; g < tab.groups; ++g)
+        tab.tile_start[g + 1] = tab.tile_start[g] + ((tab.m[g] + 255) / 256) * tiles_n;
+    if (variant == TILE_256x192)
+        return launch_large_grouped<192, Tail::NONE>(tab, n, k, workgroups, s);
+    switch (large_tile_tail(tab.tile_start[tab.groups], k, workgroups)) {
+    case Tail::QUARTERS: return launch_large_grouped<256, Tail::QUARTERS>(tab, n, k, workgroups, s);
+    case Tail::HALVES: return launch_large_grouped<256, Tail::HALVES>(tab, n, k, workgroups, s);
+    default: return launch_large_grouped<256, Tail::NONE>(tab, n, k, workgroups, s);
+    }
 }
 
 }  // namespace fp8gemm

@@ -86,6 +86,10 @@ struct GroupTable {
 bool tile_grouped_supports(const GroupTable& tab, int n, int k, int variant);
 hipError_t launch_tile_grouped(GroupTable& tab, int n, int k, int variant, int workgroups, hipStream_t s);
 // ... of the two large tiles, 256x192 and 256x256 (called by the two functions above, which check the arguments)
+// The tiles of a last round of 256x256 that would leave half the workgroups or more without one are cut into halves
+// (256x128) or quarters (128x128), one for each workgroup.
+enum class Tail { NONE, HALVES, QUARTERS };
+Tail large_tile_tail(long tiles, int k, int workgroups);
 hipError_t launch_tile_large(const GemmArgs& g, int variant, int workgroups, hipStream_t s);
 hipError_t launch_tile_large_grouped(GroupTable& tab, int n, int k, int variant, int workgroups, hipStream_t s);
 hipError_t launch_splitk_reduce(const GemmArgs& g, int ksplit, const float* partial, hipStream_t s);

@@ -100,13 +100,32 @@ struct TileProblem {
     int lda;  // elements between consecutive k-rows of a and of a_scale (>= M, a multiple of 16)
 };
 
+// Which part of a launch a walk covers.  All tiles of BM x BN; or, of a grid of such tiles, the rounds in which every
+// workgroup of an XCD gets one; or the ones left over, each cut into sub-tiles of SM x SN.
+template <int BM_, int BN_>
+struct AllTiles {
+    static constexpr int BM = BM_, BN = BN_, SM = BM_, SN = BN_;
+    static constexpr bool FULL_ROUNDS = false, LEFT_OVER = false;
+};
+template <int BM_, int BN_>
+struct FullRounds {
+    static constexpr int BM = BM_, BN = BN_, SM = BM_, SN = BN_;
+    static constexpr bool FULL_ROUNDS = true, LEFT_OVER = false;
+};
+template <int BM_, int BN_, int SM_, int SN_>
+struct LeftOver {
+    static constexpr int BM = BM_, BN = BN_, SM = SM_, SN = SN_;
+    static constexpr bool FULL_ROUNDS = false, LEFT_OVER = true;
+};
+
 // The tiles of one persistent workgroup.  Workgroup ids go round the 8 XCDs (id % 8); each XCD owns a contiguous run
 // of the tile order (groups of GROUP_M tile rows, as in k_tile.hip) and its workgroups take the run's tiles in turn, so that
 // the tiles an XCD works on at any moment are neighbours and share A and B panels in its L2.
 // GROUPED = false: one problem, tiles_m x tiles_n tiles.  GROUPED = true: the problems of `tab` (same N and K, own M),
 // whose tiles are numbered one group after the other.
-template <int BM, int BN, bool GROUPED>
+template <typename SHARE, bool GROUPED>
 struct TileWalk {
+    static constexpr int BM = SHARE::BM, BN = SHARE::BN, SUBS_N = BN / SHARE::SN, SUBS = BM / SHARE::SM * SUBS_N;
     const TileProblem& one;
     const GroupTable* tab;
     int tiles_m, tiles_n;
@@ -121,13 +140,23 @@ struct TileWalk {
         run0 = xcd * q8 + (xcd < r8 ? xcd : r8);
         run_len = q8 + (xcd < r8 ? 1 : 0);
         li = pid >> 3;
+        if (SHARE::FULL_ROUNDS || SHARE::LEFT_OVER) {
+            const int in_rounds = run_len / per_xcd * per_xcd;
+            if (SHARE::FULL_ROUNDS) {
+                run_len = in_rounds;
+            } else {
+                run0 += in_rounds;
+                run_len = (run_len - in_rounds) * SUBS;
+            }
+        }
     }
     __device__ __forceinline__ int count() const { return li < run_len ? (run_len - li + per_xcd - 1) / per_xcd : 0; }
     // tile number j of this workgroup: its problem and its origin in that problem's C
     __device__ __forceinline__ void origin(int j, TileProblem& pr, int& m0, int& n0) const
     {
         const int per_group = GROUP_M * tiles_n;
-        int logical = run0 + li + j * per_xcd;
+        const int number = li + j * per_xcd;
+        int logical = run0 + number / SUBS;
         int tm = tiles_m;
         if (GROUPED) {
             int g = 0;
@@ -143,8 +172,9 @@ struct TileWalk {
         const int first_m = group * GROUP_M;
         const int gsz = (tm - first_m < GROUP_M) ? (tm - first_m) : GROUP_M;
         const int in_group = logical - group * per_group;
-        m0 = (first_m + in_group % gsz) * BM;
-        n0 = (in_group / gsz) * BN;
+        const int sub = number % SUBS;
+        m0 = (first_m + in_group % gsz) * BM + sub / SUBS_N * SHARE::SM;
+        n0 = (in_group / gsz) * BN + sub % SUBS_N * SHARE::SN;
     }
 };
 

@@ -191,6 +191,20 @@ def test_tile_kernel_256x256(pkg, m, n, k):
     assert np.array_equal(got, plain), "both tiles fold the same block sums in the same order"
 
 
+# Tiles of 256 x 256 beyond full rounds of 32 per XCD, cut into quarters or halves: one and eight left over on every XCD,
+# one on three XCDs only, sixteen, as few K blocks as the pieces' ring takes and fewer, odd K blocks over several tiles,
+# ragged edges in the last pieces (some of them wholly outside the matrix)
+@pytest.mark.parametrize("m,n,k", [(6128, 2800, 384), (5120, 4096, 640), (9456, 1776, 384), (6032, 4048, 1024), (6032, 4048, 896),
+                                   (5104, 3856, 256), (12288, 2800, 384)])
+def test_tile_kernel_256x256_tiles_left_over(pkg, m, n, k):
+    a, b, sa, sb = oracle.make_inputs(m, n, k, 3 * m + n + k, 0.5, 30.0)
+    got, name = _run(pkg, a, b, sa, sb, m, n, k, kernel=pkg.KERNEL_LARGE, variant=6)
+    assert name == "tile256x256_k1_persistent", name
+    _assert_every_element(got, a, b, sa, sb, m, n, k, name)
+    plain, _ = _run(pkg, a, b, sa, sb, m, n, k, kernel=pkg.KERNEL_LARGE, variant=0, persistent=0)
+    assert np.array_equal(got, plain), "whole tiles and pieces fold the same block sums in the same order"
+
+
 @pytest.mark.parametrize("variant,ksplit,m,n,k", [(2, 2, 256, 256, 512), (2, 4, 512, 512, 1024),
                                                    (1, 3, 272, 576, 896), (0, 8, 256, 576, 2048),
                                                    (2, 7, 128, 640, 7168), (1, 16, 256, 128, 2048), (3, 5, 384, 576, 1280),
@@ -984,6 +998,9 @@ def _grouped_case(pkg, ms, n, k, variant, seed):
                                             (1, [512] * 9 + [48, 2064], 1024, 384),
                                             (3, [144] * 40, 384, 640),
                                             (6, [2048, 272, 16, 1024, 4096], 1280, 512),
+                                            (6, [1040, 2320, 16, 0, 1536, 528, 2048], 2064, 384),   # 297 tiles: quarters
+                                            (6, [2064, 1280, 4096, 784, 1040], 2576, 1024),         # 429 tiles: 22 of 32 left over, whole
+                                            (6, [2064, 1280, 4096, 256], 3056, 1024),               # 372 tiles: halves
                                             (2, [128], 128, 384)])
 def test_grouped_gemm_equals_the_problems_one_by_one(pkg, variant, ms, n, k):
     host, dev, outs, name = _grouped_case(pkg, ms, n, k, variant, 7000 + n + k)
