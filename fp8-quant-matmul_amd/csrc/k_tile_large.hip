@@ -23,7 +23,8 @@
 // Bound by power on operands that toggle: 8192 x 4096 x 7168 (256 x 256) runs at a clock of 1.98 GHz with the matrix pipes
 // 62 % busy; without its copies it takes 160 us.  Against 32x32x64 MFMAs with the barrier at the block's end and the
 // tile leaving through a slot: 8192 x 4096 x 7168 212.7 -> 189 us = 51 % of 5033 TFLOP/s; 8192 x 4608 x 7168 (256 x 192) 252.8 ->
-// 239; 8192 x 7168 x 2048 (256 x 192 and 256 x 256) 136.7 -> 129.5 and 123.8 -> 117; 8192 x 7168 x 256 32.8 -> 29.
+// 239; 8192 x 7168 x 2048 (256 x 192 and 256 x 256) 136.7 -> 129.5 and 123.8 -> 117; 8192 x 7168 x 256 32.8 -> 29; with C's
+// stores past the caches (c_streams) 8192 x 4096 x 7168 180 us = 53 %.
 #include "tile_persistent_body.h"
 
 namespace fp8gemm {
@@ -64,7 +65,7 @@ __device__ __forceinline__ int lane_now()
 
 template <int BN, bool GROUPED, typename SHARE>
 __device__ __forceinline__ void large_tile_body(const TileProblem& one, const GroupTable* tab, int N, int K, int tiles_m,
-                                                int tiles_n)
+                                                int tiles_n, bool stream_c)
 {
     using L = LargeShape<BN>;
     using S = typename L::S;
@@ -314,7 +315,10 @@ __device__ __forceinline__ void large_tile_body(const TileProblem& one, const Gr
                     const int mrow = m_wave + 16 * i + row, ncol = n_wave + part * L::SCOLS + 8 * ch;
                     const v4i v = *LDS_PTR(v4i, lds + at(row, ch));
                     const uint32_t off = mrow < pr.M && ncol < N ? ((uint32_t)mrow * (uint32_t)N + (uint32_t)ncol) * 2u : 0xFFFFFFF0u;
-                    __builtin_amdgcn_raw_buffer_store_b128(v, rc, off, 0, 0);
+                    if (stream_c)
+                        __builtin_amdgcn_raw_buffer_store_b128(v, rc, off, 0, 2);  // nt
+                    else
+                        __builtin_amdgcn_raw_buffer_store_b128(v, rc, off, 0, 0);
                 }
                 asm volatile("" ::: "memory");
             }
@@ -392,14 +396,14 @@ constexpr int tail_lds_bytes()
 
 template <int BN, bool GROUPED, Tail TAIL>
 __device__ __forceinline__ void large_kernel_body(const TileProblem& one, const GroupTable* tab, int N, int K, int tiles_m,
-                                                  int tiles_n)
+                                                  int tiles_n, bool stream_c)
 {
     if constexpr (TAIL == Tail::NONE) {
-        large_tile_body<BN, GROUPED, AllTiles<256, BN>>(one, tab, N, K, tiles_m, tiles_n);
+        large_tile_body<BN, GROUPED, AllTiles<256, BN>>(one, tab, N, K, tiles_m, tiles_n, stream_c);
     } else {
         static_assert(BN == 256, "halves and quarters of 256x256");
         const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-        large_tile_body<BN, GROUPED, FullRounds<256, BN>>(one, tab, N, K, tiles_m, tiles_n);
+        large_tile_body<BN, GROUPED, FullRounds<256, BN>>(one, tab, N, K, tiles_m, tiles_n, stream_c);
         __syncthreads();  // nobody reads the slots any more
         const int thread = 64 * wave + lane_now();
         if constexpr (TAIL == Tail::HALVES)
@@ -415,18 +419,30 @@ template <int BN, Tail TAIL>
 __global__ void __launch_bounds__(NTHREADS)
 tile_gemm_large_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b, const float* __restrict__ a_scale,
                        const float* __restrict__ b_scale, uint16_t* __restrict__ c, int M, int lda, int N, int K, int tiles_m,
-                       int tiles_n)
+                       int tiles_n, int stream_c)
 {
     const TileProblem one{a, b, a_scale, b_scale, c, M, lda};
-    large_kernel_body<BN, false, TAIL>(one, nullptr, N, K, tiles_m, tiles_n);
+    large_kernel_body<BN, false, TAIL>(one, nullptr, N, K, tiles_m, tiles_n, stream_c != 0);
 }
 
 template <int BN, Tail TAIL>
 __global__ void __launch_bounds__(NTHREADS)
-tile_gemm_large_grouped_kernel(const GroupTable tab, int N, int K, int tiles_n)
+tile_gemm_large_grouped_kernel(const GroupTable tab, int N, int K, int tiles_n, int stream_c)
 {
     const TileProblem none{nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0};
-    large_kernel_body<BN, true, TAIL>(none, &tab, N, K, 0, tiles_n);
+    large_kernel_body<BN, true, TAIL>(none, &tab, N, K, 0, tiles_n, stream_c != 0);
+}
+
+// Whether C leaves with stores that tell the caches not to keep it.  The tiles of a round are stored together, 32 MB in a few
+// microseconds, and the lines that the L2s and the Infinity Cache then hold have to leave under the next rounds' reads.
+// Where the launch's data are small enough to stay, so does C.  Kept / not kept, us, three sets of operands in turn,
+// bytes of A, B and C together: 92 MB 8192 x 4096 x 2048 61.1 / 63.2; 108 MB 4608 x 4608 x 7168 139.0 / 137.0; 111 MB 8192 x
+// 5120 x 2048 79.5 / 80.8; 117 MB 8192 x 4096 x 4096 112.2 / 108.1, 4096 x 8192 x 4096 113.3 / 108.4; 130 MB 8192 x 6144 x 2048
+// 91.3 / 88.2; 155 MB 8192 x 4096 x 7168 187.7 / 180.2; 167 MB 8192 x 4608 x 7168 232.9 / 226.0; with the quantiser in front 8192
+// x 7168 x 2048 129.4 / 120.6.
+int c_streams(long rows, long weights, int n, int k)
+{
+    return (double)rows * k + (double)weights * n * k + 2.0 * rows * n >= 115e6 ? 1 : 0;
 }
 
 template <int BN, Tail TAIL>
@@ -436,7 +452,7 @@ hipError_t launch_large(const GemmArgs& g, int workgroups, hipStream_t s)
     auto kern = tile_gemm_large_kernel<BN, TAIL>;
     FP8GEMM_ALLOW_LDS(kern, LDS);
     hipLaunchKernelGGL(kern, dim3(workgroups), dim3(NTHREADS), LDS, s, g.a, g.b, g.a_scale, g.b_scale, g.c, g.m,
-                       leading_dim(g), g.n, g.k, (g.m + 255) / 256, (g.n + BN - 1) / BN);
+                       leading_dim(g), g.n, g.k, (g.m + 255) / 256, (g.n + BN - 1) / BN, c_streams(g.m, 1, g.n, g.k));
     return hipGetLastError();
 }
 
@@ -446,7 +462,11 @@ hipError_t launch_large_grouped(const GroupTable& tab, int n, int k, int workgro
     constexpr int LDS = LargeShape<BN>::LDS_BYTES > tail_lds_bytes<TAIL>() ? LargeShape<BN>::LDS_BYTES : tail_lds_bytes<TAIL>();
     auto kern = tile_gemm_large_grouped_kernel<BN, TAIL>;
     FP8GEMM_ALLOW_LDS(kern, LDS);
-    hipLaunchKernelGGL(kern, dim3(workgroups), dim3(NTHREADS), LDS, s, tab, n, k, (n + BN - 1) / BN);
+    long rows = 0;
+    for (int g = 0; g < tab.groups; ++g)
+        rows += tab.m[g];
+    hipLaunchKernelGGL(kern, dim3(workgroups), dim3(NTHREADS), LDS, s, tab, n, k, (n + BN - 1) / BN,
+                       c_streams(rows, tab.groups, n, k));
     return hipGetLastError();
 }
 
