@@ -79,7 +79,20 @@ __device__ __forceinline__ void lds_dma16(v4i rsrc, uint32_t voffset, uint32_t l
                  : "memory");
 }
 
-// The same where `skip` (wave-uniform) is zero.  The branch sits inside the statement: as one of the compiler's it would
+// The same; ONCE = bytes that the launch reads once, which the caches are told not to keep (nt).
+template <bool ONCE>
+__device__ __forceinline__ void lds_dma16_of(v4i rsrc, uint32_t voffset, uint32_t lds_addr, uint32_t soffset = 0)
+{
+    if constexpr (ONCE)
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %3 offen nt lds"
+                     :
+                     : "v"(voffset), "s"(rsrc), "s"(lds_addr), "s"(soffset)
+                     : "memory");
+    else
+        lds_dma16(rsrc, voffset, lds_addr, soffset);
+}
+
+// lds_dma16 where `skip` (wave-uniform) is zero.  The branch sits inside the statement: as one of the compiler's it would
 // end the block of instructions that LDS reads, MFMAs and folds are scheduled in.
 __device__ __forceinline__ void lds_dma16_unless(uint32_t skip, v4i rsrc, uint32_t voffset, uint32_t lds_addr, uint32_t soffset)
 {

@@ -47,6 +47,9 @@
 // holds workgroups and no K split: 256 workgroups walk through the strips -- of one problem or of all groups --
 // and the K blocks of all strips of a workgroup form one copy stream.
 //
+// ONCE: the caches are told not to keep B's bytes, which no other workgroup reads, and the streaming form's stores of C do the
+// same (b_read_once).
+//
 // LDS stage: 128 k-rows x 128 B of B (chunk c of row r at position c ^ ((r >> 1) & 7)), 128 x 32 B
 // of A (chunk c at c ^ ((r >> 3) & 1); 64-byte rows: c ^ ((r >> 2) & 3)), the block's a_scale and b_scale values; six stages form a
 // ring, up to five in flight while one is multiplied.  A CU takes in about 50 bytes per clock through
@@ -129,7 +132,7 @@ struct DecodeProblem {
 // blockIdx.y = split: gridDim.x is a multiple of 8, so their linear ids agree modulo 8 and they share an XCD.
 // TILES = the number of 16-row tiles when the launch knows it (a single problem: the count is then a constant
 // in the epilogue as well), 0 = read from the problem (grouped launches).
-template <int MT, bool GROUPED, int DS_NS, ARows FORM, int TILES, int NB, int STEP>
+template <int MT, bool GROUPED, int DS_NS, ARows FORM, int TILES, int NB, int STEP, bool ONCE>
 __device__ __forceinline__ void decode_body(const DecodeProblem& one, const GroupTable* tab, float* mailbox, int N, int K,
                                             int strips, int units, int ksplit, int kb_per_split)
 {
@@ -226,8 +229,8 @@ __device__ __forceinline__ void decode_body(const DecodeProblem& one, const Grou
         const uint32_t skip_b = (uint32_t)kb * KBLOCK * (uint32_t)N;
 #pragma unroll
         for (int h = 0; h < NB; ++h) {
-            lds_dma16(rsrc_b, voff_b[h][0], stage + (uint32_t)(h * S::HALF_B + (2 * wave) * 1024), skip_b);
-            lds_dma16(rsrc_b, voff_b[h][1], stage + (uint32_t)(h * S::HALF_B + (2 * wave + 1) * 1024), skip_b);
+            lds_dma16_of<ONCE>(rsrc_b, voff_b[h][0], stage + (uint32_t)(h * S::HALF_B + (2 * wave) * 1024), skip_b);
+            lds_dma16_of<ONCE>(rsrc_b, voff_b[h][1], stage + (uint32_t)(h * S::HALF_B + (2 * wave + 1) * 1024), skip_b);
         }
         if (RAGGED)
             issue_slab(slot + STEP >= DS_NS ? slot + STEP - DS_NS : slot + STEP, kb + STEP);
@@ -544,7 +547,7 @@ __device__ __forceinline__ void decode_body(const DecodeProblem& one, const Grou
     store_c(sum);
 }
 
-template <int MT, int DS_NS, ARows FORM, int TILES, int NB, int STEP>
+template <int MT, int DS_NS, ARows FORM, int TILES, int NB, int STEP, bool ONCE>
 __global__ void __launch_bounds__(DS_THREADS)
 decode_strip_kernel(const uint8_t* __restrict__ b, const uint8_t* __restrict__ a, int N, int K, int M, int lda,
                     int kb_per_split, int strips, const float* __restrict__ a_scale, const float* __restrict__ b_scale,
@@ -552,16 +555,16 @@ decode_strip_kernel(const uint8_t* __restrict__ b, const uint8_t* __restrict__ a
 {
     // (the first 14 words of the arguments are in registers when a wave starts: what the copies need comes first)
     const DecodeProblem one{a, b, a_scale, b_scale, c, M, lda};
-    decode_body<MT, false, DS_NS, FORM, TILES, NB, STEP>(one, nullptr, mailbox, N, K, strips, strips, ksplit, kb_per_split);
+    decode_body<MT, false, DS_NS, FORM, TILES, NB, STEP, ONCE>(one, nullptr, mailbox, N, K, strips, strips, ksplit, kb_per_split);
 }
 
-template <int MT, int DS_NS, bool RAGGED, int STEP>
+template <int MT, int DS_NS, bool RAGGED, int STEP, bool ONCE>
 __global__ void __launch_bounds__(DS_THREADS)
 decode_strip_grouped_kernel(const GroupTable tab, float* mailbox, int N, int K, int strips, int ksplit, int kb_per_split)
 {
     const DecodeProblem none{nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0};
     constexpr ARows FORM = RAGGED ? ARows::SPREAD : ARows::GRID;
-    decode_body<MT, true, DS_NS, FORM, 0, 1, STEP>(none, &tab, mailbox, N, K, strips, strips * tab.groups, ksplit, kb_per_split);
+    decode_body<MT, true, DS_NS, FORM, 0, 1, STEP, ONCE>(none, &tab, mailbox, N, K, strips, strips * tab.groups, ksplit, kb_per_split);
 }
 
 // The streaming form, for a single problem without a K split whose strips outnumber the workgroups the
@@ -579,7 +582,7 @@ decode_strip_grouped_kernel(const GroupTable tab, float* mailbox, int N, int K, 
 // writes to HBM among the reads, whatever their shape).  Needs c on a 16-byte boundary.
 // GROUPED: units run through the strips of all problems of `tab` (TILES = 0: the tile count is the unit's own, and
 // the stage's math is chosen by it -- one straight-line copy per count).
-template <int MT, int DS_NS, int TILES, bool STAGED, int NB, bool GROUPED>
+template <int MT, int DS_NS, int TILES, bool STAGED, int NB, bool GROUPED, bool ONCE>
 __device__ __forceinline__ void decode_stream_body(const DecodeProblem& one, const GroupTable* tab, int N, int K, int strips,
                                                    int units)
 {
@@ -641,8 +644,8 @@ __device__ __forceinline__ void decode_stream_body(const DecodeProblem& one, con
         const v4i rb = make_rsrc_words(cp.b + skip_b, b_bytes - skip_b);
 #pragma unroll
         for (int h = 0; h < NB; ++h) {
-            lds_dma16(rb, voff_b[h][0], stage + (uint32_t)(h * S::HALF_B + (2 * wave) * 1024));
-            lds_dma16(rb, voff_b[h][1], stage + (uint32_t)(h * S::HALF_B + (2 * wave + 1) * 1024));
+            lds_dma16_of<ONCE>(rb, voff_b[h][0], stage + (uint32_t)(h * S::HALF_B + (2 * wave) * 1024));
+            lds_dma16_of<ONCE>(rb, voff_b[h][1], stage + (uint32_t)(h * S::HALF_B + (2 * wave + 1) * 1024));
         }
         const int scale_wave = MT == 2 ? wave - 4 : wave;
         if (MT == 4 || wave < 4)
@@ -665,6 +668,13 @@ __device__ __forceinline__ void decode_stream_body(const DecodeProblem& one, con
             cp_kb = 0;
             cp_unit += G;
         }
+    };
+
+    auto store_c = [](auto v, uint16_t* to) __attribute__((always_inline)) {
+        if (ONCE)
+            __builtin_nontemporal_store(v, reinterpret_cast<decltype(v)*>(to));
+        else
+            *reinterpret_cast<decltype(v)*>(to) = v;
     };
 
     // ---- multiply side
@@ -765,8 +775,7 @@ __device__ __forceinline__ void decode_stream_body(const DecodeProblem& one, con
                     const int row = idx / CPR, ch = idx % CPR;
                     const int ncol = mp_strip * BN + 8 * ch;
                     if (row < mp.M && ncol < N)
-                        *reinterpret_cast<v4i*>(mp.c + (size_t)row * N + ncol) =
-                            *LDS_PTR(v4i, lds + cbase + row * C_STAGE_ROW + 16 * ch);
+                        store_c(*LDS_PTR(v4i, lds + cbase + row * C_STAGE_ROW + 16 * ch), mp.c + (size_t)row * N + ncol);
                 }
             } else {
 #pragma unroll
@@ -776,10 +785,9 @@ __device__ __forceinline__ void decode_stream_body(const DecodeProblem& one, con
                     for (int i = 0; i < MT; ++i) {
                         const int mrow = 16 * i + i16;
                         if (mrow < mp.M && ncol < N) {
-                            uint2 pk;
-                            pk.x = pack_bf16x2(acc[h][i][0], acc[h][i][1]);
-                            pk.y = pack_bf16x2(acc[h][i][2], acc[h][i][3]);
-                            *reinterpret_cast<uint2*>(mp.c + (size_t)mrow * N + ncol) = pk;
+                            const v2i pk = {(int)pack_bf16x2(acc[h][i][0], acc[h][i][1]),
+                                            (int)pack_bf16x2(acc[h][i][2], acc[h][i][3])};
+                            store_c(pk, mp.c + (size_t)mrow * N + ncol);
                         }
                     }
                 }
@@ -790,22 +798,22 @@ __device__ __forceinline__ void decode_stream_body(const DecodeProblem& one, con
     }
 }
 
-template <int MT, int DS_NS, bool STAGED, int NB>
+template <int MT, int DS_NS, bool STAGED, int NB, bool ONCE>
 __global__ void __launch_bounds__(DS_THREADS)
 decode_stream_grouped_kernel(const GroupTable tab, int N, int K, int strips, int units)
 {
     const DecodeProblem none{};
-    decode_stream_body<MT, DS_NS, 0, STAGED, NB, true>(none, &tab, N, K, strips, units);
+    decode_stream_body<MT, DS_NS, 0, STAGED, NB, true, ONCE>(none, &tab, N, K, strips, units);
 }
 
-template <int MT, int DS_NS, int TILES, bool STAGED, int NB>
+template <int MT, int DS_NS, int TILES, bool STAGED, int NB, bool ONCE>
 __global__ void __launch_bounds__(DS_THREADS)
 decode_stream_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b, const float* __restrict__ a_scale,
                      const float* __restrict__ b_scale, uint16_t* __restrict__ c, int M, int lda, int N, int K,
                      int strips)
 {
     const DecodeProblem one{a, b, a_scale, b_scale, c, M, lda};
-    decode_stream_body<MT, DS_NS, TILES, STAGED, NB, false>(one, nullptr, N, K, strips, strips);
+    decode_stream_body<MT, DS_NS, TILES, STAGED, NB, false, ONCE>(one, nullptr, N, K, strips, strips);
 }
 
 // records the XCC (XCD) id each workgroup of a probe grid runs on
@@ -850,6 +858,14 @@ inline bool stages_in_pairs(long workgroups, int kb_per_split, int ring)
 // Measured on grouped launches: 64 groups x 56 strips, 16 K blocks each: 221 against 236 us; with 768-1152
 // workgroups (1.5-2.25 rounds of 512 resident ones) 1-3 % slower than three to four and a half rounds of 256.
 inline bool shallow_ring_pays(long workgroups, int kb_per_split) { return workgroups >= 2048 && kb_per_split >= 6; }
+
+// Whether the caches are told not to keep B.  Kept / not kept, us: from HBM 32 x 7168 x 2048 7.00 / 6.79, 24 x 4608 x 7168
+// 11.34 / 11.02, 16 x 16384 x 7168 25.2 / 23.7, 8 x 49152 x 4096 37.5 / 35.5, 16 groups of up to 32 rows, 7168 x 2048, 50.9 /
+// 46.5, 64 of 1 - 63 rows 190.7 / 179.7; from the Infinity Cache 1 x 7168 x 2048 5.68 / 5.43, 16 x 4608 x 7168 9.00 / 8.90.
+// A smaller B, whose launches leave most CUs without a strip, stays in the caches and is not helped: 16 x 1536 x 7168 from
+// HBM 7.02 / 6.98, from the Infinity Cache 6.03 / 6.60.  Strips that are no whole 128-byte lines share some: 16 x 576 x 7168 6.92 /
+// 7.27 and 5.87 / 6.68, 64 groups of up to 32 rows, 7152 x 2048, 189.6 / 215.0.
+inline bool b_read_once(int groups, int n, int k) { return n % 128 == 0 && (double)groups * n * k >= 12e6; }
 
 }  // namespace
 
@@ -963,6 +979,7 @@ hipError_t launch_decode_strips(const GemmArgs& g, int ksplit, int halves, float
     const int kb_per_split = (nkb + ksplit - 1) / ksplit;
     if ((ksplit - 1) * kb_per_split >= nkb)  // every split owns at least one K block
         return hipErrorInvalidValue;
+    const bool once = b_read_once(1, g.n, g.k);
     const dim3 grid(8 * ((strips + 7) / 8), ksplit);
     auto go = [&](auto kern, int lds) -> hipError_t {
         FP8GEMM_ALLOW_LDS(kern, lds);
@@ -986,11 +1003,13 @@ hipError_t launch_decode_strips(const GemmArgs& g, int ksplit, int halves, float
             constexpr bool ST = decltype(staged_c)::value;
             constexpr int lds = DecodeShape<MT, NS, false, NB>::LDS + (ST ? 16 * T * (2 * DS_BN * NB + 16) : 0);
             static_assert(lds <= 160 * 1024, "ring and staged C exceed the LDS");
-            auto kern = decode_stream_kernel<MT, NS, T, ST, NB>;
-            FP8GEMM_ALLOW_LDS(kern, lds);
-            hipLaunchKernelGGL(kern, dim3(STREAM_WORKGROUPS), dim3(DS_THREADS), lds, s, g.a, g.b, g.a_scale, g.b_scale, g.c,
-                               g.m, leading_dim(g), g.n, g.k, units);
-            return hipGetLastError();
+            auto with = [&](auto kern) -> hipError_t {
+                FP8GEMM_ALLOW_LDS(kern, lds);
+                hipLaunchKernelGGL(kern, dim3(STREAM_WORKGROUPS), dim3(DS_THREADS), lds, s, g.a, g.b, g.a_scale, g.b_scale,
+                                   g.c, g.m, leading_dim(g), g.n, g.k, units);
+                return hipGetLastError();
+            };
+            return once ? with(decode_stream_kernel<MT, NS, T, ST, NB, true>) : with(decode_stream_kernel<MT, NS, T, ST, NB, false>);
         };
         auto by_staging = [&](auto shape, auto tiles_c) -> hipError_t {
             return staged ? stream(shape, tiles_c, std::true_type{}) : stream(shape, tiles_c, std::false_type{});
@@ -1015,8 +1034,9 @@ hipError_t launch_decode_strips(const GemmArgs& g, int ksplit, int halves, float
         auto wide = [&](auto mt_c, auto form_c, auto tiles_c) -> hipError_t {
             constexpr int MT = decltype(mt_c)::value, T = decltype(tiles_c)::value;
             constexpr ARows F = decltype(form_c)::value;
-            return go(decode_strip_kernel<MT, STREAM_NS_WIDE, F, T, 2, 1>,
-                      DecodeShape<MT, STREAM_NS_WIDE, F == ARows::SPREAD, 2>::LDS);
+            constexpr int lds = DecodeShape<MT, STREAM_NS_WIDE, F == ARows::SPREAD, 2>::LDS;
+            return once ? go(decode_strip_kernel<MT, STREAM_NS_WIDE, F, T, 2, 1, true>, lds)
+                        : go(decode_strip_kernel<MT, STREAM_NS_WIDE, F, T, 2, 1, false>, lds);
         };
         auto by_tiles = [&](auto form_c) -> hipError_t {
             switch (tiles) {
@@ -1043,8 +1063,10 @@ hipError_t launch_decode_strips(const GemmArgs& g, int ksplit, int halves, float
         constexpr int lds = DecodeShape<MT, NS, F == ARows::SPREAD>::LDS;
         if constexpr (NS % 2 == 0)
             if (stages_in_pairs((long)strips * ksplit, kb_per_split, NS))
-                return go(decode_strip_kernel<MT, NS, F, T, 1, 2>, lds);
-        return go(decode_strip_kernel<MT, NS, F, T, 1, 1>, lds);
+                return once ? go(decode_strip_kernel<MT, NS, F, T, 1, 2, true>, lds)
+                            : go(decode_strip_kernel<MT, NS, F, T, 1, 2, false>, lds);
+        return once ? go(decode_strip_kernel<MT, NS, F, T, 1, 1, true>, lds)
+                    : go(decode_strip_kernel<MT, NS, F, T, 1, 1, false>, lds);
     };
     using std::integral_constant;
     auto by_tiles = [&](auto ns2, auto ns4, auto form_c) -> hipError_t {
@@ -1141,6 +1163,7 @@ hipError_t launch_decode_grouped(const GroupTable& tab, int n, int k, int ksplit
         mmax = tab.lda[g] > mmax ? tab.lda[g] : mmax;
         ragged |= tab.lda[g] % 16 != 0;
     }
+    const bool once = b_read_once(tab.groups, n, k);
     // many strips, rows on the 16-byte grid, no K split: the streaming form with 256-column strips
     const int wide_strips = (n + 2 * DS_BN - 1) / (2 * DS_BN);
     const long wide_units = (long)wide_strips * tab.groups;
@@ -1153,11 +1176,14 @@ hipError_t launch_decode_grouped(const GroupTable& tab, int n, int k, int ksplit
             constexpr bool ST = decltype(staged_c)::value;
             constexpr int lds = DecodeShape<MT, NS, false, NB>::LDS + (ST ? 16 * MT * (2 * DS_BN * NB + 16) : 0);
             static_assert(lds <= 160 * 1024, "ring and staged C exceed the LDS");
-            auto kern = decode_stream_grouped_kernel<MT, NS, ST, NB>;
-            FP8GEMM_ALLOW_LDS(kern, lds);
-            hipLaunchKernelGGL(kern, dim3(STREAM_WORKGROUPS), dim3(DS_THREADS), lds, s, tab, n, k, wide_strips,
-                               (int)wide_units);
-            return hipGetLastError();
+            auto with = [&](auto kern) -> hipError_t {
+                FP8GEMM_ALLOW_LDS(kern, lds);
+                hipLaunchKernelGGL(kern, dim3(STREAM_WORKGROUPS), dim3(DS_THREADS), lds, s, tab, n, k, wide_strips,
+                                   (int)wide_units);
+                return hipGetLastError();
+            };
+            return once ? with(decode_stream_grouped_kernel<MT, NS, ST, NB, true>)
+                        : with(decode_stream_grouped_kernel<MT, NS, ST, NB, false>);
         };
         if (row_tiles(mmax) == 2)
             return staged ? stream(StreamShape<2, STREAM_NS_WIDE, 2>{}, std::true_type{})
@@ -1182,8 +1208,10 @@ hipError_t launch_decode_grouped(const GroupTable& tab, int n, int k, int ksplit
         constexpr int lds = DecodeShape<MT, NS, RG>::LDS;
         if constexpr (NS % 2 == 0)
             if (stages_in_pairs(units * ksplit, kb_per_split, NS) && !(RG && (kb_per_split == 1 || kb_per_split == 3)))
-                return go(decode_strip_grouped_kernel<MT, NS, RG, 2>, lds);
-        return go(decode_strip_grouped_kernel<MT, NS, RG, 1>, lds);
+                return once ? go(decode_strip_grouped_kernel<MT, NS, RG, 2, true>, lds)
+                            : go(decode_strip_grouped_kernel<MT, NS, RG, 2, false>, lds);
+        return once ? go(decode_strip_grouped_kernel<MT, NS, RG, 1, true>, lds)
+                    : go(decode_strip_grouped_kernel<MT, NS, RG, 1, false>, lds);
     };
     using std::integral_constant;
     const integral_constant<int, 2> two{};
