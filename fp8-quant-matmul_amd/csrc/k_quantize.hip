@@ -32,16 +32,29 @@ namespace fp8gemm {
 namespace {
 
 // eight consecutive k of one row as they lie in memory: four words of bf16 pairs, or eight of fp32
+// ONCE = the caches are told not to keep them
+template <bool ONCE>
+__device__ __forceinline__ v4i load_piece(const void* p)
+{
+    return ONCE ? __builtin_nontemporal_load(static_cast<const v4i*>(p)) : *static_cast<const v4i*>(p);
+}
+template <bool ONCE>
 __device__ __forceinline__ void load_raw(const uint16_t* p, uint32_t (&w)[4])
 {
-    const uint4 v = *reinterpret_cast<const uint4*>(p);
-    w[0] = v.x; w[1] = v.y; w[2] = v.z; w[3] = v.w;
+    const v4i v = load_piece<ONCE>(p);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        w[i] = (uint32_t)v[i];
 }
+template <bool ONCE>
 __device__ __forceinline__ void load_raw(const float* p, uint32_t (&w)[8])
 {
-    const uint4 lo = reinterpret_cast<const uint4*>(p)[0], hi = reinterpret_cast<const uint4*>(p)[1];
-    w[0] = lo.x; w[1] = lo.y; w[2] = lo.z; w[3] = lo.w;
-    w[4] = hi.x; w[5] = hi.y; w[6] = hi.z; w[7] = hi.w;
+    const v4i lo = load_piece<ONCE>(p), hi = load_piece<ONCE>(p + 4);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        w[i] = (uint32_t)lo[i];
+        w[4 + i] = (uint32_t)hi[i];
+    }
 }
 template <int J>
 __device__ __forceinline__ float value(const uint32_t (&w)[4])
@@ -105,7 +118,8 @@ __device__ __forceinline__ float scale_of(float amax)
 
 // BLOCK = false: one scale per row and 128 k (1 x 128).  BLOCK = true: one per 128 x 128.
 // QTILE = rows of a workgroup's tile, 16 per wave (4 rows x 8 k per thread).
-template <typename TIn, bool BLOCK, bool BF16MATH, int QTILE>
+// ONCE = x is read past the caches.
+template <typename TIn, bool BLOCK, bool BF16MATH, int QTILE, bool ONCE>
 __global__ void __launch_bounds__(QTILE * 4)
 quantize_kernel(const TIn* __restrict__ x, uint8_t* __restrict__ q, float* __restrict__ scale_out,
                 int rows, int K, int grid)
@@ -136,7 +150,7 @@ quantize_kernel(const TIn* __restrict__ x, uint8_t* __restrict__ q, float* __res
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int row = row0 + 16 * wave + 4 * g + i;
-        load_raw(x + (size_t)(row < rows ? row : rows - 1) * K + (size_t)kb * 128 + 8 * c, raw[i]);
+        load_raw<ONCE>(x + (size_t)(row < rows ? row : rows - 1) * K + (size_t)kb * 128 + 8 * c, raw[i]);
     }
 
     float amax[4];
@@ -279,11 +293,11 @@ int output_grid(const uint8_t* q, int rows)
     return ends % 16 == 0 ? 16 : ends % 8 == 0 ? 8 : 0;
 }
 
-template <typename TIn, bool BLOCK, bool BF16MATH, int QTILE>
+template <typename TIn, bool BLOCK, bool BF16MATH, int QTILE, bool ONCE = false>
 void launch_quantize_tile(const TIn* x, uint8_t* q, float* scale_out, int rows, int k, hipStream_t s)
 {
     const int grid = output_grid(q, rows);
-    hipLaunchKernelGGL((quantize_kernel<TIn, BLOCK, BF16MATH, QTILE>), dim3((rows + QTILE - 1) / QTILE, k / 128),
+    hipLaunchKernelGGL((quantize_kernel<TIn, BLOCK, BF16MATH, QTILE, ONCE>), dim3((rows + QTILE - 1) / QTILE, k / 128),
                        dim3(QTILE * 4), 0, s, x, q, scale_out, rows, k, grid);
 }
 
@@ -300,13 +314,23 @@ void launch_quantize_tile(const TIn* x, uint8_t* q, float* scale_out, int rows, 
 //   Multiples of 8 rows leave in 8-byte stores, without the shifting and the single bytes, and count as on the grid
 //   (with the GEMM behind it: 24 x 512 x 7168 10.43 -> 10.09, 200 x 512 x 7168 13.84 -> 13.25, 1032 x 512 x 7168 25.97 ->
 //   24.13, 8184 x 1536 x 2048 46.4 -> 45.3; 24 rows of fp32 10.52 -> 10.04).
+//   Values and codes of 115 MB or more together, nearly half of the Infinity Cache, do not stay there beside whatever else
+//   runs: the values are read past it (kept / not kept, us, three sets in turn, 1 x 128 with the GEMM behind it: bf16 129 MB
+//   6000 x 1536 x 7168 114.5 / 100.8, 176 MB 8192 x 512 x 7168 71.7 / 65.5; blocks of bf16 99 MB 4608 x 7168 17.88 / 18.17,
+//   176 MB 8192 x 7168 36.6 / 31.0; fp32 84 MB 8192 x 576 x 2048 36.3 / 40.3, 147 MB 4096 x 1536 x 7168 79.9 / 80.2, 168 MB
+//   8192 x 576 x 4096 75.4 / 74.0, 215 MB 6000 x 1536 x 7168 131.8 / 119.2; blocks of fp32 106 MB 4608 x 4608 20.6 / 22.7, 126
+//   MB 8192 x 3072 27.5 / 26.5, 165 MB 4608 x 7168 34.3 / 32.5.  bf16 with its GEMM gains from 97 MB on: 4500 x 4608 x 7168
+//   182.7 / 178.8).
 template <typename TIn, bool BF16MATH>
 void launch_quantize_typed(const TIn* x, uint8_t* q, float* scale_out, int rows, int k, bool block128, hipStream_t s)
 {
     const bool on_grid = rows % 16 == 0 || output_grid(q, rows) == 8;
     const long nkb = k / 128;
     auto tiles = [&](int qtile) { return (rows + qtile - 1) / qtile * nkb; };
-    if (block128)
+    const bool once = (double)rows * k * (sizeof(TIn) + 1) >= 115e6;
+    if (block128 && once)
+        launch_quantize_tile<TIn, true, BF16MATH, 128, true>(x, q, scale_out, rows, k, s);
+    else if (block128)
         launch_quantize_tile<TIn, true, BF16MATH, 128>(x, q, scale_out, rows, k, s);
     else if (rows <= (on_grid ? 32 : 16))
         launch_quantize_tile<TIn, false, BF16MATH, 16>(x, q, scale_out, rows, k, s);
@@ -314,6 +338,8 @@ void launch_quantize_typed(const TIn* x, uint8_t* q, float* scale_out, int rows,
         launch_quantize_tile<TIn, false, BF16MATH, 64>(x, q, scale_out, rows, k, s);
     else if (tiles(256) < 256)
         launch_quantize_tile<TIn, false, BF16MATH, 128>(x, q, scale_out, rows, k, s);
+    else if (once)
+        launch_quantize_tile<TIn, false, BF16MATH, 256, true>(x, q, scale_out, rows, k, s);
     else
         launch_quantize_tile<TIn, false, BF16MATH, 256>(x, q, scale_out, rows, k, s);
 }

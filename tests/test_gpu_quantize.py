@@ -192,3 +192,11 @@ def test_quantize_tile_sizes_and_ends(pkg, rows, k, offset, source):
 @pytest.mark.parametrize("source", ["bf16", "f32"])
 def test_quantize_rows_on_an_8_byte_grid(pkg, rows, k, offset, source):
     test_quantize_tile_sizes_and_ends(pkg, rows, k, offset, source)
+
+
+@pytest.mark.parametrize("source,rows,k,offset", [("bf16", 18733, 2048, 3), ("bf16", 18720, 2048, 0), ("f32", 11232, 2048, 0),
+                                                  ("f32", 11233, 2048, 5)])
+def test_quantize_values_read_past_the_caches(pkg, source, rows, k, offset):
+    """values and codes of 115 MB and a little more: the instances that take over from there, on the grid and off it"""
+    assert rows * k * (3 if source == "bf16" else 5) >= 115e6
+    test_quantize_tile_sizes_and_ends(pkg, rows, k, offset, source)
