@@ -28,18 +28,28 @@
 //     the K loop holds no compiler-visible global load and every wait on the copies is the
 //     explicit one below.  b_scale is asked for by scalar loads one K block ahead: in the block that
 //     needs it its trip to the L2 would stand in front of the MFMAs (from the Infinity Cache, 128 x 128
-//     tiles, 336 x 4608 x 7168: 27.1 -> 22.6 us; 1024 x 1536 x 7168: 24.9 -> 21.6 us).  The smallest tile is
-//     done before that trip is: there a wave that does not multiply copies b_scale into the stage
-//     (48 x 4608 x 7168: 14.2 -> 10.9 us).
+//     tiles, 336 x 4608 x 7168: 27.1 -> 22.6 us; 1024 x 1536 x 7168: 24.9 -> 21.6 us).  Where only four waves
+//     multiply, a wave that does not copies b_scale into the stage (64x64 tiles, which are done before that
+//     trip is: 48 x 4608 x 7168 14.2 -> 10.9 us).
+//   * The two smaller tiles, 64x64 and 128x128, are multiplied by four waves, one per SIMD, and copied by the other
+//     four.  What bounds a K block of them is the LDS: in a block of its own, every wave's reads come first (all waves',
+//     640 clocks for 128x128 in eight waves of 64x32) and its MFMAs, 512 clocks, behind them.  Four waves of 64x64 read
+//     two thirds of that, and they read block kb + 1 into a second set of registers between the MFMAs of block kb, so that
+//     a block takes the longer of the two and not their sum; the folds of a block's last four sums cross the barrier.
+//     Before (eight waves, reads at the head of the block) / after, from the Infinity Cache: 5504 x 512 x 7168 30.7 -> 26.7 us,
+//     2048 x 2048 x 7168 36.1 -> 32.0, 1024 x 1536 x 7168 21.4 -> 19.6, 352 x 3072 x 1536 9.4 -> 8.9, 350 x 3072 x 1536
+//     (RAGGED) 11.3 -> 10.5, 64x64 tiles 1024 x 512 x 2048 6.1 -> 5.9; 64 x 4608 x 7168, bound by the copies, 10.4 -> 10.5.
+//     Copies between the MFMAs of a lone wave hold them up (RAGGED with B copied there: 350 x 3072 x 1536 12.3 us), so
+//     they are the other waves'.  Eight stages of 64x64 instead of four: slower, 5.9 -> 6.8 us.
 //   * NS LDS stages form a ring: the copies of K blocks kb+1 .. kb+NS-1 are in flight while
 //     block kb is multiplied.  Large tiles fit two stages; smaller tiles get three or four,
 //     which is what hides the global latency when a K block is only a few MFMAs long.
-//   * The copy instructions of a K block ride on the first MFMAs of an earlier block instead
+//   * Where all eight waves multiply, the copy instructions of a K block ride on the first MFMAs of an earlier block instead
 //     of being issued in one burst after the barrier (a burst queues up in the address unit
 //     and holds every wave back from its LDS reads).
 //
 //   * RAGGED: M is no multiple of 16, so A's k-rows start anywhere and 16-byte copies straight to LDS are out.  Four of
-//     the eight waves load A's pieces into registers from where they lie (a load takes any address; measured: no slower
+//     the eight waves (two of the four that do not multiply) load A's pieces into registers from where they lie (a load takes any address; measured: no slower
 //     off the grid than on it) and write them to the ring a step before they are multiplied, two or three register
 //     sets ahead; the other four copy B and the scales as ever.  Each kind has a loop of its own, so that the compiler's
 //     waits count the loads of A alone.  A K block takes 0.05 - 0.1 us more than with copies throughout (128 x 128, 336 x
@@ -69,11 +79,10 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
                  int M, int lda, int N, int K, int tiles_m, int tiles_n, int kb_per_split, int group_m)
 {
     using S = TileShape<BM, BN, WM, WN, NS>;
-    // Eight waves copy; WM x WN of them (all eight, or the first four for the smallest tile)
-    // also multiply.
+    // WM x WN waves multiply: all eight, or the first four of the two smaller tiles (AHEAD)
     static_assert(WM * WN == 8 || WM * WN == 4, "eight or four multiplying waves");
     constexpr int NCW = WM * WN;
-    static_assert(NS >= 2 && NS <= 4, "two to four LDS stages");
+    static_assert(NCW == 4 ? NS == 4 : NS == 2 || NS == 3, "LDS stages");
     constexpr int TM = BM / WM, TN = BN / WN;      // wave tile
     constexpr int MI = TM / 16, NJ = TN / 16;      // 16x16 patches per wave
     static_assert(TM % 16 == 0 && TN % 32 == 0, "wave tile is made of 16x16 patches, pairs of them along n");
@@ -81,15 +90,14 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
     static_assert(BM <= 256 && BN <= 256, "LDS rows hold at most 256 bytes");
     constexpr int RSA = S::RSA, RSB = S::RSB, NA = S::NA, NB = S::NB, NCOPY = S::NCOPY;
     static_assert(!RAGGED || NS >= 3, "A's registers are written a step ahead of the multiply");
-    // RAGGED: waves 0 - 3 copy B and the scales, waves 4 - 7 load A, twice as much per wave each
-    constexpr int A_WAVE = 4, NAW = 2 * NA, NBW = RAGGED ? 2 * NB : NB;
+    // Who copies: all eight waves; the four that do not multiply, if there are such.  RAGGED: waves 0 - 3 copy B and the
+    // scales and waves 4 - 7 load A; where those do not multiply, waves 4 and 5 load A and waves 6 and 7 copy.
+    constexpr bool AHEAD = NCW == 4;
+    constexpr int A_WAVE = 4, A_WAVES = AHEAD ? 2 : 4, NAW = 8 / A_WAVES * NA;
+    constexpr int COPIERS = !AHEAD && !RAGGED ? 8 : AHEAD && RAGGED ? 2 : 4;
+    constexpr int NBW = 8 / COPIERS * NB, NAC = RAGGED ? 0 : 8 / COPIERS * NA;  // copies of such a wave per K block
     constexpr int SETS = NS - 1, LEAD = SETS + 1;  // register sets of A, and K blocks that they run ahead
-    // A's registers are emptied behind the first MFMA of a block; with two sets only behind its last one, a step is short
-    // for the loads' trip (128x192, per K block from the Infinity Cache: 0.83 us early, 0.76 us late; 128x128 with three
-    // sets 0.59 and 0.61 us)
-    constexpr bool A_EARLY = SETS >= 3;
-    static_assert(!RAGGED || BM <= 64 * A_WAVE, "a wave that copies for every 64 rows of a_scale");
-    constexpr int SCALE_WAVE = NCW == 4 ? 4 : 0;  // brings the a_scale slice: a wave that does not multiply, if there is one
+    static_assert(!RAGGED || BM <= 64 * COPIERS, "a wave that copies for every 64 rows of a_scale");
 
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
     auto lds = LDS_PTR(uint8_t, smem);
@@ -97,8 +105,9 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int copier = wave & (COPIERS - 1);
     const int wm = wave % WM, wn = (wave / WM) % WN;
-    const bool compute = NCW == 8 || wave < NCW;
+    const bool compute = !AHEAD || wave < NCW;
 
     // ---- which tile: consecutive workgroup ids land on different XCDs (id % 8), so give
     // each XCD a contiguous run of tile numbers, and walk tiles in groups of group_m rows
@@ -130,14 +139,14 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
     uint32_t voff_a[S::NVA], voff_b[S::NVB];  // RAGGED: voff_a is not used, voff_b by the waves that copy
 #pragma unroll
     for (int q = 0; q < S::NVA; ++q) {
-        const int r = (NA * wave + q) * (1024 / RSA) + S::template copy_row<RSA>(lane);
+        const int r = (NAC * copier + q) * (1024 / RSA) + S::template copy_row<RSA>(lane);
         const int cc = S::template copy_pos<RSA>(lane) ^ row_swizzle<RSA>(r);
         const bool ok = (16 * cc < BM) && (m0 + 16 * cc < M);
         voff_a[q] = ok ? (uint32_t)(r * lda + m0 + 16 * cc) : 0x80000000u;
     }
 #pragma unroll
     for (int q = 0; q < S::NVB; ++q) {
-        const int r = (NBW * wave + q) * (1024 / RSB) + S::template copy_row<RSB>(lane);
+        const int r = (NBW * copier + q) * (1024 / RSB) + S::template copy_row<RSB>(lane);
         const int cc = S::template copy_pos<RSB>(lane) ^ row_swizzle<RSB>(r);
         const bool ok = (16 * cc < BN) && (n0 + 16 * cc < N);
         voff_b[q] = ok ? (uint32_t)(r * N + n0 + 16 * cc) : 0x80000000u;
@@ -146,14 +155,14 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
     const uint32_t as_bytes = (uint32_t)nkb * (uint32_t)lda * 4u;
     // a_scale: 16 bytes per lane by one wave; rows that do not start on the 16-byte grid by 4 bytes per lane and a wave
     // for every 64 of them
-    const int scale_m = RAGGED ? m0 + 64 * wave + lane : m0 + 4 * lane;
-    const uint32_t voff_s = (RAGGED ? 64 * wave < BM : 4 * lane < BM) && scale_m < M ? (uint32_t)(scale_m * 4) : 0x80000000u;
+    const int scale_m = RAGGED ? m0 + 64 * copier + lane : m0 + 4 * lane;
+    const uint32_t voff_s = (RAGGED ? 64 * copier < BM : 4 * lane < BM) && scale_m < M ? (uint32_t)(scale_m * 4) : 0x80000000u;
 
     // RAGGED: the 16 bytes per lane that a copy instruction would bring, by a load from wherever they lie; pieces
     // without a row of the matrix bring the tile's first one instead
     uint32_t off_a[NAW];
     v4i set_a[SETS][NAW];
-    const bool loads_a = wave >= A_WAVE;
+    const bool loads_a = wave >= A_WAVE && wave < A_WAVE + A_WAVES;
     const int a_first = NAW * (wave - A_WAVE);  // first KiB of the A tile that the wave brings
     if constexpr (RAGGED) {
 #pragma unroll
@@ -193,7 +202,7 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
     const v4i rsrc_bs = make_rsrc_words(b_scale, (uint32_t)nkb * (uint32_t)sn * 4u);
     const uint32_t voff_sb = lane == 0 ? (uint32_t)((n0 >> 7) * 4) : 0x80000000u;  // staged: the tile is at most 128 wide
     auto copy_b = [&](uint32_t stage, int kb, int q) __attribute__((always_inline)) {
-        lds_dma16(rsrc_b, voff_b[S::template voff_index<RSB>(q)], stage + S::MAT_A + (uint32_t)((NBW * wave + q) * 1024),
+        lds_dma16(rsrc_b, voff_b[S::template voff_index<RSB>(q)], stage + S::MAT_A + (uint32_t)((NBW * copier + q) * 1024),
                   (uint32_t)(kb * KBLOCK + S::template extra_rows<RSB>(q)) * (uint32_t)N);
     };
     auto copy_step = [&](int slot, int kb, int q) __attribute__((always_inline)) {
@@ -203,23 +212,32 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
                       (uint32_t)(kb * KBLOCK + S::template extra_rows<RSA>(q)) * (uint32_t)lda);
         } else if (q < NA + NB) {
             copy_b(stage, kb, q - NA);
-        } else if (SCALE_WAVE == 0) {
+        } else {
             lds_dma16_unless((uint32_t)wave, rsrc_s, voff_s, stage + S::SCALE_OFF, (uint32_t)kb * (uint32_t)lda * 4u);
-        } else if (wave == SCALE_WAVE) {
-            lds_dma16(rsrc_s, voff_s, stage + S::SCALE_OFF, (uint32_t)kb * (uint32_t)lda * 4u);
-        } else if (S::SB_STAGED && wave == SCALE_WAVE + 1) {
-            lds_dma4(rsrc_bs, voff_sb, stage + S::SB_OFF, (uint32_t)kb * (uint32_t)sn * 4u);
         }
     };
-    // RAGGED: all copies of a wave at once
+    // RAGGED and AHEAD: all copies of a wave at once
     auto copy_all = [&](int slot, int kb) __attribute__((always_inline)) {
         const uint32_t stage = lds_base + (uint32_t)(slot * S::STAGE);
+        if constexpr (!RAGGED) {
+#pragma unroll
+            for (int q = 0; q < NAC; ++q)
+                lds_dma16(rsrc_a, voff_a[S::template voff_index<RSA>(q)], stage + (uint32_t)((NAC * copier + q) * 1024),
+                          (uint32_t)(kb * KBLOCK + S::template extra_rows<RSA>(q)) * (uint32_t)lda);
+        }
 #pragma unroll
         for (int q = 0; q < NBW; ++q)
             copy_b(stage, kb, q);
-        if (64 * wave < BM)
-            lds_dma4(rsrc_s, voff_s, stage + S::SCALE_OFF + (uint32_t)(256 * wave), (uint32_t)kb * (uint32_t)M * 4u);
-        else if (S::SB_STAGED && wave == A_WAVE - 1)
+        if constexpr (!RAGGED) {
+            if (copier == 0)
+                lds_dma16(rsrc_s, voff_s, stage + S::SCALE_OFF, (uint32_t)kb * (uint32_t)lda * 4u);
+            else if (copier == 1)
+                lds_dma4(rsrc_bs, voff_sb, stage + S::SB_OFF, (uint32_t)kb * (uint32_t)sn * 4u);
+            return;
+        }
+        if (64 * copier < BM)
+            lds_dma4(rsrc_s, voff_s, stage + S::SCALE_OFF + (uint32_t)(256 * copier), (uint32_t)kb * (uint32_t)M * 4u);
+        if (S::SB_STAGED && copier == COPIERS - 1)
             lds_dma4(rsrc_bs, voff_sb, stage + S::SB_OFF, (uint32_t)kb * (uint32_t)sn * 4u);
     };
 
@@ -252,202 +270,338 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
         for (int j = 0; j < NJ; ++j)
             acc[i][j] = (v4f){0.f, 0.f, 0.f, 0.f};
 
-    // ---- prologue: the first NS-1 K blocks go into ring slots 0 .. NS-2
-#pragma unroll
-    for (int p = 0; p < NS - 1; ++p)
-        if (kb0 + p < kb1) {
-            if constexpr (RAGGED) {
-                if (!loads_a)
-                    copy_all(p, kb0 + p);
-            } else {
-#pragma unroll
-                for (int q = 0; q < NCOPY; ++q)
-                    copy_step(p, kb0 + p, q);
-            }
-        }
-    int slot = 0;             // ring slot of block kb
-    int slot_fill = NS - 1;   // ring slot that block kb + NS - 1 goes into (= slot of kb - 1)
-
-    // b_scale of the next block (wave-uniform addresses: scalar loads)
-    float next_lo = 0.f, next_hi = 0.f;
-    if (!S::SB_STAGED) {
-        next_lo = b_scale[__builtin_amdgcn_readfirstlane(kb0 * sn + nb_lo)];
-        next_hi = b_scale[__builtin_amdgcn_readfirstlane(kb0 * sn + nb_hi)];
-    }
-
-    // One K block.  MORE = block kb+NS-1 exists and is copied here; two instantiations keep the
-    // steady-state body free of branches.
-    auto k_block = [&](auto more_tag, auto loads_tag, auto set_tag, int kb) __attribute__((always_inline)) {
-        constexpr bool loads_a = decltype(loads_tag)::value;
-        constexpr bool steady = decltype(more_tag)::value;
-        const bool more = steady || (RAGGED && kb + NS - 1 < kb1);
-        // RAGGED: A of the next block into its slot, and its registers filled again
-        auto next_a = [&]() __attribute__((always_inline)) {
-            if constexpr (loads_a) {
-                constexpr int set = (decltype(set_tag)::value + 1) % SETS;
-                if (steady || kb + 1 < kb1)
-                    write_a(more_tag, set_a[set], slot + 1 == NS ? 0 : slot + 1, kb + 1);  // steady: not the last block
-                if (steady || kb + LEAD < kb1)
-                    load_a(set_a[set], kb + LEAD);
-            }
-        };
-        // Block kb has landed once at most the copies of the younger blocks in flight are
-        // outstanding (loads complete in order).  NCOPY - 1 per block is exact for waves 1..7
-        // and one short for wave 0, which then waits for one more copy than it must.
-        // RAGGED: the waves that load A have written it, the others' copies are B's, two of which bring one more.
-        constexpr int PER_BLOCK = RAGGED ? NBW : NCOPY - 1;
-        if (loads_a) {
-        } else if (steady) {
-            wait_vmcnt<(NS - 2) * PER_BLOCK>();
-        } else {
-            const int younger = (kb1 - 1 - kb < NS - 2) ? (kb1 - 1 - kb) : (NS - 2);
-            if (NS >= 4 && younger >= 2)
-                wait_vmcnt<2 * PER_BLOCK>();
-            else if (NS >= 3 && younger >= 1)
+    if constexpr (AHEAD) {
+        // Iteration kb multiplies what the last one read into registers and reads block kb + 1; the slot of block kb is
+        // free behind its barrier and gets block kb + NS.
+        constexpr int PER_BLOCK = NAC + NBW;  // copies of a wave per block, or one or two short
+        auto wait_block = [&](int kb) __attribute__((always_inline)) {  // at most the copies of the younger blocks are out
+            const int younger = kb1 - 1 - kb;
+            if (younger >= NS - 2)
+                wait_vmcnt<(NS - 2) * PER_BLOCK>();
+            else if (younger == 1)
                 wait_vmcnt<PER_BLOCK>();
             else
                 wait_vmcnt<0>();
+        };
+        // The first blocks are copied by all waves that have nothing else to do: the first two by those that multiply
+        // (RAGGED: by two of them each), the others by those that copy later on.
+        if (compute) {
+            if constexpr (RAGGED) {
+                if (kb0 + (wave >> 1) < kb1)
+                    copy_all(wave >> 1, kb0 + (wave >> 1));
+                if (wave < 2)
+                    wait_vmcnt<0>();
+            } else {
+                if (kb0 < kb1)
+                    copy_all(0, kb0);
+                if (kb0 + 1 < kb1) {
+                    copy_all(1, kb0 + 1);
+                    wait_vmcnt<PER_BLOCK>();
+                } else {
+                    wait_vmcnt<0>();
+                }
+            }
+        } else if (!(RAGGED && loads_a)) {
+#pragma unroll
+            for (int p = 2; p < NS; ++p)
+                if (kb0 + p < kb1)
+                    copy_all(p, kb0 + p);
         }
-        __syncthreads();  // everyone's copies of block kb landed; slot_fill is no longer read
-        if (!compute) {  // copy-only wave
-            if (more) {
+        if (RAGGED && loads_a) {
+#pragma unroll
+            for (int p = 0; p < SETS; ++p)
+                if (kb0 + p < kb1)
+                    load_a(set_a[p], kb0 + p);
+            write_a(std::false_type{}, set_a[0], 0, kb0);
+            if (kb0 + SETS < kb1)
+                load_a(set_a[0], kb0 + SETS);
+            __syncthreads();
+            int slot_w = 1;
+            auto step = [&](auto more_tag, auto set_tag, int at) __attribute__((always_inline)) {  // block at into the ring
+                constexpr int set = decltype(set_tag)::value;
+                constexpr bool steady = decltype(more_tag)::value;
+                if (steady || at < kb1)
+                    write_a(more_tag, set_a[set], slot_w, at);
+                if (steady || at + SETS < kb1)
+                    load_a(set_a[set], at + SETS);
+                slot_w = slot_w + 1 == NS ? 0 : slot_w + 1;
+                if (steady || at <= kb1)
+                    __syncthreads();
+            };
+            static_assert(SETS == 3, "unrolled");
+            int at = kb0 + 1;
+            for (; at + 2 + SETS < kb1; at += SETS) {
+                step(std::true_type{}, std::integral_constant<int, 1>{}, at);
+                step(std::true_type{}, std::integral_constant<int, 2>{}, at + 1);
+                step(std::true_type{}, std::integral_constant<int, 0>{}, at + 2);
+            }
+            for (; at <= kb1; at += SETS) {
+                step(std::false_type{}, std::integral_constant<int, 1>{}, at);
+                step(std::false_type{}, std::integral_constant<int, 2>{}, at + 1);
+                step(std::false_type{}, std::integral_constant<int, 0>{}, at + 2);
+            }
+        } else if (!compute) {
+            __syncthreads();
+            int slot = 0, kb = kb0;
+            for (; kb < kb1; ++kb) {
+                if (kb + 1 < kb1)
+                    wait_block(kb + 1);
+                __syncthreads();
+                if (kb + NS < kb1)
+                    copy_all(slot, kb + NS);
+                slot = slot + 1 == NS ? 0 : slot + 1;
+            }
+        } else {
+            constexpr int T = MI * NJ, LAG = 4, FRAGS = MI + NJ, PER_MFMA = T >= 16 ? 1 : 2;
+            static_assert(T % LAG == 0, "sums keep their registers from block to block");
+            v8i fa[2][MI], fb[2][NJ];
+            float sa[2][MI], sb[2], sc[2][MI];
+            v4f blk[LAG];
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+                sc[1][i] = 0.f;
+#pragma unroll
+            for (int i = 0; i < LAG; ++i)
+                blk[i] = (v4f){0.f, 0.f, 0.f, 0.f};
+            auto read = [&](int set, int f, uint32_t so) __attribute__((always_inline)) {
+                if (f == 0)
+                    fb[set][0] = read_frag<RSB>(lds + (addr_b[0] + so));
+                else if (f <= MI)
+                    fa[set][f - 1] = read_frag<RSA>(lds + (addr_a[f - 1] + so));
+                else
+                    fb[set][f - MI] = read_frag<RSB>(lds + (addr_b[f - MI] + so));
+            };
+            auto read_scales = [&](int set, uint32_t so) __attribute__((always_inline)) {
+#pragma unroll
+                for (int i = 0; i < MI; ++i)
+                    sa[set][i] = *LDS_PTR(float, lds + so + addr_s + 64 * i);
+                sb[set] = *LDS_PTR(float, lds + so + S::SB_OFF);
+            };
+            auto fold = [&](int set, int t) __attribute__((always_inline)) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    acc[t % MI][t / MI][e] = fmaf(sc[set][t % MI], blk[t % LAG][e], acc[t % MI][t / MI][e]);
+            };
+            __syncthreads();
+#pragma unroll
+            for (int f = 0; f < FRAGS; ++f)
+                read(0, f, 0);
+            read_scales(0, 0);
+            wait_vmcnt<0>();
+            int slot = 0;
+            auto block = [&](auto set_tag) __attribute__((always_inline)) {
+                constexpr int s = decltype(set_tag)::value;
+                __syncthreads();
+                slot = slot + 1 == NS ? 0 : slot + 1;
+                const uint32_t so = (uint32_t)(slot * S::STAGE);
+#pragma unroll
+                for (int i = 0; i < MI; ++i)
+                    sc[s][i] = sa[s][i] * sb[s];
+#pragma unroll
+                for (int t = 0; t < T; ++t) {
+                    const int u = t < LAG ? T - LAG + t : t - LAG;
+                    fold(t < LAG ? 1 - s : s, u);
+                    if (t + 1 < T)
+                        asm volatile("" : "+v"(acc[u % MI][u / MI]), "+v"(fa[s][(t + 1) % MI]));
+                    else
+                        asm volatile("" : "+v"(acc[u % MI][u / MI]));
+                    blk[t % LAG] = block_sum(fb[s][t / MI], fa[s][t % MI]);
+#pragma unroll
+                    for (int f = t * PER_MFMA; f < (t + 1) * PER_MFMA; ++f)
+                        if (f < FRAGS)
+                            read(1 - s, f, so);
+                    if (t == (FRAGS + PER_MFMA - 1) / PER_MFMA - 1)
+                        read_scales(1 - s, so);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            };
+            int kb = kb0;
+            for (; kb + 1 < kb1; kb += 2) {
+                block(std::integral_constant<int, 0>{});
+                block(std::integral_constant<int, 1>{});
+            }
+            if (kb < kb1) {
+                block(std::integral_constant<int, 0>{});
+#pragma unroll
+                for (int t = T - LAG; t < T; ++t)
+                    fold(0, t);
+            } else {
+#pragma unroll
+                for (int t = T - LAG; t < T; ++t)
+                    fold(1, t);
+            }
+        }
+    } else {
+        // ---- prologue: the first NS-1 K blocks go into ring slots 0 .. NS-2
+#pragma unroll
+        for (int p = 0; p < NS - 1; ++p)
+            if (kb0 + p < kb1) {
                 if constexpr (RAGGED) {
                     if (!loads_a)
-                        copy_all(slot_fill, kb + NS - 1);
+                        copy_all(p, kb0 + p);
                 } else {
 #pragma unroll
                     for (int q = 0; q < NCOPY; ++q)
-                        copy_step(slot_fill, kb + NS - 1, q);
+                        copy_step(p, kb0 + p, q);
                 }
             }
+        int slot = 0;             // ring slot of block kb
+        int slot_fill = NS - 1;   // ring slot that block kb + NS - 1 goes into (= slot of kb - 1)
+
+        // b_scale of the next block (wave-uniform addresses: scalar loads)
+        float next_lo = 0.f, next_hi = 0.f;
+        next_lo = b_scale[__builtin_amdgcn_readfirstlane(kb0 * sn + nb_lo)];
+        next_hi = b_scale[__builtin_amdgcn_readfirstlane(kb0 * sn + nb_hi)];
+
+        // One K block.  MORE = block kb+NS-1 exists and is copied here; two instantiations keep the
+        // steady-state body free of branches.
+        auto k_block = [&](auto more_tag, auto loads_tag, auto set_tag, int kb) __attribute__((always_inline)) {
+            constexpr bool loads_a = decltype(loads_tag)::value;
+            constexpr bool steady = decltype(more_tag)::value;
+            const bool more = steady || (RAGGED && kb + NS - 1 < kb1);
+            // RAGGED: A of the next block into its slot, and its registers filled again
+            auto next_a = [&]() __attribute__((always_inline)) {
+                if constexpr (loads_a) {
+                    constexpr int set = (decltype(set_tag)::value + 1) % SETS;
+                    if (steady || kb + 1 < kb1)
+                        write_a(more_tag, set_a[set], slot + 1 == NS ? 0 : slot + 1, kb + 1);  // steady: not the last block
+                    if (steady || kb + LEAD < kb1)
+                        load_a(set_a[set], kb + LEAD);
+                }
+            };
+            // Block kb has landed once at most the copies of the younger blocks in flight are
+            // outstanding (loads complete in order).  NCOPY - 1 per block is exact for waves 1..7
+            // and one short for wave 0, which then waits for one more copy than it must.
+            // RAGGED: the waves that load A have written it, the others' copies are B's, two of which bring one more.
+            constexpr int PER_BLOCK = RAGGED ? NBW : NCOPY - 1;
+            if (loads_a) {
+            } else if (steady) {
+                wait_vmcnt<(NS - 2) * PER_BLOCK>();
+            } else {
+                const int younger = (kb1 - 1 - kb < NS - 2) ? (kb1 - 1 - kb) : (NS - 2);
+                if (NS >= 4 && younger >= 2)
+                    wait_vmcnt<2 * PER_BLOCK>();
+                else if (NS >= 3 && younger >= 1)
+                    wait_vmcnt<PER_BLOCK>();
+                else
+                    wait_vmcnt<0>();
+            }
+            __syncthreads();  // everyone's copies of block kb landed; slot_fill is no longer read
+            // b_scale of this block, asked for during the last one: waited for here, before any LDS read is in flight (behind
+            // a scalar load that is still out every wait for an LDS read is a wait for all of them)
+            const float sb_lo = next_lo, sb_hi = next_hi;
+            asm volatile("" ::"s"(sb_lo), "s"(sb_hi));
+            const uint32_t so = (uint32_t)(slot * S::STAGE);
+            // The first column's fragments of B and all of A's, then the second column's; the later ones a column ahead.
+            v8i fa[MI], fb[NJ];
+            fb[0] = read_frag<RSB>(lds + (addr_b[0] + so));
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+                fa[i] = read_frag<RSA>(lds + (addr_a[i] + so));
+            fb[1] = read_frag<RSB>(lds + (addr_b[1] + so));
+            float sa[MI], sc[MI];
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+                sa[i] = *LDS_PTR(float, lds + so + addr_s + 64 * i);
+
+            // MFMA number t multiplies patch (t % MI, t / MI).  Patches are folded LAG MFMAs behind their own, in the order that
+            // stands here (the next MFMA's operand passes through the fold's empty asm statement).  The wave's copy instructions
+            // of block kb + NS - 1 ride on the first MFMAs.
+            constexpr int T = MI * NJ, PER_MFMA = (NCOPY + T - 1) / T;
+            // two patch rows: six behind (128x192: 300 x 12288 x 2048 17.16 -> 17.02 us, four behind 17.05)
+            constexpr int LAG = MI < 4 ? 6 : MI;
+            v4f blk[LAG];
+            auto fold = [&](int t) __attribute__((always_inline)) {
+                if (t % MI == 0) {
+                    // wave-uniform choice of the b_scale value on the scalar unit (bit select), then one product per patch
+                    const float sbj = __uint_as_float((__float_as_uint(sb_hi) & hi_mask[t / MI / 2]) |
+                                                      (__float_as_uint(sb_lo) & ~hi_mask[t / MI / 2]));
+#pragma unroll
+                    for (int i = 0; i < MI; ++i)
+                        sc[i] = sa[i] * sbj;
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    acc[t % MI][t / MI][e] = fmaf(sc[t % MI], blk[t % LAG][e], acc[t % MI][t / MI][e]);
+            };
+#pragma unroll
+            for (int t = 0; t < T; ++t) {
+                if (t % MI == 0 && t > 0 && t / MI + 1 < NJ)
+                    fb[t / MI + 1] = read_frag<RSB>(lds + (addr_b[t / MI + 1] + so));
+                if (t >= LAG) {
+                    fold(t - LAG);
+                    if (t + 1 < T)
+                        asm volatile("" : "+v"(acc[(t - LAG) % MI][(t - LAG) / MI]), "+v"(fa[(t + 1) % MI]));
+                }
+                blk[t % LAG] = block_sum(fb[t / MI], fa[t % MI]);
+                if (RAGGED) {
+                    if (t == 1 && !loads_a && more)
+                        copy_all(slot_fill, kb + NS - 1);
+                } else if (more) {
+#pragma unroll
+                    for (int q = t * PER_MFMA; q < (t + 1) * PER_MFMA; ++q)
+                        if (q < NCOPY)
+                            copy_step(slot_fill, kb + NS - 1, q);
+                }
+                if (t == T - 1) {
+                    // the next block's b_scale, behind this block's last LDS read: its trip to the L2 (a block's values share
+                    // no cache line with the next one's unless N is small) is covered by the folds and the barrier
+                    int next = kb + 1 < kb1 ? kb + 1 : kb;
+                    asm volatile("" : "+s"(next));
+                    next_lo = b_scale[next * sn + nb_lo];
+                    next_hi = b_scale[next * sn + nb_hi];
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int t = T - LAG; t < T; ++t) {
+                fold(t);
+                asm volatile("" : "+v"(acc[t % MI][t / MI]));
+            }
+            // A's registers are emptied behind the block's last MFMA: with two sets a step is short for the loads' trip (128x192,
+            // per K block from the Infinity Cache: 0.83 us behind the first MFMA, 0.76 us here)
             next_a();
+
             slot_fill = slot;
             slot = (slot + 1 == NS) ? 0 : slot + 1;
-            return;
-        }
-        // b_scale of this block, asked for during the last one: waited for here, before any LDS read is in flight (behind
-        // a scalar load that is still out every wait for an LDS read is a wait for all of them)
-        const float sb_lo = next_lo, sb_hi = next_hi;
-        if (!S::SB_STAGED)
-            asm volatile("" ::"s"(sb_lo), "s"(sb_hi));
-        const uint32_t so = (uint32_t)(slot * S::STAGE);
-        // The first column's fragments of B and all of A's, then the second column's; the later ones a column ahead.
-        v8i fa[MI], fb[NJ];
-        fb[0] = read_frag<RSB>(lds + (addr_b[0] + so));
-#pragma unroll
-        for (int i = 0; i < MI; ++i)
-            fa[i] = read_frag<RSA>(lds + (addr_a[i] + so));
-        if (NJ > 1)
-            fb[1] = read_frag<RSB>(lds + (addr_b[1] + so));
-        const float sb_stage = S::SB_STAGED ? *LDS_PTR(float, lds + so + S::SB_OFF) : 0.f;
-        float sa[MI], sc[MI];
-#pragma unroll
-        for (int i = 0; i < MI; ++i)
-            sa[i] = *LDS_PTR(float, lds + so + addr_s + 64 * i);
-
-        // MFMA number t multiplies patch (t % MI, t / MI).  Patches are folded LAG MFMAs behind their own, in the order that
-        // stands here (the next MFMA's operand passes through the fold's empty asm statement).  The wave's copy instructions
-        // of block kb + NS - 1 ride on the first MFMAs.
-        constexpr int T = MI * NJ, PER_MFMA = (NCOPY + T - 1) / T;
-        // two patch rows: six behind where there are that many (128x192: 300 x 12288 x 2048 17.16 -> 17.02 us, four behind 17.05),
-        // four of four (64x64: 1024 x 512 x 2048 6.15 -> 6.03, 244 x 3072 x 1536 7.13 -> 7.00)
-        constexpr int LAG = T == 4 ? 4 : MI < 4 && T >= 12 ? 6 : MI;
-        v4f blk[LAG];
-        auto fold = [&](int t) __attribute__((always_inline)) {
-            if (t % MI == 0) {
-                // wave-uniform choice of the b_scale value on the scalar unit (bit select), then one product per patch
-                const float sbj = __uint_as_float((__float_as_uint(sb_hi) & hi_mask[t / MI / 2]) |
-                                                  (__float_as_uint(sb_lo) & ~hi_mask[t / MI / 2]));
-#pragma unroll
-                for (int i = 0; i < MI; ++i)
-                    sc[i] = sa[i] * (S::SB_STAGED ? sb_stage : sbj);
-            }
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                acc[t % MI][t / MI][e] = fmaf(sc[t % MI], blk[t % LAG][e], acc[t % MI][t / MI][e]);
         };
+        int kb = kb0;
+        using Set0 = std::integral_constant<int, 0>;
+        if constexpr (RAGGED) {
+            // a loop for either kind of wave: with the loads of A in a branch of a common one, the compiler has to expect that
+            // an earlier block's were not followed by any, and waits for all of them
+            auto blocks = [&](auto loads_tag) __attribute__((always_inline)) {
+                if constexpr (decltype(loads_tag)::value) {  // A: block 0 into its slot, the next ones on their way
 #pragma unroll
-        for (int t = 0; t < T; ++t) {
-            if (t % MI == 0 && t > 0 && t / MI + 1 < NJ)
-                fb[t / MI + 1] = read_frag<RSB>(lds + (addr_b[t / MI + 1] + so));
-            if (t >= LAG) {
-                fold(t - LAG);
-                if (t + 1 < T)
-                    asm volatile("" : "+v"(acc[(t - LAG) % MI][(t - LAG) / MI]), "+v"(fa[(t + 1) % MI]));
-            }
-            blk[t % LAG] = block_sum(fb[t / MI], fa[t % MI]);
-            if (RAGGED) {
-                if (t == 1) {
-                    if (loads_a && A_EARLY)
-                        next_a();
-                    if (!loads_a && more)
-                        copy_all(slot_fill, kb + NS - 1);
+                    for (int p = 0; p < SETS; ++p)
+                        if (kb0 + p < kb1)
+                            load_a(set_a[p], kb0 + p);
+                    write_a(std::false_type{}, set_a[0], 0, kb0);
+                    if (kb0 + SETS < kb1)
+                        load_a(set_a[0], kb0 + SETS);
                 }
-            } else if (more) {
-#pragma unroll
-                for (int q = t * PER_MFMA; q < (t + 1) * PER_MFMA; ++q)
-                    if (q < NCOPY)
-                        copy_step(slot_fill, kb + NS - 1, q);
-            }
-            if (t == T - 1 && !S::SB_STAGED) {
-                // the next block's b_scale, behind this block's last LDS read: its trip to the L2 (a block's values share
-                // no cache line with the next one's unless N is small) is covered by the folds and the barrier
-                int next = kb + 1 < kb1 ? kb + 1 : kb;
-                asm volatile("" : "+s"(next));
-                next_lo = b_scale[next * sn + nb_lo];
-                next_hi = b_scale[next * sn + nb_hi];
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-#pragma unroll
-        for (int t = T - LAG; t < T; ++t) {
-            fold(t);
-            asm volatile("" : "+v"(acc[t % MI][t / MI]));
-        }
-        if (!A_EARLY)
-            next_a();
-
-        slot_fill = slot;
-        slot = (slot + 1 == NS) ? 0 : slot + 1;
-    };
-    int kb = kb0;
-    using Set0 = std::integral_constant<int, 0>;
-    if constexpr (RAGGED) {
-        // a loop for either kind of wave: with the loads of A in a branch of a common one, the compiler has to expect that
-        // an earlier block's were not followed by any, and waits for all of them
-        auto blocks = [&](auto loads_tag) __attribute__((always_inline)) {
-            if constexpr (decltype(loads_tag)::value) {  // A: block 0 into its slot, the next ones on their way
-#pragma unroll
-                for (int p = 0; p < SETS; ++p)
-                    if (kb0 + p < kb1)
-                        load_a(set_a[p], kb0 + p);
-                write_a(std::false_type{}, set_a[0], 0, kb0);
-                if (kb0 + SETS < kb1)
-                    load_a(set_a[0], kb0 + SETS);
-            }
-            auto round = [&](auto more_tag, int at) __attribute__((always_inline)) {  // the sets are numbered at compile time
-                constexpr bool steady = decltype(more_tag)::value;
-                k_block(more_tag, loads_tag, Set0{}, at);
-                if (steady || at + 1 < kb1)
-                    k_block(more_tag, loads_tag, std::integral_constant<int, 1>{}, at + 1);
-                if (SETS == 3 && (steady || at + 2 < kb1))
-                    k_block(more_tag, loads_tag, std::integral_constant<int, SETS - 1>{}, at + 2);
+                auto round = [&](auto more_tag, int at) __attribute__((always_inline)) {  // the sets are numbered at compile time
+                    constexpr bool steady = decltype(more_tag)::value;
+                    k_block(more_tag, loads_tag, Set0{}, at);
+                    if (steady || at + 1 < kb1)
+                        k_block(more_tag, loads_tag, std::integral_constant<int, 1>{}, at + 1);
+                };
+                static_assert(SETS == 2, "unrolled above");
+                for (; kb + SETS - 1 + LEAD < kb1; kb += SETS)
+                    round(std::true_type{}, kb);
+                for (; kb < kb1; kb += SETS)
+                    round(std::false_type{}, kb);
             };
-            static_assert(SETS == 2 || SETS == 3, "unrolled above");
-            for (; kb + SETS - 1 + LEAD < kb1; kb += SETS)
-                round(std::true_type{}, kb);
-            for (; kb < kb1; kb += SETS)
-                round(std::false_type{}, kb);
-        };
-        if (loads_a)
-            blocks(std::true_type{});
-        else
-            blocks(std::false_type{});
-    } else {
-        for (; kb + NS - 1 < kb1; ++kb)
-            k_block(std::true_type{}, std::false_type{}, Set0{}, kb);
-        for (; kb < kb1; ++kb)
-            k_block(std::false_type{}, std::false_type{}, Set0{}, kb);
+            if (loads_a)
+                blocks(std::true_type{});
+            else
+                blocks(std::false_type{});
+        } else {
+            for (; kb + NS - 1 < kb1; ++kb)
+                k_block(std::true_type{}, std::false_type{}, Set0{}, kb);
+            for (; kb < kb1; ++kb)
+                k_block(std::false_type{}, std::false_type{}, Set0{}, kb);
+        }
     }
 
     // ---- K splits added inside the kernel (mailbox != nullptr).  grid.x is a multiple of 8, so the
@@ -815,7 +969,7 @@ hipError_t launch_tile(const GemmArgs& g, int variant, int ksplit, float* partia
     case TILE_256x192: return launch_variant<256, 192, 4, 2, 2>(g, ksplit, partial, mailbox, s);
     case TILE_256x128: return launch_variant<256, 128, 4, 2, 3>(g, ksplit, partial, mailbox, s);
     case TILE_128x192: return launch_variant<128, 192, 4, 2, 3>(g, ksplit, partial, mailbox, s);
-    case TILE_128x128: return launch_variant<128, 128, 2, 4, 4>(g, ksplit, partial, mailbox, s);
+    case TILE_128x128: return launch_variant<128, 128, 2, 2, 4>(g, ksplit, partial, mailbox, s);
     case TILE_64x64: return launch_variant<64, 64, 2, 2, 4>(g, ksplit, partial, mailbox, s);
     default: return hipErrorInvalidValue;
     }

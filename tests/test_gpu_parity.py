@@ -119,6 +119,22 @@ def test_tile_kernel(pkg, variant, m, n, k):
     _assert_every_element(got, a, b, sa, sb, m, n, k, name)
 
 
+# the tiles of four multiplying waves, which read a K block while they multiply the one before: chains shorter and longer
+# than the ring of four, odd and even (the registers alternate), with copied rows of A and with loaded ones (m off the grid)
+@pytest.mark.parametrize("variant", [2, 4])
+@pytest.mark.parametrize("kb", [1, 2, 3, 4, 5, 6, 7, 11])
+def test_tile_kernel_of_four_waves_chains(pkg, variant, kb):
+    n, k = 336, 128 * kb
+    for m in (208, 203):
+        a, b, sa, sb = oracle.make_inputs(m, n, k, 3 * m + n + k, 0.5, 30.0)
+        got, name = _run(pkg, a, b, sa, sb, m, n, k, variant=variant, ksplit=1)
+        assert name == {2: "tile128x128_k1", 4: "tile64x64_k1"}[variant], name
+        _assert_every_element(got, a, b, sa, sb, m, n, k, name)
+        other, name1 = _run(pkg, a, b, sa, sb, m, n, k, variant=1, ksplit=1, persistent=0)
+        assert name1.endswith("tile256x128_k1"), name1
+        assert np.array_equal(got, other), "both tiles fold the same block sums in the same order"
+
+
 # persistent form: several tiles per workgroup (more than 256 tiles), ragged edges, K ranges from
 # the shortest the ring allows to many blocks, and a launch with fewer tiles than workgroups
 @pytest.mark.parametrize("variant,m,n,k", [(0, 4096, 3456, 512), (0, 1040, 1232, 256), (0, 4112, 3472, 128),
