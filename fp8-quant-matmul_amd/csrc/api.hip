@@ -206,8 +206,16 @@ double tile_cost(const GemmArgs& g, int variant, int ksplit, bool fused = false)
     // says, or slower.)
     const bool light = variant == TILE_64x64 && !streams_b && tiles <= 64;
     // (256x192 in the persistent form: the fit knows the kernel before its barrier moved, 5 % slower)
+    // (unsplit 128x128 tiles in one round: the fit knows the kernel before four waves read ahead of themselves, 10 - 15 %
+    // slower from the caches, and level from HBM, where the copies bound it: they do also where a row of B starts
+    // anywhere on a line of 128 bytes, so that each row of a tile is two of them, 2896 x 704 x 5760 26.4 us against 24.9 as
+    // 256x128 with three splits.  At 0.94 shapes change from two or three splits of 128x192 or 256x128 tiles: 20
+    // random ones with whole lines of B all faster from the caches, by 16 - 31 % (640 x 4480 x 6144 30.7 -> 23.5 us), and
+    // -1 ... +22 % from HBM, 6 % on average; five without -6 ... +9 % there.  At 0.88 more change, down to -14 % from HBM.)
+    const bool ahead = variant == TILE_128x128 && ksplit == 1 && g.m > 256 && tiles <= NUM_CU &&
+                       leading_dim(g) % 16 == 0 && g.n % 128 == 0;
     const double per_kb = (1.19 * area + 0.267) * (variant == TILE_256x192 && ksplit == 1 && tiles > NUM_CU ? 0.95 : 1.0) *
-                          (streams_b ? 1.25 : 1.0) * (light ? 0.8 : 1.0);
+                          (streams_b ? 1.25 : 1.0) * (light ? 0.8 : 1.0) * (ahead ? 0.94 : 1.0);
     // (unsplit 128x192 tiles in more than one round of workgroups: the fit has them 8 % too fast against the 256-row
     // tiles -- 36 random shapes of 512 ... 8192 rows where that margin decides, before / after: the 256x256 or
     // 256x128 plan +5.6 % with B cached, +10.3 % with B from HBM on average, worst -2.3 %)
@@ -283,7 +291,10 @@ inline bool persistent_only(int variant) { return variant == TILE_256x192_W4 || 
 // ... of which the dispatcher may pick this one by itself
 inline bool persistent_only_auto(int variant) { return variant == TILE_256x256; }
 
-// A persistent launch pays off when a CU gets more than one tile.
+// A persistent launch pays off when a CU gets more than one tile -- but for 128x128 tiles, whose plain form multiplies
+// with four waves that read ahead, only while the K range is short (5000 x 1664 x 384 10.0 us persistent, 10.2 plain; 4096 x
+// 4096 x 1024 26.2, 26.2; 1664 x 4864 x 1408 18.0, 16.5; 2688 x 3072 x 3840 40.7, 35.3; 1040 x 6912 x 7552 75.9, 64.2; 13
+// more random shapes of K = 2176 ... 6144 all 4 - 16 % faster plain).
 void decide_persistent(const GemmArgs& g, Plan& p, const Config& cfg)
 {
     p.persistent = false;
@@ -297,7 +308,7 @@ void decide_persistent(const GemmArgs& g, Plan& p, const Config& cfg)
     int bm, bn;
     tile_variant_dims(p.variant, &bm, &bn);
     const long tiles = (long)((g.m + bm - 1) / bm) * ((g.n + bn - 1) / bn);
-    p.persistent = mode == 1 || tiles > NUM_CU;
+    p.persistent = mode == 1 || (tiles > NUM_CU && (p.variant != TILE_128x128 || g.k < 1024));
 }
 
 // Whether a tile plan that splits K adds the partial tiles inside the GEMM kernel (the last workgroup of
