@@ -32,15 +32,16 @@
 //     multiply, a wave that does not copies b_scale into the stage (64x64 tiles, which are done before that
 //     trip is: 48 x 4608 x 7168 14.2 -> 10.9 us).
 //   * The two smaller tiles, 64x64 and 128x128, are multiplied by four waves, one per SIMD, and copied by the other
-//     four.  What bounds a K block of them is the LDS: in a block of its own, every wave's reads come first (all waves',
-//     640 clocks for 128x128 in eight waves of 64x32) and its MFMAs, 512 clocks, behind them.  Four waves of 64x64 read
-//     two thirds of that, and they read block kb + 1 into a second set of registers between the MFMAs of block kb, so that
-//     a block takes the longer of the two and not their sum; the folds of a block's last four sums cross the barrier.
-//     Before (eight waves, reads at the head of the block) / after, from the Infinity Cache: 5504 x 512 x 7168 30.7 -> 26.7 us,
-//     2048 x 2048 x 7168 36.1 -> 32.0, 1024 x 1536 x 7168 21.4 -> 19.6, 352 x 3072 x 1536 9.4 -> 8.9, 350 x 3072 x 1536
-//     (RAGGED) 11.3 -> 10.5, 64x64 tiles 1024 x 512 x 2048 6.1 -> 5.9; 64 x 4608 x 7168, bound by the copies, 10.4 -> 10.5.
-//     Copies between the MFMAs of a lone wave hold them up (RAGGED with B copied there: 350 x 3072 x 1536 12.3 us), so
-//     they are the other waves'.  Eight stages of 64x64 instead of four: slower, 5.9 -> 6.8 us.
+//     four (128x128 with ragged rows and split K: by eight, see launch_tile).  What bounds a K block of them is the
+//     LDS: where a block stands by itself, the reads of all waves come first (640 clocks for 128x128 in eight waves of
+//     64x32) and the MFMAs, 512 clocks, behind them.  Four waves of 64x64 read two thirds of that, and they read
+//     block kb + 1 into a second set of registers between the MFMAs of block kb, so that a block takes the longer of
+//     the two and not their sum; the folds of a block's last four sums cross the barrier.  Eight waves with the reads
+//     at the head of the block / this, from the Infinity Cache: 5504 x 512 x 7168 30.7 / 26.7 us, 2048 x 2048 x 7168
+//     36.1 / 32.0, 1024 x 1536 x 7168 21.4 / 19.2, 352 x 3072 x 1536 9.4 / 8.9, 350 x 3072 x 1536 (RAGGED) 11.3 / 10.5;
+//     64x64 tiles 1024 x 512 x 2048 6.1 / 5.9, 64 x 4608 x 7168, bound by the copies, 10.4 / 10.5.  Copies between the
+//     MFMAs of a lone wave hold them up (RAGGED with B copied there: 350 x 3072 x 1536 12.3 us), so they are the other
+//     waves'.  Eight stages of 64x64 instead of four: 5.9 -> 6.8 us.
 //   * NS LDS stages form a ring: the copies of K blocks kb+1 .. kb+NS-1 are in flight while
 //     block kb is multiplied.  Large tiles fit two stages; smaller tiles get three or four,
 //     which is what hides the global latency when a K block is only a few MFMAs long.
@@ -49,12 +50,13 @@
 //     and holds every wave back from its LDS reads).
 //
 //   * RAGGED: M is no multiple of 16, so A's k-rows start anywhere and 16-byte copies straight to LDS are out.  Four of
-//     the eight waves (two of the four that do not multiply) load A's pieces into registers from where they lie (a load takes any address; measured: no slower
-//     off the grid than on it) and write them to the ring a step before they are multiplied, two or three register
-//     sets ahead; the other four copy B and the scales as ever.  Each kind has a loop of its own, so that the compiler's
-//     waits count the loads of A alone.  A K block takes 0.05 - 0.1 us more than with copies throughout (128 x 128, 336 x
-//     4608 from the Infinity Cache: 0.53 -> 0.59 us), and the launch that copied A into padded rows is gone: 121 x 7168
-//     x 256 5.6 -> 3.8 us, 244 x 3072 x 1536 9.2 -> 7.0, 1021 x 512 x 2048 11.4 -> 7.7, 2204 x 512 x 7168 26.9 -> 21.2.
+//     the eight waves (two of the four that do not multiply) load A's pieces into registers from where they lie (a load
+//     takes any address; measured: no slower off the grid than on it) and write them to the ring a step before they are
+//     read, two or three register sets ahead; the others copy B and the scales as ever.  Each kind has a loop of its own,
+//     so that the compiler's waits count the loads of A alone.  A K block takes 0.05 - 0.1 us more than with copies
+//     throughout (128 x 128 in eight waves, 336 x 4608 from the Infinity Cache: 0.53 -> 0.59 us), and the launch that
+//     copied A into padded rows is gone: 121 x 7168 x 256 5.6 -> 3.8 us, 244 x 3072 x 1536 9.2 -> 7.0, 1021 x 512 x 2048
+//     11.4 -> 7.7, 2204 x 512 x 7168 26.9 -> 21.2.
 //
 // Work decomposition: grid.x = tiles (XCD-aware order), grid.y = K splits.
 #include "tile_common.h"
@@ -82,7 +84,7 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
     // WM x WN waves multiply: all eight, or the first four of the two smaller tiles (AHEAD)
     static_assert(WM * WN == 8 || WM * WN == 4, "eight or four multiplying waves");
     constexpr int NCW = WM * WN;
-    static_assert(NCW == 4 ? NS == 4 : NS == 2 || NS == 3, "LDS stages");
+    static_assert(NCW == 4 ? NS == 4 : NS >= 2 && NS <= 4, "LDS stages");
     constexpr int TM = BM / WM, TN = BN / WN;      // wave tile
     constexpr int MI = TM / 16, NJ = TN / 16;      // 16x16 patches per wave
     static_assert(TM % 16 == 0 && TN % 32 == 0, "wave tile is made of 16x16 patches, pairs of them along n");
@@ -97,6 +99,10 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
     constexpr int COPIERS = !AHEAD && !RAGGED ? 8 : AHEAD && RAGGED ? 2 : 4;
     constexpr int NBW = 8 / COPIERS * NB, NAC = RAGGED ? 0 : 8 / COPIERS * NA;  // copies of such a wave per K block
     constexpr int SETS = NS - 1, LEAD = SETS + 1;  // register sets of A, and K blocks that they run ahead
+    // RAGGED, eight waves multiply: A's registers are emptied behind the first MFMA of a block; with two sets only behind its
+    // last one, a step is short for the loads' trip (128x192, per K block from the Infinity Cache: 0.83 us early, 0.76 us
+    // late; 128x128 with three sets 0.59 and 0.61 us)
+    constexpr bool A_EARLY = SETS >= 3;
     static_assert(!RAGGED || BM <= 64 * COPIERS, "a wave that copies for every 64 rows of a_scale");
 
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
@@ -535,8 +541,12 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
                 }
                 blk[t % LAG] = block_sum(fb[t / MI], fa[t % MI]);
                 if (RAGGED) {
-                    if (t == 1 && !loads_a && more)
-                        copy_all(slot_fill, kb + NS - 1);
+                    if (t == 1) {
+                        if (loads_a && A_EARLY)
+                            next_a();
+                        if (!loads_a && more)
+                            copy_all(slot_fill, kb + NS - 1);
+                    }
                 } else if (more) {
 #pragma unroll
                     for (int q = t * PER_MFMA; q < (t + 1) * PER_MFMA; ++q)
@@ -558,9 +568,8 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
                 fold(t);
                 asm volatile("" : "+v"(acc[t % MI][t / MI]));
             }
-            // A's registers are emptied behind the block's last MFMA: with two sets a step is short for the loads' trip (128x192,
-            // per K block from the Infinity Cache: 0.83 us behind the first MFMA, 0.76 us here)
-            next_a();
+            if (!A_EARLY)
+                next_a();
 
             slot_fill = slot;
             slot = (slot + 1 == NS) ? 0 : slot + 1;
@@ -585,8 +594,10 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
                     k_block(more_tag, loads_tag, Set0{}, at);
                     if (steady || at + 1 < kb1)
                         k_block(more_tag, loads_tag, std::integral_constant<int, 1>{}, at + 1);
+                    if (SETS == 3 && (steady || at + 2 < kb1))
+                        k_block(more_tag, loads_tag, std::integral_constant<int, SETS - 1>{}, at + 2);
                 };
-                static_assert(SETS == 2, "unrolled above");
+                static_assert(SETS == 2 || SETS == 3, "unrolled above");
                 for (; kb + SETS - 1 + LEAD < kb1; kb += SETS)
                     round(std::true_type{}, kb);
                 for (; kb < kb1; kb += SETS)
@@ -644,8 +655,9 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
             }
             if (compute) {
                 // PG patches at a time (all of them when there are at most eight: one trip to the L2 for everything that
-                // is there), ZB splits at a time
-                constexpr int PG = MI * NJ <= 8 ? MI * NJ : 4, ZB = MI * NJ <= 4 ? 3 : 2;
+                // is there), ZB splits at a time.  Of sixteen in four waves, eight: 333 x 4608 x 7168 in two splits 24.3 us four
+                // at a time, 23.9 eight, 24.2 sixteen; 777 x 2048 x 4096 18.4, 17.9, 18.2.
+                constexpr int PG = MI * NJ <= 8 ? MI * NJ : AHEAD ? 8 : 4, ZB = MI * NJ <= 4 ? 3 : 2;
                 static_assert(MI * NJ % PG == 0, "whole groups of patches");
                 const __amdgpu_buffer_rsrc_t rp = make_rsrc(reinterpret_cast<const v4i*>(mailbox) + first, mail_span);
                 const unsigned long long t_first = __builtin_amdgcn_s_memrealtime();
@@ -865,7 +877,7 @@ int choose_group_m(int tiles_m, int tiles_n, int bm, int bn)
 // the tile shapes that have a form for row counts off the 16-byte grid
 constexpr bool tile_takes_ragged_rows(int bm, int ns) { return bm <= 128 && ns >= 3; }
 
-template <int BM, int BN, int WM, int WN, int NS, bool RAGGED>
+template <int BM, int BN, int WM, int WN, int NS, bool SPLIT, bool RAGGED>
 hipError_t launch_typed(const GemmArgs& g, int ksplit, float* partial, float* mailbox, hipStream_t s)
 {
     using S = TileShape<BM, BN, WM, WN, NS>;
@@ -875,33 +887,28 @@ hipError_t launch_typed(const GemmArgs& g, int ksplit, float* partial, float* ma
     const int kb_per_split = (nkb + ksplit - 1) / ksplit;
     const int tiles = tiles_m * tiles_n;
     const int group_m = choose_group_m(tiles_m, tiles_n, BM, BN);
-    if (ksplit > 1) {
-        // in-kernel reduction: the other splits' patches of every tile fit the mailbox
-        if (mailbox && (size_t)tiles * (ksplit - 1) * BM * BN * 4 > SPLIT_MAILBOX_BYTES)
-            return hipErrorInvalidValue;
-        dim3 grid(mailbox ? (tiles + 7) & ~7 : tiles, ksplit);
-        auto kern = tile_gemm_kernel<BM, BN, WM, WN, NS, true, RAGGED>;
-        FP8GEMM_ALLOW_LDS(kern, LDS_TOTAL);
-        hipLaunchKernelGGL(kern, grid, dim3(NTHREADS), LDS_TOTAL, s, g.a, g.b, g.a_scale, g.b_scale, g.c, partial,
-                           mailbox, g.m, leading_dim(g), g.n, g.k, tiles_m, tiles_n, kb_per_split, group_m);
-    } else {
-        auto kern = tile_gemm_kernel<BM, BN, WM, WN, NS, false, RAGGED>;
-        FP8GEMM_ALLOW_LDS(kern, LDS_TOTAL);
-        hipLaunchKernelGGL(kern, dim3(tiles, 1), dim3(NTHREADS), LDS_TOTAL, s, g.a, g.b, g.a_scale, g.b_scale, g.c,
-                           partial, static_cast<float*>(nullptr), g.m, leading_dim(g), g.n, g.k, tiles_m,
-                           tiles_n, kb_per_split, group_m);
-    }
+    // in-kernel reduction: the other splits' patches of every tile fit the mailbox
+    if (SPLIT && mailbox && (size_t)tiles * (ksplit - 1) * BM * BN * 4 > SPLIT_MAILBOX_BYTES)
+        return hipErrorInvalidValue;
+    const dim3 grid(SPLIT && mailbox ? (tiles + 7) & ~7 : tiles, SPLIT ? ksplit : 1);
+    auto kern = tile_gemm_kernel<BM, BN, WM, WN, NS, SPLIT, RAGGED>;
+    FP8GEMM_ALLOW_LDS(kern, LDS_TOTAL);
+    hipLaunchKernelGGL(kern, grid, dim3(NTHREADS), LDS_TOTAL, s, g.a, g.b, g.a_scale, g.b_scale, g.c, partial,
+                       SPLIT ? mailbox : nullptr, g.m, leading_dim(g), g.n, g.k, tiles_m, tiles_n, kb_per_split, group_m);
     return hipGetLastError();
 }
 
-template <int BM, int BN, int WM, int WN, int NS>
+// WMS x WNS: the waves of the form that takes ragged rows and splits K
+template <int BM, int BN, int WM, int WN, int NS, int WMS = WM, int WNS = WN>
 hipError_t launch_variant(const GemmArgs& g, int ksplit, float* partial, float* mailbox, hipStream_t s)
 {
     if (leading_dim(g) % 16 == 0)
-        return launch_typed<BM, BN, WM, WN, NS, false>(g, ksplit, partial, mailbox, s);
+        return ksplit > 1 ? launch_typed<BM, BN, WM, WN, NS, true, false>(g, ksplit, partial, mailbox, s)
+                          : launch_typed<BM, BN, WM, WN, NS, false, false>(g, ksplit, partial, mailbox, s);
     if constexpr (tile_takes_ragged_rows(BM, NS)) {
         if (leading_dim(g) == g.m && g.m >= 16)
-            return launch_typed<BM, BN, WM, WN, NS, true>(g, ksplit, partial, mailbox, s);
+            return ksplit > 1 ? launch_typed<BM, BN, WMS, WNS, NS, true, true>(g, ksplit, partial, mailbox, s)
+                              : launch_typed<BM, BN, WM, WN, NS, false, true>(g, ksplit, partial, mailbox, s);
     }
     return hipErrorInvalidValue;
 }
@@ -969,7 +976,11 @@ hipError_t launch_tile(const GemmArgs& g, int variant, int ksplit, float* partia
     case TILE_256x192: return launch_variant<256, 192, 4, 2, 2>(g, ksplit, partial, mailbox, s);
     case TILE_256x128: return launch_variant<256, 128, 4, 2, 3>(g, ksplit, partial, mailbox, s);
     case TILE_128x192: return launch_variant<128, 192, 4, 2, 3>(g, ksplit, partial, mailbox, s);
-    case TILE_128x128: return launch_variant<128, 128, 2, 2, 4>(g, ksplit, partial, mailbox, s);
+    // (ragged rows and K split: eight waves multiply.  Four of them bring A there, and all take part in the hand-over,
+    // which the short chains of a split do not make up for: 250 x 7168 x 2048 in two splits, B from HBM, 14.1 us by four
+    // waves and 12.9 by eight, 2204 x 512 x 7168 in three 23.4 and 22.0, 333 x 4608 x 7168 in two 30.9 and 30.0; unsplit
+    // 500 x 4608 x 2048 12.9 and 13.8)
+    case TILE_128x128: return launch_variant<128, 128, 2, 2, 4, 2, 4>(g, ksplit, partial, mailbox, s);
     case TILE_64x64: return launch_variant<64, 64, 2, 2, 4>(g, ksplit, partial, mailbox, s);
     default: return hipErrorInvalidValue;
     }
