@@ -1,4 +1,5 @@
-// Persistent form of the MFMA tile kernel for shapes with more tiles than compute units.
+// Persistent form of the MFMA tile kernel for shapes with more tiles than compute units (256 x 192 and 256 x 256 tiles have a
+// body of their own: k_tile_large.hip).
 //
 // The plain kernel (k_tile.hip) runs one tile per workgroup: with one workgroup per CU (the LDS
 // ring fills the CU) every round of 256 tiles pays the launch of a new workgroup, an empty
