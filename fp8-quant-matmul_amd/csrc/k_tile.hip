@@ -37,9 +37,9 @@
 //     64x32) and the MFMAs, 512 clocks, behind them.  Four waves of 64x64 read two thirds of that, and they read
 //     block kb + 1 into a second set of registers between the MFMAs of block kb, so that a block takes the longer of
 //     the two and not their sum; the folds of a block's last four sums cross the barrier.  Eight waves with the reads
-//     at the head of the block / this, from the Infinity Cache: 5504 x 512 x 7168 30.7 / 26.7 us, 2048 x 2048 x 7168
-//     36.1 / 32.0, 1024 x 1536 x 7168 21.4 / 19.2, 352 x 3072 x 1536 9.4 / 8.9, 350 x 3072 x 1536 (RAGGED) 11.3 / 10.5;
-//     64x64 tiles 1024 x 512 x 2048 6.1 / 5.9, 64 x 4608 x 7168, bound by the copies, 10.4 / 10.5.  Copies between the
+//     at the head of the block / this, from the Infinity Cache: 5504 x 512 x 7168 30.7 / 26.4 us, 2048 x 2048 x 7168
+//     36.1 / 32.0, 1024 x 1536 x 7168 21.4 / 19.1, 352 x 3072 x 1536 9.4 / 8.6, 350 x 3072 x 1536 (RAGGED) 11.3 / 10.4;
+//     64x64 tiles 1024 x 512 x 2048 6.1 / 5.85, 64 x 4608 x 7168, bound by the copies, 10.4 / 10.6.  Copies between the
 //     MFMAs of a lone wave hold them up (RAGGED with B copied there: 350 x 3072 x 1536 12.3 us), so they are the other
 //     waves'.  Eight stages of 64x64 instead of four: 5.9 -> 6.8 us.
 //   * NS LDS stages form a ring: the copies of K blocks kb+1 .. kb+NS-1 are in flight while
@@ -365,7 +365,7 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
             v4f blk[LAG];
 #pragma unroll
             for (int i = 0; i < MI; ++i)
-                sc[1][i] = 0.f;
+                sc[0][i] = sc[1][i] = 0.f;
 #pragma unroll
             for (int i = 0; i < LAG; ++i)
                 blk[i] = (v4f){0.f, 0.f, 0.f, 0.f};
@@ -393,11 +393,17 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
             for (int f = 0; f < FRAGS; ++f)
                 read(0, f, 0);
             read_scales(0, 0);
-            wait_vmcnt<0>();
             int slot = 0;
-            auto block = [&](auto set_tag) __attribute__((always_inline)) {
+            // The first block: the barrier, behind which the next one has landed, stands behind half of the MFMAs, which need
+            // not wait for those copies (before / after: 352 x 3072 x 1536 8.87 / 8.60 us, 1024 x 512 x 2048 5.99 / 5.85, 5504 x 512
+            // x 7168 26.7 / 26.4, 64 x 4608 x 7168 10.5 / 10.6)
+            auto block = [&](auto set_tag, auto first_tag) __attribute__((always_inline)) {
                 constexpr int s = decltype(set_tag)::value;
-                __syncthreads();
+                constexpr bool first = decltype(first_tag)::value;
+                constexpr int R0 = first ? T / 2 : 0;  // the MFMA that the reads start with
+                static_assert((T - R0) * PER_MFMA >= FRAGS, "all fragments are read");
+                if (!first)
+                    __syncthreads();
                 slot = slot + 1 == NS ? 0 : slot + 1;
                 const uint32_t so = (uint32_t)(slot * S::STAGE);
 #pragma unroll
@@ -406,6 +412,10 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
 #pragma unroll
                 for (int t = 0; t < T; ++t) {
                     const int u = t < LAG ? T - LAG + t : t - LAG;
+                    if (first && t == R0) {
+                        wait_vmcnt<0>();
+                        __syncthreads();
+                    }
                     fold(t < LAG ? 1 - s : s, u);
                     if (t + 1 < T)
                         asm volatile("" : "+v"(acc[u % MI][u / MI]), "+v"(fa[s][(t + 1) % MI]));
@@ -413,28 +423,34 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
                         asm volatile("" : "+v"(acc[u % MI][u / MI]));
                     blk[t % LAG] = block_sum(fb[s][t / MI], fa[s][t % MI]);
 #pragma unroll
-                    for (int f = t * PER_MFMA; f < (t + 1) * PER_MFMA; ++f)
-                        if (f < FRAGS)
+                    for (int f = (t - R0) * PER_MFMA; f < (t - R0 + 1) * PER_MFMA; ++f)
+                        if (t >= R0 && f < FRAGS)
                             read(1 - s, f, so);
-                    if (t == (FRAGS + PER_MFMA - 1) / PER_MFMA - 1)
+                    if (t - R0 == (FRAGS + PER_MFMA - 1) / PER_MFMA - 1)
                         read_scales(1 - s, so);
                     __builtin_amdgcn_sched_barrier(0);
                 }
             };
+            using Set0 = std::integral_constant<int, 0>;
+            using Set1 = std::integral_constant<int, 1>;
             int kb = kb0;
+            if (kb < kb1) {
+                block(Set0{}, std::true_type{});
+                ++kb;
+            }
             for (; kb + 1 < kb1; kb += 2) {
-                block(std::integral_constant<int, 0>{});
-                block(std::integral_constant<int, 1>{});
+                block(Set1{}, std::false_type{});
+                block(Set0{}, std::false_type{});
             }
             if (kb < kb1) {
-                block(std::integral_constant<int, 0>{});
-#pragma unroll
-                for (int t = T - LAG; t < T; ++t)
-                    fold(0, t);
-            } else {
+                block(Set1{}, std::false_type{});
 #pragma unroll
                 for (int t = T - LAG; t < T; ++t)
                     fold(1, t);
+            } else {
+#pragma unroll
+                for (int t = T - LAG; t < T; ++t)
+                    fold(0, t);
             }
         }
     } else {
