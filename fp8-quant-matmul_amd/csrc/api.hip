@@ -292,7 +292,7 @@ inline bool persistent_only(int variant) { return variant == TILE_256x192_W4 || 
 inline bool persistent_only_auto(int variant) { return variant == TILE_256x256; }
 
 // A persistent launch pays off when a CU gets more than one tile -- but for 128x128 tiles, whose plain form multiplies
-// with four waves that read ahead, only while the K range is short (5000 x 1664 x 384 10.0 us persistent, 10.2 plain; 4096 x
+// with four waves that read ahead, only while the K range is short (4992 x 1664 x 384 10.0 us persistent, 10.2 plain; 4096 x
 // 4096 x 1024 26.2, 26.2; 1664 x 4864 x 1408 18.0, 16.5; 2688 x 3072 x 3840 40.7, 35.3; 1040 x 6912 x 7552 75.9, 64.2; 13
 // more random shapes of K = 2176 ... 6144 all 4 - 16 % faster plain).
 void decide_persistent(const GemmArgs& g, Plan& p, const Config& cfg)
