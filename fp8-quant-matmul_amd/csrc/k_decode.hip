@@ -862,6 +862,9 @@ inline bool shallow_ring_pays(long workgroups, int kb_per_split) { return workgr
 // Whether the caches are told not to keep B.  Kept / not kept, us: from HBM 32 x 7168 x 2048 7.00 / 6.79, 24 x 4608 x 7168
 // 11.34 / 11.02, 16 x 16384 x 7168 25.2 / 23.7, 8 x 49152 x 4096 37.5 / 35.5, 16 groups of up to 32 rows, 7168 x 2048, 50.9 /
 // 46.5, 64 of 1 - 63 rows 190.7 / 179.7; from the Infinity Cache 1 x 7168 x 2048 5.68 / 5.43, 16 x 4608 x 7168 9.00 / 8.90.
+// The price: a B that the Infinity Cache does hold from call to call comes slower, 32 x 7168 x 2048 twelve of them in turn 6.34 /
+// 6.58, one alone 5.15 / 5.31, 32 x 4096 x 7168 alone 8.71 / 9.35 (twelve in turn, from HBM: 11.02 / 10.31); the weights of a
+// model that a decode step reads are more than the 256 MB it has.
 // A smaller B, whose launches leave most CUs without a strip, stays in the caches and is not helped: 16 x 1536 x 7168 from
 // HBM 7.02 / 6.98, from the Infinity Cache 6.03 / 6.60.  Strips that are no whole 128-byte lines share some: 16 x 576 x 7168 6.92 /
 // 7.27 and 5.87 / 6.68, 64 groups of up to 32 rows, 7152 x 2048, 189.6 / 215.0.

@@ -320,7 +320,7 @@ void launch_quantize_tile(const TIn* x, uint8_t* q, float* scale_out, int rows, 
 //   176 MB 8192 x 7168 36.6 / 31.0; fp32 84 MB 8192 x 576 x 2048 36.3 / 40.3, 147 MB 4096 x 1536 x 7168 79.9 / 80.2, 168 MB
 //   8192 x 576 x 4096 75.4 / 74.0, 215 MB 6000 x 1536 x 7168 131.8 / 119.2; blocks of fp32 106 MB 4608 x 4608 20.6 / 22.7, 126
 //   MB 8192 x 3072 27.5 / 26.5, 165 MB 4608 x 7168 34.3 / 32.5.  bf16 with its GEMM gains from 97 MB on: 4500 x 4608 x 7168
-//   182.7 / 178.8).
+//   182.7 / 178.8).  The price: the same 8192 x 7168 quantised over and over, nothing between, 27.2 / 30.6.
 template <typename TIn, bool BF16MATH>
 void launch_quantize_typed(const TIn* x, uint8_t* q, float* scale_out, int rows, int k, bool block128, hipStream_t s)
 {
