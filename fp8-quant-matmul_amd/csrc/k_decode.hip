@@ -863,12 +863,18 @@ inline bool shallow_ring_pays(long workgroups, int kb_per_split) { return workgr
 // 11.34 / 11.02, 16 x 16384 x 7168 25.2 / 23.7, 8 x 49152 x 4096 37.5 / 35.5, 16 groups of up to 32 rows, 7168 x 2048, 50.9 /
 // 46.5, 64 of 1 - 63 rows 190.7 / 179.7; from the Infinity Cache 1 x 7168 x 2048 5.68 / 5.43, 16 x 4608 x 7168 9.00 / 8.90.
 // The price: a B that the Infinity Cache does hold from call to call comes slower, 32 x 7168 x 2048 twelve of them in turn 6.34 /
-// 6.58, one alone 5.15 / 5.31, 32 x 4096 x 7168 alone 8.71 / 9.35 (twelve in turn, from HBM: 11.02 / 10.31); the weights of a
-// model that a decode step reads are more than the 256 MB it has.
-// A smaller B, whose launches leave most CUs without a strip, stays in the caches and is not helped: 16 x 1536 x 7168 from
+// 6.58, one alone 5.15 / 5.31, 32 x 4096 x 7168 alone 8.71 / 9.35 (twelve in turn, from HBM: 11.02 / 10.31), 32 x 7168 x 7168
+// three in turn 11.9 / 13.2 (twelve: 14.04 / 13.31); the weights of a model that a decode step reads are more than the 256 MB
+// it has.  With a strip for fewer than 200 of the 256 CUs the price is as high and the gain less: three in turn 32 x
+// 2048 x 7168 (128 workgroups) 8.2 / 8.9, 24 x 7168 x 2304 (168) 6.9 / 7.3, and the decode step whose projections are both
+// such and larger 95.5 us with those kept and 96.7 without.
+// A smaller B stays in the caches and is not helped: 16 x 1536 x 7168 from
 // HBM 7.02 / 6.98, from the Infinity Cache 6.03 / 6.60.  Strips that are no whole 128-byte lines share some: 16 x 576 x 7168 6.92 /
 // 7.27 and 5.87 / 6.68, 64 groups of up to 32 rows, 7152 x 2048, 189.6 / 215.0.
-inline bool b_read_once(int groups, int n, int k) { return n % 128 == 0 && (double)groups * n * k >= 12e6; }
+inline bool b_read_once(int groups, int n, int k, long workgroups)
+{
+    return n % 128 == 0 && (double)groups * n * k >= 12e6 && workgroups >= 200;
+}
 
 }  // namespace
 
@@ -982,7 +988,7 @@ hipError_t launch_decode_strips(const GemmArgs& g, int ksplit, int halves, float
     const int kb_per_split = (nkb + ksplit - 1) / ksplit;
     if ((ksplit - 1) * kb_per_split >= nkb)  // every split owns at least one K block
         return hipErrorInvalidValue;
-    const bool once = b_read_once(1, g.n, g.k);
+    const bool once = b_read_once(1, g.n, g.k, (long)strips * ksplit);
     const dim3 grid(8 * ((strips + 7) / 8), ksplit);
     auto go = [&](auto kern, int lds) -> hipError_t {
         FP8GEMM_ALLOW_LDS(kern, lds);
@@ -1166,7 +1172,7 @@ hipError_t launch_decode_grouped(const GroupTable& tab, int n, int k, int ksplit
         mmax = tab.lda[g] > mmax ? tab.lda[g] : mmax;
         ragged |= tab.lda[g] % 16 != 0;
     }
-    const bool once = b_read_once(tab.groups, n, k);
+    const bool once = b_read_once(tab.groups, n, k, (long)tab.groups * (n / DS_BN));
     // many strips, rows on the 16-byte grid, no K split: the streaming form with 256-column strips
     const int wide_strips = (n + 2 * DS_BN - 1) / (2 * DS_BN);
     const long wide_units = (long)wide_strips * tab.groups;
