@@ -39,9 +39,10 @@
 //     the two and not their sum; the folds of a block's last four sums cross the barrier.  Eight waves with the reads
 //     at the head of the block / this, from the Infinity Cache: 5504 x 512 x 7168 30.7 / 26.4 us, 2048 x 2048 x 7168
 //     36.1 / 32.0, 1024 x 1536 x 7168 21.4 / 19.1, 352 x 3072 x 1536 9.4 / 8.6, 350 x 3072 x 1536 (RAGGED) 11.3 / 10.4;
-//     64x64 tiles 1024 x 512 x 2048 6.1 / 5.85, 64 x 4608 x 7168, bound by the copies, 10.4 / 10.6.  Copies between the
-//     MFMAs of a lone wave hold them up (RAGGED with B copied there: 350 x 3072 x 1536 12.3 us), so they are the other
-//     waves'.  Eight stages of 64x64 instead of four: 5.9 -> 6.8 us.
+//     64x64 tiles 1024 x 512 x 2048 6.1 / 5.85, 64 x 4608 x 7168, bound by the copies, 10.4 / 10.6.  From HBM the
+//     copies bound a block: 5504 x 512 x 7168 35.0 / 36.1, 2048 x 2048 x 7168 39.9 / 39.4, 1024 x 1536 x 7168 21.3 / 20.0.
+//     Copies between the MFMAs of a lone wave hold them up (RAGGED with B copied there: 350 x 3072 x 1536 12.3 us), so
+//     they are the other waves'.  Eight stages of 64x64 instead of four: 5.9 -> 6.8 us.
 //   * NS LDS stages form a ring: the copies of K blocks kb+1 .. kb+NS-1 are in flight while
 //     block kb is multiplied.  Large tiles fit two stages; smaller tiles get three or four,
 //     which is what hides the global latency when a K block is only a few MFMAs long.
