@@ -1,3 +1,4 @@
+import gc
 import os
 import sys
 
@@ -23,6 +24,13 @@ def orc():
     import oracle
     oracle.lib()
     return oracle
+
+
+@pytest.fixture
+def garbage_collected():
+    """for tests that capture a stream: nothing that an earlier test left in a reference cycle, a graph above all, is
+    destroyed while the capture runs"""
+    gc.collect()
 
 
 def _have_gpu():

@@ -14,7 +14,7 @@ import pytest
 
 import oracle
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("garbage_collected")]
 
 
 def _say(msg):
