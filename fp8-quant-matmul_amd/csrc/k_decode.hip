@@ -990,7 +990,8 @@ hipError_t launch_decode_strips(const GemmArgs& g, int ksplit, int halves, float
         return hipErrorInvalidValue;
     const bool once = b_read_once(1, g.n, g.k, (long)strips * ksplit);
     const dim3 grid(8 * ((strips + 7) / 8), ksplit);
-    auto go = [&](auto kern, int lds) -> hipError_t {
+    auto go = [&](auto kernel, int lds) -> hipError_t {
+        constexpr auto kern = decltype(kernel)::value;
         FP8GEMM_ALLOW_LDS(kern, lds);
         hipLaunchKernelGGL(kern, grid, dim3(DS_THREADS), lds, s, g.b, g.a, g.n, g.k, g.m, leading_dim(g), kb_per_split, strips,
                            g.a_scale, g.b_scale, g.c, mailbox, ksplit);
@@ -1012,13 +1013,15 @@ hipError_t launch_decode_strips(const GemmArgs& g, int ksplit, int halves, float
             constexpr bool ST = decltype(staged_c)::value;
             constexpr int lds = DecodeShape<MT, NS, false, NB>::LDS + (ST ? 16 * T * (2 * DS_BN * NB + 16) : 0);
             static_assert(lds <= 160 * 1024, "ring and staged C exceed the LDS");
-            auto with = [&](auto kern) -> hipError_t {
+            auto with = [&](auto kernel) -> hipError_t {
+                constexpr auto kern = decltype(kernel)::value;
                 FP8GEMM_ALLOW_LDS(kern, lds);
                 hipLaunchKernelGGL(kern, dim3(STREAM_WORKGROUPS), dim3(DS_THREADS), lds, s, g.a, g.b, g.a_scale, g.b_scale,
                                    g.c, g.m, leading_dim(g), g.n, g.k, units);
                 return hipGetLastError();
             };
-            return once ? with(decode_stream_kernel<MT, NS, T, ST, NB, true>) : with(decode_stream_kernel<MT, NS, T, ST, NB, false>);
+            return once ? with(Kernel<decode_stream_kernel<MT, NS, T, ST, NB, true>>{})
+                        : with(Kernel<decode_stream_kernel<MT, NS, T, ST, NB, false>>{});
         };
         auto by_staging = [&](auto shape, auto tiles_c) -> hipError_t {
             return staged ? stream(shape, tiles_c, std::true_type{}) : stream(shape, tiles_c, std::false_type{});
@@ -1044,8 +1047,8 @@ hipError_t launch_decode_strips(const GemmArgs& g, int ksplit, int halves, float
             constexpr int MT = decltype(mt_c)::value, T = decltype(tiles_c)::value;
             constexpr ARows F = decltype(form_c)::value;
             constexpr int lds = DecodeShape<MT, STREAM_NS_WIDE, F == ARows::SPREAD, 2>::LDS;
-            return once ? go(decode_strip_kernel<MT, STREAM_NS_WIDE, F, T, 2, 1, true>, lds)
-                        : go(decode_strip_kernel<MT, STREAM_NS_WIDE, F, T, 2, 1, false>, lds);
+            return once ? go(Kernel<decode_strip_kernel<MT, STREAM_NS_WIDE, F, T, 2, 1, true>>{}, lds)
+                        : go(Kernel<decode_strip_kernel<MT, STREAM_NS_WIDE, F, T, 2, 1, false>>{}, lds);
         };
         auto by_tiles = [&](auto form_c) -> hipError_t {
             switch (tiles) {
@@ -1072,10 +1075,10 @@ hipError_t launch_decode_strips(const GemmArgs& g, int ksplit, int halves, float
         constexpr int lds = DecodeShape<MT, NS, F == ARows::SPREAD>::LDS;
         if constexpr (NS % 2 == 0)
             if (stages_in_pairs((long)strips * ksplit, kb_per_split, NS))
-                return once ? go(decode_strip_kernel<MT, NS, F, T, 1, 2, true>, lds)
-                            : go(decode_strip_kernel<MT, NS, F, T, 1, 2, false>, lds);
-        return once ? go(decode_strip_kernel<MT, NS, F, T, 1, 1, true>, lds)
-                    : go(decode_strip_kernel<MT, NS, F, T, 1, 1, false>, lds);
+                return once ? go(Kernel<decode_strip_kernel<MT, NS, F, T, 1, 2, true>>{}, lds)
+                            : go(Kernel<decode_strip_kernel<MT, NS, F, T, 1, 2, false>>{}, lds);
+        return once ? go(Kernel<decode_strip_kernel<MT, NS, F, T, 1, 1, true>>{}, lds)
+                    : go(Kernel<decode_strip_kernel<MT, NS, F, T, 1, 1, false>>{}, lds);
     };
     using std::integral_constant;
     auto by_tiles = [&](auto ns2, auto ns4, auto form_c) -> hipError_t {
@@ -1185,14 +1188,15 @@ hipError_t launch_decode_grouped(const GroupTable& tab, int n, int k, int ksplit
             constexpr bool ST = decltype(staged_c)::value;
             constexpr int lds = DecodeShape<MT, NS, false, NB>::LDS + (ST ? 16 * MT * (2 * DS_BN * NB + 16) : 0);
             static_assert(lds <= 160 * 1024, "ring and staged C exceed the LDS");
-            auto with = [&](auto kern) -> hipError_t {
+            auto with = [&](auto kernel) -> hipError_t {
+                constexpr auto kern = decltype(kernel)::value;
                 FP8GEMM_ALLOW_LDS(kern, lds);
                 hipLaunchKernelGGL(kern, dim3(STREAM_WORKGROUPS), dim3(DS_THREADS), lds, s, tab, n, k, wide_strips,
                                    (int)wide_units);
                 return hipGetLastError();
             };
-            return once ? with(decode_stream_grouped_kernel<MT, NS, ST, NB, true>)
-                        : with(decode_stream_grouped_kernel<MT, NS, ST, NB, false>);
+            return once ? with(Kernel<decode_stream_grouped_kernel<MT, NS, ST, NB, true>>{})
+                        : with(Kernel<decode_stream_grouped_kernel<MT, NS, ST, NB, false>>{});
         };
         if (row_tiles(mmax) == 2)
             return staged ? stream(StreamShape<2, STREAM_NS_WIDE, 2>{}, std::true_type{})
@@ -1201,7 +1205,8 @@ hipError_t launch_decode_grouped(const GroupTable& tab, int n, int k, int ksplit
                       : stream(StreamShape<4, STREAM_NS_WIDE, 2>{}, std::false_type{});
     }
     const dim3 grid((unsigned)(8 * ((units + 7) / 8)), (unsigned)ksplit);
-    auto go = [&](auto kern, int lds) -> hipError_t {
+    auto go = [&](auto kernel, int lds) -> hipError_t {
+        constexpr auto kern = decltype(kernel)::value;
         FP8GEMM_ALLOW_LDS(kern, lds);
         hipLaunchKernelGGL(kern, grid, dim3(DS_THREADS), lds, s, tab, mailbox, n, k, strips, ksplit, kb_per_split);
         return hipGetLastError();
@@ -1217,10 +1222,10 @@ hipError_t launch_decode_grouped(const GroupTable& tab, int n, int k, int ksplit
         constexpr int lds = DecodeShape<MT, NS, RG>::LDS;
         if constexpr (NS % 2 == 0)
             if (stages_in_pairs(units * ksplit, kb_per_split, NS) && !(RG && (kb_per_split == 1 || kb_per_split == 3)))
-                return once ? go(decode_strip_grouped_kernel<MT, NS, RG, 2, true>, lds)
-                            : go(decode_strip_grouped_kernel<MT, NS, RG, 2, false>, lds);
-        return once ? go(decode_strip_grouped_kernel<MT, NS, RG, 1, true>, lds)
-                    : go(decode_strip_grouped_kernel<MT, NS, RG, 1, false>, lds);
+                return once ? go(Kernel<decode_strip_grouped_kernel<MT, NS, RG, 2, true>>{}, lds)
+                            : go(Kernel<decode_strip_grouped_kernel<MT, NS, RG, 2, false>>{}, lds);
+        return once ? go(Kernel<decode_strip_grouped_kernel<MT, NS, RG, 1, true>>{}, lds)
+                    : go(Kernel<decode_strip_grouped_kernel<MT, NS, RG, 1, false>>{}, lds);
     };
     using std::integral_constant;
     const integral_constant<int, 2> two{};

@@ -235,7 +235,7 @@ hipError_t launch_skinny(const GemmArgs& g, int ksplit, float* partial, hipStrea
     dim3 grid(tiles_n, ksplit);
     hipError_t e;
     if (ksplit > 1) {
-        auto kern = skinny_gemm_kernel<true>;
+        constexpr auto kern = skinny_gemm_kernel<true>;
         FP8GEMM_ALLOW_LDS(kern, SK_LDS);
         hipLaunchKernelGGL(kern, grid, dim3(SK_THREADS), SK_LDS, s, g.a, g.b, g.a_scale, g.b_scale,
                            g.c, partial, g.m, g.n, g.k, tiles_n, kb_per_split);
@@ -244,7 +244,7 @@ hipError_t launch_skinny(const GemmArgs& g, int ksplit, float* partial, hipStrea
             return e;
         return launch_splitk_reduce(g, ksplit, partial, s);
     }
-    auto kern = skinny_gemm_kernel<false>;
+    constexpr auto kern = skinny_gemm_kernel<false>;
     FP8GEMM_ALLOW_LDS(kern, SK_LDS);
     hipLaunchKernelGGL(kern, grid, dim3(SK_THREADS), SK_LDS, s, g.a, g.b, g.a_scale, g.b_scale, g.c,
                        partial, g.m, g.n, g.k, tiles_n, kb_per_split);

@@ -908,7 +908,7 @@ hipError_t launch_typed(const GemmArgs& g, int ksplit, float* partial, float* ma
     if (SPLIT && mailbox && (size_t)tiles * (ksplit - 1) * BM * BN * 4 > SPLIT_MAILBOX_BYTES)
         return hipErrorInvalidValue;
     const dim3 grid(SPLIT && mailbox ? (tiles + 7) & ~7 : tiles, SPLIT ? ksplit : 1);
-    auto kern = tile_gemm_kernel<BM, BN, WM, WN, NS, SPLIT, RAGGED>;
+    constexpr auto kern = tile_gemm_kernel<BM, BN, WM, WN, NS, SPLIT, RAGGED>;
     FP8GEMM_ALLOW_LDS(kern, LDS_TOTAL);
     hipLaunchKernelGGL(kern, grid, dim3(NTHREADS), LDS_TOTAL, s, g.a, g.b, g.a_scale, g.b_scale, g.c, partial,
                        SPLIT ? mailbox : nullptr, g.m, leading_dim(g), g.n, g.k, tiles_m, tiles_n, kb_per_split, group_m);

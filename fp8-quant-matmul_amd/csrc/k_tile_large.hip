@@ -449,7 +449,7 @@ template <int BN, Tail TAIL>
 hipError_t launch_large(const GemmArgs& g, int workgroups, hipStream_t s)
 {
     constexpr int LDS = LargeShape<BN>::LDS_BYTES > tail_lds_bytes<TAIL>() ? LargeShape<BN>::LDS_BYTES : tail_lds_bytes<TAIL>();
-    auto kern = tile_gemm_large_kernel<BN, TAIL>;
+    constexpr auto kern = tile_gemm_large_kernel<BN, TAIL>;
     FP8GEMM_ALLOW_LDS(kern, LDS);
     hipLaunchKernelGGL(kern, dim3(workgroups), dim3(NTHREADS), LDS, s, g.a, g.b, g.a_scale, g.b_scale, g.c, g.m,
                        leading_dim(g), g.n, g.k, (g.m + 255) / 256, (g.n + BN - 1) / BN, c_streams(g.m, 1, g.n, g.k));
@@ -460,7 +460,7 @@ template <int BN, Tail TAIL>
 hipError_t launch_large_grouped(const GroupTable& tab, int n, int k, int workgroups, hipStream_t s)
 {
     constexpr int LDS = LargeShape<BN>::LDS_BYTES > tail_lds_bytes<TAIL>() ? LargeShape<BN>::LDS_BYTES : tail_lds_bytes<TAIL>();
-    auto kern = tile_gemm_large_grouped_kernel<BN, TAIL>;
+    constexpr auto kern = tile_gemm_large_grouped_kernel<BN, TAIL>;
     FP8GEMM_ALLOW_LDS(kern, LDS);
     long rows = 0;
     for (int g = 0; g < tab.groups; ++g)

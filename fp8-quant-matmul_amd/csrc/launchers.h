@@ -23,23 +23,35 @@ struct GemmArgs {
 inline int leading_dim(const GemmArgs& g) { return g.lda ? g.lda : g.m; }
 
 // Kernels with more than 64 KiB of dynamic LDS need the attribute raised before their first launch
-// on a device.  Once per kernel and device (a bit per device in a word the call site owns) instead of
+// on a device.  Once per kernel and device (a bit per device in a word of each kernel's own) instead of
 // once per launch: the runtime call costs as much as a short kernel takes.
+template <auto KERNEL>
+hipError_t allow_lds(int bytes)
+{
+    static std::atomic<uint64_t> done{0};
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess)
+        return e;
+    const uint64_t bit = 1ull << (dev & 63);
+    if (done.load(std::memory_order_acquire) & bit)
+        return hipSuccess;
+    e = hipFuncSetAttribute(reinterpret_cast<const void*>(KERNEL), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    if (e == hipSuccess)
+        done.fetch_or(bit, std::memory_order_release);
+    return e;
+}
+// A kernel as an argument of a generic lambda: kernels with the same parameters have one type, so the function
+// pointer itself would leave them one instantiation, and one word of allow_lds, between them.
+template <auto KERNEL>
+struct Kernel {
+    static constexpr auto value = KERNEL;
+};
 #define FP8GEMM_ALLOW_LDS(kern, bytes)                                                                       \
     do {                                                                                                     \
-        static std::atomic<uint64_t> done_{0};                                                               \
-        int dev_ = 0;                                                                                        \
-        hipError_t e_ = hipGetDevice(&dev_);                                                                 \
+        const hipError_t e_ = allow_lds<kern>(bytes);                                                        \
         if (e_ != hipSuccess)                                                                                \
             return e_;                                                                                       \
-        const uint64_t bit_ = 1ull << (dev_ & 63);                                                           \
-        if (!(done_.load(std::memory_order_acquire) & bit_)) {                                               \
-            e_ = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),                                    \
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, (bytes));                   \
-            if (e_ != hipSuccess)                                                                            \
-                return e_;                                                                                   \
-            done_.fetch_or(bit_, std::memory_order_release);                                                 \
-        }                                                                                                    \
     } while (0)
 
 // one thread per C element (check.cu:30-49)
