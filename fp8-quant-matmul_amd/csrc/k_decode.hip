@@ -859,19 +859,50 @@ inline bool stages_in_pairs(long workgroups, int kb_per_split, int ring)
 // workgroups (1.5-2.25 rounds of 512 resident ones) 1-3 % slower than three to four and a half rounds of 256.
 inline bool shallow_ring_pays(long workgroups, int kb_per_split) { return workgroups >= 2048 && kb_per_split >= 6; }
 
-// Whether the caches are told not to keep B.  Kept / not kept, us: from HBM 32 x 7168 x 2048 7.00 / 6.79, 24 x 4608 x 7168
-// 11.34 / 11.02, 16 x 16384 x 7168 25.2 / 23.7, 8 x 49152 x 4096 37.5 / 35.5, 16 groups of up to 32 rows, 7168 x 2048, 50.9 /
-// 46.5, 64 of 1 - 63 rows 190.7 / 179.7; from the Infinity Cache 1 x 7168 x 2048 5.68 / 5.43, 16 x 4608 x 7168 9.00 / 8.90.
-// The price: a B that the Infinity Cache does hold from call to call comes slower, 32 x 7168 x 2048 twelve of them in turn 6.34 /
-// 6.58, one alone 5.15 / 5.31, 32 x 4096 x 7168 alone 8.71 / 9.35 (twelve in turn, from HBM: 11.02 / 10.31), 32 x 7168 x 7168
-// three in turn 11.9 / 13.2 (twelve: 14.04 / 13.31); the weights of a model that a decode step reads are more than the 256 MB
-// it has.  With a strip for fewer than 200 of the 256 CUs the price is as high and the gain less: three in turn 32 x
-// 2048 x 7168 (128 workgroups) 8.2 / 8.9, 24 x 7168 x 2304 (168) 6.9 / 7.3, and the decode step whose projections are both
-// such and larger 95.5 us with those kept and 96.7 without.
-// A smaller B stays in the caches and is not helped: 16 x 1536 x 7168 from
-// HBM 7.02 / 6.98, from the Infinity Cache 6.03 / 6.60.  Strips that are no whole 128-byte lines share some: 16 x 576 x 7168 6.92 /
-// 7.27 and 5.87 / 6.68, 64 groups of up to 32 rows, 7152 x 2048, 189.6 / 215.0.
-inline bool b_read_once(int groups, int n, int k, long workgroups)
+// Whether the caches are told not to keep B.  From HBM that is a little faster, and what such a B does not displace stays
+// in the caches for the rest of a decode step; but a B that the caches do hold from call to call comes slower, as from
+// HBM.  us kept / not kept, "alone" one B over and over, "in turn" as many as take 140 MB and so stay in the Infinity
+// Cache, HBM 800 MB of them in turn (graphs of 48 and more launches, medians of nine):
+//                                  alone          in turn        HBM
+//   16 x 7168 x 2048 (15 MB)     4.10 /  4.10   5.62 /  5.84   6.05 /  5.94   three in turn, more than the L2s hold, 5.58 / 5.37
+//   32 x 7168 x 2048             5.16 /  5.16   6.66 /  6.79   6.92 /  6.85   (alone 5.48 on other boxes; three 6.46 / 6.44)
+//   16 x 10240 x 2048 (21 MB)    4.59 /  4.59   6.78 /  7.31   7.68 /  7.56
+//   32 x 9216 x 3072 (28 MB)     6.94 /  7.75   8.46 /  9.13   9.75 /  9.46
+//   24 x 4608 x 7168 (33 MB)     9.74 / 10.08  10.54 / 10.83  11.56 / 11.10
+//   16 x 8192 x 4096 (34 MB)     6.79 /  6.87   8.51 /  8.66   9.53 /  8.93
+//   32 x 7168 x 7168 (51 MB)    12.00 / 12.60  12.02 / 13.50  14.28 / 13.89
+//   32 x 10240 x 7168 (73 MB)   15.46 / 17.56  15.49 / 18.25  19.56 / 18.81
+//   16 x 16384 x 7168 (117 MB)  20.64 / 21.59                 25.34 / 23.03
+//   48 x 16384 x 7168           23.48 / 25.89                 27.87 / 26.56
+//   unsplit: 16 x 28672 x 2048 (59 MB) 11.14 / 11.39, 11.12 / 12.63, 13.43 / 13.17; 48 x 28672 x 4096 (117 MB) 20.23 / 25.57,
+//   HBM 26.77 / 26.74; in strips of 256 columns 16 x 57344 x 2048 (117 MB) 18.93 / 19.30, HBM 21.84 / 20.94; 16 x 65536 x
+//   3072 (201 MB) HBM 34.39 / 31.81, 16 x 131072 x 4096 91.8 / 82.9
+// So: always where the Infinity Cache (256 MB) cannot hold B anyway; from half of that on, which does not stay beside
+// much else, where HBM gains (K split over up to 32 rows, strips of 256 columns); and up to 36 MB where the L2s' 32 MB
+// decide and the price is small: a single row tile, whose three in turn gain, or 30 MB and more, whose gain from HBM is
+// 4 - 6 %.  A decode step of nine projections with 24 rows, 92 MB of weights, three of them in turn: 100.3 us with every B
+// kept, 93.5 with the one of 33 MB not kept and all others kept, of which then 175 MB stay.  With a strip for fewer than
+// 200 of the 256 CUs the price is as high and the gain less: three in turn 32 x 2048 x 7168 (128 workgroups) 8.2 / 8.9, 24 x
+// 7168 x 2304 (168) 6.9 / 7.3.  Strips that are no whole 128-byte lines share some: 16 x 576 x 7168 6.92 / 7.27.
+inline bool b_read_once(const GemmArgs& g, int ksplit, bool wide, long workgroups)
+{
+    const double b = (double)g.n * g.k;
+    if (g.n % 128 != 0)
+        return false;
+    if (b >= 192e6)
+        return true;
+    if (b >= 115e6)
+        return ksplit > 1 ? g.m <= 32 : wide;
+    const bool in_turn = g.m <= 16 && b >= 12e6 && b <= 20e6, large_enough = b >= 30e6 && b <= 36e6;
+    return ksplit > 1 && workgroups >= 200 && (in_turn || large_enough);
+}
+
+// The same for a grouped launch, whose B are as many as its groups.  Kept / not kept, us, alone / in turn / from HBM: two groups
+// of 9 - 12 rows, 7168 x 2048, 7.66 / 7.76, 8.91 / 9.36, 10.29 / 9.44; four of 20 - 29 13.01 / 13.22, 13.00 / 14.10, 15.68 / 14.80;
+// seven of 20 - 31, 1536 x 2048, 8.47 / 8.55, 9.36 / 9.40, 9.95 / 9.28; 64 of 2 - 16, 1536 x 1024, 23.56 / 22.95, HBM 25.95 / 23.90;
+// 16 of up to 32, 7168 x 2048, HBM 50.2 / 46.4; 64 of 1 - 62 200.8 / 186.5.  64 of up to 32 rows, 7152 x 2048, whose strips
+// share lines, 189.6 / 215.0.
+inline bool grouped_b_read_once(int groups, int n, int k, long workgroups)
 {
     return n % 128 == 0 && (double)groups * n * k >= 12e6 && workgroups >= 200;
 }
@@ -988,7 +1019,14 @@ hipError_t launch_decode_strips(const GemmArgs& g, int ksplit, int halves, float
     const int kb_per_split = (nkb + ksplit - 1) / ksplit;
     if ((ksplit - 1) * kb_per_split >= nkb)  // every split owns at least one K block
         return hipErrorInvalidValue;
-    const bool once = b_read_once(1, g.n, g.k, (long)strips * ksplit);
+    // more strips than resident workgroups, no K split: one copy stream per workgroup (the streaming form chooses
+    // its strip width itself).  Strips of the width asked for: 57344 columns are 448 strips of 128 -- two turns of
+    // the streaming workgroups, the second three quarters full, 96.9 us for 16 x 57344 x 8192 -- but 224 strips of
+    // 256, one round of plain workgroups, 80.8 us.
+    const bool streams = ksplit == 1 && strips > STREAM_WORKGROUPS && leading_dim(g) % 16 == 0;
+    const int wide_units = (g.n + 2 * DS_BN - 1) / (2 * DS_BN);
+    const bool wide_stream = wide_units >= STREAM_WORKGROUPS;  // 256-column strips while every CU gets one
+    const bool once = b_read_once(g, ksplit, streams ? wide_stream : halves == 2, (long)strips * ksplit);
     const dim3 grid(8 * ((strips + 7) / 8), ksplit);
     auto go = [&](auto kernel, int lds) -> hipError_t {
         constexpr auto kern = decltype(kernel)::value;
@@ -997,16 +1035,10 @@ hipError_t launch_decode_strips(const GemmArgs& g, int ksplit, int halves, float
                            g.a_scale, g.b_scale, g.c, mailbox, ksplit);
         return hipGetLastError();
     };
-    // more strips than resident workgroups, no K split: one copy stream per workgroup (the streaming form chooses
-    // its strip width itself).  Strips of the width asked for: 57344 columns are 448 strips of 128 -- two turns of
-    // the streaming workgroups, the second three quarters full, 96.9 us for 16 x 57344 x 8192 -- but 224 strips of
-    // 256, one round of plain workgroups, 80.8 us.
     const int strips128 = (g.n + DS_BN - 1) / DS_BN;
-    if (ksplit == 1 && strips > STREAM_WORKGROUPS && leading_dim(g) % 16 == 0) {
+    if (streams) {
         const bool staged = reinterpret_cast<uintptr_t>(g.c) % 16 == 0;
-        const int wide_units = (g.n + 2 * DS_BN - 1) / (2 * DS_BN);
-        const bool wide = wide_units >= STREAM_WORKGROUPS;  // 256-column strips while every CU gets one
-        const int units = wide ? wide_units : strips128;
+        const int units = wide_stream ? wide_units : strips128;
         auto stream = [&](auto shape, auto tiles_c, auto staged_c) -> hipError_t {
             constexpr int MT = decltype(shape)::MT, NS = decltype(shape)::NS, NB = decltype(shape)::NB;
             constexpr int T = decltype(tiles_c)::value;
@@ -1034,8 +1066,8 @@ hipError_t launch_decode_strips(const GemmArgs& g, int ksplit, int halves, float
             default: return by_staging(shape4, std::integral_constant<int, 4>{});
             }
         };
-        return wide ? by_tiles(StreamShape<2, STREAM_NS_WIDE, 2>{}, StreamShape<4, STREAM_NS_WIDE, 2>{})
-                    : by_tiles(StreamShape<2, STREAM_NS, 1>{}, StreamShape<4, STREAM_NS4, 1>{});
+        return wide_stream ? by_tiles(StreamShape<2, STREAM_NS_WIDE, 2>{}, StreamShape<4, STREAM_NS_WIDE, 2>{})
+                           : by_tiles(StreamShape<2, STREAM_NS, 1>{}, StreamShape<4, STREAM_NS4, 1>{});
     }
     using Grid = std::integral_constant<ARows, ARows::GRID>;
     using Spread = std::integral_constant<ARows, ARows::SPREAD>;
@@ -1175,7 +1207,7 @@ hipError_t launch_decode_grouped(const GroupTable& tab, int n, int k, int ksplit
         mmax = tab.lda[g] > mmax ? tab.lda[g] : mmax;
         ragged |= tab.lda[g] % 16 != 0;
     }
-    const bool once = b_read_once(tab.groups, n, k, (long)tab.groups * (n / DS_BN));
+    const bool once = grouped_b_read_once(tab.groups, n, k, (long)tab.groups * (n / DS_BN));
     // many strips, rows on the 16-byte grid, no K split: the streaming form with 256-column strips
     const int wide_strips = (n + 2 * DS_BN - 1) / (2 * DS_BN);
     const long wide_units = (long)wide_strips * tab.groups;

@@ -1,7 +1,9 @@
 /* A program that carries its own stand-ins for the HIP runtime's calls (the library's references resolve to them first),
  * takes the decode kernels' entry points through many shapes without a device and prints what the launches asked for:
  * "kernels K raised R again A missing M" -- kernels launched with more than 64 KiB of dynamic LDS, kernels whose limit was
- * raised, times it was raised again for one, launches above their kernel's limit. */
+ * raised, times it was raised again for one, launches above their kernel's limit.
+ * With arguments "rows n k split groups" (split 0 = automatic; groups 0 = a single problem) only that call, and the mangled
+ * names of the kernels that it launches. */
 #include <stddef.h>
 #include <stdint.h>
 #include <stdio.h>
@@ -15,7 +17,19 @@ static struct { dim3 grid, block; size_t lds; void *stream; } cfg;
 
 enum { MAX_KERNELS = 1024 };
 static struct { const void *kernel; int raised, times, large; } seen[MAX_KERNELS];
-static int kernels, missing;
+static int kernels, missing, say_names;
+static struct { const void *kernel; const char *name; } known[8192];
+static int registered;
+
+void __hipRegisterFunction(void **modules, const void *kernel, char *a, const char *name, unsigned b, void *c, void *d, void *e,
+                           void *f, int *g)
+{
+    (void)modules, (void)a, (void)b, (void)c, (void)d, (void)e, (void)f, (void)g;
+    if (registered == 8192)
+        abort();
+    known[registered].kernel = kernel;
+    known[registered++].name = name;
+}
 
 static int number_of(const void *kernel)
 {
@@ -40,6 +54,9 @@ int hipFuncSetAttribute(const void *kernel, int attribute, int value)
 int hipLaunchKernel(const void *kernel, dim3 grid, dim3 block, void **args, size_t lds, void *stream)
 {
     (void)grid, (void)block, (void)args, (void)stream;
+    for (int i = 0; say_names && i < registered; ++i)
+        if (known[i].kernel == kernel)
+            printf("%s\n", known[i].name);
     if (lds > 64 * 1024) {
         const int i = number_of(kernel);
         seen[i].large = 1;
@@ -70,10 +87,42 @@ int hipMemcpy(void *to, const void *from, size_t bytes, int kind)
     return 0;
 }
 
-int main(void)
+/* never read: nothing is launched */
+static void *const p = (void *)(uintptr_t)(1 << 20), *const odd = (void *)(uintptr_t)((1 << 20) + 8);
+
+/* groups problems of m rows each; c = not on a 16-byte boundary if odd_c, the first one with other rows if first > 0 */
+static int grouped(int groups, int m, int first, int n, int k, int split, int odd_c)
 {
-    /* never read: nothing is launched */
-    void *const p = (void *)(uintptr_t)(1 << 20), *const odd = (void *)(uintptr_t)((1 << 20) + 8);
+    const void *ptr[64];
+    void *out[64];
+    int rows[64];
+    for (int g = 0; g < groups; ++g) {
+        ptr[g] = p;
+        out[g] = odd_c ? odd : p;
+        rows[g] = first > 0 && g == 0 ? first : m;
+    }
+    const fp8gemm_options opt = {FP8GEMM_KERNEL_AUTO, -1, split, -1, FP8GEMM_FLAG_WORKSPACE_ZEROED};
+    return fp8_block_gemm_grouped_ex(groups, ptr, ptr, (const float *const *)ptr, (const float *const *)ptr, out, rows, n, k, &opt,
+                                     p, (size_t)1 << 36, 0);
+}
+
+static int one_call(char **word)
+{
+    const int m = atoi(word[1]), n = atoi(word[2]), k = atoi(word[3]), split = atoi(word[4]), groups = atoi(word[5]);
+    const fp8gemm_options opt = {split ? FP8GEMM_KERNEL_SKINNY : FP8GEMM_KERNEL_AUTO, split ? 1 : -1, split, -1,
+                                 FP8GEMM_FLAG_WORKSPACE_ZEROED};
+    /* the first call looks at the placement of workgroups */
+    fp8_block_gemm_ex(p, p, p, p, p, 32, 7168, 2048, 0, p, (size_t)1 << 32, 0);
+    grouped(2, 16, 0, 7168, 2048, 2, 0);
+    say_names = 1;
+    return groups ? grouped(groups, m, 0, n, k, split, 0)
+                  : fp8_block_gemm_ex(p, p, p, p, p, m, n, k, &opt, p, (size_t)1 << 32, 0);
+}
+
+int main(int argc, char **argv)
+{
+    if (argc == 6)
+        return one_call(argv);
     const int rows[] = {1, 8, 15, 16, 24, 31, 32, 40, 47, 48, 56, 63, 64};
     const int ns[] = {128, 1536, 4608, 7152, 7168, 16384, 28672, 33024, 49152, 65536, 65664, 131072};
     const int ks[] = {128, 384, 512, 1024, 2048, 4096, 7168, 8192};
@@ -91,19 +140,9 @@ int main(void)
                 for (int groups = 2; groups <= 64; groups *= 2)
                     for (int split = 0; split <= 4; split += 4)
                         for (int ragged = 0; ragged < 2; ++ragged)
-                            for (int c = 0; c < 2; ++c) {
-                                const void *ptr[64];
-                                void *out[64];
-                                int m[64];
-                                for (int g = 0; g < groups; ++g) {
-                                    ptr[g] = p;
-                                    out[g] = c ? odd : p;
-                                    m[g] = ragged && g == 0 ? (rows[i] > 1 ? rows[i] - 1 : 1) : (rows[i] + 15) / 16 * 16;
-                                }
-                                const fp8gemm_options opt = {FP8GEMM_KERNEL_AUTO, -1, split, -1, FP8GEMM_FLAG_WORKSPACE_ZEROED};
-                                calls += fp8_block_gemm_grouped_ex(groups, ptr, ptr, (const float *const *)ptr, (const float *const *)ptr,
-                                                                   out, m, ns[j], ks[l], &opt, p, (size_t)1 << 36, 0) == 0;
-                            }
+                            for (int c = 0; c < 2; ++c)
+                                calls += grouped(groups, (rows[i] + 15) / 16 * 16, ragged ? (rows[i] > 1 ? rows[i] - 1 : 1) : 0, ns[j],
+                                                 ks[l], split, c) == 0;
             }
     int large = 0, raised = 0, again = 0;
     for (int i = 0; i < kernels; ++i) {

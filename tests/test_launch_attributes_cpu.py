@@ -1,16 +1,42 @@
-"""The dynamic-LDS limit of the decode kernels, with stand-ins for the runtime's calls: no device, nothing runs."""
+"""What the decode kernels' launches ask for, with stand-ins for the runtime's calls: no device, nothing runs."""
 import os
 import subprocess
+
+import pytest
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 
 
-def test_the_lds_limit_is_raised_once_for_each_kernel(pkg, tmp_path):
+@pytest.fixture(scope="module")
+def program(pkg, tmp_path_factory):
     lib = pkg.lib_path()
-    exe = str(tmp_path / "stand_in_runtime")
+    exe = str(tmp_path_factory.mktemp("stand_in") / "stand_in_runtime")
     subprocess.run(["gcc", "-O1", "-Wall", "-rdynamic", os.path.join(HERE, "stand_in_runtime.c"), lib, "-Wl,-rpath," + os.path.dirname(lib),
                     "-Wl,--unresolved-symbols=ignore-in-shared-libs", "-o", exe], check=True)
-    words = subprocess.run([exe], check=True, capture_output=True, text=True, timeout=120).stdout.split()
+    return lambda *args: subprocess.run([exe, *map(str, args)], check=True, capture_output=True, text=True, timeout=120).stdout.split()
+
+
+def test_the_lds_limit_is_raised_once_for_each_kernel(program):
+    words = program()
     count = {name: int(value) for name, value in zip(words[::2], words[1::2])}
     assert count["calls"] > 1000 and count["kernels"] > 60, count
     assert count["missing"] == 0 and count["again"] == 0 and count["raised"] >= count["kernels"], count
+
+
+def reads_past_the_caches(program, m, n, k, split=0, groups=0):
+    kernels = [name for name in program(m, n, k, split, groups) if "decode_" in name]
+    assert len(kernels) == 1, kernels
+    name = subprocess.run(["c++filt", kernels[0]], check=True, capture_output=True, text=True).stdout
+    assert ", true>(" in name or ", false>(" in name, name   # ONCE is the last template argument
+    return ", true>(" in name
+
+
+# B that the caches hold from call to call stays there where it comes slower past them: two row tiles over a small B, mid-sized
+# ones, unsplit launches of 128-column strips; what does not fit the Infinity Cache is read past it whatever the launch
+@pytest.mark.parametrize("m,n,k,past", [(1, 7168, 2048, True), (16, 7168, 2048, True), (24, 7168, 2048, False), (32, 7168, 2048, False),
+                                        (24, 4608, 7168, True), (8, 10240, 2048, False), (32, 9216, 3072, False), (16, 7168, 7168, False),
+                                        (24, 7168, 2304, False), (16, 28672, 2048, False), (16, 28672, 4096, False), (32, 16384, 7168, True),
+                                        (48, 16384, 7168, False), (16, 57344, 2048, True), (48, 65536, 3072, True), (31, 28672, 8192, True),
+                                        (16, 7152, 2048, False)])
+def test_which_b_is_read_past_the_caches(program, m, n, k, past):
+    assert reads_past_the_caches(program, m, n, k) == past
