@@ -900,7 +900,9 @@ inline bool b_read_once(const GemmArgs& g, int ksplit, bool wide, long workgroup
 // The same for a grouped launch, whose B are as many as its groups.  Kept / not kept, us, alone / in turn / from HBM: two groups
 // of 9 - 12 rows, 7168 x 2048, 7.66 / 7.76, 8.91 / 9.36, 10.29 / 9.44; four of 20 - 29 13.01 / 13.22, 13.00 / 14.10, 15.68 / 14.80;
 // seven of 20 - 31, 1536 x 2048, 8.47 / 8.55, 9.36 / 9.40, 9.95 / 9.28; 64 of 2 - 16, 1536 x 1024, 23.56 / 22.95, HBM 25.95 / 23.90;
-// 16 of up to 32, 7168 x 2048, HBM 50.2 / 46.4; 64 of 1 - 62 200.8 / 186.5.  64 of up to 32 rows, 7152 x 2048, whose strips
+// 16 of up to 32, 7168 x 2048, HBM 50.2 / 46.4; 64 of 1 - 62 200.8 / 186.5; with K split three of 1 - 12, 3072 x 2048 (216
+// workgroups), 6.21 / 6.22, 7.73 / 7.79, 8.39 / 7.77; four of 19 - 31, 2048 x 7168 (256), 14.63 / 14.05, 14.62 / 14.91, 17.02 /
+// 15.42; 16 of 1 - 31, 1024 x 2048 (256), 10.63 / 9.33, 10.67 / 10.46, 11.79 / 10.60.  64 of up to 32 rows, 7152 x 2048, whose strips
 // share lines, 189.6 / 215.0.
 inline bool grouped_b_read_once(int groups, int n, int k, long workgroups)
 {
@@ -1207,7 +1209,7 @@ hipError_t launch_decode_grouped(const GroupTable& tab, int n, int k, int ksplit
         mmax = tab.lda[g] > mmax ? tab.lda[g] : mmax;
         ragged |= tab.lda[g] % 16 != 0;
     }
-    const bool once = grouped_b_read_once(tab.groups, n, k, (long)tab.groups * (n / DS_BN));
+    const bool once = grouped_b_read_once(tab.groups, n, k, units * ksplit);
     // many strips, rows on the 16-byte grid, no K split: the streaming form with 256-column strips
     const int wide_strips = (n + 2 * DS_BN - 1) / (2 * DS_BN);
     const long wide_units = (long)wide_strips * tab.groups;

@@ -40,3 +40,10 @@ def reads_past_the_caches(program, m, n, k, split=0, groups=0):
                                         (16, 7152, 2048, False)])
 def test_which_b_is_read_past_the_caches(program, m, n, k, past):
     assert reads_past_the_caches(program, m, n, k) == past
+
+
+# 72 strips in four splits and 84 in three are launches of more than 200 workgroups, 84 unsplit are not
+@pytest.mark.parametrize("groups,m,n,k,split,past", [(3, 16, 3072, 2048, 4, True), (7, 32, 1536, 2048, 3, True), (7, 32, 1536, 2048, 1, False),
+                                                     (16, 32, 7168, 2048, 1, True), (2, 16, 1536, 2048, 4, False), (64, 32, 7152, 2048, 1, False)])
+def test_grouped_launches_count_their_workgroups(program, groups, m, n, k, split, past):
+    assert reads_past_the_caches(program, m, n, k, split, groups) == past
