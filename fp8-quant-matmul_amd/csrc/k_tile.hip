@@ -32,7 +32,7 @@
 //     multiply, a wave that does not copies b_scale into the stage (64x64 tiles, which are done before that
 //     trip is: 48 x 4608 x 7168 14.2 -> 10.9 us).
 //   * The two smaller tiles, 64x64 and 128x128, are multiplied by four waves, one per SIMD, and copied by the other
-//     four (128x128 with ragged rows and split K: by eight, see launch_tile).  What bounds a K block of them is the
+//     four (128x128 with short chains: by eight, see four_waves).  What bounds a K block of them is the
 //     LDS: where a block stands by itself, the reads of all waves come first (640 clocks for 128x128 in eight waves of
 //     64x32) and the MFMAs, 512 clocks, behind them.  Four waves of 64x64 read two thirds of that, and they read
 //     block kb + 1 into a second set of registers between the MFMAs of block kb, so that a block takes the longer of
@@ -915,19 +915,39 @@ hipError_t launch_typed(const GemmArgs& g, int ksplit, float* partial, float* ma
     return hipGetLastError();
 }
 
-// WMS x WNS: the waves of the form that takes ragged rows and splits K
-template <int BM, int BN, int WM, int WN, int NS, int WMS = WM, int WNS = WN>
+template <int BM, int BN, int WM, int WN, int NS, bool RAGGED_SPLITS = true>
 hipError_t launch_variant(const GemmArgs& g, int ksplit, float* partial, float* mailbox, hipStream_t s)
 {
     if (leading_dim(g) % 16 == 0)
         return ksplit > 1 ? launch_typed<BM, BN, WM, WN, NS, true, false>(g, ksplit, partial, mailbox, s)
                           : launch_typed<BM, BN, WM, WN, NS, false, false>(g, ksplit, partial, mailbox, s);
     if constexpr (tile_takes_ragged_rows(BM, NS)) {
-        if (leading_dim(g) == g.m && g.m >= 16)
-            return ksplit > 1 ? launch_typed<BM, BN, WMS, WNS, NS, true, true>(g, ksplit, partial, mailbox, s)
-                              : launch_typed<BM, BN, WM, WN, NS, false, true>(g, ksplit, partial, mailbox, s);
+        if (leading_dim(g) == g.m && g.m >= 16) {
+            if (ksplit == 1)
+                return launch_typed<BM, BN, WM, WN, NS, false, true>(g, ksplit, partial, mailbox, s);
+            if constexpr (RAGGED_SPLITS)
+                return launch_typed<BM, BN, WM, WN, NS, true, true>(g, ksplit, partial, mailbox, s);
+        }
     }
     return hipErrorInvalidValue;
+}
+
+// Whether 128x128 tiles are multiplied by four waves that read ahead, or by eight.  us by four / by eight:
+//   Ragged rows with K split: eight.  Four of them bring A there, and all take part in the hand-over, which the short chains
+//   of a split do not make up for: 250 x 7168 x 2048 in two splits, B from HBM, 14.1 / 12.9, 2204 x 512 x 7168 in three
+//   23.4 / 22.0, 333 x 4608 x 7168 in two 30.9 / 30.0; unsplit 500 x 4608 x 2048 12.9 / 13.8.
+//   Splits added in the kernel: eight while a split has fewer than 16 K blocks.  752 x 1360 x 1536 in three of four 12.09 /
+//   11.01, 3824 x 272 x 2176 in two of nine 12.40 / 11.68, 1520 x 768 x 3840 in three of ten 14.82 / 13.97, 1376 x 624 x 5760 in
+//   three of 15 18.20 / 17.11 (30 shapes of 4 - 15: eight ahead on 27, by up to 11 %, 2 % behind at worst); from 16 on either
+//   way, 384 x 3456 x 6144 in three of 16 24.75 / 26.12, 1520 x 640 x 6144 17.62 / 16.62, 2048 x 576 x 7168 in three of 19
+//   18.63 / 19.04, 208 x 4352 x 6144 in two of 24 17.14 / 18.53.  With the reduction kernel behind them, which needs no
+//   hand-over, four: 512 x 1024 x 7168 in five 13.99 / 14.77.
+//   A single K block: eight, there is nothing to read ahead of.  5104 x 720 x 128 4.72 / 4.41, 413 x 3824 x 128 4.47 / 4.37; two:
+//   5104 x 720 x 256 5.14 / 5.19.
+bool four_waves(const GemmArgs& g, int ksplit, bool fused)
+{
+    const int kb_per_split = (g.k / KBLOCK + ksplit - 1) / ksplit;
+    return kb_per_split > 1 && (ksplit == 1 || (leading_dim(g) % 16 == 0 && (!fused || kb_per_split >= 16)));
 }
 
 }  // namespace
@@ -993,11 +1013,9 @@ hipError_t launch_tile(const GemmArgs& g, int variant, int ksplit, float* partia
     case TILE_256x192: return launch_variant<256, 192, 4, 2, 2>(g, ksplit, partial, mailbox, s);
     case TILE_256x128: return launch_variant<256, 128, 4, 2, 3>(g, ksplit, partial, mailbox, s);
     case TILE_128x192: return launch_variant<128, 192, 4, 2, 3>(g, ksplit, partial, mailbox, s);
-    // (ragged rows and K split: eight waves multiply.  Four of them bring A there, and all take part in the hand-over,
-    // which the short chains of a split do not make up for: 250 x 7168 x 2048 in two splits, B from HBM, 14.1 us by four
-    // waves and 12.9 by eight, 2204 x 512 x 7168 in three 23.4 and 22.0, 333 x 4608 x 7168 in two 30.9 and 30.0; unsplit
-    // 500 x 4608 x 2048 12.9 and 13.8)
-    case TILE_128x128: return launch_variant<128, 128, 2, 2, 4, 2, 4>(g, ksplit, partial, mailbox, s);
+    case TILE_128x128:
+        return four_waves(g, ksplit, mailbox != nullptr) ? launch_variant<128, 128, 2, 2, 4, false>(g, ksplit, partial, mailbox, s)
+                                                         : launch_variant<128, 128, 2, 4, 4>(g, ksplit, partial, mailbox, s);
     case TILE_64x64: return launch_variant<64, 64, 2, 2, 4>(g, ksplit, partial, mailbox, s);
     default: return hipErrorInvalidValue;
     }

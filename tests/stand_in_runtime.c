@@ -2,8 +2,8 @@
  * takes the decode kernels' entry points through many shapes without a device and prints what the launches asked for:
  * "kernels K raised R again A missing M" -- kernels launched with more than 64 KiB of dynamic LDS, kernels whose limit was
  * raised, times it was raised again for one, launches above their kernel's limit.
- * With arguments "rows n k split groups" (split 0 = automatic; groups 0 = a single problem) only that call, and the mangled
- * names of the kernels that it launches. */
+ * With arguments "rows n k split groups [tile]" (split 0 = automatic; groups 0 = a single problem, by the decode kernels if
+ * split; tile = a tile variant) only that call, and the mangled names of the kernels that it launches. */
 #include <stddef.h>
 #include <stdint.h>
 #include <stdio.h>
@@ -106,11 +106,12 @@ static int grouped(int groups, int m, int first, int n, int k, int split, int od
                                      p, (size_t)1 << 36, 0);
 }
 
-static int one_call(char **word)
+static int one_call(int words, char **word)
 {
     const int m = atoi(word[1]), n = atoi(word[2]), k = atoi(word[3]), split = atoi(word[4]), groups = atoi(word[5]);
-    const fp8gemm_options opt = {split ? FP8GEMM_KERNEL_SKINNY : FP8GEMM_KERNEL_AUTO, split ? 1 : -1, split, -1,
-                                 FP8GEMM_FLAG_WORKSPACE_ZEROED};
+    const int tile = words > 6 ? atoi(word[6]) : -1;
+    const fp8gemm_options opt = {split && tile < 0 ? FP8GEMM_KERNEL_SKINNY : FP8GEMM_KERNEL_AUTO, tile >= 0 ? tile : split ? 1 : -1,
+                                 split, -1, FP8GEMM_FLAG_WORKSPACE_ZEROED};
     /* the first call looks at the placement of workgroups */
     fp8_block_gemm_ex(p, p, p, p, p, 32, 7168, 2048, 0, p, (size_t)1 << 32, 0);
     grouped(2, 16, 0, 7168, 2048, 2, 0);
@@ -121,8 +122,8 @@ static int one_call(char **word)
 
 int main(int argc, char **argv)
 {
-    if (argc == 6)
-        return one_call(argv);
+    if (argc >= 6)
+        return one_call(argc, argv);
     const int rows[] = {1, 8, 15, 16, 24, 31, 32, 40, 47, 48, 56, 63, 64};
     const int ns[] = {128, 1536, 4608, 7152, 7168, 16384, 28672, 33024, 49152, 65536, 65664, 131072};
     const int ks[] = {128, 384, 512, 1024, 2048, 4096, 7168, 8192};

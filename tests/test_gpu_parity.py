@@ -135,6 +135,21 @@ def test_tile_kernel_of_four_waves_chains(pkg, variant, kb):
         assert np.array_equal(got, other), "both tiles fold the same block sums in the same order"
 
 
+# 128x128 tiles with K split: splits added in the kernel are multiplied by eight waves up to 15 K blocks and by four from 16
+# on, splits for the reduction kernel by four; splits of unequal length, a single K block each
+@pytest.mark.parametrize("ksplit,kb", [(2, 2), (3, 3), (2, 5), (2, 29), (2, 30), (2, 31), (2, 33), (3, 47)])
+def test_tile_kernel_128x128_splits_by_four_and_eight_waves(pkg, ksplit, kb):
+    n, k = 272, 128 * kb
+    for m in (304, 299):
+        a, b, sa, sb = oracle.make_inputs(m, n, k, 5 * m + k, 0.5, 30.0)
+        got, name = _run(pkg, a, b, sa, sb, m, n, k, variant=2, ksplit=ksplit, fused=1)
+        assert name == f"tile128x128_k{ksplit}f", name
+        _assert_every_element(got, a, b, sa, sb, m, n, k, name)
+        other, name = _run(pkg, a, b, sa, sb, m, n, k, variant=2, ksplit=ksplit, fused=0)
+        assert name == f"tile128x128_k{ksplit}", name
+        assert np.array_equal(got, other), "both add the same sums in the same order"
+
+
 # persistent form: several tiles per workgroup (more than 256 tiles), ragged edges, K ranges from
 # the shortest the ring allows to many blocks, and a launch with fewer tiles than workgroups
 @pytest.mark.parametrize("variant,m,n,k", [(0, 4096, 3456, 512), (0, 1040, 1232, 256), (0, 4112, 3472, 128),

@@ -1,4 +1,5 @@
-"""What the decode kernels' launches ask for, with stand-ins for the runtime's calls: no device, nothing runs."""
+"""Which kernels calls launch and what the launches ask for, with stand-ins for the runtime's calls: no device, nothing
+runs."""
 import os
 import subprocess
 
@@ -47,3 +48,13 @@ def test_which_b_is_read_past_the_caches(program, m, n, k, past):
                                                      (16, 32, 7168, 2048, 1, True), (2, 16, 1536, 2048, 4, False), (64, 32, 7152, 2048, 1, False)])
 def test_grouped_launches_count_their_workgroups(program, groups, m, n, k, split, past):
     assert reads_past_the_caches(program, m, n, k, split, groups) == past
+
+
+# 128x128 tiles: four waves of 64x64, or eight of 64x32 where the chains are short
+@pytest.mark.parametrize("m,n,k,split,waves", [(1392, 720, 1024, 2, 8), (3824, 272, 2176, 2, 8), (1376, 624, 5760, 3, 8),
+                                               (2048, 576, 7168, 3, 4), (256, 1024, 4096, 2, 4), (253, 1024, 4096, 2, 8),
+                                               (416, 3824, 128, 1, 8), (413, 3824, 128, 1, 8), (416, 3824, 256, 1, 4), (413, 3824, 256, 1, 4),
+                                               (1024, 4096, 2048, 4, 4)])   # the last: more than the mailbox holds, a reduction kernel
+def test_waves_of_128x128_tiles(program, m, n, k, split, waves):
+    names = subprocess.run(["c++filt"], input="\n".join(program(m, n, k, split, 0, 2)), check=True, capture_output=True, text=True).stdout
+    assert f"tile_gemm_kernel<128, 128, 2, {waves // 2}, 4, {'true' if split > 1 else 'false'}, {'true' if m % 16 else 'false'}>" in names, names
