@@ -295,6 +295,10 @@ inline bool persistent_only_auto(int variant) { return variant == TILE_256x256; 
 // with four waves that read ahead, only while the K range is short (4992 x 1664 x 384 10.0 us persistent, 10.2 plain; 4096 x
 // 4096 x 1024 26.2, 26.2; 1664 x 4864 x 1408 18.0, 16.5; 2688 x 3072 x 3840 40.7, 35.3; 1040 x 6912 x 7552 75.9, 64.2; 13
 // more random shapes of K = 2176 ... 6144 all 4 - 16 % faster plain).
+// For 256x192 tiles over more than eight K blocks it pays in a single round too: that kernel's barrier does not hold its
+// MFMAs up (k_tile_large.hip).  Plain / persistent, us: 928 x 8640 x 2048 25.6 / 23.6, 3792 x 3072 x 3072 41.2 / 37.2, 4032 x 2640 x
+// 5120 61.1 / 54.5, 3328 x 2496 x 1536 20.3 / 19.2, 2272 x 2864 x 1152 16.7 / 16.5; eight blocks 4064 x 752 x 1024 14.06 / 14.48,
+// 1264 x 9536 x 1024 18.0 / 17.6, five 2288 x 1520 x 640 10.74 / 11.45.
 void decide_persistent(const GemmArgs& g, Plan& p, const Config& cfg)
 {
     p.persistent = false;
@@ -308,7 +312,7 @@ void decide_persistent(const GemmArgs& g, Plan& p, const Config& cfg)
     int bm, bn;
     tile_variant_dims(p.variant, &bm, &bn);
     const long tiles = (long)((g.m + bm - 1) / bm) * ((g.n + bn - 1) / bn);
-    p.persistent = mode == 1 || (tiles > NUM_CU && (p.variant != TILE_128x128 || g.k < 1024));
+    p.persistent = mode == 1 || (tiles > NUM_CU ? p.variant != TILE_128x128 || g.k < 1024 : p.variant == TILE_256x192 && g.k > 1024);
 }
 
 // Whether a tile plan that splits K adds the partial tiles inside the GEMM kernel (the last workgroup of

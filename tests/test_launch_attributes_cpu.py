@@ -58,3 +58,11 @@ def test_grouped_launches_count_their_workgroups(program, groups, m, n, k, split
 def test_waves_of_128x128_tiles(program, m, n, k, split, waves):
     names = subprocess.run(["c++filt"], input="\n".join(program(m, n, k, split, 0, 2)), check=True, capture_output=True, text=True).stdout
     assert f"tile_gemm_kernel<128, 128, 2, {waves // 2}, 4, {'true' if split > 1 else 'false'}, {'true' if m % 16 else 'false'}>" in names, names
+
+
+# 256x192 tiles in a single round: the persistent kernel over more than eight K blocks, also on padded copies
+@pytest.mark.parametrize("m,n,k,persistent", [(1424, 7168, 2048, True), (2512, 4608, 7168, True), (3608, 3072, 1536, True),
+                                              (2272, 2864, 1152, True), (4064, 752, 1024, False), (2288, 1520, 640, False), (80, 80, 2048, True)])
+def test_256x192_tiles_in_one_round(program, m, n, k, persistent):
+    names = subprocess.run(["c++filt"], input="\n".join(program(m, n, k, 1, 0, 0)), check=True, capture_output=True, text=True).stdout
+    assert ("tile_gemm_large_kernel<192" in names) == persistent and ("tile_gemm_kernel<256, 192" in names) != persistent, names
