@@ -905,10 +905,14 @@ double grouped_tile_cost(const GroupTable& tab, int n, int k, int variant)
     const double area = (double)bm * bn / 65536.0;
     if (variant == TILE_256x256)
         return large_tile_cost(grouped_tiles(tab, n, variant), k, 1.2);
-    const double from_hbm = variant == TILE_256x192 ? 1.43 : bm == 256 ? 1.5 : 1.7;
+    const long tiles = grouped_tiles(tab, n, variant);
+    // (256x192 tiles in a single round, where 256x256 tiles are fewer still: 18 of 20 random launches are 1 - 13 % faster in
+    // the smaller ones and two 1 % slower, 384 - 624 rows, 4960 x 1664, 140 or 182 tiles, 25.3 / 22.3 us, 16 of 96 - 656, 1232 x
+    // 1792, 28.3 / 24.9, six of 80 - 336, 4608 x 7168, 93.1 / 88.3; and fewer of them are too few for one launch, below)
+    const double from_hbm = variant == TILE_256x192 ? (tiles <= NUM_CU ? 1.32 : 1.43) : bm == 256 ? 1.5 : 1.7;
     const double per_kb = (1.19 * area + 0.267) * from_hbm;
     const double per_item = 0.95 + 4.38 * area + (k / 128) * per_kb;
-    const long rounds = (grouped_tiles(tab, n, variant) + NUM_CU - 1) / NUM_CU;
+    const long rounds = (tiles + NUM_CU - 1) / NUM_CU;
     return 1.79 + rounds * per_item;
 }
 

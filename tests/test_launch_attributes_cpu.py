@@ -66,3 +66,13 @@ def test_waves_of_128x128_tiles(program, m, n, k, split, waves):
 def test_256x192_tiles_in_one_round(program, m, n, k, persistent):
     names = subprocess.run(["c++filt"], input="\n".join(program(m, n, k, 1, 0, 0)), check=True, capture_output=True, text=True).stdout
     assert ("tile_gemm_large_kernel<192" in names) == persistent and ("tile_gemm_kernel<256, 192" in names) != persistent, names
+
+
+# tall groups that are a single round of 256x192 tiles: those, in one launch (of 256x256 tiles, 147 would be too few for one);
+# more than a round of them: 256x256
+@pytest.mark.parametrize("groups,m,n,k,columns", [(7, 768, 1664, 2176, 192), (4, 512, 4960, 1664, 192), (8, 512, 3584, 2048, 256)])
+def test_tall_groups_in_one_round(program, groups, m, n, k, columns):
+    names = [name for name in program(m, n, k, 0, groups) if "tile_gemm" in name]
+    assert len(names) == 1, names
+    name = subprocess.run(["c++filt", names[0]], check=True, capture_output=True, text=True).stdout
+    assert f"tile_gemm_large_grouped_kernel<{columns}," in name, name
