@@ -50,14 +50,14 @@ CHALLENGE_REF_GEOMEAN_US = 136.0
 # scaled by what the same counter reads for a 1 GiB copy kernel in the same session: FETCH_SIZE
 # reads 0.5 of the bytes copied (factor 2.0), WRITE_SIZE reads them exactly (factor 1.0).
 # profiles/counters_cfg1_to_cfg5.md holds the table; the kernels measured are those of the commit
-# named here (the kernels of these plans have not changed since).
-TRAFFIC_MEASURED_AT_COMMIT = "4b917b7"
+# named here.
+TRAFFIC_MEASURED_AT_COMMIT = "b744ed8"
 MEASURED_TRAFFIC_BYTES = {
-    "cfg1": int((5243 * 2.0 + 3072 * 1.0) * 1024),       # 13.9 MB: C + the mailbox traffic of the K split
-    "cfg2": int((115833 * 2.0 + 114688 * 1.0) * 1024),   # 355 MB
-    "cfg3": int((28716 * 2.0 + 22239 * 1.0) * 1024),     # 81.6 MB, one kernel (K splits added inside it)
-    "cfg4": int((242079 * 2.0 + 73728 * 1.0) * 1024),    # 571 MB: 8 L2s refetch A/B panels
-    "cfg5": int((8845 * 2.0 + 3136 * 1.0) * 1024),       # 21.3 MB: B once (1.23 x the reads) + mailbox write-back
+    "cfg1": int((5252 * 2.0 + 3072 * 1.0) * 1024),       # 13.9 MB: C + the mailbox traffic of the K split
+    "cfg2": int((96494 * 2.0 + 114759 * 1.0) * 1024),    # 315 MB
+    "cfg3": int((28775 * 2.0 + 22252 * 1.0) * 1024),     # 81.7 MB, one kernel (K splits added inside it)
+    "cfg4": int((242248 * 2.0 + 73746 * 1.0) * 1024),    # 572 MB: 8 L2s refetch A/B panels
+    "cfg5": int((8844 * 2.0 + 3136 * 1.0) * 1024),       # 21.3 MB: B once (1.23 x the reads) + mailbox write-back
 }
 
 

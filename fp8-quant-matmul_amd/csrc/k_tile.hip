@@ -6,7 +6,7 @@
 //     global -> LDS with 16-byte buffer loads that write LDS directly (no VGPR round trip),
 //     keeping the global orientation: one LDS row per k, 128 or 256 bytes per row.  The
 //     16-byte column chunk c of row r is stored at chunk position c ^ swizzle(r), which makes
-//     the transposing reads below bank-conflict free (measured: 0 conflicts).
+//     the transposing reads below bank-conflict free (measured: the conflicts of a launch do not grow with K).
 //   * Operands are fetched with ds_read_b64_tr_b8: 16 lanes read an 8(k) x 16(m|n) byte
 //     patch and receive it transposed, i.e. lane i holds 8 consecutive k of column i.  Four
 //     such reads give the 32 bytes per lane that v_mfma_f32_16x16x128_f8f6f4 consumes.

@@ -20,8 +20,8 @@
 //     is one for the stores (both count in vmcnt, in order; the stores are buffer stores that every wave issues, rows
 //     and columns beyond C addressed outside the buffer, so their number is known).
 //
-// Bound by power on operands that toggle: 8192 x 4096 x 7168 (256 x 256) runs at a clock of 1.98 GHz with the matrix pipes
-// 62 % busy; without its copies it takes 160 us.  Against 32x32x64 MFMAs with the barrier at the block's end and the
+// Bound by power on operands that toggle: 8192 x 4096 x 7168 (256 x 256) runs at a clock of 1.91 GHz with the matrix pipes
+// 65 % busy; without its copies it takes 160 us.  Against 32x32x64 MFMAs with the barrier at the block's end and the
 // tile leaving through a slot: 8192 x 4096 x 7168 212.7 -> 189 us = 51 % of 5033 TFLOP/s; 8192 x 4608 x 7168 (256 x 192) 252.8 ->
 // 239; 8192 x 7168 x 2048 (256 x 192 and 256 x 256) 136.7 -> 129.5 and 123.8 -> 117; 8192 x 7168 x 256 32.8 -> 29; with C's
 // stores past the caches (c_streams) 8192 x 4096 x 7168 180 us = 53 %.
@@ -433,7 +433,7 @@ tile_gemm_large_grouped_kernel(const GroupTable tab, int N, int K, int tiles_n, 
     large_kernel_body<BN, true, TAIL>(none, &tab, N, K, 0, tiles_n, stream_c != 0);
 }
 
-// Whether C leaves with stores that tell the caches not to keep it.  The tiles of a round are stored together, 32 MB in a few
+// Whether C leaves with stores that tell the caches not to keep it (whole tiles; halves and quarters are stored as ever).  The tiles of a round are stored together, 32 MB in a few
 // microseconds, and the lines that the L2s and the Infinity Cache then hold have to leave under the next rounds' reads.
 // Where the launch's data are small enough to stay, so does C.  Kept / not kept, us, three sets of operands in turn,
 // bytes of A, B and C together: 92 MB 8192 x 4096 x 2048 61.1 / 63.2; 108 MB 4608 x 4608 x 7168 139.0 / 137.0; 111 MB 8192 x
