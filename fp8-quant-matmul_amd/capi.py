@@ -222,7 +222,7 @@ def gemm_grouped_ex(a, b, a_scale, b_scale, c, m, n, k, options=None, workspace=
 
 
 def set_persistent(mode=-1):
-    """-1: persistent tile kernel when tiles outnumber the CUs, 0: never, 1: whenever possible"""
+    """-1: persistent tile kernel where it pays (mostly when tiles outnumber the CUs), 0: never, 1: whenever possible"""
     _check(lib().fp8_block_gemm_set_persistent(mode), "fp8_block_gemm_set_persistent")
 
 

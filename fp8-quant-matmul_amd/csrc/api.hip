@@ -22,7 +22,7 @@ constexpr int NUM_CU = 256;
 std::atomic<int> g_selected{FP8GEMM_KERNEL_AUTO};
 std::atomic<int> g_force_variant{-1};
 std::atomic<int> g_force_ksplit{0};
-std::atomic<int> g_persistent{-1};  // -1 = when tiles outnumber the CUs, 0 = never, 1 = whenever possible
+std::atomic<int> g_persistent{-1};  // -1 = where it pays (decide_persistent), 0 = never, 1 = whenever possible
 std::atomic<int> g_fused{-1};       // K splits added inside the GEMM kernel: -1 = by cost, 0 = never, 1 = whenever possible
 thread_local const char* t_last_kernel = "none";
 thread_local char t_name_buf[96];

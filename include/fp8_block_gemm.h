@@ -105,8 +105,8 @@ int fp8_block_gemm_force_config(int tile_variant, int ksplit);
 
 /* The tile kernels have a persistent form (ksplit = 1): 256 workgroups walk through all
  * tiles and copy a tile's first K blocks while the previous tile is stored.  mode -1 = use it
- * when there are more tiles than compute units (default), 0 = never, 1 = whenever the shape
- * allows.  The reference names such a kernel as future work (/root/reference/README.md:29). */
+ * where it pays, mostly when there are more tiles than compute units (default), 0 = never, 1 =
+ * whenever the shape allows.  The reference names such a kernel as future work (/root/reference/README.md:29). */
 int fp8_block_gemm_set_persistent(int mode);
 
 /* Plans that split K ("..._kN") write fp32 partial results; they are added either by a second kernel or

@@ -148,3 +148,28 @@ def test_quantise_then_gemm_graph_replays_equal_eager(pkg):
     ref = oracle.ref_gemm(a, b, sa, sb, m, n, k)
     r = oracle.compare_bf16(eager[2].view(np.uint16), ref, 1e-2, 1e-3)
     assert r["bad"] == 0, r
+
+
+@pytest.mark.parametrize("m,k,ksplit", [(7, 384, 1), (24, 384, 1), (31, 640, 1), (40, 384, 1), (47, 640, 1), (64, 384, 1), (16, 3712, 1)])
+def test_first_launch_of_a_kernel_under_capture(pkg, m, k, ksplit):
+    """a decode kernel whose dynamic-LDS limit nobody has raised yet, first launched into a graph"""
+    import torch
+    n = 528
+    a, b, sa, sb = oracle.make_inputs(m, n, k, 7400 + m)
+    da, db, dsa, dsb = [torch.from_numpy(np.ascontiguousarray(x)).cuda() for x in (a, b, sa, sb)]
+    c0, c1 = [torch.full((m, n), -1, dtype=torch.int16, device="cuda") for _ in range(2)]
+    opt = pkg.Options(pkg.KERNEL_SKINNY, 1, ksplit)
+    _say(f"[gpu case] first launch under capture m={m} n={n} k={k}")
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        pkg.gemm_ex(da, db, dsa, dsb, c0, m, n, k, opt, None, 0, torch.cuda.current_stream().cuda_stream)
+    for rep in range(3):
+        c0.fill_(-1)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        pkg.gemm_ex(da, db, dsa, dsb, c1, m, n, k, opt, None, 0, torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        assert torch.equal(c0, c1), rep
+    ref = oracle.ref_gemm(a, b, sa, sb, m, n, k)
+    assert oracle.compare_bf16(c0.cpu().numpy().view(np.uint16), ref, 1e-2, 1e-3)["bad"] == 0
