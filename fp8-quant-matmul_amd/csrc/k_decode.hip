@@ -865,7 +865,7 @@ inline bool shallow_ring_pays(long workgroups, int kb_per_split) { return workgr
 // Cache, HBM 800 MB of them in turn (graphs of 48 and more launches, medians of nine):
 //                                  alone          in turn        HBM
 //   16 x 7168 x 2048 (15 MB)     4.10 /  4.10   5.62 /  5.84   6.05 /  5.94   three in turn, more than the L2s hold, 5.58 / 5.37
-//   32 x 7168 x 2048             5.16 /  5.16   6.66 /  6.79   6.92 /  6.85   (alone 5.48 on other boxes; three 6.46 / 6.44)
+//   32 x 7168 x 2048             5.16 /  5.16   6.66 /  6.79   6.92 /  6.85   (alone 5.48 on other machines; three 6.46 / 6.44)
 //   16 x 10240 x 2048 (21 MB)    4.59 /  4.59   6.78 /  7.31   7.68 /  7.56
 //   32 x 9216 x 3072 (28 MB)     6.94 /  7.75   8.46 /  9.13   9.75 /  9.46
 //   24 x 4608 x 7168 (33 MB)     9.74 / 10.08  10.54 / 10.83  11.56 / 11.10
