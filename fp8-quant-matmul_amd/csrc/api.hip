@@ -37,6 +37,7 @@ struct Config {
     // and the device places workgroups on XCDs as those kernels assume (set by run())
     bool fused_ok = true;
     int fused_mode = -1;  // -1 = by cost, 0 = never, 1 = whenever fused_ok and the plan allows
+    bool strips_for_tiles = true;  // 64-column strips may take the place of 64x64 tiles (strips_for_tiles below)
 };
 Config global_config()
 {
@@ -98,7 +99,7 @@ struct Plan {
     bool padded = false;      // the plan is for the problem with m and n rounded up to 16 (run_padded)
     bool wide = false;        // decode family: 128-column strips, K splits added inside the kernel (k_decode.hip)
     bool fused = false;       // tile family, ksplit > 1: the last workgroup of a tile adds the partial tiles (no reduction launch)
-    int halves = 1;           // wide decode strips: 128-column halves per strip (2 = 256-column strips)
+    int halves = 1;           // wide decode strips: 128-column halves per strip (2 = 256-column strips, 0 = 64-column ones)
 };
 
 // Shapes or addresses the MFMA kernels cannot take (m or n not a multiple of 16, a base not
@@ -332,12 +333,12 @@ struct PlanKey {
     int m, n, k, lda;
     uint32_t low_bits;  // 6 low address bits of a, b, a_scale, b_scale and c
     int selected, force_variant, force_ksplit, persistent, fused_mode;
-    int fused_ok;
+    int allowed;  // bit 0: fused_ok, bit 1: strips_for_tiles
     bool operator==(const PlanKey& o) const
     {
         return m == o.m && n == o.n && k == o.k && lda == o.lda && low_bits == o.low_bits && selected == o.selected &&
                force_variant == o.force_variant && force_ksplit == o.force_ksplit && persistent == o.persistent &&
-               fused_mode == o.fused_mode && fused_ok == o.fused_ok;
+               fused_mode == o.fused_mode && allowed == o.allowed;
     }
 };
 struct PlanSlot {
@@ -351,7 +352,8 @@ Plan make_plan(const GemmArgs& g, const Config& cfg)
     auto low6 = [](const void* p) { return (uint32_t)(reinterpret_cast<uintptr_t>(p) & 63); };
     const PlanKey key{g.m, g.n, g.k, g.lda,
                       low6(g.a) | low6(g.b) << 6 | low6(g.a_scale) << 12 | low6(g.b_scale) << 18 | low6(g.c) << 24,
-                      cfg.selected, cfg.force_variant, cfg.force_ksplit, cfg.persistent, cfg.fused_mode, cfg.fused_ok ? 1 : 0};
+                      cfg.selected, cfg.force_variant, cfg.force_ksplit, cfg.persistent, cfg.fused_mode,
+                      (cfg.fused_ok ? 1 : 0) | (cfg.strips_for_tiles ? 2 : 0)};
     const uint32_t h = ((uint32_t)g.m * 2654435761u) ^ ((uint32_t)g.n * 40503u) ^ ((uint32_t)g.k * 2246822519u) ^
                        (cfg.fused_ok ? 0x9E3779B9u : 0u);
     PlanSlot& slot = slots[(h >> 16 ^ h) & 63];
@@ -383,6 +385,25 @@ Plan off_grid_plan(const GemmArgs& g, const Config& cfg)
     return p;
 }
 
+// 33 ... 56 rows, multiples of 8, over weights that want five splits or more of 64x64 tiles: the 64-column strips, whose stages
+// are shorter (a fragment of B is read once for all row tiles), in their own number of splits.  16 random problems, from
+// the Infinity Cache / from HBM: 8 / 9 % faster on average, 4 - 16 % (48 x 1232 x 1920 6.2 -> 5.4, 48 x 1536 x 7168 9.0 -> 8.3 /
+// 10.0 -> 9.4).  Left with the tiles: rows that are spread (36 x 576 x 7168 8.2 -> 8.7, 45 x 576 x 1792 5.95 -> 5.62), 57 rows and
+// more (64 x 2464 x 4736 8.2 -> 9.4 / 9.5 -> 9.8, 64 x 1680 x 2560 level) and fewer splits (one to three 2 - 20 % slower).
+Plan strips_for_tiles(const GemmArgs& g, const Plan& tiles)
+{
+    if (tiles.variant != TILE_64x64 || !tiles.fused || g.m <= 32 || g.m > 56 || leading_dim(g) % 8 != 0 || tiles.ksplit < 5 ||
+        !decode_strip_supports(g))
+        return tiles;
+    const int ks = decode64_ksplit(g);
+    if (ks <= 1)
+        return tiles;
+    Plan strips{FP8GEMM_KERNEL_SKINNY, 0, ks};
+    strips.wide = true;
+    strips.halves = 0;
+    return strips;
+}
+
 Plan compute_plan(const GemmArgs& g, const Config& cfg)
 {
     const int selected = cfg.selected;
@@ -391,7 +412,7 @@ Plan compute_plan(const GemmArgs& g, const Config& cfg)
         return p;
     // The decode kernels (M <= 32): narrow strips (k_skinny.hip) or wide strips whose K splits are added
     // inside the kernel (k_decode.hip), whichever the cost model prefers; with the family asked for by name,
-    // tile_variant 0 / 1 pins the narrow / wide form.  Under automatic dispatch the family has to hold its own
+    // tile_variant 0 / 1 / 2 / 3 pins the narrow strips / the wide ones of 128, 256, 64 columns.  Under automatic dispatch the family has to hold its own
     // against the best tile plan by cost: with a long K range and many column strips 64x64 tiles with the K
     // range split are faster than the narrow kernel (measured: 12-14 us against 15-20 us for M = 16 / 32,
     // N >= 4608, K = 7168).
@@ -415,6 +436,21 @@ Plan compute_plan(const GemmArgs& g, const Config& cfg)
         double narrow_us = 1e300, wide_us = 1e300;
         Plan narrow = decode, wide = decode;
         wide.wide = true;
+        auto strips64 = [&](int ksplit) {
+            Plan strips = wide;
+            strips.ksplit = ksplit;
+            strips.halves = 0;
+            return strips;
+        };
+        if (by_name && cfg.force_variant == 3 && wide_ok) {  // pins the 64-column strips
+            const int ks = forced_ks ? forced_ks : cfg.fused_ok ? decode64_ksplit(g) : 1;
+            if (ks <= 1)
+                return strips64(1);
+            if (ks <= MAX_KSPLIT && cfg.fused_ok && decode_strip_can_split(g, ks, 0))
+                return strips64(ks);
+            p.family = -1;
+            return p;
+        }
         if (narrow_ok && !(by_name && cfg.force_variant >= 1)) {
             narrow.ksplit = forced_ks ? forced_ks : skinny_ksplit(g);
             narrow_us = skinny_cost(g, narrow.ksplit);
@@ -467,14 +503,18 @@ Plan compute_plan(const GemmArgs& g, const Config& cfg)
         // average and 21 % at worst.  No tiles that need padded copies (12 shapes: 6.8 - 16.9 us against 10.8 - 23.8 us).
         if (!by_name && g.m > 32 && g.m % 16 != 0 && b_bytes < 16000000ll && cfg.force_variant < 0 &&
             cfg.force_ksplit <= 0 && cfg.fused_ok) {
-            const Plan tiles = off_grid_plan(g, cfg);
+            Config tiles_cfg = cfg;
+            tiles_cfg.strips_for_tiles = false;  // decided below for the rows as they are
+            const Plan tiles = off_grid_plan(g, tiles_cfg);
             const bool header_only = tiles.ksplit == 1 || tiles.fused;  // as the strips: no partial sums in the workspace
             if (!tiles.padded && header_only && (tiles.family == FP8GEMM_KERNEL_LARGE || tiles.family == FP8GEMM_KERNEL_SPLITK))
-                return tiles;
+                return strips_for_tiles(g, tiles);
         }
 
-        if (!by_name && cfg.force_variant < 0 && cfg.force_ksplit <= 0 && wide_us < 1e300 && cfg.fused_ok)
-            return wide;
+        if (!by_name && cfg.force_variant < 0 && cfg.force_ksplit <= 0 && wide_us < 1e300 && cfg.fused_ok) {
+            const int ks = wide.halves == 1 ? decode64_ksplit(g) : 0;
+            return decode64_pays(g, ks, wide.ksplit) ? strips64(ks) : wide;
+        }
         if (!by_name && !cfg.fused_ok)
             wide_us = 1e300;  // unsplit wide strips leave most CUs idle: the narrow kernel and the tile plans compete
         if (narrow_us == 1e300 && wide_us == 1e300) {
@@ -595,6 +635,8 @@ Plan compute_plan(const GemmArgs& g, const Config& cfg)
     decide_fused(g, p, cfg);
     if (persistent_only(p.variant) && !p.persistent)
         p.family = -1;
+    if (cfg.strips_for_tiles && selected == FP8GEMM_KERNEL_AUTO && fv < 0 && fk <= 0)
+        return strips_for_tiles(g, p);
     return p;
 }
 
@@ -690,7 +732,7 @@ void plan_name(const Plan& p, char* out, size_t cap)
     if (p.family == FP8GEMM_KERNEL_SCALAR)
         snprintf(out, cap, "scalar");
     else if (p.family == FP8GEMM_KERNEL_SKINNY)
-        snprintf(out, cap, p.wide ? (p.halves == 2 ? "%sdecode256_k%d" : "%sdecode128_k%d") : "%sskinny_k%d", pre, p.ksplit);
+        snprintf(out, cap, p.wide ? (p.halves == 2 ? "%sdecode256_k%d" : p.halves == 0 ? "%sdecode64_k%d" : "%sdecode128_k%d") : "%sskinny_k%d", pre, p.ksplit);
     else
         snprintf(out, cap, "%s%s_k%d%s", pre, tile_variant_name(p.variant), p.ksplit,
                  p.persistent ? "_persistent" : (p.fused ? "f" : ""));

@@ -934,6 +934,8 @@ size_t decode_strip_mailbox_bytes(const GemmArgs& g, int ksplit, int halves)
 {
     if (ksplit <= 1)
         return 0;
+    if (halves == 0)
+        return decode64_mailbox_bytes(g, ksplit);
     const size_t strips = (size_t)(g.n + DS_BN * halves - 1) / (DS_BN * halves);
     return strips * (size_t)(ksplit - 1) * 8 * halves * row_tiles(g.m) * 64 * 16;
 }
@@ -1011,6 +1013,8 @@ int xcd_placement_confirmed(bool may_probe)
 
 hipError_t launch_decode_strips(const GemmArgs& g, int ksplit, int halves, float* mailbox, hipStream_t s)
 {
+    if (halves == 0)
+        return launch_decode64(g, ksplit, mailbox, s);
     if (halves != 1 && halves != 2)
         return hipErrorInvalidValue;
     const int strips = (g.n + DS_BN * halves - 1) / (DS_BN * halves);

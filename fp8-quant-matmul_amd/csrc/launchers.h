@@ -117,11 +117,17 @@ hipError_t launch_skinny(const GemmArgs& g, int ksplit, float* partial, hipStrea
 // decode_strip_can_split.
 constexpr int DECODE_MAX_KSPLIT = 16;
 bool decode_strip_supports(const GemmArgs& g);
-// halves = 128-column halves of a strip: 1, or 2 (256-column strips: 256 contiguous bytes of every k-row of B)
+// halves = 128-column halves of a strip: 1, or 2 (256-column strips: 256 contiguous bytes of every k-row of B), or 0: strips
+// of 64 columns (k_decode64.hip)
 size_t decode_strip_mailbox_bytes(const GemmArgs& g, int ksplit, int halves = 1);
 bool decode_strip_can_split(const GemmArgs& g, int ksplit, int halves = 1);
 double decode_strip_cost(const GemmArgs& g, int ksplit, int halves = 1);
 hipError_t launch_decode_strips(const GemmArgs& g, int ksplit, int halves, float* mailbox, hipStream_t s);
+// ... in strips of 64 columns (called by the functions above for halves = 0)
+size_t decode64_mailbox_bytes(const GemmArgs& g, int ksplit);
+int decode64_ksplit(const GemmArgs& g);  // the split that it would run with; 0: more strips than the device holds at once
+bool decode64_pays(const GemmArgs& g, int ksplit, int ksplit128);  // against 128-column strips in ksplit128 splits
+hipError_t launch_decode64(const GemmArgs& g, int ksplit, float* mailbox, hipStream_t s);
 // The same kernel on several problems with common n and k and their own m <= 64 (multiples of 16), whose
 // strips form one list of work items; tile_start of the table is not used.
 bool decode_grouped_supports(const GroupTable& tab, int n, int k);
