@@ -67,6 +67,17 @@ __device__ __forceinline__ float value(const uint32_t (&w)[8])
     return __uint_as_float(w[J]);
 }
 
+template <int J>
+__device__ __forceinline__ float pair_value(const uint32_t (&w)[1])
+{
+    return __uint_as_float(J ? w[0] & 0xFFFF0000u : w[0] << 16);
+}
+template <int J>
+__device__ __forceinline__ float pair_value(const uint32_t (&w)[2])
+{
+    return __uint_as_float(w[J]);
+}
+
 template <bool BF16MATH>
 __device__ __forceinline__ float q_round(float v)
 {
@@ -97,6 +108,13 @@ template <int J>
 __device__ __forceinline__ float quad_lane(float v)
 {
     return __uint_as_float((uint32_t)__builtin_amdgcn_mov_dpp((int)__float_as_uint(v), J * 0x55, 0xF, 0xF, true));
+}
+
+// v of lane l ^ X of the same group of four
+template <int X>
+__device__ __forceinline__ float quad_swap(float v)
+{
+    return __uint_as_float((uint32_t)__builtin_amdgcn_mov_dpp((int)__float_as_uint(v), X == 1 ? 0xB1 : 0x4E, 0xF, 0xF, true));
 }
 
 __device__ __forceinline__ float row_max(float a)
@@ -140,9 +158,6 @@ quantize_kernel(const TIn* __restrict__ x, uint8_t* __restrict__ q, float* __res
     const int g = lane >> 4;   // four rows
     const int row0 = blockIdx.x * QTILE;
     const int kb = blockIdx.y;
-    // One tile holds all rows (a decode batch): the K block's output, [128][rows] bytes, is one contiguous piece of
-    // memory.  The tile is kept packed like it in the LDS and leaves as it lies.
-    const bool packed = QTILE <= 64 && rows <= QTILE && grid == 0 && (reinterpret_cast<uintptr_t>(q) & 15) == 0;
 
     // rows past the last are read as the last one: no branch around a load, all of them are in flight together (they
     // do not change the block's amax, and their bytes are not stored)
@@ -200,15 +215,7 @@ quantize_kernel(const TIn* __restrict__ x, uint8_t* __restrict__ q, float* __res
         int w = q_pair<BF16MATH, false>(value<j>(raw[0]) * scale[0], value<j>(raw[1]) * scale[1], 0);
         w = q_pair<BF16MATH, true>(value<j>(raw[2]) * scale[2], value<j>(raw[3]) * scale[3], w);
         const int k = 8 * c + j;
-        if (packed) {
-            const int r = 16 * wave + 4 * g;
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                if (r + i < rows)
-                    tile[k * rows + r + i] = (uint8_t)((uint32_t)w >> (8 * i));
-        } else {
-            *reinterpret_cast<int*>(tile + k * STRIDE + ((wave ^ ((k >> KSH) & (CH - 1))) << 4) + 4 * g) = w;
-        }
+        *reinterpret_cast<int*>(tile + k * STRIDE + ((wave ^ ((k >> KSH) & (CH - 1))) << 4) + 4 * g) = w;
     };
     put(Index<0>{});
     put(Index<1>{});
@@ -220,25 +227,54 @@ quantize_kernel(const TIn* __restrict__ x, uint8_t* __restrict__ q, float* __res
     put(Index<7>{});
     __syncthreads();
 
-    if (packed) {
-        for (int idx = t; idx < 8 * rows; idx += NT)
-            reinterpret_cast<uint4*>(q + (size_t)kb * 128 * rows)[idx] = reinterpret_cast<const uint4*>(tile)[idx];
-        return;
-    }
-
-    // k-row kk of the tile: QTILE bytes, one per source row
-    if (grid == 16) {  // every k-row starts on a 16-byte boundary: a lane takes 16 of its bytes
-        const int dq = t % CH, first = row0 + 16 * dq;
+    // k-row kk of the tile: QTILE bytes, one per source row; a lane takes 16 of them
+    const int dq = t % CH, first = row0 + 16 * dq;
+    auto piece = [&](int kk) __attribute__((always_inline)) { return tile + kk * STRIDE + ((dq ^ ((kk >> KSH) & (CH - 1))) << 4); };
+    if (grid == 16) {  // every k-row starts on a 16-byte boundary
 #pragma unroll
         for (int pass = 0; pass < 128 * CH / NT; ++pass) {
             const int kk = t / CH + (NT / CH) * pass;
-            const uint4 v = *reinterpret_cast<const uint4*>(tile + kk * STRIDE + ((dq ^ ((kk >> KSH) & (CH - 1))) << 4));
+            const uint4 v = *reinterpret_cast<const uint4*>(piece(kk));
             if (first < rows)
                 *reinterpret_cast<uint4*>(q + (size_t)(kb * 128 + kk) * rows + first) = v;
         }
         return;
     }
-    if (grid == 8) {  // the same in pieces of 8 bytes
+    // The small tiles: the same, since a store takes any address, and of a row's last bytes what there is.  Where the memory
+    // system is not what bounds the launch that is the shortest way (128 rows of a tile, shifted into aligned pieces as
+    // below / this, bf16 from the Infinity Cache: 100 x 7168 4.18 / 2.95 us, 333 x 2048 4.29 / 3.07, 1023 x 7168 8.48 / 7.14,
+    // blocks of 4607 x 7168 27.1 / 24.7; 256 rows: 4095 x 7168 22.3 / 23.6, fp32 34.6 / 38.5).
+    if (QTILE != 256) {
+#pragma unroll
+        for (int pass = 0; pass < 128 * CH / NT; ++pass) {
+            const int kk = t / CH + (NT / CH) * pass;
+            const uint8_t* const from = piece(kk);
+            uint8_t* const to = q + (size_t)(kb * 128 + kk) * rows + first;
+            if (first + 16 <= rows) {
+                const uint4 v = *reinterpret_cast<const uint4*>(from);
+                __builtin_memcpy(to, &v, 16);
+            } else if (first < rows) {
+                const int left = rows - first;
+                int at = 0;
+                if (left & 8) {
+                    __builtin_memcpy(to, __builtin_assume_aligned(from, 8), 8);
+                    at = 8;
+                }
+                if (left & 4) {
+                    __builtin_memcpy(to + at, __builtin_assume_aligned(from + at, 4), 4);
+                    at += 4;
+                }
+                if (left & 2) {
+                    __builtin_memcpy(to + at, __builtin_assume_aligned(from + at, 2), 2);
+                    at += 2;
+                }
+                if (left & 1)
+                    to[at] = from[at];
+            }
+        }
+        return;
+    }
+    if (grid == 8) {  // in pieces of 8 bytes
 #pragma unroll 4
         for (int idx = t; idx < 128 * 2 * CH; idx += NT) {
             const int kk = idx / (2 * CH), h = idx % (2 * CH), first = row0 + 8 * h;
@@ -286,6 +322,73 @@ quantize_kernel(const TIn* __restrict__ x, uint8_t* __restrict__ q, float* __res
     }
 }
 
+// 1 x 128 groups of a decode batch, up to 4 * NW <= 64 rows: a workgroup owns a K block of all of them, whose output, [128][rows]
+// bytes, is one contiguous piece of memory (q on a 16-byte boundary).  Bound by a chain, launch, load, arithmetic, store, of which
+// only the arithmetic can be shortened: a wave takes four rows, a lane two k of each (the tile kernel's lanes: eight), and the
+// condition for the rows that do not exist is the wave's, so that no lane is masked.  The four bytes of one k leave the
+// conversion as a dword again; the 16-byte pieces of the output are permuted in the LDS, low four bits of a piece's number
+// by the next four, which spreads the lanes' writes, rows bytes apart, over 16 banks.
+template <typename TIn, bool BF16MATH, int NW>
+__global__ void __launch_bounds__(64 * NW)
+quantize_batch_kernel(const TIn* __restrict__ x, uint8_t* __restrict__ q, float* __restrict__ scale_out, int rows, int K)
+{
+    __shared__ __attribute__((aligned(16))) uint8_t tile[128 * 4 * NW];
+    const int t = threadIdx.x;
+    const int lane = t & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int kb = blockIdx.x;
+    const int row0 = 4 * wave;
+    if (row0 < rows) {
+        constexpr int WORDS = sizeof(TIn) / 2;  // of two values
+        uint32_t raw[4][WORDS];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {  // rows past the last are read as the last one, and their bytes are not stored
+            const int row = row0 + i < rows ? row0 + i : rows - 1;
+            __builtin_memcpy(raw[i], x + (size_t)row * K + (size_t)kb * 128 + 2 * lane, sizeof(raw[i]));
+        }
+        float v[4][2], amax[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            v[i][0] = pair_value<0>(raw[i]);
+            v[i][1] = pair_value<1>(raw[i]);
+            amax[i] = fmaxf(fmaxf(__builtin_fabsf(v[i][0]), __builtin_fabsf(v[i][1])), 0.0f);  // a group of NaNs has amax 0
+        }
+        // lane l ends with the maximum of row l & 3: two exchanges that halve the rows, then over the 16 lanes that have it
+        const bool odd = lane & 1, high = lane & 2;
+        const float lo = fmaxf(odd ? amax[1] : amax[0], quad_swap<1>(odd ? amax[0] : amax[1]));
+        const float hi = fmaxf(odd ? amax[3] : amax[2], quad_swap<1>(odd ? amax[2] : amax[3]));
+        float a = fmaxf(high ? hi : lo, quad_swap<2>(high ? lo : hi));
+        a = fmaxf(a, row_rotate<4>(a));
+        a = fmaxf(a, row_rotate<8>(a));
+        const auto p16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(a), false, false);
+        a = fmaxf(__uint_as_float(p16[0]), __uint_as_float(p16[1]));
+        const auto p32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(a), false, false);
+        a = fmaxf(__uint_as_float(p32[0]), __uint_as_float(p32[1]));
+        const float mine = scale_of<BF16MATH>(a);
+        const float scale[4] = {quad_lane<0>(mine), quad_lane<1>(mine), quad_lane<2>(mine), quad_lane<3>(mine)};
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            int w = q_pair<BF16MATH, false>(v[0][j] * scale[0], v[1][j] * scale[1], 0);
+            w = q_pair<BF16MATH, true>(v[2][j] * scale[2], v[3][j] * scale[3], w);
+            const int at = (2 * lane + j) * rows + row0;  // in the packed block
+            auto place = [](int byte) { return byte ^ ((byte >> 4) & 0xF0); };
+            if ((rows & 3) == 0) {
+                *reinterpret_cast<int*>(tile + place(at)) = w;
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (row0 + i < rows)
+                        tile[place(at + i)] = (uint8_t)((uint32_t)w >> (8 * i));
+            }
+        }
+        if (lane < 4 && row0 + lane < rows)
+            scale_out[(size_t)kb * rows + row0 + lane] = 1.0f / mine;
+    }
+    __syncthreads();
+    for (int idx = t; idx < 8 * rows; idx += 64 * NW)
+        reinterpret_cast<uint4*>(q + (size_t)kb * 128 * rows)[idx] = reinterpret_cast<const uint4*>(tile)[idx ^ ((idx >> 4) & 15)];
+}
+
 // the boundary that every k-row of the output starts on, if that is one of 16 or 8 bytes, else 0
 int output_grid(const uint8_t* q, int rows)
 {
@@ -301,19 +404,24 @@ void launch_quantize_tile(const TIn* x, uint8_t* q, float* scale_out, int rows, 
                        dim3(QTILE * 4), 0, s, x, q, scale_out, rows, k, grid);
 }
 
+template <typename TIn, bool BF16MATH, int NW>
+void launch_quantize_batch(const TIn* x, uint8_t* q, float* scale_out, int rows, int k, hipStream_t s)
+{
+    hipLaunchKernelGGL((quantize_batch_kernel<TIn, BF16MATH, NW>), dim3(k / 128), dim3(64 * NW), 0, s, x, q, scale_out, rows, k);
+}
+
 // Tile sizes, measured with every operand from HBM (us, previous kernel -> this one):
 //   128 x 128 blocks: 128 rows, eight waves of 16, whatever the size (512 x 2048 6.5 -> 3.5, 4608 x 7168 28.8 -> 22.0 =
 //   4.5 TB/s; 256-row tiles 4.5 and 23.3).
-//   1 x 128 groups, up to 64 rows: a decode batch is launch and latency.  One wave per 16 rows up to 32 rows on a
-//   16- or 8-byte grid or 16 off them (16 rows 3.8 -> 2.5, 64-row tiles 3.1), else 64-row tiles (24 rows in
-//   one of them 3.9 -> 3.2, 64 rows 4.5 -> 2.9).
+//   1 x 128 groups, up to 64 rows: quantize_batch_kernel (previous forms -> it, from the Infinity Cache, in a graph whose empty kernel
+//   takes 1.83: 1 x 7168 3.15 -> 2.12, 16 x 7168 2.48 -> 2.13, 24 x 7168 2.77 -> 2.21, 31 x 7168 3.19 -> 2.34, 50 x 7168 3.27 -> 2.68,
+//   64 x 7168 2.83 -> 2.55; fp32 the same to 0.05).  Its way of taking 65 rows and more, two passes over 128: 100 x 7168 3.37 against 2.92
+//   in tiles of 64.
 //   More rows: 256-row tiles once they make 256 workgroups, whose k-rows leave in pieces of 256 bytes (8192 x 7168
-//   46.3 -> 37.1 = 4.7 TB/s, 8191 x 7168 75 -> 48.6 against 54.1 with 128 rows).  Fewer than that, on the grid: 64 rows
-//   up to 1024 tiles (1024 x 2048 5.7 -> 3.8, with 128 rows 4.2), else 128; off the grid 128 rows, which have fewer
-//   ends of segments to store byte by byte (333 x 7168 8.1 -> 6.1, with 64 rows 7.5).
-//   Multiples of 8 rows leave in 8-byte stores, without the shifting and the single bytes, and count as on the grid
-//   (with the GEMM behind it: 24 x 512 x 7168 10.43 -> 10.09, 200 x 512 x 7168 13.84 -> 13.25, 1032 x 512 x 7168 25.97 ->
-//   24.13, 8184 x 1536 x 2048 46.4 -> 45.3; 24 rows of fp32 10.52 -> 10.04).
+//   46.3 -> 37.1 = 4.7 TB/s, 8191 x 7168 75 -> 48.6 against 54.1 with 128 rows).  Fewer than that: 64 rows
+//   up to 1024 tiles (1024 x 2048 5.7 -> 3.8, with 128 rows 4.2), off the grid up to 384 (128 / 64 rows: 130 x 512 3.59 / 2.94, 333 x
+//   2048 3.78 / 3.21, 777 x 2048 4.03 / 3.68, 333 x 7168, 336 tiles, 4.62 / 4.60, 500 x 7168, 448, 4.79 / 4.98, fp32 1023 x 7168 10.9 /
+//   14.3), else 128.  Multiples of 8 rows count as on the grid (8184 x 1536 x 2048 with its GEMM 46.4 -> 45.3).
 //   Values and codes of 115 MB or more together, nearly half of the Infinity Cache, do not stay there beside whatever else
 //   runs: the values are read past it (kept / not kept, us, three sets in turn, 1 x 128 with the GEMM behind it: bf16 129 MB
 //   6000 x 1536 x 7168 114.5 / 100.8, 176 MB 8192 x 512 x 7168 71.7 / 65.5; blocks of bf16 99 MB 4608 x 7168 17.88 / 18.17,
@@ -332,9 +440,11 @@ void launch_quantize_typed(const TIn* x, uint8_t* q, float* scale_out, int rows,
         launch_quantize_tile<TIn, true, BF16MATH, 128, true>(x, q, scale_out, rows, k, s);
     else if (block128)
         launch_quantize_tile<TIn, true, BF16MATH, 128>(x, q, scale_out, rows, k, s);
-    else if (rows <= (on_grid ? 32 : 16))
-        launch_quantize_tile<TIn, false, BF16MATH, 16>(x, q, scale_out, rows, k, s);
-    else if (rows <= 64 || (on_grid && tiles(64) <= 1024))
+    else if (rows <= 64 && reinterpret_cast<uintptr_t>(q) % 16 == 0)
+        rows <= 16   ? launch_quantize_batch<TIn, BF16MATH, 4>(x, q, scale_out, rows, k, s)
+        : rows <= 32 ? launch_quantize_batch<TIn, BF16MATH, 8>(x, q, scale_out, rows, k, s)
+                     : launch_quantize_batch<TIn, BF16MATH, 16>(x, q, scale_out, rows, k, s);
+    else if (rows <= 64 || tiles(64) <= (on_grid ? 1024 : 384))
         launch_quantize_tile<TIn, false, BF16MATH, 64>(x, q, scale_out, rows, k, s);
     else if (tiles(256) < 256)
         launch_quantize_tile<TIn, false, BF16MATH, 128>(x, q, scale_out, rows, k, s);
