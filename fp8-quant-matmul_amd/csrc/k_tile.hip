@@ -640,13 +640,15 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
     // split -- the workgroup with the highest id of its tile, dispatched after the others -- load the other
     // splits' patches past their L1 until no word is zero, add them in split order, their own registers last (the
     // arithmetic of splitk_reduce_kernel: adding -0.0 changes nothing), the workgroup leaves through the bf16
-    // epilogue, and zeros go back into the mailbox behind it (in front of it, the epilogue's first barrier waits until
-    // they are acknowledged).  A wave that has polled for a second gives up and
+    // epilogue, and zeros go back into the mailbox: behind it where all waves write C (in front of it, its first barrier
+    // would wait until they are acknowledged), else beside it.  A wave that has polled for a second gives up and
     // writes NaN.
     bool as_partial = SPLIT;
     constexpr int PATCHES = NCW * MI * NJ;  // 16x16 patches of a tile: 1 KiB of fp32 each
     const int senders = (int)gridDim.y - 1;
-    const size_t first = ((size_t)pid * senders * PATCHES + (size_t)wave * (MI * NJ)) * 64;  // in 16-byte units
+    const size_t first = ((size_t)pid * senders * PATCHES + (size_t)(wave & (NCW - 1)) * (MI * NJ)) * 64;  // in 16-byte units
+    constexpr uint32_t SUMS_OFF = BM * (BN * 2 + 16);  // behind the tile's bf16 rows (below)
+    static_assert(!AHEAD || SUMS_OFF + 4 * (MI * NJ / 2) * 1024 <= S::LDS_BYTES, "sums behind the rows");
     const uint32_t mail_span = (uint32_t)senders * PATCHES * 1024u;
     auto mail_at = [&](int z, int patch) __attribute__((always_inline)) {
         return (uint32_t)((z * PATCHES + patch) * 64 + lane) * 16u;
@@ -670,65 +672,85 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
                 }
                 return;
             }
-            if (compute) {
-                // PG patches at a time (all of them when there are at most eight: one trip to the L2 for everything that
-                // is there), ZB splits at a time.  Of sixteen in four waves, eight: 333 x 4608 x 7168 in two splits 24.3 us four
-                // at a time, 23.9 eight, 24.2 sixteen; 777 x 2048 x 4096 18.4, 17.9, 18.2.
-                constexpr int PG = MI * NJ <= 8 ? MI * NJ : AHEAD ? 8 : 4, ZB = MI * NJ <= 4 ? 3 : 2;
-                static_assert(MI * NJ % PG == 0, "whole groups of patches");
-                const __amdgpu_buffer_rsrc_t rp = make_rsrc(reinterpret_cast<const v4i*>(mailbox) + first, mail_span);
-                const unsigned long long t_first = __builtin_amdgcn_s_memrealtime();
-                bool gave_up = false;
+            // Who gathers.  The hand-over is bound by what one workgroup keeps in flight to the L2: where four waves multiply,
+            // the other four, idle since their last copy, take the second half of the patches of one of them each, hand
+            // the sums over through the LDS (no wave needs a fragment from it behind the last block's barrier, nor the
+            // scales) and put the zeros back while C is written.  By the four that multiply / by all eight: 64x64 tiles
+            // 64 x 1536 x 7168 in eight 9.19 / 8.29 us, 96 x 576 x 7168 in seven 8.16 / 7.40, 48 x 3136 x 1664 in four 5.53 /
+            // 5.09, 304 x 1536 x 7168 in two 14.39 / 14.16; 128x128 2464 x 512 x 7168 in three 19.35 / 18.85, 384 x 4608 x 7168 in two
+            // 19.67 / 19.41.
+            // PG patches at a time (all of them when there are at most eight: one trip to the L2 for everything that
+            // is there), ZB splits at a time.  Two patches a wave: three splits or four alike, two 1.3 % and seven 1.2 %
+            // behind (60 and 44 shapes).
+            constexpr int MINE = AHEAD ? MI * NJ / 2 : MI * NJ;  // patches that a wave gathers
+            constexpr int PG = MINE <= 8 ? MINE : 4, ZB = MINE <= 4 ? 3 : 2;
+            static_assert(MINE % PG == 0, "whole groups of patches");
+            const int part = AHEAD && !compute ? MINE : 0;  // its first patch
+            const __amdgpu_buffer_rsrc_t rp = make_rsrc(reinterpret_cast<const v4i*>(mailbox) + first, mail_span);
+            const unsigned long long t_first = __builtin_amdgcn_s_memrealtime();
+            bool gave_up = false;
 #pragma unroll
-                for (int pg = 0; pg < MI * NJ; pg += PG) {
-                    v4f sum[PG];
-                    auto gather = [&](auto count, int z0) __attribute__((always_inline)) {  // splits z0 .. z0 + ZC - 1
-                        constexpr int ZC = decltype(count)::value;
-                        v4i v[ZC][PG];
-                        for (;;) {
-                            asm volatile("" ::: "memory");  // the loads belong to this round of the loop
-#pragma unroll
-                            for (int z = 0; z < ZC; ++z)
-#pragma unroll
-                                for (int g = 0; g < PG; ++g)
-                                    v[z][g] = __builtin_amdgcn_raw_buffer_load_b128(rp, mail_at(z0 + z, pg + g), 0, 16);
-                            bool missing = false;
-#pragma unroll
-                            for (int z = 0; z < ZC; ++z)
-#pragma unroll
-                                for (int g = 0; g < PG; ++g)
-                                    missing = missing | (v[z][g][0] == 0) | (v[z][g][1] == 0) | (v[z][g][2] == 0) |
-                                              (v[z][g][3] == 0);
-                            if (__builtin_amdgcn_ballot_w64(missing) == 0)
-                                break;
-                            if (__builtin_amdgcn_s_memrealtime() - t_first > 100000000ull) {  // one second at 100 MHz
-                                gave_up = true;
-                                break;
-                            }
-                        }
+            for (int pg = 0; pg < MINE; pg += PG) {
+                v4f sum[PG];
+                auto gather = [&](auto count, int z0) __attribute__((always_inline)) {  // splits z0 .. z0 + ZC - 1
+                    constexpr int ZC = decltype(count)::value;
+                    v4i v[ZC][PG];
+                    for (;;) {
+                        asm volatile("" ::: "memory");  // the loads belong to this round of the loop
 #pragma unroll
                         for (int z = 0; z < ZC; ++z)
 #pragma unroll
-                            for (int g = 0; g < PG; ++g) {
-                                const v4f f = __builtin_bit_cast(v4f, v[z][g]);
-                                sum[g] = z0 + z == 0 ? f : sum[g] + f;
-                            }
-                    };
-                    int z0 = 0;
-                    for (; z0 + ZB <= senders; z0 += ZB)
-                        gather(std::integral_constant<int, ZB>{}, z0);
-                    if (ZB > 2 && senders - z0 == 2) {
-                        gather(std::integral_constant<int, 2>{}, z0);
-                        z0 += 2;
+                            for (int g = 0; g < PG; ++g)
+                                v[z][g] = __builtin_amdgcn_raw_buffer_load_b128(rp, mail_at(z0 + z, part + pg + g), 0, 16);
+                        bool missing = false;
+#pragma unroll
+                        for (int z = 0; z < ZC; ++z)
+#pragma unroll
+                            for (int g = 0; g < PG; ++g)
+                                missing = missing | (v[z][g][0] == 0) | (v[z][g][1] == 0) | (v[z][g][2] == 0) |
+                                          (v[z][g][3] == 0);
+                        if (__builtin_amdgcn_ballot_w64(missing) == 0)
+                            break;
+                        if (__builtin_amdgcn_s_memrealtime() - t_first > 100000000ull) {  // one second at 100 MHz
+                            gave_up = true;
+                            break;
+                        }
                     }
-                    if (z0 < senders)
-                        gather(std::integral_constant<int, 1>{}, z0);
 #pragma unroll
-                    for (int g = 0; g < PG; ++g) {
-                        v4f& own = acc[(pg + g) / NJ][(pg + g) % NJ];
+                    for (int z = 0; z < ZC; ++z)
 #pragma unroll
-                        for (int e = 0; e < 4; ++e)
-                            own[e] = gave_up ? __builtin_nanf("") : sum[g][e] + own[e];
+                        for (int g = 0; g < PG; ++g) {
+                            const v4f f = __builtin_bit_cast(v4f, v[z][g]);
+                            sum[g] = z0 + z == 0 ? f : sum[g] + f;
+                        }
+                };
+                int z0 = 0;
+                for (; z0 + ZB <= senders; z0 += ZB)
+                    gather(std::integral_constant<int, ZB>{}, z0);
+                auto rest = [&](auto count) __attribute__((always_inline)) {
+                    constexpr int ZC = decltype(count)::value;
+                    if (ZB > ZC && senders - z0 == ZC)
+                        gather(count, z0);
+                };
+                rest(std::integral_constant<int, 2>{});
+                rest(std::integral_constant<int, 1>{});
+#pragma unroll
+                for (int g = 0; g < PG; ++g) {
+                    if (gave_up)
+                        sum[g] = (v4f){__builtin_nanf(""), __builtin_nanf(""), __builtin_nanf(""), __builtin_nanf("")};
+                    if (AHEAD && !compute)
+                        *LDS_PTR(v4f, lds + SUMS_OFF + (uint32_t)(((wave & 3) * MINE + pg + g) * 1024 + lane * 16)) = sum[g];
+                    else
+                        acc[(pg + g) / NJ][(pg + g) % NJ] = sum[g] + acc[(pg + g) / NJ][(pg + g) % NJ];
+                }
+            }
+            if (AHEAD) {
+                __syncthreads();
+                if (compute) {
+#pragma unroll
+                    for (int g = 0; g < MINE; ++g) {
+                        v4f& own = acc[(MINE + g) / NJ][(MINE + g) % NJ];
+                        own = *LDS_PTR(v4f, lds + SUMS_OFF + (uint32_t)((wave * MINE + g) * 1024 + lane * 16)) + own;
                     }
                 }
             }
@@ -741,6 +763,13 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
     // padded row stride that keeps the writes conflict free, and leaves as 16 bytes per lane
     // along whole rows of the tile.  A tile larger than the ring is written in two halves.
     // PARTIAL = fp32 into this split's partial tile (the reduction kernel follows), else bf16 into c.
+    auto zeros = [&]() __attribute__((always_inline)) {
+        const __amdgpu_buffer_rsrc_t rp = make_rsrc(reinterpret_cast<const v4i*>(mailbox) + first, mail_span);
+        for (int z = 0; z < senders; ++z)
+#pragma unroll
+            for (int patch = 0; patch < MI * NJ; ++patch)
+                __builtin_amdgcn_raw_buffer_store_b128((v4i){0, 0, 0, 0}, rp, mail_at(z, patch), 0, 0);
+    };
     auto write_tile = [&](auto partial_tag) __attribute__((always_inline)) {
         constexpr bool PARTIAL = decltype(partial_tag)::value;
         constexpr int ESZ = PARTIAL ? 4 : 2;
@@ -751,9 +780,13 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
         static_assert(HROWS % 16 == 0, "a patch lies in one half");
         constexpr int CPR = BN * ESZ / 16;                 // 16-byte chunks per tile row
         constexpr int CHUNKS = HROWS * CPR;
+        constexpr bool GATHERED = AHEAD && SPLIT && !PARTIAL;  // a barrier has passed since the ring was read
+        constexpr int STORERS = GATHERED ? 64 * NCW : NTHREADS;
+        static_assert(!GATHERED || HALVES == 1, "one pass");
 #pragma unroll
         for (int h = 0; h < HALVES; ++h) {
-            __syncthreads();  // nobody reads the ring (or the previous half) any more
+            if (!GATHERED)
+                __syncthreads();  // nobody reads the ring (or the previous half) any more
 #pragma unroll
             for (int i = 0; i < MI; ++i) {
                 const int prow = wm * TM + 16 * i;  // first tile row of the patch
@@ -772,10 +805,19 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
                     }
                 }
             }
-            __syncthreads();
+            if (GATHERED) {
+                if (!compute) {
+                    zeros();
+                    asm volatile("s_barrier" ::: "memory");
+                    return;
+                }
+                asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // the rows are in the LDS
+            } else {
+                __syncthreads();
+            }
 #pragma unroll
-            for (int it = 0; it < (CHUNKS + NTHREADS - 1) / NTHREADS; ++it) {
-                const int idx = it * NTHREADS + (int)threadIdx.x;
+            for (int it = 0; it < (CHUNKS + STORERS - 1) / STORERS; ++it) {
+                const int idx = it * STORERS + (int)threadIdx.x;
                 const int row = idx / CPR, ch = idx - row * CPR;
                 const int mrow = m0 + h * HROWS + row;
                 const int ncol = n0 + ch * (16 / ESZ);
@@ -796,13 +838,8 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
             write_tile(std::true_type{});
         } else {
             write_tile(std::false_type{});
-            if (compute) {  // zeros back into the mailbox, behind the tile
-                const __amdgpu_buffer_rsrc_t rp = make_rsrc(reinterpret_cast<const v4i*>(mailbox) + first, mail_span);
-                for (int z = 0; z < senders; ++z)
-#pragma unroll
-                    for (int patch = 0; patch < MI * NJ; ++patch)
-                        __builtin_amdgcn_raw_buffer_store_b128((v4i){0, 0, 0, 0}, rp, mail_at(z, patch), 0, 0);
-            }
+            if (!AHEAD)
+                zeros();
         }
     } else {
         write_tile(std::false_type{});
