@@ -201,11 +201,16 @@ double tile_cost(const GemmArgs& g, int variant, int ksplit, bool fused = false)
     // share an XCD: the workgroups beyond the tiles exit at once but take their turn -- 85 tiles x 3 splits are
     // 264 workgroups, and the last of them start when a CU frees up: 20.2 us against 13.9 us with two splits)
     const long items = (ksplit > 1 && fused ? (tiles + 7) / 8 * 8 : tiles) * ksplit;
-    // (a problem of at most 64 tiles of 64x64: a K block takes 0.265 us whether 4 or 64 tiles run -- M, N = 96 ... 512
-    // with K = 1536 ... 8192 -- where the fit, made on launches of several rounds, says 0.34, and the hand-over of
-    // the splits inside the kernel starts 0.3 us earlier.  Problems of 96 ... 256 such tiles measure as the fit
-    // says, or slower.)
-    const bool light = variant == TILE_64x64 && !streams_b && tiles <= 64;
+    // (64x64 tiles: the fit knows the kernel before four waves read ahead and all eight hand splits over.  Fill and store
+    // take 0.72 us less, and with 64 tiles or fewer a K block takes 0.285 us for 32 of them and 0.015 more for every 32
+    // beyond, the hand-over starts 0.3 us earlier; with more tiles a block takes 9 % longer than the fit says.  649 random
+    // problems of 48 ... 4096 rows, every plan measured: the one chosen was 1.4 / 1.7 % behind the best one from the Infinity
+    // Cache / HBM and is 0.7 / 0.9 %; the 110 that change are 6 and 8 % faster on average (149 x 7168 x 256 as 128x128 5.07 us,
+    // now 4.32; 224 x 2336 x 4096 as 128x128 in four 14.7 / 17.0, now in three 12.1 / 15.1; 256 x 336 x 1536 unsplit 4.69 / 6.60,
+    // now in three 4.49 / 5.30), at worst 800 x 576 x 7168 as 128x128 in seven 15.6 / 15.4, now in two 13.6 / 17.9.)
+    const bool small = variant == TILE_64x64;
+    const bool light = small && !streams_b && tiles <= 64;
+    const double of_small = !small ? 1.0 : light ? 0.838 : tiles > 64 ? 1.087 : 1.035;
     // (256x192 in the persistent form: the fit knows the kernel before its barrier moved, 5 % slower)
     // (unsplit 128x128 tiles in one round: the fit knows the kernel before four waves read ahead of themselves, 10 - 15 %
     // slower from the caches, and level from HBM, where the copies bound it: they do also where a row of B starts
@@ -216,12 +221,13 @@ double tile_cost(const GemmArgs& g, int variant, int ksplit, bool fused = false)
     const bool ahead = variant == TILE_128x128 && ksplit == 1 && g.m > 256 && tiles <= NUM_CU &&
                        leading_dim(g) % 16 == 0 && g.n % 128 == 0;
     const double per_kb = (1.19 * area + 0.267) * (variant == TILE_256x192 && ksplit == 1 && tiles > NUM_CU ? 0.95 : 1.0) *
-                          (streams_b ? 1.25 : 1.0) * (light ? 0.8 : 1.0) * (ahead ? 0.94 : 1.0);
+                          (streams_b ? 1.25 : 1.0) * of_small * (ahead ? 0.94 : 1.0) +
+                          (light ? 0.015 * (double)(tiles - 32) / 32.0 : 0.0);
     // (unsplit 128x192 tiles in more than one round of workgroups: the fit has them 8 % too fast against the 256-row
     // tiles -- 36 random shapes of 512 ... 8192 rows where that margin decides, before / after: the 256x256 or
     // 256x128 plan +5.6 % with B cached, +10.3 % with B from HBM on average, worst -2.3 %)
     const double in_rounds = variant == TILE_128x192 && ksplit == 1 && tiles > NUM_CU ? 1.08 : 1.0;
-    const double per_item = 0.95 + 4.38 * area + kbs * per_kb * in_rounds;
+    const double per_item = (small ? 0.23 : variant == TILE_128x128 ? 1.01 : 0.95) + 4.38 * area + kbs * per_kb * in_rounds;
     // (two 64x64 workgroups share a CU, but a single row of tiles with B from HBM is fastest with at most one
     // workgroup per CU: M = 48, 64 on 12 shapes, the split that keeps tiles x splits within 256 is the best
     // measured or within 2 % of it)

@@ -342,3 +342,10 @@ def test_generated_k_loop_is_what_its_generator_writes():
                          check=True).stdout
     with open(os.path.join(csrc, "w4_loop.inc")) as f:
         assert f.read() == out
+
+
+@pytest.mark.parametrize("m,n,k,plan", [(160, 7168, 256, "tile64x64_k1"), (224, 2336, 4096, "tile64x64_k3f"), (256, 336, 1536, "tile64x64_k3f"),
+                                        (149, 7168, 256, "tile64x64_k1"), (1744, 576, 7168, "tile128x128_k3f"), (592, 2048, 4096, "tile128x128_k3f")])
+def test_plans_of_small_tiles(pkg, m, n, k, plan):
+    """64x64 tiles where they are the best measured plan, and shapes on the other side of the line"""
+    assert pkg.plan(m, n, k) == plan
