@@ -11,6 +11,7 @@ import subprocess
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 _LIB = None
+_CALL = None  # csrc/pycall.cpp: the calls of a serving loop without ctypes
 
 KERNEL_AUTO, KERNEL_SCALAR, KERNEL_LARGE, KERNEL_SPLITK, KERNEL_SKINNY = range(5)
 DTYPE_BF16, DTYPE_F32, DTYPE_BF16_F32MATH = 0, 1, 2
@@ -119,6 +120,20 @@ def lib():
     return L
 
 
+def _load_call():
+    """The native entry points of gemm, gemm_ex and the quantisers.  They answer None to arguments that are not tensors,
+    plain integers or None; those calls go through ctypes."""
+    global _CALL
+    lib()
+    path = os.path.join(_HERE, "_pycall.so")
+    if not os.path.exists(path):
+        raise FileNotFoundError(f"{path} is missing: build it with __graft_entry__.build() or `make -C {_HERE}`")
+    from . import _pycall
+    _pycall.setup(Options)
+    _CALL = _pycall
+    return _CALL
+
+
 def error_string(code):
     return lib().fp8_block_gemm_error_string(int(code)).decode()
 
@@ -139,22 +154,23 @@ def _check(rc, where):
 def gemm(a, b, a_scale, b_scale, c, m, n, k, stream=None):
     """C[m,n] bf16 = block-scaled A.B^T.  `stream` is a raw hipStream_t (int) or None for the
     null stream."""
-    L = lib()
-    if stream is None:
-        rc = L.fp8_block_gemm(_ptr(a), _ptr(b), _ptr(a_scale), _ptr(b_scale), _ptr(c), m, n, k)
-    else:
-        rc = L.fp8_block_gemm_stream(_ptr(a), _ptr(b), _ptr(a_scale), _ptr(b_scale), _ptr(c), m, n, k,
-                                     stream)
-    _check(rc, "fp8_block_gemm")
+    rc = (_CALL or _load_call()).gemm(a, b, a_scale, b_scale, c, m, n, k, stream)
+    if rc is None:
+        rc = lib().fp8_block_gemm_stream(_ptr(a), _ptr(b), _ptr(a_scale), _ptr(b_scale), _ptr(c), m, n, k, stream)
+    if rc != 0:
+        raise Fp8GemmError(rc, "fp8_block_gemm")
 
 
 def gemm_ex(a, b, a_scale, b_scale, c, m, n, k, options=None, workspace=None, workspace_bytes=0, stream=None):
     """Per-call form: `options` (Options or None = automatic), `workspace` (device tensor / pointer or
     None) of `workspace_bytes`.  Allocates nothing, reads no process-wide switch."""
-    opt = C.byref(options) if options is not None else None
-    rc = lib().fp8_block_gemm_ex(_ptr(a), _ptr(b), _ptr(a_scale), _ptr(b_scale), _ptr(c), m, n, k, opt,
-                                 _ptr(workspace), workspace_bytes, stream)
-    _check(rc, "fp8_block_gemm_ex")
+    rc = (_CALL or _load_call()).gemm_ex(a, b, a_scale, b_scale, c, m, n, k, options, workspace, workspace_bytes, stream)
+    if rc is None:
+        opt = C.byref(options) if options is not None else None
+        rc = lib().fp8_block_gemm_ex(_ptr(a), _ptr(b), _ptr(a_scale), _ptr(b_scale), _ptr(c), m, n, k, opt,
+                                     _ptr(workspace), workspace_bytes, stream)
+    if rc != 0:
+        raise Fp8GemmError(rc, "fp8_block_gemm_ex")
 
 
 NOALLOC_MAX_BYTES = 32 << 20
@@ -263,15 +279,21 @@ def quantize_a_1x128(x, a, a_scale, m, k, dtype=DTYPE_BF16, stream=None):
     """x [m][k] row-major (bf16 bits or fp32) -> a (fp8, element (m,k) at m + k*M) and
     a_scale ([k/128][m]): to_float8_rowwise_scale of /root/reference/quantize.py:43-67 written
     in the GEMM's layouts."""
-    _check(lib().fp8_quantize_a_1x128(_ptr(x), dtype, _ptr(a), _ptr(a_scale), m, k, stream),
-           "fp8_quantize_a_1x128")
+    rc = (_CALL or _load_call()).quantize_a(x, dtype, a, a_scale, m, k, stream)
+    if rc is None:
+        rc = lib().fp8_quantize_a_1x128(_ptr(x), dtype, _ptr(a), _ptr(a_scale), m, k, stream)
+    if rc != 0:
+        raise Fp8GemmError(rc, "fp8_quantize_a_1x128")
 
 
 def quantize_b_128x128(x, b, b_scale, n, k, dtype=DTYPE_BF16, stream=None):
     """x [n][k] row-major -> b (fp8 at n + k*N) and b_scale ([k/128][ceil(n/128)]):
     to_float8_block_scale of /root/reference/quantize.py:16-41 written in the GEMM's layouts."""
-    _check(lib().fp8_quantize_b_128x128(_ptr(x), dtype, _ptr(b), _ptr(b_scale), n, k, stream),
-           "fp8_quantize_b_128x128")
+    rc = (_CALL or _load_call()).quantize_b(x, dtype, b, b_scale, n, k, stream)
+    if rc is None:
+        rc = lib().fp8_quantize_b_128x128(_ptr(x), dtype, _ptr(b), _ptr(b_scale), n, k, stream)
+    if rc != 0:
+        raise Fp8GemmError(rc, "fp8_quantize_b_128x128")
 
 
 def custom_kernel(data, stream=None):
