@@ -333,7 +333,7 @@ Plan compute_plan(const GemmArgs& g, const Config& cfg);
 
 // The plan of a problem depends on its sizes, on the low address bits of its operands and on the switches: a
 // serving loop asks for the same few again and again, and working one out costs a microsecond or two of host
-// time (three are worked out per call), which is what a launch-bound decode loop runs on.  Each thread keeps the
+// time (three are looked up in a call until the workgroups' placement is known, one from then on), which is what a launch-bound decode loop runs on.  Each thread keeps the
 // last plans it worked out, 64 slots indexed by a hash of the sizes.
 struct PlanKey {
     int m, n, k, lda;
@@ -744,6 +744,19 @@ void plan_name(const Plan& p, char* out, size_t cap)
                  p.persistent ? "_persistent" : (p.fused ? "f" : ""));
 }
 
+// The thread's last launch by name; a plan's is put together when somebody asks (0.06 us of a call).
+thread_local Plan t_last_plan;
+thread_local bool t_plan_unnamed = false;  // t_last_plan is newer than t_last_kernel
+const char* last_kernel_name()
+{
+    if (t_plan_unnamed) {
+        plan_name(t_last_plan, t_name_buf, sizeof(t_name_buf));
+        t_last_kernel = t_name_buf;
+        t_plan_unnamed = false;
+    }
+    return t_last_kernel;
+}
+
 // the kernels of a plan on operands they can take; `partial` holds plan_workspace_bytes, `w` is the
 // workspace whose zeroed header the plans use that add their K splits inside the kernel
 hipError_t launch_plan(const GemmArgs& g, const Plan& p, float* partial, const Workspace& w, hipStream_t stream)
@@ -848,7 +861,7 @@ int run(const void* a, const void* b, const float* as, const float* bs, void* c,
     // in-kernel K-split reduction: a zeroed header (every process-wide workspace has one; a per-call
     // one when the caller says so) and a confirmed workgroup placement
     cfg.fused_ok = cfg.fused_ok && (!explicit_ws || explicit_ws->zeroed);
-    if (cfg.fused_ok) {
+    if (cfg.fused_ok && xcd_placement_confirmed(false) != 1) {  // not known yet, or not as they assume
         Config probe = cfg;
         probe.fused_ok = false;
         const Plan with = make_plan(g, cfg), without = make_plan(g, probe);
@@ -889,8 +902,8 @@ int run(const void* a, const void* b, const float* as, const float* bs, void* c,
     }
     const int rc = p.padded ? run_padded(g, p, w, stream) : (int)launch_plan(g, p, ws_data(w), w, stream);
     if (rc == FP8GEMM_OK) {
-        plan_name(p, t_name_buf, sizeof(t_name_buf));
-        t_last_kernel = t_name_buf;
+        t_last_plan = p;
+        t_plan_unnamed = true;
     }
     return rc;
 }
@@ -1140,6 +1153,7 @@ int run_grouped_table(const GroupTable& tab, int n, int k, bool decode, hipStrea
             snprintf(t_name_buf, sizeof(t_name_buf), "%s%s_k1_grouped%d", padded ? "padded_" : "", tile_variant_name(variant),
                      tab.groups);
         t_last_kernel = t_name_buf;
+        t_plan_unnamed = false;
     }
     return (int)e;
 }
@@ -1381,6 +1395,7 @@ static int run_grouped(int groups, const void* const* a, const void* const* b, c
             }
             if (rc != FP8GEMM_OK)
                 break;
+            (void)last_kernel_name();  // into t_name_buf
             if (launches > 1) {  // the last launch's name and how many there were
                 char many[sizeof(t_name_buf)];
                 snprintf(many, sizeof(many), "%.88sx%d", t_name_buf, launches);
@@ -1443,7 +1458,7 @@ int fp8_block_gemm_set_persistent(int mode)
     return FP8GEMM_OK;
 }
 
-const char* fp8_block_gemm_last_kernel(void) { return t_last_kernel; }
+const char* fp8_block_gemm_last_kernel(void) { return last_kernel_name(); }
 
 int fp8_block_gemm_plan(int m, int n, int k, char* name, size_t cap)
 {

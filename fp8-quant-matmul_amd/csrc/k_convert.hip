@@ -41,7 +41,7 @@ hipError_t launch_convert(const float* in, uint8_t* out, size_t count, hipStream
         blocks = 1;
     if (blocks > 256 * 16)
         blocks = 256 * 16;
-    hipLaunchKernelGGL(convert_kernel, dim3((unsigned)blocks), dim3(256), 0, s, in, out, count);
+    launch_kernel(convert_kernel, dim3((unsigned)blocks), dim3(256), 0, s, in, out, count);
     return hipGetLastError();
 }
 

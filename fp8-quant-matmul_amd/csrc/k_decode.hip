@@ -1002,7 +1002,7 @@ int xcd_placement_confirmed(bool may_probe)
     unsigned int h[XCC_PROBE];
     bool ok = hipGetSymbolAddress(reinterpret_cast<void**>(&out), HIP_SYMBOL(xcc_probe_out)) == hipSuccess;
     for (int rep = 0; rep < 2 && ok; ++rep) {
-        hipLaunchKernelGGL(xcc_probe_kernel, dim3(XCC_PROBE), dim3(64), 0, nullptr, out);
+        launch_kernel(xcc_probe_kernel, dim3(XCC_PROBE), dim3(64), 0, nullptr, out);
         ok = hipMemcpy(h, out, sizeof(h), hipMemcpyDeviceToHost) == hipSuccess;
         for (int i = 8; i < XCC_PROBE && ok; ++i)
             ok = h[i] == h[i & 7];
@@ -1037,7 +1037,7 @@ hipError_t launch_decode_strips(const GemmArgs& g, int ksplit, int halves, float
     auto go = [&](auto kernel, int lds) -> hipError_t {
         constexpr auto kern = decltype(kernel)::value;
         FP8GEMM_ALLOW_LDS(kern, lds);
-        hipLaunchKernelGGL(kern, grid, dim3(DS_THREADS), lds, s, g.b, g.a, g.n, g.k, g.m, leading_dim(g), kb_per_split, strips,
+        launch_kernel(kern, grid, dim3(DS_THREADS), lds, s, g.b, g.a, g.n, g.k, g.m, leading_dim(g), kb_per_split, strips,
                            g.a_scale, g.b_scale, g.c, mailbox, ksplit);
         return hipGetLastError();
     };
@@ -1054,7 +1054,7 @@ hipError_t launch_decode_strips(const GemmArgs& g, int ksplit, int halves, float
             auto with = [&](auto kernel) -> hipError_t {
                 constexpr auto kern = decltype(kernel)::value;
                 FP8GEMM_ALLOW_LDS(kern, lds);
-                hipLaunchKernelGGL(kern, dim3(STREAM_WORKGROUPS), dim3(DS_THREADS), lds, s, g.a, g.b, g.a_scale, g.b_scale,
+                launch_kernel(kern, dim3(STREAM_WORKGROUPS), dim3(DS_THREADS), lds, s, g.a, g.b, g.a_scale, g.b_scale,
                                    g.c, g.m, leading_dim(g), g.n, g.k, units);
                 return hipGetLastError();
             };
@@ -1229,7 +1229,7 @@ hipError_t launch_decode_grouped(const GroupTable& tab, int n, int k, int ksplit
             auto with = [&](auto kernel) -> hipError_t {
                 constexpr auto kern = decltype(kernel)::value;
                 FP8GEMM_ALLOW_LDS(kern, lds);
-                hipLaunchKernelGGL(kern, dim3(STREAM_WORKGROUPS), dim3(DS_THREADS), lds, s, tab, n, k, wide_strips,
+                launch_kernel(kern, dim3(STREAM_WORKGROUPS), dim3(DS_THREADS), lds, s, tab, n, k, wide_strips,
                                    (int)wide_units);
                 return hipGetLastError();
             };
@@ -1246,7 +1246,7 @@ hipError_t launch_decode_grouped(const GroupTable& tab, int n, int k, int ksplit
     auto go = [&](auto kernel, int lds) -> hipError_t {
         constexpr auto kern = decltype(kernel)::value;
         FP8GEMM_ALLOW_LDS(kern, lds);
-        hipLaunchKernelGGL(kern, grid, dim3(DS_THREADS), lds, s, tab, mailbox, n, k, strips, ksplit, kb_per_split);
+        launch_kernel(kern, grid, dim3(DS_THREADS), lds, s, tab, mailbox, n, k, strips, ksplit, kb_per_split);
         return hipGetLastError();
     };
     // One or three K blocks with slabs to spread are not taken in pairs, where the last turn handles a slab that does not

@@ -478,7 +478,7 @@ hipError_t launch_decode64(const GemmArgs& g, int ksplit, float* mailbox, hipStr
         constexpr int T = decltype(tiles_c)::value, lds = Strip64<T, F>::LDS;
         constexpr auto kern = decode64_kernel<T, F>;
         FP8GEMM_ALLOW_LDS(kern, lds);
-        hipLaunchKernelGGL(kern, grid, dim3(NTHREADS), lds, s, g.b, g.a, g.n, g.k, g.m, leading_dim(g), kb_per_split, strips,
+        launch_kernel(kern, grid, dim3(NTHREADS), lds, s, g.b, g.a, g.n, g.k, g.m, leading_dim(g), kb_per_split, strips,
                            g.a_scale, g.b_scale, g.c, mailbox, ksplit, paired ? 1 : 0);
         return hipGetLastError();
     };

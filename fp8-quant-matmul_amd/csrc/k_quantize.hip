@@ -400,14 +400,14 @@ template <typename TIn, bool BLOCK, bool BF16MATH, int QTILE, bool ONCE = false>
 void launch_quantize_tile(const TIn* x, uint8_t* q, float* scale_out, int rows, int k, hipStream_t s)
 {
     const int grid = output_grid(q, rows);
-    hipLaunchKernelGGL((quantize_kernel<TIn, BLOCK, BF16MATH, QTILE, ONCE>), dim3((rows + QTILE - 1) / QTILE, k / 128),
+    launch_kernel((quantize_kernel<TIn, BLOCK, BF16MATH, QTILE, ONCE>), dim3((rows + QTILE - 1) / QTILE, k / 128),
                        dim3(QTILE * 4), 0, s, x, q, scale_out, rows, k, grid);
 }
 
 template <typename TIn, bool BF16MATH, int NW>
 void launch_quantize_batch(const TIn* x, uint8_t* q, float* scale_out, int rows, int k, hipStream_t s)
 {
-    hipLaunchKernelGGL((quantize_batch_kernel<TIn, BF16MATH, NW>), dim3(k / 128), dim3(64 * NW), 0, s, x, q, scale_out, rows, k);
+    launch_kernel((quantize_batch_kernel<TIn, BF16MATH, NW>), dim3(k / 128), dim3(64 * NW), 0, s, x, q, scale_out, rows, k);
 }
 
 // Tile sizes, measured with every operand from HBM (us, previous kernel -> this one):

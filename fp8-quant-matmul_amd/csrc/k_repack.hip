@@ -132,10 +132,10 @@ hipError_t launch_pad_typed(PadJobs<MAX>& jobs, hipStream_t s)
     }
     if constexpr (MAX > 4)
         if ((uint64_t)most * jobs.count <= JOB_ROWS_MAX_WORKGROUPS) {
-            hipLaunchKernelGGL((pad_kernel<MAX, PER_THREAD, true>), dim3(most, jobs.count), dim3(256), 0, s, jobs);
+            launch_kernel((pad_kernel<MAX, PER_THREAD, true>), dim3(most, jobs.count), dim3(256), 0, s, jobs);
             return hipGetLastError();
         }
-    hipLaunchKernelGGL((pad_kernel<MAX, PER_THREAD, false>), dim3(blocks), dim3(256), 0, s, jobs);
+    launch_kernel((pad_kernel<MAX, PER_THREAD, false>), dim3(blocks), dim3(256), 0, s, jobs);
     return hipGetLastError();
 }
 
@@ -205,7 +205,7 @@ hipError_t launch_crop_bf16(const uint16_t* src, uint16_t* dst, int m, int n, in
 {
     if (m == 0 || n == 0)
         return hipSuccess;
-    hipLaunchKernelGGL(crop_kernel, dim3(crop_blocks(m, n)), dim3(256), 0, s, src, dst, m, n, ld_src);
+    launch_kernel(crop_kernel, dim3(crop_blocks(m, n)), dim3(256), 0, s, src, dst, m, n, ld_src);
     return hipGetLastError();
 }
 
@@ -220,7 +220,7 @@ hipError_t launch_crop_bf16_batched(const CropTable& tab, hipStream_t s)
     }
     if (most == 0)
         return hipSuccess;
-    hipLaunchKernelGGL(crop_batched_kernel, dim3(most, (unsigned)tab.groups), dim3(256), 0, s, tab);
+    launch_kernel(crop_batched_kernel, dim3(most, (unsigned)tab.groups), dim3(256), 0, s, tab);
     return hipGetLastError();
 }
 

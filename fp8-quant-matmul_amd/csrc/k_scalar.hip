@@ -44,7 +44,7 @@ hipError_t launch_scalar(const GemmArgs& g, hipStream_t s)
     if (strips > 65535u)  // n beyond 4 M columns: not a shape this kernel is for
         return hipErrorInvalidConfiguration;
     dim3 grid((unsigned)((g.m + 3) / 4), strips);
-    hipLaunchKernelGGL(scalar_gemm_kernel, grid, dim3(256), 0, s, g.a, g.b, g.a_scale, g.b_scale,
+    launch_kernel(scalar_gemm_kernel, grid, dim3(256), 0, s, g.a, g.b, g.a_scale, g.b_scale,
                        g.c, g.m, g.n, g.k);
     return hipGetLastError();
 }

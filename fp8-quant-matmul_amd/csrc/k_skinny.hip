@@ -237,7 +237,7 @@ hipError_t launch_skinny(const GemmArgs& g, int ksplit, float* partial, hipStrea
     if (ksplit > 1) {
         constexpr auto kern = skinny_gemm_kernel<true>;
         FP8GEMM_ALLOW_LDS(kern, SK_LDS);
-        hipLaunchKernelGGL(kern, grid, dim3(SK_THREADS), SK_LDS, s, g.a, g.b, g.a_scale, g.b_scale,
+        launch_kernel(kern, grid, dim3(SK_THREADS), SK_LDS, s, g.a, g.b, g.a_scale, g.b_scale,
                            g.c, partial, g.m, g.n, g.k, tiles_n, kb_per_split);
         e = hipGetLastError();
         if (e != hipSuccess)
@@ -246,7 +246,7 @@ hipError_t launch_skinny(const GemmArgs& g, int ksplit, float* partial, hipStrea
     }
     constexpr auto kern = skinny_gemm_kernel<false>;
     FP8GEMM_ALLOW_LDS(kern, SK_LDS);
-    hipLaunchKernelGGL(kern, grid, dim3(SK_THREADS), SK_LDS, s, g.a, g.b, g.a_scale, g.b_scale, g.c,
+    launch_kernel(kern, grid, dim3(SK_THREADS), SK_LDS, s, g.a, g.b, g.a_scale, g.b_scale, g.c,
                        partial, g.m, g.n, g.k, tiles_n, kb_per_split);
     return hipGetLastError();
 }

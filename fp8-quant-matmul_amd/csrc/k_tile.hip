@@ -947,7 +947,7 @@ hipError_t launch_typed(const GemmArgs& g, int ksplit, float* partial, float* ma
     const dim3 grid(SPLIT && mailbox ? (tiles + 7) & ~7 : tiles, SPLIT ? ksplit : 1);
     constexpr auto kern = tile_gemm_kernel<BM, BN, WM, WN, NS, SPLIT, RAGGED>;
     FP8GEMM_ALLOW_LDS(kern, LDS_TOTAL);
-    hipLaunchKernelGGL(kern, grid, dim3(NTHREADS), LDS_TOTAL, s, g.a, g.b, g.a_scale, g.b_scale, g.c, partial,
+    launch_kernel(kern, grid, dim3(NTHREADS), LDS_TOTAL, s, g.a, g.b, g.a_scale, g.b_scale, g.c, partial,
                        SPLIT ? mailbox : nullptr, g.m, leading_dim(g), g.n, g.k, tiles_m, tiles_n, kb_per_split, group_m);
     return hipGetLastError();
 }
@@ -1062,7 +1062,7 @@ hipError_t launch_splitk_reduce(const GemmArgs& g, int ksplit, const float* part
 {
     size_t mn = (size_t)g.m * g.n;
     unsigned blocks = (unsigned)((mn / 4 + 255) / 256);
-    hipLaunchKernelGGL(splitk_reduce_kernel, dim3(blocks), dim3(256), 0, s, partial, g.c, mn, ksplit);
+    launch_kernel(splitk_reduce_kernel, dim3(blocks), dim3(256), 0, s, partial, g.c, mn, ksplit);
     return hipGetLastError();
 }
 

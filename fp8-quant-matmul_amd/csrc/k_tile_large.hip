@@ -451,7 +451,7 @@ hipError_t launch_large(const GemmArgs& g, int workgroups, hipStream_t s)
     constexpr int LDS = LargeShape<BN>::LDS_BYTES > tail_lds_bytes<TAIL>() ? LargeShape<BN>::LDS_BYTES : tail_lds_bytes<TAIL>();
     constexpr auto kern = tile_gemm_large_kernel<BN, TAIL>;
     FP8GEMM_ALLOW_LDS(kern, LDS);
-    hipLaunchKernelGGL(kern, dim3(workgroups), dim3(NTHREADS), LDS, s, g.a, g.b, g.a_scale, g.b_scale, g.c, g.m,
+    launch_kernel(kern, dim3(workgroups), dim3(NTHREADS), LDS, s, g.a, g.b, g.a_scale, g.b_scale, g.c, g.m,
                        leading_dim(g), g.n, g.k, (g.m + 255) / 256, (g.n + BN - 1) / BN, c_streams(g.m, 1, g.n, g.k));
     return hipGetLastError();
 }
@@ -465,7 +465,7 @@ hipError_t launch_large_grouped(const GroupTable& tab, int n, int k, int workgro
     long rows = 0;
     for (int g = 0; g < tab.groups; ++g)
         rows += tab.m[g];
-    hipLaunchKernelGGL(kern, dim3(workgroups), dim3(NTHREADS), LDS, s, tab, n, k, (n + BN - 1) / BN,
+    launch_kernel(kern, dim3(workgroups), dim3(NTHREADS), LDS, s, tab, n, k, (n + BN - 1) / BN,
                        c_streams(rows, tab.groups, n, k));
     return hipGetLastError();
 }

@@ -50,7 +50,7 @@ hipError_t launch_persistent_variant(const GemmArgs& g, int workgroups, hipStrea
     const int tiles_m = (g.m + BM - 1) / BM, tiles_n = (g.n + BN - 1) / BN;
     constexpr auto kern = tile_gemm_persistent_kernel<BM, BN, WM, WN, NS, PR>;
     FP8GEMM_ALLOW_LDS(kern, LDS_TOTAL);
-    hipLaunchKernelGGL(kern, dim3(workgroups), dim3(64 * WM * WN), LDS_TOTAL, s, g.a, g.b, g.a_scale,
+    launch_kernel(kern, dim3(workgroups), dim3(64 * WM * WN), LDS_TOTAL, s, g.a, g.b, g.a_scale,
                        g.b_scale, g.c, g.m, leading_dim(g), g.n, g.k, tiles_m, tiles_n);
     return hipGetLastError();
 }
@@ -66,7 +66,7 @@ hipError_t launch_grouped_variant(GroupTable& tab, int n, int k, int workgroups,
         tab.tile_start[g + 1] = tab.tile_start[g] + ((tab.m[g] + BM - 1) / BM) * tiles_n;
     constexpr auto kern = tile_gemm_grouped_kernel<BM, BN, WM, WN, NS, PR>;
     FP8GEMM_ALLOW_LDS(kern, LDS_TOTAL);
-    hipLaunchKernelGGL(kern, dim3(workgroups), dim3(NTHREADS), LDS_TOTAL, s, tab, n, k, tiles_n);
+    launch_kernel(kern, dim3(workgroups), dim3(NTHREADS), LDS_TOTAL, s, tab, n, k, tiles_n);
     return hipGetLastError();
 }
 
