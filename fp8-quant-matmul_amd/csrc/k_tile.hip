@@ -952,39 +952,42 @@ hipError_t launch_typed(const GemmArgs& g, int ksplit, float* partial, float* ma
     return hipGetLastError();
 }
 
-template <int BM, int BN, int WM, int WN, int NS, bool RAGGED_SPLITS = true>
+template <int BM, int BN, int WM, int WN, int NS>
 hipError_t launch_variant(const GemmArgs& g, int ksplit, float* partial, float* mailbox, hipStream_t s)
 {
     if (leading_dim(g) % 16 == 0)
         return ksplit > 1 ? launch_typed<BM, BN, WM, WN, NS, true, false>(g, ksplit, partial, mailbox, s)
                           : launch_typed<BM, BN, WM, WN, NS, false, false>(g, ksplit, partial, mailbox, s);
     if constexpr (tile_takes_ragged_rows(BM, NS)) {
-        if (leading_dim(g) == g.m && g.m >= 16) {
-            if (ksplit == 1)
-                return launch_typed<BM, BN, WM, WN, NS, false, true>(g, ksplit, partial, mailbox, s);
-            if constexpr (RAGGED_SPLITS)
-                return launch_typed<BM, BN, WM, WN, NS, true, true>(g, ksplit, partial, mailbox, s);
-        }
+        if (leading_dim(g) == g.m && g.m >= 16)
+            return ksplit > 1 ? launch_typed<BM, BN, WM, WN, NS, true, true>(g, ksplit, partial, mailbox, s)
+                              : launch_typed<BM, BN, WM, WN, NS, false, true>(g, ksplit, partial, mailbox, s);
     }
     return hipErrorInvalidValue;
 }
 
-// Whether 128x128 tiles are multiplied by four waves that read ahead, or by eight.  us by four / by eight:
-//   Ragged rows with K split: eight.  Four of them bring A there, and all take part in the hand-over, which the short chains
-//   of a split do not make up for: 250 x 7168 x 2048 in two splits, B from HBM, 14.1 / 12.9, 2204 x 512 x 7168 in three
-//   23.4 / 22.0, 333 x 4608 x 7168 in two 30.9 / 30.0; unsplit 500 x 4608 x 2048 12.9 / 13.8.
-//   Splits added in the kernel: eight while a split has fewer than 16 K blocks.  752 x 1360 x 1536 in three of four 12.09 /
-//   11.01, 3824 x 272 x 2176 in two of nine 12.40 / 11.68, 1520 x 768 x 3840 in three of ten 14.82 / 13.97, 1376 x 624 x 5760 in
-//   three of 15 18.20 / 17.11 (30 shapes of 4 - 15: eight ahead on 27, by up to 11 %, 2 % behind at worst); from 16 on either
-//   way, 384 x 3456 x 6144 in three of 16 24.75 / 26.12, 1520 x 640 x 6144 17.62 / 16.62, 2048 x 576 x 7168 in three of 19
-//   18.63 / 19.04, 208 x 4352 x 6144 in two of 24 17.14 / 18.53.  With the reduction kernel behind them, which needs no
-//   hand-over, four: 512 x 1024 x 7168 in five 13.99 / 14.77.
-//   A single K block: eight, there is nothing to read ahead of.  5104 x 720 x 128 4.72 / 4.41, 413 x 3824 x 128 4.47 / 4.37; two:
-//   5104 x 720 x 256 5.14 / 5.19.
+// Whether 128x128 tiles are multiplied by four waves that read ahead, or by eight.  us by eight / by four:
+//   K splits: four for long chains.  They start later (a K block more is read before the first MFMA) and, with rows of B that
+//   share lines of 128 bytes with their neighbours' (N no multiple of 128), gain nothing per K block, which the copies
+//   bound then.  Added in the kernel, rows on the grid, N a multiple of 128, 8 ... 15 K blocks to a split: 192 x 7168 x 2048 in
+//   two 11.03 / 10.84, 256 x 7168 x 2048 11.17 / 10.89, 144 x 7168 x 2304 11.52 / 11.26 (18 of 20 ahead, 1.5 % on average);
+//   other N 1504 x 832 x 2816 in two 12.55 / 12.94, 3728 x 288 x 2560 12.19 / 12.53, from 16 blocks on 2000 ... 3000 x 576
+//   x 7168 1 - 3 % ahead.  Rows off the grid, where two of the copy waves bring A by way of registers, N a multiple of 128:
+//   334 x 4608 x 7168 in two of 28 blocks 24.00 / 22.76, 2340 x 512 x 7168 in three 20.82 / 20.08, 397 x 1536 x 7168 in five of
+//   twelve (reduction kernel) 18.25 / 17.81, 129 x 7168 x 2304 in two of nine 13.08 / 13.37; other N 1621 x 576 x 7168 21.03 /
+//   21.42, 3065 x 576 x 7168 25.07 / 24.76 (30 shapes level).  With the reduction kernel behind them and rows on the grid,
+//   four: 512 x 1024 x 7168 in five 14.77 / 13.99.
+//   Unsplit, four: 500 x 4608 x 2048 (off the grid) 13.8 / 12.9 -- but for a single K block, where there is nothing to read
+//   ahead of: 5104 x 720 x 128 4.41 / 4.72, 413 x 3824 x 128 4.37 / 4.47; two: 5104 x 720 x 256 5.19 / 5.14.
 bool four_waves(const GemmArgs& g, int ksplit, bool fused)
 {
     const int kb_per_split = (g.k / KBLOCK + ksplit - 1) / ksplit;
-    return kb_per_split > 1 && (ksplit == 1 || (leading_dim(g) % 16 == 0 && (!fused || kb_per_split >= 16)));
+    const bool whole_lines = g.n % 128 == 0;
+    if (ksplit == 1)
+        return kb_per_split > 1;
+    if (leading_dim(g) % 16 != 0)
+        return whole_lines && kb_per_split >= 12;
+    return kb_per_split >= (!fused ? 2 : whole_lines ? 8 : 16);
 }
 
 }  // namespace
@@ -1051,7 +1054,7 @@ hipError_t launch_tile(const GemmArgs& g, int variant, int ksplit, float* partia
     case TILE_256x128: return launch_variant<256, 128, 4, 2, 3>(g, ksplit, partial, mailbox, s);
     case TILE_128x192: return launch_variant<128, 192, 4, 2, 3>(g, ksplit, partial, mailbox, s);
     case TILE_128x128:
-        return four_waves(g, ksplit, mailbox != nullptr) ? launch_variant<128, 128, 2, 2, 4, false>(g, ksplit, partial, mailbox, s)
+        return four_waves(g, ksplit, mailbox != nullptr) ? launch_variant<128, 128, 2, 2, 4>(g, ksplit, partial, mailbox, s)
                                                          : launch_variant<128, 128, 2, 4, 4>(g, ksplit, partial, mailbox, s);
     case TILE_64x64: return launch_variant<64, 64, 2, 2, 4>(g, ksplit, partial, mailbox, s);
     default: return hipErrorInvalidValue;
