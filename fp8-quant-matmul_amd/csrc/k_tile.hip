@@ -974,7 +974,7 @@ hipError_t launch_variant(const GemmArgs& g, int ksplit, float* partial, float* 
 //   other N 1504 x 832 x 2816 in two 12.55 / 12.94, 3728 x 288 x 2560 12.19 / 12.53, from 16 blocks on 2000 ... 3000 x 576
 //   x 7168 1 - 3 % ahead.  Rows off the grid, where two of the copy waves bring A by way of registers, N a multiple of 128:
 //   334 x 4608 x 7168 in two of 28 blocks 24.00 / 22.76, 2340 x 512 x 7168 in three 20.82 / 20.08, 397 x 1536 x 7168 in five of
-//   twelve (reduction kernel) 18.25 / 17.81, 129 x 7168 x 2304 in two of nine 13.08 / 13.37; other N 1621 x 576 x 7168 21.03 /
+//   twelve (reduction kernel) 18.25 / 17.81 (all of 150 workgroups and more; fewer than 128: as before, eight), 129 x 7168 x 2304 in two of nine 13.08 / 13.37; other N 1621 x 576 x 7168 21.03 /
 //   21.42, 3065 x 576 x 7168 25.07 / 24.76 (30 shapes level).  With the reduction kernel behind them and rows on the grid,
 //   four: 512 x 1024 x 7168 in five 14.77 / 13.99.
 //   Unsplit, four: 500 x 4608 x 2048 (off the grid) 13.8 / 12.9 -- but for a single K block, where there is nothing to read
@@ -985,8 +985,10 @@ bool four_waves(const GemmArgs& g, int ksplit, bool fused)
     const bool whole_lines = g.n % 128 == 0;
     if (ksplit == 1)
         return kb_per_split > 1;
-    if (leading_dim(g) % 16 != 0)
-        return whole_lines && kb_per_split >= 12;
+    if (leading_dim(g) % 16 != 0) {
+        const long tiles = (long)((g.m + 127) / 128) * ((g.n + 127) / 128);
+        return whole_lines && kb_per_split >= 12 && tiles * ksplit >= 128;
+    }
     return kb_per_split >= (!fused ? 2 : whole_lines ? 8 : 16);
 }
 

@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("variant,ksplit,m,n,k", [
     *((4, s, 80, 144, 128 * (2 * s - 1)) for s in (2, 3, 4, 5, 6, 7, 8)),   # the last split a block short
     (4, 4, 64, 64, 512), (4, 3, 77, 208, 1024), (4, 8, 117, 80, 2048),              # one block each; rows off the grid
-    (2, 2, 77, 256, 3072), (2, 3, 333, 128, 4736), (2, 2, 145, 384, 7168),          # rows off the grid in 128x128 tiles
+    (2, 2, 333, 2816, 3072), (2, 3, 269, 2048, 4736), (2, 5, 141, 1664, 7680), (2, 2, 145, 384, 7168),  # rows off the grid
     (2, 2, 144, 256, 2048), (2, 2, 144, 256, 1792), (2, 2, 333, 256, 2816),          # either side of where four waves take over
     (2, 2, 144, 208, 4096), (2, 3, 256, 144, 6016), (2, 4, 128, 128, 8192), (2, 2, 400, 272, 3968)])
 def test_splits_added_by_eight_waves(pkg, variant, ksplit, m, n, k):
