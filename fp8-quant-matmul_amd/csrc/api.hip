@@ -1018,15 +1018,134 @@ int workspace_for(size_t need, hipStream_t stream, const Workspace* explicit_ws,
     return acquire_workspace(need, stream, out);
 }
 
+constexpr int GROUPED_NOT_APPLICABLE = -1000;
+
+// A grouped launch of the persistent kernels that leaves a third of the CUs without a tile while each tile walks a long K
+// range is not made: single problems split K (one group of 200 x 4096 x 7168: 19 us against 52 us, two: 42 against 56 us;
+// four groups of 1536 x 7168: level; with K = 2048 one group 13.4 against 15.6 us, two 26 against 19 us).
+bool grouped_leaves_cus_idle(const GroupTable& tab, int n, int k, int variant)
+{
+    return tab.groups <= 8 && k >= 2048 && grouped_tiles(tab, n, variant) < 160;
+}
+
+// What the persistent kernels take for a grouped launch of tall groups: their cheapest shape, and the copies of A into
+// padded rows; no end where they would not run it.
+double grouped_persistent_cost(const GroupTable& tab, int n, int k)
+{
+    double best = 1e300;
+    int variant = -1;
+    for (int v = 0; v < TILE_VARIANT_COUNT; ++v) {
+        if (v == TILE_64x64 || (persistent_only(v) && !persistent_only_auto(v)))
+            continue;
+        const double cost = grouped_tile_cost(tab, n, k, v);
+        if (cost < best)
+            best = cost, variant = v;
+    }
+    if (grouped_leaves_cus_idle(tab, n, k, variant))
+        return 1e300;
+    double copied = 0;
+    for (int g = 0; g < tab.groups; ++g)
+        copied += tab.m[g] % 16 != 0 ? 2.0 * tab.m[g] * k : 0.0;
+    return best + (copied > 0 ? 2.9 + copied / 4.5e6 : 0.0);
+}
+
+// What a tile of 64x64 or 128x128 per workgroup takes, us: launch, rounds of 256 workgroups (two small ones share a CU, so a
+// round begun is not a whole one) x (start and store + K blocks), the hand-over of K splits, and the operands' way.  Fitted
+// to 784 plans of 220 random grouped launches (2 - 64 groups of 65 - 2048 rows, 256 ... 8192 x 256 ... 7168, three quarters
+// off the row grid, three sets of operands in turn), which it reproduces within 8.5 % (standard deviation).
+double grouped_each_cost(const GroupTable& tab, int n, int k, int variant, int ksplit, bool ragged)
+{
+    const bool small = variant == TILE_64x64;
+    const long tiles = grouped_tiles(tab, n, variant);
+    const long items = (ksplit > 1 ? (tiles + 7) / 8 * 8 : tiles) * ksplit, rounds = (items + NUM_CU - 1) / NUM_CU;
+    const int blocks = (k / 128 + ksplit - 1) / ksplit;
+    double m = 0;
+    for (int g = 0; g < tab.groups; ++g)
+        m += tab.m[g];
+    const double megabytes = (m * k + (double)tab.groups * n * k + 2.0 * m * n) * 1e-6;
+    const double handed = ksplit - 1;
+    if (small) {
+        const double turns = rounds > 1 ? 0.66 * (double)rounds + 0.34 * (double)items / NUM_CU : 1.0;
+        return 2.8 + turns * (0.93 + blocks * (ragged ? 0.4 : 0.35)) + (ksplit > 1 ? 0.57 + 0.4 * handed : 0.0) + 0.02 * megabytes;
+    }
+    return 1.4 + (double)rounds * (3.3 + blocks * (ragged ? 0.6 : 0.42) * (n % 128 ? 1.06 : 1.0)) +
+           (ksplit > 1 ? 1.0 + 1.67 * handed : 0.0) + 0.11 * megabytes;
+}
+
+struct EachPlan { int variant; int ksplit; double cost; };
+EachPlan grouped_each_plan(const GroupTable& tab, int n, int k, const Config& cfg, bool can_split, bool ragged)
+{
+    const int nkb = k / 128;
+    EachPlan best{-1, 1, 1e300};
+    for (const int v : {TILE_64x64, TILE_128x128}) {
+        if (cfg.force_variant >= 0 && v != cfg.force_variant)
+            continue;
+        const size_t mail = (size_t)grouped_tiles(tab, n, v) * (v == TILE_64x64 ? 1 : 4) * 16384;
+        for (int ks = 1; ks <= (v == TILE_64x64 ? 8 : 3); ++ks) {
+            if (cfg.force_ksplit > 0 && can_split && ks != cfg.force_ksplit)
+                continue;
+            // (off the row grid, where A comes through registers, not over a hundred K blocks for a CU: six groups of 3741 rows,
+            // 1536 x 7168, 79.7 us with copies and 256x128 tiles, 91.3 with 128x128; 35 of 27064, 576 x 7168, 243 / 246)
+            const long items = grouped_tiles(tab, n, v) * ks;
+            if (ragged && cfg.force_variant < 0 && (items + NUM_CU - 1) / NUM_CU * ((nkb + ks - 1) / ks) > 100)
+                continue;
+            if (ks > 1 && (!can_split || (ks - 1) * ((nkb + ks - 1) / ks) >= nkb || mail * (ks - 1) > SPLIT_MAILBOX_BYTES))
+                continue;
+            const double cost = grouped_each_cost(tab, n, k, v, ks, ragged);
+            if (cost < best.cost)
+                best = EachPlan{v, ks, cost};
+        }
+    }
+    return best;
+}
+
+// Tall groups with a tile of 64x64 or 128x128 per workgroup (launch_tile_each): A's rows as they are, K split where the
+// tiles are few.  Against the persistent kernels behind copies of A into padded rows, or the groups one by one, where the
+// estimates have it ahead: the 220 launches above 21 % faster in the geometric mean, none slower by more than 1 % (three groups
+// of 705 rows, 448 x 5632, one by one 27.0 us, now 14.0; 31 of 65 - 180, 576 x 7168, 72.9 / 34.1; four of 4608 x 2304 59.6 / 26.3;
+// 14 of 528 x 640 14.9 / 9.5).  N < 256 is not measured and stays.  A pinned shape comes here with persistent = 0.
+int run_grouped_each(GroupTable tab, int n, int k, hipStream_t s, const Config& cfg, const Workspace* explicit_ws)
+{
+    const bool pinned = cfg.force_variant >= 0;
+    bool ragged;
+    if (n < 256 || cfg.persistent == 1 || (pinned ? cfg.persistent != 0 : cfg.force_ksplit > 0) ||
+        !tile_each_supports(tab, n, k, pinned ? cfg.force_variant : TILE_64x64, &ragged))
+        return GROUPED_NOT_APPLICABLE;
+    const double other = pinned ? 1e300 : grouped_persistent_cost(tab, n, k);
+    const bool one_by_one = !pinned && other == 1e300;  // there, single problems may split K with the reduction kernel
+    bool can_split = cfg.fused_ok && cfg.fused_mode != 0 && (!explicit_ws || explicit_ws->zeroed);
+    EachPlan p{-1, 1, 1e300};
+    Workspace w{nullptr, 0, false};
+    for (;; can_split = false) {
+        p = grouped_each_plan(tab, n, k, cfg, can_split, ragged);
+        if (p.variant < 0 || p.cost >= other || (one_by_one && !can_split))
+            return GROUPED_NOT_APPLICABLE;
+        if (p.ksplit == 1 || (placement_ok(s) && workspace_for(with_header(0, true), s, explicit_ws, &w) == FP8GEMM_OK))
+            break;
+    }
+    const hipError_t e = launch_tile_each(tab, n, k, p.variant, p.ksplit, p.ksplit > 1 ? ws_mailbox(w) : nullptr, s);
+    if (e == hipSuccess) {
+        snprintf(t_name_buf, sizeof(t_name_buf), "%s_k%d%s_grouped%d", tile_variant_name(p.variant), p.ksplit,
+                 p.ksplit > 1 ? "f" : "", tab.groups);
+        t_last_kernel = t_name_buf;
+        t_plan_unnamed = false;
+    }
+    return (int)e;
+}
+
 // One grouped launch for the problems of `tab` (same n and k): the decode kernel when every group has at
 // most 64 rows (decode = true), else the persistent tile kernel.  Groups off the 16-byte grid (n, or for the
 // tile kernel m, not a multiple of 16; an operand off a 16-byte boundary) run on zero-padded copies in the
 // workspace: one launch for those of a and a_scale, one each for b and c where they need it.  Returns GROUPED_NOT_APPLICABLE when it cannot run (the caller
 // then takes the groups one by one).
-constexpr int GROUPED_NOT_APPLICABLE = -1000;
 int run_grouped_table(const GroupTable& tab, int n, int k, bool decode, hipStream_t s, const Config& cfg,
                       const Workspace* explicit_ws)
 {
+    if (!decode) {
+        const int rc = run_grouped_each(tab, n, k, s, cfg, explicit_ws);
+        if (rc != GROUPED_NOT_APPLICABLE)
+            return rc;
+    }
     const long long lim = 0x7FFFFFFFll;
     const int n16 = (n + 15) & ~15;
     const size_t nkb = (size_t)k / 128;
@@ -1125,10 +1244,7 @@ int run_grouped_table(const GroupTable& tab, int n, int k, bool decode, hipStrea
         variant = grouped_variant(pt, n16, k, cfg);
         if (variant < 0)
             return GROUPED_NOT_APPLICABLE;
-        // A launch that leaves a third of the CUs without a tile while each tile walks a long K range: single
-        // problems split K (one group of 200 x 4096 x 7168: 19 us against 52 us, two: 42 against 56 us; four groups
-        // of 1536 x 7168: level; with K = 2048 one group 13.4 against 15.6 us, two 26 against 19 us).
-        if (cfg.force_variant < 0 && tab.groups <= 8 && k >= 2048 && grouped_tiles(pt, n16, variant) < 160)
+        if (cfg.force_variant < 0 && grouped_leaves_cus_idle(pt, n16, k, variant))
             return GROUPED_NOT_APPLICABLE;
     }
     hipError_t e = hipSuccess;

@@ -73,13 +73,13 @@ __device__ __forceinline__ v4i shift_right_bytes(v4i v, uint32_t by)
     return __builtin_bit_cast(v4i, x >> (8 * by));
 }
 
-// RAGGED: M is no multiple of 16 (see the head of this file)
+// One tile of one problem, in K blocks blockIdx.y * kb_per_split ...: the tile at (m0, n0), number `pid` of the launch.
+// RAGGED: M may be no multiple of 16 (see the head of this file)
 template <int BM, int BN, int WM, int WN, int NS, bool SPLIT, bool RAGGED>
-__global__ void __launch_bounds__(NTHREADS)
-tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
-                 const float* __restrict__ a_scale, const float* __restrict__ b_scale,
-                 uint16_t* __restrict__ c, float* __restrict__ partial, float* mailbox,
-                 int M, int lda, int N, int K, int tiles_m, int tiles_n, int kb_per_split, int group_m)
+__device__ __forceinline__ void
+tile_body(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b, const float* __restrict__ a_scale,
+          const float* __restrict__ b_scale, uint16_t* __restrict__ c, float* __restrict__ partial, float* mailbox,
+          int M, int lda, int N, int K, int m0, int n0, int pid, int kb_per_split)
 {
     using S = TileShape<BM, BN, WM, WN, NS>;
     // WM x WN waves multiply: all eight, or the first four of the two smaller tiles (AHEAD)
@@ -115,24 +115,6 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
     const int copier = wave & (COPIERS - 1);
     const int wm = wave % WM, wn = (wave / WM) % WN;
     const bool compute = !AHEAD || wave < NCW;
-
-    // ---- which tile: consecutive workgroup ids land on different XCDs (id % 8), so give
-    // each XCD a contiguous run of tile numbers, and walk tiles in groups of group_m rows
-    // so that the tiles an XCD works on together share A and B panels in its L2 (the host picks
-    // group_m so that an XCD's co-resident tiles form a block that is about square in bytes).
-    const int T = tiles_m * tiles_n;
-    const int pid = blockIdx.x;
-    if (pid >= T)  // grid.x is rounded up to a multiple of 8 when the K splits of a tile have to share an XCD
-        return;
-    const int xcd = pid & 7, q8 = T >> 3, r8 = T & 7;
-    const int logical = xcd * q8 + (xcd < r8 ? xcd : r8) + (pid >> 3);
-    const int per_group = group_m * tiles_n;
-    const int group = logical / per_group;
-    const int first_m = group * group_m;
-    const int gsz = (tiles_m - first_m < group_m) ? (tiles_m - first_m) : group_m;
-    const int in_group = logical - group * per_group;
-    const int m0 = (first_m + in_group % gsz) * BM;
-    const int n0 = (in_group / gsz) * BN;
 
     const int nkb = K / KBLOCK;
     const int kb0 = blockIdx.y * kb_per_split;
@@ -846,6 +828,73 @@ tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
     }
 }
 
+// Which tile: consecutive workgroup ids land on different XCDs (id % 8), so each XCD gets a contiguous run of tile
+// numbers.  -1: grid.x is rounded up to a multiple of 8 when the K splits of a tile have to share an XCD.
+__device__ __forceinline__ int tile_number(int T)
+{
+    const int pid = blockIdx.x;
+    if (pid >= T)
+        return -1;
+    const int xcd = pid & 7, q8 = T >> 3, r8 = T & 7;
+    return xcd * q8 + (xcd < r8 ? xcd : r8) + (pid >> 3);
+}
+
+// ... walked in groups of group_m rows so that the tiles an XCD works on together share A and B panels in its L2 (the host
+// picks group_m so that an XCD's co-resident tiles form a block that is about square in bytes).
+template <int BM, int BN>
+__device__ __forceinline__ void tile_origin(int logical, int tiles_m, int tiles_n, int group_m, int& m0, int& n0)
+{
+    const int per_group = group_m * tiles_n;
+    const int group = logical / per_group;
+    const int first_m = group * group_m;
+    const int gsz = (tiles_m - first_m < group_m) ? (tiles_m - first_m) : group_m;
+    const int in_group = logical - group * per_group;
+    m0 = (first_m + in_group % gsz) * BM;
+    n0 = (in_group / gsz) * BN;
+}
+
+template <int BM, int BN, int WM, int WN, int NS, bool SPLIT, bool RAGGED>
+__global__ void __launch_bounds__(NTHREADS)
+tile_gemm_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
+                 const float* __restrict__ a_scale, const float* __restrict__ b_scale,
+                 uint16_t* __restrict__ c, float* __restrict__ partial, float* mailbox,
+                 int M, int lda, int N, int K, int tiles_m, int tiles_n, int kb_per_split, int group_m)
+{
+    const int logical = tile_number(tiles_m * tiles_n);
+    if (logical < 0)
+        return;
+    int m0, n0;
+    tile_origin<BM, BN>(logical, tiles_m, tiles_n, group_m, m0, n0);
+    tile_body<BM, BN, WM, WN, NS, SPLIT, RAGGED>(a, b, a_scale, b_scale, c, partial, mailbox, M, lda, N, K, m0, n0,
+                                                 blockIdx.x, kb_per_split);
+}
+
+// The problems of `tab` (same N and K, own M), a tile per workgroup and K split, tiles numbered one problem after the other.
+// What small grouped launches of tall groups are bound by is latency and idle CUs: the persistent kernels want A's rows on the
+// grid (a copy launch, 3 - 6 us), start in tiles of 128 rows and more, and don't split K, for which the groups used to run
+// one by one.  Here A comes as it lies, in tiles of 64 or 128 rows, K split where the tiles are few; the look-up is one trip to
+// the kernel arguments.  22 groups of 67 - 172 rows, 576 x 7168, 64.9 -> 53.7 us; nine of 2637 rows in all, 48.3 -> 36.8; three of 705,
+// 448 x 5632, 27.0 -> 14.0; eight of 68 - 139, 832 x 384, 8.5 -> 4.5.  In more than a few rounds the persistent kernels, which
+// copy the next tile's blocks while one is stored, are ahead again (seven groups of 4048 rows, 4608 x 7168, 170 against 190).
+template <int BM, int BN, int WM, int WN, int NS, bool SPLIT, bool RAGGED>
+__global__ void __launch_bounds__(NTHREADS)
+tile_gemm_each_kernel(const GroupTable tab, float* mailbox, int N, int K, int tiles_n, int kb_per_split)
+{
+    int logical = tile_number(tab.tile_start[tab.groups]);
+    if (logical < 0)
+        return;
+    // tile_start ascends: how many problems end at or before this tile, looked up by a lane each
+    static_assert(GroupTable::MAX_GROUPS == 64, "a lane for every problem");
+    const int lane = threadIdx.x & 63;
+    const int g = __builtin_popcountll(__builtin_amdgcn_ballot_w64(lane < tab.groups && tab.tile_start[lane + 1] <= logical));
+    logical -= tab.tile_start[g];
+    const int M = tab.m[g];
+    int m0, n0;
+    tile_origin<BM, BN>(logical, (M + BM - 1) / BM, tiles_n, GROUP_M, m0, n0);
+    tile_body<BM, BN, WM, WN, NS, SPLIT, RAGGED>(tab.a[g], tab.b[g], tab.a_scale[g], tab.b_scale[g], tab.c[g], nullptr,
+                                                 mailbox, M, tab.lda[g], N, K, m0, n0, blockIdx.x, kb_per_split);
+}
+
 // sum of the K-split partials in split order, then bf16
 __global__ void __launch_bounds__(256) splitk_reduce_kernel(const float* __restrict__ partial,
                                                             uint16_t* __restrict__ c, size_t mn,
@@ -1061,6 +1110,67 @@ hipError_t launch_tile(const GemmArgs& g, int variant, int ksplit, float* partia
     case TILE_64x64: return launch_variant<64, 64, 2, 2, 4>(g, ksplit, partial, mailbox, s);
     default: return hipErrorInvalidValue;
     }
+}
+
+namespace {
+
+template <int BM, int BN, int WM, int WN, int NS, bool SPLIT, bool RAGGED>
+hipError_t launch_each_typed(GroupTable& tab, int n, int k, int ksplit, float* mailbox, hipStream_t s)
+{
+    using S = TileShape<BM, BN, WM, WN, NS>;
+    const int tiles_n = (n + BN - 1) / BN, nkb = k / KBLOCK;
+    tab.tile_start[0] = 0;
+    for (int g = 0; g < tab.groups; ++g)
+        tab.tile_start[g + 1] = tab.tile_start[g] + ((tab.m[g] + BM - 1) / BM) * tiles_n;
+    const int tiles = tab.tile_start[tab.groups];
+    if (SPLIT && (!mailbox || (size_t)tiles * (ksplit - 1) * BM * BN * 4 > SPLIT_MAILBOX_BYTES))
+        return hipErrorInvalidValue;
+    constexpr auto kern = tile_gemm_each_kernel<BM, BN, WM, WN, NS, SPLIT, RAGGED>;
+    FP8GEMM_ALLOW_LDS(kern, S::LDS_BYTES);
+    launch_kernel(kern, dim3(SPLIT ? (tiles + 7) & ~7 : tiles, ksplit), dim3(NTHREADS), S::LDS_BYTES, s, tab,
+                  SPLIT ? mailbox : nullptr, n, k, tiles_n, (nkb + ksplit - 1) / ksplit);
+    return hipGetLastError();
+}
+
+template <int BM, int BN, int WM, int WN, int NS>
+hipError_t launch_each_variant(GroupTable& tab, bool ragged, int n, int k, int ksplit, float* mailbox, hipStream_t s)
+{
+    if (ragged)
+        return ksplit > 1 ? launch_each_typed<BM, BN, WM, WN, NS, true, true>(tab, n, k, ksplit, mailbox, s)
+                          : launch_each_typed<BM, BN, WM, WN, NS, false, true>(tab, n, k, 1, nullptr, s);
+    return ksplit > 1 ? launch_each_typed<BM, BN, WM, WN, NS, true, false>(tab, n, k, ksplit, mailbox, s)
+                      : launch_each_typed<BM, BN, WM, WN, NS, false, false>(tab, n, k, 1, nullptr, s);
+}
+
+}  // namespace
+
+// every problem as a single one, for the form that takes it; one off the 16-row grid takes all to the form for such
+bool tile_each_supports(const GroupTable& tab, int n, int k, int variant, bool* ragged)
+{
+    if ((variant != TILE_64x64 && variant != TILE_128x128) || tab.groups < 1 || tab.groups > GroupTable::MAX_GROUPS)
+        return false;
+    *ragged = false;
+    for (int g = 0; g < tab.groups; ++g)
+        *ragged = *ragged || tab.m[g] % 16 != 0;
+    for (int g = 0; g < tab.groups; ++g) {
+        GemmArgs ga{tab.a[g], tab.b[g], tab.a_scale[g], tab.b_scale[g], tab.c[g], tab.m[g], n, k, tab.lda[g]};
+        if (tab.m[g] < 16 || tab.lda[g] != tab.m[g])
+            return false;
+        ga.m = ga.lda = tab.m[g] & ~15;  // the addresses and n
+        if (!tile_supports(ga))
+            return false;
+    }
+    return true;
+}
+
+hipError_t launch_tile_each(GroupTable& tab, int n, int k, int variant, int ksplit, float* mailbox, hipStream_t s)
+{
+    bool ragged;
+    const int nkb = k / KBLOCK;
+    if (ksplit < 1 || (ksplit - 1) * ((nkb + ksplit - 1) / ksplit) >= nkb || !tile_each_supports(tab, n, k, variant, &ragged))
+        return hipErrorInvalidValue;
+    return variant == TILE_64x64 ? launch_each_variant<64, 64, 2, 2, 4>(tab, ragged, n, k, ksplit, mailbox, s)
+                                 : launch_each_variant<128, 128, 2, 2, 4>(tab, ragged, n, k, ksplit, mailbox, s);
 }
 
 hipError_t launch_splitk_reduce(const GemmArgs& g, int ksplit, const float* partial, hipStream_t s)

@@ -109,6 +109,10 @@ struct GroupTable {
 };
 bool tile_grouped_supports(const GroupTable& tab, int n, int k, int variant);
 hipError_t launch_tile_grouped(GroupTable& tab, int n, int k, int variant, int workgroups, hipStream_t s);
+// The same problems with a tile of 64x64 or 128x128 per workgroup, rows off the 16-row grid as they are (`ragged`), their K
+// splits added inside the kernel: mailbox = SPLIT_MAILBOX_BYTES as above, not used with ksplit 1.  lda has to be m.
+bool tile_each_supports(const GroupTable& tab, int n, int k, int variant, bool* ragged);
+hipError_t launch_tile_each(GroupTable& tab, int n, int k, int variant, int ksplit, float* mailbox, hipStream_t s);
 // ... of the two large tiles, 256x192 and 256x256 (called by the two functions above, which check the arguments)
 // The tiles of a last round of 256x256 that would leave half the workgroups or more without one are cut into halves
 // (256x128) or quarters (128x128), one for each workgroup.

@@ -142,11 +142,13 @@ int fp8_block_gemm_set_fused_reduction(int mode);
  * own (its own tile count, K blocks priced for operands from HBM: mostly the 256x256 tile, which streams a
  * group's B once per 256 rows in pieces of 256 bytes).  A tile launch of at most 8 groups that
  * would leave more than a third of the CUs without a tile while K >= 2048 is not made: those groups run one by
- * one, where the dispatcher splits K.  A launch holds FP8GEMM_MAX_GROUPS problems; more of a kind run as
+ * one, where the dispatcher splits K.  Where an estimate has it ahead, tall groups run instead as ONE launch of the plain
+ * tile kernel, a tile of 64x64 or 128x128 per workgroup ("tile64x64_kNf_groupedG"; n >= 256, m[g] >=
+ * 16, operands 16-byte aligned): row counts off the grid as they are, without copies, and the K range of few tiles split and added inside the kernel,
+ * given a zeroed workspace header as for a single problem.  A launch holds FP8GEMM_MAX_GROUPS problems; more of a kind run as
  * the fewest launches that hold them, of equal size, one after the other on the stream ("...groupedGxL":
  * L launches, the last of G groups).  Each C[g] is bit-identical to
- * what fp8_block_gemm_stream gives for that problem with the same tile shape (decode kernel: with the
- * same K split).  No counterpart in the
+ * what fp8_block_gemm_stream gives for that problem with the same tile shape and K split.  No counterpart in the
  * reference, which launches one problem at a time (/root/reference/check.cu:106-114). */
 #define FP8GEMM_MAX_GROUPS 64
 int fp8_block_gemm_grouped(int groups, const void* const* a, const void* const* b,
@@ -197,7 +199,7 @@ size_t fp8_block_gemm_workspace_bytes_ex(int m, int n, int k, const fp8gemm_opti
  * several host threads on several streams with distinct workspaces, and under stream capture).
  * fp8_block_gemm_grouped_workspace_bytes_ex bounds the workspace for any alignment of the operands;
  * with less than that (or none) the groups that need a workspace run one by one, or the call returns
- * FP8GEMM_E_WORKSPACE when a single group needs more than it was given.  The decode kernel splits K
+ * FP8GEMM_E_WORKSPACE when a single group needs more than it was given.  Grouped launches split K
  * only with FP8GEMM_FLAG_WORKSPACE_ZEROED.  No counterpart in the reference (one problem at a time on
  * stream 0, /root/reference/check.cu:106-119). */
 int fp8_block_gemm_grouped_ex(int groups, const void* const* a, const void* const* b,

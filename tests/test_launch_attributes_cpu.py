@@ -76,3 +76,15 @@ def test_tall_groups_in_one_round(program, groups, m, n, k, columns):
     assert len(names) == 1, names
     name = subprocess.run(["c++filt", names[0]], check=True, capture_output=True, text=True).stdout
     assert f"tile_gemm_large_grouped_kernel<{columns}," in name, name
+
+
+# small launches of tall groups: a tile per workgroup, with K split where the tiles are few; large ones, narrow N, rows off the
+# grid over a hundred K blocks for a CU, a header that is not there: the persistent kernels
+@pytest.mark.parametrize("groups,m,n,k,kernel", [(8, 100, 512, 512, "tile_gemm_each_kernel<64, 64, 2, 2, 4, false, true>"),
+                                                 (20, 112, 576, 1024, "tile_gemm_each_kernel<64, 64, 2, 2, 4, false, false>"),
+                                                 (9, 333, 976, 2048, "tile_gemm_each_kernel<128, 128, 2, 2, 4, false, true>"),
+                                                 (8, 1024, 7168, 2048, "tile_gemm_large_grouped_kernel<256"), (8, 100, 240, 512, "tile_gemm_grouped_kernel<"),
+                                                 (35, 773, 576, 7168, "tile_gemm_large_grouped_kernel<256")])
+def test_tall_groups_with_a_tile_per_workgroup(program, groups, m, n, k, kernel):
+    names = subprocess.run(["c++filt"], input="\n".join(program(m, n, k, 0, groups)), check=True, capture_output=True, text=True).stdout
+    assert kernel in names, names
