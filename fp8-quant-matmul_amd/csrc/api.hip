@@ -967,6 +967,17 @@ double grouped_tile_cost(const GroupTable& tab, int n, int k, int variant)
     if (variant == TILE_256x256)
         return large_tile_cost(grouped_tiles(tab, n, variant), k, 1.2);
     const long tiles = grouped_tiles(tab, n, variant);
+    // 128x256 tiles where they are no more than tiles of 256x256 would be, every group's last 256 rows being 128 at most: half
+    // of A's slots go to a third stage, more of B is on its way (19 launches of up to 128 rows a group 0.2 - 15 % ahead of 256x256,
+    // 10 % on average).  Where they are more it is open, 15 of 25 with 1.08 to 1.65 times as many behind by up to 50 %.
+    if (variant == TILE_128x256) {
+        const int nkb = k / 128;
+        if (nkb < 3 || tiles != grouped_tiles(tab, n, TILE_256x256))
+            return 1e300;
+        const bool tail = large_tile_tail(tiles, k, NUM_CU) != Tail::NONE;
+        const long whole = tail ? tiles / NUM_CU : (tiles + NUM_CU - 1) / NUM_CU;
+        return 1.79 + (double)whole * 0.89 * (4.5 + nkb * 1.6) + (tail ? 3.0 + nkb * 0.7 : 0.0);
+    }
     // (256x192 tiles in a single round, where 256x256 tiles are fewer still: 18 of 20 random launches are 1 - 13 % faster in
     // the smaller ones and two 1 % slower, 384 - 624 rows, 4960 x 1664, 140 or 182 tiles, 25.3 / 22.3 us, 16 of 96 - 656, 1232 x
     // 1792, 28.3 / 24.9, six of 80 - 336, 4608 x 7168, 93.1 / 88.3; and fewer of them are too few for one launch, below)
@@ -989,7 +1000,7 @@ int grouped_variant(const GroupTable& tab, int n, int k, const Config& cfg)
     int best_v = -1;
     double best = 1e300;
     const int fv = cfg.force_variant;
-    for (int v = 0; v < TILE_VARIANT_COUNT; ++v) {
+    for (int v = 0; v <= TILE_128x256; ++v) {
         if ((fv >= 0 && v != fv) || !tile_grouped_supports(tab, n, k, v))
             continue;
         if (fv < 0 && persistent_only(v) && !persistent_only_auto(v))
@@ -1034,7 +1045,7 @@ double grouped_persistent_cost(const GroupTable& tab, int n, int k)
 {
     double best = 1e300;
     int variant = -1;
-    for (int v = 0; v < TILE_VARIANT_COUNT; ++v) {
+    for (int v = 0; v <= TILE_128x256; ++v) {
         if (v == TILE_64x64 || (persistent_only(v) && !persistent_only_auto(v)))
             continue;
         const double cost = grouped_tile_cost(tab, n, k, v);

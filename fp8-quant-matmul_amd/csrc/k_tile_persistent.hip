@@ -70,9 +70,48 @@ hipError_t launch_grouped_variant(GroupTable& tab, int n, int k, int workgroups,
     return hipGetLastError();
 }
 
+// 128x256 tiles for groups of at most 128 rows, which bring more B than anything else: a launch streams every B once, from
+// HBM, and is bound by the bytes that its CUs keep on their way there.  Tiles of 256x256 ask for B in the same whole pieces of
+// 256 bytes, but half of their two slots is for rows that do not exist; here three slots fit, and a tile has half the MFMAs.
+// A last round that leaves half of the workgroups idle is cut into 128x128 halves (large_tile_tail).  256x256 / this: 28 groups
+// of 68 - 128 rows, 4608 x 7168, 229 / 206 us (925 MB of B: 4.5 TB/s); 64 of 3504 x 2944 208 / 185; 31 of 7168 x 2304 154 / 140; without
+// halves 233 / 209 and 152 / 146.  B past the caches on top: -5.6 ... +2 %, +15 % where B fits the caches; not kept.
+template <bool HALVES>
+__global__ void __launch_bounds__(NTHREADS) tile_gemm_grouped_wide_kernel(const GroupTable tab, int N, int K, int tiles_n)
+{
+    const TileProblem none{nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0};
+    using Whole = std::conditional_t<HALVES, FullRounds<128, 256>, AllTiles<128, 256>>;
+    persistent_body<128, 256, 2, 4, 3, 64, true, Whole>(none, &tab, N, K, 0, tiles_n, (int)threadIdx.x);
+    if constexpr (HALVES) {
+        __syncthreads();  // nobody reads the ring any more
+        persistent_body<128, 128, 2, 4, 4, 128, true, LeftOver<128, 256, 128, 128>>(none, &tab, N, K, 0, tiles_n, (int)threadIdx.x);
+    }
+}
+
+hipError_t launch_grouped_wide(GroupTable& tab, int n, int k, int workgroups, hipStream_t s)
+{
+    constexpr int WHOLE = TileShape<128, 256, 2, 4, 3>::LDS_BYTES, PIECES = TileShape<128, 128, 2, 4, 4>::LDS_BYTES;
+    constexpr int LDS_TOTAL = WHOLE > PIECES ? WHOLE : PIECES;
+    const int tiles_n = (n + 255) / 256;
+    tab.tile_start[0] = 0;
+    for (int g = 0; g < tab.groups; ++g)
+        tab.tile_start[g + 1] = tab.tile_start[g] + ((tab.m[g] + 127) / 128) * tiles_n;
+    if (large_tile_tail(tab.tile_start[tab.groups], k, workgroups) == Tail::NONE) {
+        constexpr auto kern = tile_gemm_grouped_wide_kernel<false>;
+        FP8GEMM_ALLOW_LDS(kern, LDS_TOTAL);
+        launch_kernel(kern, dim3(workgroups), dim3(NTHREADS), LDS_TOTAL, s, tab, n, k, tiles_n);
+    } else {
+        constexpr auto kern = tile_gemm_grouped_wide_kernel<true>;
+        FP8GEMM_ALLOW_LDS(kern, LDS_TOTAL);
+        launch_kernel(kern, dim3(workgroups), dim3(NTHREADS), LDS_TOTAL, s, tab, n, k, tiles_n);
+    }
+    return hipGetLastError();
+}
+
 int persistent_stages(int variant)
 {
     switch (variant) {
+    case TILE_128x256: return 4;  // of the halves
     case TILE_256x192: return 2;
     case TILE_256x128: return 3;
     case TILE_128x192: return 3;
@@ -88,7 +127,7 @@ int persistent_stages(int variant)
 bool tile_persistent_supports(const GemmArgs& g, int variant)
 {
     const int stages = persistent_stages(variant);
-    return stages > 0 && tile_supports(g) && g.k / KBLOCK >= stages - 1;
+    return stages > 0 && variant < TILE_VARIANT_COUNT && tile_supports(g) && g.k / KBLOCK >= stages - 1;
 }
 
 hipError_t launch_tile_persistent(const GemmArgs& g, int variant, int workgroups, hipStream_t s)
@@ -131,6 +170,7 @@ hipError_t launch_tile_grouped(GroupTable& tab, int n, int k, int variant, int w
     case TILE_256x128: return launch_grouped_variant<256, 128, 4, 2, 3, 128>(tab, n, k, workgroups, s);
     case TILE_128x192: return launch_grouped_variant<128, 192, 4, 2, 3, 128>(tab, n, k, workgroups, s);
     case TILE_128x128: return launch_grouped_variant<128, 128, 2, 4, 4, 128>(tab, n, k, workgroups, s);
+    case TILE_128x256: return launch_grouped_wide(tab, n, k, workgroups, s);
     default: return hipErrorInvalidValue;
     }
 }

@@ -80,7 +80,8 @@ constexpr size_t SPLIT_MAILBOX_BYTES = (size_t)16 << 20;
 // adds the other splits' accumulators itself and writes c, with the same arithmetic, and `partial` is
 // not used.  The latter needs xcd_placement_confirmed() and tile_mailbox_bytes() <= SPLIT_MAILBOX_BYTES.
 enum TileVariant { TILE_256x192 = 0, TILE_256x128 = 1, TILE_128x128 = 2, TILE_128x192 = 3,
-                   TILE_64x64 = 4, TILE_256x192_W4 = 5, TILE_256x256 = 6, TILE_VARIANT_COUNT };
+                   TILE_64x64 = 4, TILE_256x192_W4 = 5, TILE_256x256 = 6, TILE_VARIANT_COUNT,
+                   TILE_128x256 = TILE_VARIANT_COUNT };  // grouped launches only, not to be asked for by number
 bool tile_supports(const GemmArgs& g);
 // row counts off the 16-byte grid, taken as they are (launch_tile, plain form)
 bool tile_ragged_supports(const GemmArgs& g, int variant);

@@ -140,7 +140,7 @@ int fp8_block_gemm_set_fused_reduction(int mode);
  * both kinds launches each kernel once, unless the small groups are few beside the taller ones (at most a third
  * as many), which then join the tile launch.  The tile shape of a grouped launch comes from a cost model of its
  * own (its own tile count, K blocks priced for operands from HBM: mostly the 256x256 tile, which streams a
- * group's B once per 256 rows in pieces of 256 bytes).  A tile launch of at most 8 groups that
+ * group's B once per 256 rows in pieces of 256 bytes; 128x256 where no group has more rows).  A tile launch of at most 8 groups that
  * would leave more than a third of the CUs without a tile while K >= 2048 is not made: those groups run one by
  * one, where the dispatcher splits K.  Where an estimate has it ahead, tall groups run instead as ONE launch of the plain
  * tile kernel, a tile of 64x64 or 128x128 per workgroup ("tile64x64_kNf_groupedG"; n >= 256, m[g] >=

@@ -1,4 +1,4 @@
-"""Tall groups in one launch with a tile per workgroup: both tile shapes, rows on and off the 16-row grid, with and without K
+"""Tall groups in one launch, with a tile per workgroup and in 128x256 tiles: both tile shapes, rows on and off the 16-row grid, with and without K
 splits, against the oracle element by element and bit for bit against the groups one by one; and the launches that dispatch
 makes of them."""
 import numpy as np
@@ -70,3 +70,18 @@ def test_automatic_dispatch(pkg, ms, n, k, splits):
         assert "f_grouped" not in name, name
         for g, (h, m) in enumerate(zip(host, ms)):
             _assert_every_element(again[g], *h, m, n, k, f"{name} group {g}")
+
+
+# whole rounds; halves of a last round that would leave a quarter of the workgroups or less, or half of them, with a tile; columns
+# that end in either half of a tile, rows on and off the grid, the fewest and the most that a group of one tile has
+@pytest.mark.parametrize("ms,n,k", [([65 + 7 * g for g in range(9)], 7168, 384), ([128] * 8 + [16], 7216, 2048), ([72 + g for g in range(12)], 7168, 1024),
+                                    ([80] * 12 + [128], 6640, 1152), ([127] * 20, 2576, 896)])
+def test_groups_of_one_128x256_tile_row(pkg, ms, n, k):
+    host, got, name = _call(pkg, ms, n, k, pkg.Options(persistent=1))
+    assert name.endswith(f"tile128x256_k1_grouped{len(ms)}"), name
+    _, general, pinned = _call(pkg, ms, n, k, pkg.Options(tile_variant=6))
+    assert pinned.endswith(f"tile256x256_k1_grouped{len(ms)}"), pinned
+    for g, m in enumerate(ms):
+        assert np.array_equal(got[g], general[g]), f"group {g}: {name} and {pinned} differ"
+        if g in (0, len(ms) - 1):
+            _assert_every_element(got[g], *host[g], m, n, k, f"{name} group {g}")
