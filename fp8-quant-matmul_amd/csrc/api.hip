@@ -1145,7 +1145,7 @@ int run_grouped_each(GroupTable tab, int n, int k, hipStream_t s, const Config& 
 }
 
 // One grouped launch for the problems of `tab` (same n and k): the decode kernel when every group has at
-// most 64 rows (decode = true), else the persistent tile kernel.  Groups off the 16-byte grid (n, or for the
+// most 64 rows (decode = true), else a tile kernel (run_grouped_each, or the persistent one).  For the latter, groups off the 16-byte grid (n, or for the
 // tile kernel m, not a multiple of 16; an operand off a 16-byte boundary) run on zero-padded copies in the
 // workspace: one launch for those of a and a_scale, one each for b and c where they need it.  Returns GROUPED_NOT_APPLICABLE when it cannot run (the caller
 // then takes the groups one by one).
@@ -1445,7 +1445,7 @@ static int run_grouped(int groups, const void* const* a, const void* const* b, c
     if (!a || !b || !a_scale || !b_scale || !c || !m)
         return FP8GEMM_E_NULLPTR;
     // Groups of at most 64 rows (an MoE layer in a decode step) go to the decode kernel, which streams
-    // every group's B once in whole lines; taller groups to the persistent tile kernel.  A pinned tile
+    // every group's B once in whole lines; taller groups to the tile kernels.  A pinned tile
     // shape sends everything to the tile kernel.
     // A few small groups beside many taller ones ride along in the tile launch: their tiles fill its last round,
     // which costs less than a launch of their own (15 small + 49 tall groups, N = 2048, K = 7168: 258 us against

@@ -85,3 +85,32 @@ def test_groups_of_one_128x256_tile_row(pkg, ms, n, k):
         assert np.array_equal(got[g], general[g]), f"group {g}: {name} and {pinned} differ"
         if g in (0, len(ms) - 1):
             _assert_every_element(got[g], *host[g], m, n, k, f"{name} group {g}")
+
+
+@pytest.mark.parametrize("ms,n,k,name", [([67, 83, 99], 528, 3840, "f_grouped3"), ([90] * 12, 6640, 1152, "tile128x256_k1_grouped12")])
+def test_in_a_graph(pkg, ms, n, k, name):
+    """every replay, eager work in between, has the eager result"""
+    import torch
+    dev = [_dev(*oracle.make_inputs(m, n, k, 4700 + g + m, 0.5, 30.0)) for g, m in enumerate(ms)]
+    outs = [torch.zeros((m, n), dtype=torch.bfloat16, device="cuda") for m in ms]
+    ws = torch.zeros(pkg.grouped_workspace_bytes(ms, n, k), dtype=torch.uint8, device="cuda")
+    opt = pkg.Options(persistent=1 if "256" in name else -1, flags=pkg.FLAG_WORKSPACE_ZEROED)
+
+    def call():
+        pkg.gemm_grouped_ex(*[[d[i] for d in dev] for i in range(4)], outs, ms, n, k, opt, ws, ws.numel(),
+                            torch.cuda.current_stream().cuda_stream)
+    _say(f"[gpu case] grouped in a graph ms={ms} n={n} k={k}")
+    call()
+    torch.cuda.synchronize()
+    assert pkg.last_kernel().endswith(name), pkg.last_kernel()
+    want = [o.clone() for o in outs]
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call()
+    for _ in range(4):
+        for o in outs:
+            o.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(o, w) for o, w in zip(outs, want))
+        call()
