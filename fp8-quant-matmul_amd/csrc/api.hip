@@ -38,6 +38,7 @@ struct Config {
     bool fused_ok = true;
     int fused_mode = -1;  // -1 = by cost, 0 = never, 1 = whenever fused_ok and the plan allows
     bool strips_for_tiles = true;  // 64-column strips may take the place of 64x64 tiles (strips_for_tiles below)
+    size_t partial_room = SIZE_MAX;  // automatic plans keep no more bytes of partial sums in the workspace (fitting_plan)
 };
 Config global_config()
 {
@@ -100,6 +101,7 @@ struct Plan {
     bool wide = false;        // decode family: 128-column strips, K splits added inside the kernel (k_decode.hip)
     bool fused = false;       // tile family, ksplit > 1: the last workgroup of a tile adds the partial tiles (no reduction launch)
     int halves = 1;           // wide decode strips: 128-column halves per strip (2 = 256-column strips, 0 = 64-column ones)
+    double us = 0.0;          // the estimate that chose the plan
 };
 
 // Shapes or addresses the MFMA kernels cannot take (m or n not a multiple of 16, a base not
@@ -340,11 +342,12 @@ struct PlanKey {
     uint32_t low_bits;  // 6 low address bits of a, b, a_scale, b_scale and c
     int selected, force_variant, force_ksplit, persistent, fused_mode;
     int allowed;  // bit 0: fused_ok, bit 1: strips_for_tiles
+    size_t partial_room;
     bool operator==(const PlanKey& o) const
     {
         return m == o.m && n == o.n && k == o.k && lda == o.lda && low_bits == o.low_bits && selected == o.selected &&
                force_variant == o.force_variant && force_ksplit == o.force_ksplit && persistent == o.persistent &&
-               fused_mode == o.fused_mode && allowed == o.allowed;
+               fused_mode == o.fused_mode && allowed == o.allowed && partial_room == o.partial_room;
     }
 };
 struct PlanSlot {
@@ -359,9 +362,9 @@ Plan make_plan(const GemmArgs& g, const Config& cfg)
     const PlanKey key{g.m, g.n, g.k, g.lda,
                       low6(g.a) | low6(g.b) << 6 | low6(g.a_scale) << 12 | low6(g.b_scale) << 18 | low6(g.c) << 24,
                       cfg.selected, cfg.force_variant, cfg.force_ksplit, cfg.persistent, cfg.fused_mode,
-                      (cfg.fused_ok ? 1 : 0) | (cfg.strips_for_tiles ? 2 : 0)};
+                      (cfg.fused_ok ? 1 : 0) | (cfg.strips_for_tiles ? 2 : 0), cfg.partial_room};
     const uint32_t h = ((uint32_t)g.m * 2654435761u) ^ ((uint32_t)g.n * 40503u) ^ ((uint32_t)g.k * 2246822519u) ^
-                       (cfg.fused_ok ? 0x9E3779B9u : 0u);
+                       (cfg.fused_ok ? 0x9E3779B9u : 0u) ^ (cfg.partial_room != SIZE_MAX ? 0x85EBCA6Bu : 0u);
     PlanSlot& slot = slots[(h >> 16 ^ h) & 63];
     if (slot.used && slot.key == key)
         return slot.plan;
@@ -425,6 +428,7 @@ Plan compute_plan(const GemmArgs& g, const Config& cfg)
     Plan decode{FP8GEMM_KERNEL_SKINNY, 0, 1};
     double decode_us = -1.0;  // >= 0: the decode family is a candidate, at this cost
     const bool narrow_ok = skinny_supports(g), wide_ok = decode_strip_supports(g);
+    auto has_room = [&](int ks) { return ks == 1 || (size_t)ks * g.m * g.n * sizeof(float) <= cfg.partial_room; };
     if (selected == FP8GEMM_KERNEL_SKINNY && !narrow_ok && !wide_ok) {
         p.family = -1;
         return p;
@@ -459,6 +463,8 @@ Plan compute_plan(const GemmArgs& g, const Config& cfg)
         }
         if (narrow_ok && !(by_name && cfg.force_variant >= 1)) {
             narrow.ksplit = forced_ks ? forced_ks : skinny_ksplit(g);
+            if (!has_room(narrow.ksplit))
+                narrow.ksplit = 1;
             narrow_us = skinny_cost(g, narrow.ksplit);
         }
         if (wide_ok && (by_name ? cfg.force_variant != 0 : cfg.force_variant < 0)) {
@@ -531,6 +537,7 @@ Plan compute_plan(const GemmArgs& g, const Config& cfg)
         } else {
             decode = wide_us < narrow_us ? wide : narrow;
             decode_us = wide_us < narrow_us ? wide_us : narrow_us;
+            decode.us = decode_us;
             if (by_name || cfg.force_variant >= 0 || cfg.force_ksplit > 0 || !tile_supports(g))
                 return decode;
             // one pass of one round of workgroups: nothing here is faster
@@ -555,6 +562,9 @@ Plan compute_plan(const GemmArgs& g, const Config& cfg)
                 p.ksplit = t.ksplit;
                 decide_persistent(g, p, cfg);
                 decide_fused(g, p, cfg);
+                p.us = tile_cost(g, p.variant, p.ksplit, p.fused);
+                if (!p.fused && !has_room(p.ksplit))
+                    break;
                 return p;
             }
     double best = 1e300, best_256x128 = 1e300;
@@ -598,7 +608,10 @@ Plan compute_plan(const GemmArgs& g, const Config& cfg)
             if (v == TILE_128x128 && ks > 1 && kbs < 8 && fk <= 0 && selected == FP8GEMM_KERNEL_AUTO &&
                 tile_plan_fused(g, v, ks, cfg))
                 continue;
-            const double cst = tile_cost(g, v, ks, tile_plan_fused(g, v, ks, cfg));
+            const bool fused = tile_plan_fused(g, v, ks, cfg);
+            if (!fused && !has_room(ks))
+                continue;
+            const double cst = tile_cost(g, v, ks, fused);
             if (cst < best) {
                 best = cst;
                 p.family = ks > 1 ? FP8GEMM_KERNEL_SPLITK : FP8GEMM_KERNEL_LARGE;
@@ -639,6 +652,7 @@ Plan compute_plan(const GemmArgs& g, const Config& cfg)
         p.variant = TILE_256x128;
     decide_persistent(g, p, cfg);
     decide_fused(g, p, cfg);
+    p.us = best;
     if (persistent_only(p.variant) && !p.persistent)
         p.family = -1;
     if (cfg.strips_for_tiles && selected == FP8GEMM_KERNEL_AUTO && fv < 0 && fk <= 0)
@@ -649,11 +663,13 @@ Plan compute_plan(const GemmArgs& g, const Config& cfg)
 // The process-wide workspace for a call on `stream` that needs `bytes`: the caller-supplied one, else
 // the library-owned one, grown on demand (growth_target).  Growing allocates, which a stream under
 // capture does not allow (and which would leave the graph with a buffer it was not recorded with): such
-// a call gets FP8GEMM_E_WORKSPACE and the capture stays valid.  An outgrown buffer is retired, not
-// freed on the spot: kernels in flight may still use it.
-int acquire_workspace(size_t bytes, hipStream_t stream, Workspace* out)
+// a call gets FP8GEMM_E_WORKSPACE, and in *at_hand what there is, and the capture stays valid.  An outgrown buffer is
+// retired, not freed on the spot: kernels in flight may still use it.
+int acquire_workspace(size_t bytes, hipStream_t stream, Workspace* out, size_t* at_hand = nullptr)
 {
     std::lock_guard<std::mutex> lock(g_ws_mutex);
+    if (at_hand)
+        *at_hand = g_ws_user ? g_ws_user_bytes : g_ws_own_bytes;
     if (g_ws_user) {
         if (g_ws_user_bytes < bytes)
             return FP8GEMM_E_WORKSPACE;
@@ -833,6 +849,41 @@ int run_padded(const GemmArgs& g, const Plan& p, const Workspace& w, hipStream_t
     return (int)e;
 }
 
+// bytes of workspace that a call needs under a plan
+size_t call_bytes(const GemmArgs& g, const Plan& p)
+{
+    return p.padded ? padded_bytes(g, p) : with_header(plan_workspace_bytes(g, p), plan_uses_header(p));
+}
+
+// The plan of a call whose workspace of `at_hand` bytes is too small for `p`, automatic dispatch's choice: the cheapest one
+// whose partial sums find room in it, if that is next to as fast; else p, which the caller is told to bring a workspace
+// for.  Which of two plans level with each other the estimates prefer thus does not decide whether a call runs at all (639 x
+// 4608 x 7168: 128x192 tiles in two splits, 38 MiB, or 128x128 unsplit and no workspace).  The line: a new fit of the estimates
+// had taken the plan that ran without a workspace, or within the fixed array, from 0.4 % of 54 000 random problems; all of them
+// have it back from 1.08 on, all but three from 1.05 on.  Further up, calls would run that much slower where a workspace helps.
+constexpr double FITTING_PLAN_WITHIN = 1.10;
+Plan fitting_plan(const GemmArgs& g, const Plan& p, Config cfg, size_t at_hand)
+{
+    if (p.family < 0 || cfg.selected != FP8GEMM_KERNEL_AUTO || cfg.force_variant >= 0 || cfg.force_ksplit > 0 || cfg.fused_mode == 1)
+        return p;
+    GemmArgs gp = g;
+    if (p.padded) {
+        gp.m = (g.m + 15) & ~15;
+        gp.n = (g.n + 15) & ~15;
+    }
+    const size_t partial = plan_workspace_bytes(gp, p), rest = call_bytes(g, p) - partial;
+    for (;; cfg.fused_ok = false) {  // (splits added inside the kernel need the header)
+        for (const size_t taken : {WS_HEADER, rest}) {  // room beside no copies, which p may need and another plan not, and beside p's
+            cfg.partial_room = at_hand > taken ? at_hand - taken : 0;
+            const Plan fit = make_plan(g, cfg);
+            if (fit.family >= 0 && call_bytes(g, fit) <= at_hand && fit.us <= FITTING_PLAN_WITHIN * p.us)
+                return fit;
+        }
+        if (!cfg.fused_ok)
+            return p;
+    }
+}
+
 // Whether plans that add their K splits inside the kernel may run for a call on `stream`: the device
 // must place workgroups on XCDs as those kernels assume.  The first call on a device finds out with a
 // probe grid that it waits for; while `stream` is being captured nothing is probed and an unknown
@@ -874,9 +925,11 @@ int run(const void* a, const void* b, const float* as, const float* bs, void* c,
     if (p.family < 0)
         return FP8GEMM_E_KERNEL;
     Workspace w{nullptr, 0, false};
+    bool fitted = false;
     for (int attempt = 0;; ++attempt) {
-        const size_t need = p.padded ? padded_bytes(g, p) : with_header(plan_workspace_bytes(g, p), plan_uses_header(p));
+        const size_t need = call_bytes(g, p);
         int rc = FP8GEMM_OK;
+        size_t at_hand = 0;
         if (need) {
             if (explicit_ws) {
                 if (!explicit_ws->ptr || explicit_ws->bytes < need ||
@@ -884,19 +937,29 @@ int run(const void* a, const void* b, const float* as, const float* bs, void* c,
                     rc = FP8GEMM_E_WORKSPACE;
                 else
                     w = *explicit_ws;
+                at_hand = explicit_ws->ptr && (reinterpret_cast<uintptr_t>(explicit_ws->ptr) % 256) == 0 ? explicit_ws->bytes : 0;
             } else {
-                rc = acquire_workspace(need, stream, &w);
+                rc = acquire_workspace(need, stream, &w, &at_hand);
             }
         }
         if (rc == FP8GEMM_OK)
             break;
         // A plan that adds its K splits inside the kernel needs the header; when the workspace at hand cannot
         // hold it (a small caller-owned buffer, or none while the stream is being captured) the plan without
-        // it may still run -- cfg1-like shapes then need no workspace at all.  Not when that form was asked for.
-        if (rc != FP8GEMM_E_WORKSPACE || attempt > 0 || !cfg.fused_ok || cfg.fused_mode == 1 || !plan_uses_header(p))
+        // it may still run -- cfg1-like shapes then need no workspace at all.  Not when that form was asked for.  Then one
+        // that finds room (fitting_plan).
+        if (rc != FP8GEMM_E_WORKSPACE || fitted)
             return rc;
-        cfg.fused_ok = false;
-        p = make_plan(g, cfg);
+        if (attempt == 0 && cfg.fused_ok && cfg.fused_mode != 1 && plan_uses_header(p)) {
+            cfg.fused_ok = false;
+            p = make_plan(g, cfg);
+        } else {
+            cfg.fused_ok = cfg.fused_ok && placement_ok(stream);  // (not asked where p needs no more than the plan without it)
+            p = fitting_plan(g, p, cfg, at_hand);
+            if (call_bytes(g, p) > at_hand)
+                return rc;
+            fitted = true;
+        }
         if (p.family < 0)
             return FP8GEMM_E_WORKSPACE;
     }
@@ -1391,10 +1454,12 @@ int fp8_block_gemm_noalloc(const void* a, const void* b, const float* a_scale, c
     for (int fused = 0; fused < 2; ++fused) {
         Config probe = cfg;
         probe.fused_ok = fused != 0;
-        const Plan p = make_plan(g, probe);
+        Plan p = make_plan(g, probe);
         if (p.family < 0)
             return FP8GEMM_E_KERNEL;
-        const size_t bytes = p.padded ? padded_bytes(g, p) : with_header(plan_workspace_bytes(g, p), plan_uses_header(p));
+        if (call_bytes(g, p) > (size_t)FP8GEMM_NOALLOC_MAX_BYTES)
+            p = fitting_plan(g, p, probe, FP8GEMM_NOALLOC_MAX_BYTES);
+        const size_t bytes = call_bytes(g, p);
         need = bytes > need ? bytes : need;
     }
     if (need > (size_t)FP8GEMM_NOALLOC_MAX_BYTES)

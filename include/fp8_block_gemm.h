@@ -159,7 +159,8 @@ int fp8_block_gemm_grouped(int groups, const void* const* a, const void* const* 
  * this call only; `workspace` (256-byte aligned device memory of `workspace_bytes`; NULL / 0 when the
  * plan needs none) replaces the process-wide workspace: the call allocates nothing, synchronises
  * nothing and returns FP8GEMM_E_WORKSPACE when the plan needs more than it was given
- * (fp8_block_gemm_workspace_bytes_ex tells how much).  Safe to call from several host threads and on
+ * (fp8_block_gemm_workspace_bytes_ex tells how much) -- under automatic dispatch only where no plan within a tenth of
+ * the chosen one's estimated time does with that.  Safe to call from several host threads and on
  * several streams at once with distinct workspaces, and under stream capture.  No counterpart in the
  * reference, whose launcher is single-threaded on stream 0 (/root/reference/check.cu:106-119). */
 typedef struct fp8gemm_options {
@@ -213,8 +214,8 @@ size_t fp8_block_gemm_grouped_workspace_bytes_ex(int groups, const int* m, int n
  * loops, harnesses that forbid hipMalloc): the same dispatch under the same process-wide switches, but
  * the workspace of plans that split K or pad is a fixed array inside the library's device image,
  * FP8GEMM_NOALLOC_MAX_BYTES per GPU, held until the process ends.  The call allocates and frees nothing.
- * A plan that needs more than that returns FP8GEMM_E_WORKSPACE (ask fp8_block_gemm_workspace_bytes /
- * _ex beforehand; plans that neither split K nor pad need nothing and always fit).  All calls on one
+ * A plan that needs more than that returns FP8GEMM_E_WORKSPACE, as from fp8_block_gemm_ex (ask
+ * fp8_block_gemm_workspace_bytes / _ex beforehand; plans that neither split K nor pad need nothing and always fit).  All calls on one
  * GPU share that GPU's array: calls that use it and overlap on the device (different streams) race, as
  * with the process-wide workspace.  The caller clears nothing: the array starts out zero, the plans that
  * use its first FP8GEMM_WORKSPACE_HEADER_BYTES (the mailbox of the K splits) leave them zero, every other
