@@ -229,11 +229,16 @@ double tile_cost(const GemmArgs& g, int variant, int ksplit, bool fused = false)
     // tiles -- 36 random shapes of 512 ... 8192 rows where that margin decides, before / after: the 256x256 or
     // 256x128 plan +5.6 % with B cached, +10.3 % with B from HBM on average, worst -2.3 %)
     const double in_rounds = variant == TILE_128x192 && ksplit == 1 && tiles > NUM_CU ? 1.08 : 1.0;
-    const double per_item = (small ? 0.23 : variant == TILE_128x128 ? 1.01 : 0.95) + 4.38 * area + kbs * per_kb * in_rounds;
+    double per_item = (small ? 0.23 : variant == TILE_128x128 ? 1.01 : 0.95) + 4.38 * area + kbs * per_kb * in_rounds;
     // (two 64x64 workgroups share a CU, but a single row of tiles with B from HBM is fastest with at most one
     // workgroup per CU: M = 48, 64 on 12 shapes, the split that keeps tiles x splits within 256 is the best
     // measured or within 2 % of it)
     const long rounds = (items + NUM_CU - 1) / NUM_CU;
+    // (64x64 tiles over a single K block in more than one round: a round takes 1.1 to 1.6 us, the start and end of its
+    // workgroups, however little they multiply; 44 problems of 276 ... 768 such tiles.  In three rounds 128x128 tiles are ahead, 4112 x
+    // 640 x 128 4.6 us against 5.8, 1997 x 1536 x 128 5.4 against 6.5; in two they are level, 6342 x 224 x 128 4.8 and 4.9 us)
+    if (small && rounds > 1 && per_item < 1.25)
+        per_item = 1.25;
     double cost = 1.79 + rounds * per_item;
     if (ksplit > 1 && fused)  // the last split of a tile waits for the others' accumulators and reads them
         cost += (light ? 1.5 : 1.8) + 0.35 * (ksplit - 1) * (double)(bm * bn) / 4096.0;

@@ -349,3 +349,10 @@ def test_generated_k_loop_is_what_its_generator_writes():
 def test_plans_of_small_tiles(pkg, m, n, k, plan):
     """64x64 tiles where they are the best measured plan, and shapes on the other side of the line"""
     assert pkg.plan(m, n, k) == plan
+
+
+@pytest.mark.parametrize("m,n,k,plan", [(4112, 640, 128, "tile128x128_k1"), (1997, 1536, 128, "tile128x128_k1"), (384, 5712, 128, "tile128x128_k1"),
+                                        (6342, 224, 128, "tile64x64_k1"), (208, 4400, 128, "tile64x64_k1"), (2275, 864, 256, "tile64x64_k1")])
+def test_plans_over_a_single_k_block(pkg, m, n, k, plan):
+    """three rounds of 64x64 workgroups that multiply one K block each are slower than one round of 128x128; two are not"""
+    assert pkg.plan(m, n, k) == plan
