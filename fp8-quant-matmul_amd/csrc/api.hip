@@ -403,11 +403,13 @@ Plan off_grid_plan(const GemmArgs& g, const Config& cfg)
 // are shorter (a fragment of B is read once for all row tiles), in their own number of splits.  16 random problems, from
 // the Infinity Cache / from HBM: 8 / 9 % faster on average, 4 - 16 % (48 x 1232 x 1920 6.2 -> 5.4, 48 x 1536 x 7168 9.0 -> 8.3 /
 // 10.0 -> 9.4).  Left with the tiles: rows that are spread (36 x 576 x 7168 8.2 -> 8.7, 45 x 576 x 1792 5.95 -> 5.62), 57 rows and
-// more (64 x 2464 x 4736 8.2 -> 9.4 / 9.5 -> 9.8, 64 x 1680 x 2560 level) and fewer splits (one to three 2 - 20 % slower).
+// more (64 x 2464 x 4736 8.2 -> 9.4 / 9.5 -> 9.8, 64 x 1680 x 2560 level), fewer splits (one to three 2 - 20 % slower) and a B of
+// 20 MB or more, which decides there and comes slower in pieces of 64 bytes from fewer workgroups (48 x 2400 x 9984 10.5 -> 12.4 / 12.7 ->
+// 13.4, 48 x 5824 x 9088 15.8 -> 18.7 / 19.5 -> 21.1; eleven of 24 ... 53 MB 11 / 5 % slower, 55 of 1 ... 15 MB 9 / 10 % faster).
 Plan strips_for_tiles(const GemmArgs& g, const Plan& tiles)
 {
     if (tiles.variant != TILE_64x64 || !tiles.fused || g.m <= 32 || g.m > 56 || leading_dim(g) % 8 != 0 || tiles.ksplit < 5 ||
-        !decode_strip_supports(g))
+        (long long)g.n * g.k >= 20000000ll || !decode_strip_supports(g))
         return tiles;
     const int ks = decode64_ksplit(g);
     if (ks <= 1)

@@ -356,3 +356,10 @@ def test_plans_of_small_tiles(pkg, m, n, k, plan):
 def test_plans_over_a_single_k_block(pkg, m, n, k, plan):
     """three rounds of 64x64 workgroups that multiply one K block each are slower than one round of 128x128; two are not"""
     assert pkg.plan(m, n, k) == plan
+
+
+@pytest.mark.parametrize("m,n,k,plan", [(48, 2400, 9984, "tile64x64_k6f"), (48, 5824, 9088, "tile64x64_k5f"), (48, 2240, 14848, "tile64x64_k6f"),
+                                        (48, 2560, 7808, "decode64_k5"), (48, 2560, 7936, "tile64x64_k6f"), (48, 1536, 7168, "decode64_k8")])
+def test_strips_of_64_columns_in_place_of_tiles(pkg, m, n, k, plan):
+    """up to 20 MB of B"""
+    assert pkg.plan(m, n, k) == plan
