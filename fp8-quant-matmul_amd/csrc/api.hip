@@ -1195,6 +1195,16 @@ int run_grouped_each(GroupTable tab, int n, int k, hipStream_t s, const Config& 
     const double other = pinned ? 1e300 : grouped_persistent_cost(tab, n, k);
     const bool one_by_one = !pinned && other == 1e300;  // there, single problems may split K with the reduction kernel
     bool can_split = cfg.fused_ok && cfg.fused_mode != 0 && (!explicit_ws || explicit_ws->zeroed);
+    // Splits meet in the workspace, and calls that share the process-wide one must not overlap on two streams.  Groups that
+    // need none of it otherwise -- on the row grid in one launch, or each by itself in an unsplit plan -- stay without.
+    if (!explicit_ws && !pinned && can_split) {
+        bool shares = ragged && !one_by_one;
+        for (int g = 0; g < tab.groups && one_by_one && !shares; ++g) {
+            const GemmArgs ga{tab.a[g], tab.b[g], tab.a_scale[g], tab.b_scale[g], tab.c[g], tab.m[g], n, k, tab.lda[g]};
+            shares = call_bytes(ga, make_plan(ga, cfg)) > 0;
+        }
+        can_split = shares;
+    }
     EachPlan p{-1, 1, 1e300};
     Workspace w{nullptr, 0, false};
     for (;; can_split = false) {

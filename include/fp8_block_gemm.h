@@ -145,7 +145,8 @@ int fp8_block_gemm_set_fused_reduction(int mode);
  * one, where the dispatcher splits K.  Where an estimate has it ahead, tall groups run instead as ONE launch of the plain
  * tile kernel, a tile of 64x64 or 128x128 per workgroup ("tile64x64_kNf_groupedG"; n >= 256, m[g] >=
  * 16, operands 16-byte aligned): row counts off the grid as they are, without copies, and the K range of few tiles split and added inside the kernel,
- * given a zeroed workspace header as for a single problem.  A launch holds FP8GEMM_MAX_GROUPS problems; more of a kind run as
+ * given a zeroed workspace header as for a single problem.  (fp8_block_gemm_grouped splits K so only where its call uses the process-wide
+ * workspace in any case: tall groups on the grid that fill the chip touch no workspace and may run on several streams at once.)  A launch holds FP8GEMM_MAX_GROUPS problems; more of a kind run as
  * the fewest launches that hold them, of equal size, one after the other on the stream ("...groupedGxL":
  * L launches, the last of G groups).  Each C[g] is bit-identical to
  * what fp8_block_gemm_stream gives for that problem with the same tile shape and K split.  No counterpart in the

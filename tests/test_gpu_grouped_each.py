@@ -114,3 +114,21 @@ def test_in_a_graph(pkg, ms, n, k, name):
         torch.cuda.synchronize()
         assert all(torch.equal(o, w) for o, w in zip(outs, want))
         call()
+
+
+@pytest.mark.parametrize("ms,n,k", [([80 + 16 * (g % 3) for g in range(9)], 576, 7168), ([80, 96, 256, 112], 512, 1920)])
+def test_groups_on_the_grid_leave_the_process_wide_workspace_alone(pkg, ms, n, k):
+    """what calls on two streams at once would share: split in a workspace of the call's own only"""
+    import torch
+    _, _, name = _call(pkg, ms, n, k, pkg.Options(flags=pkg.FLAG_WORKSPACE_ZEROED))
+    assert "f_grouped" in name, name
+    host = [oracle.make_inputs(m, n, k, 4900 + g + m, 0.5, 30.0) for g, m in enumerate(ms)]
+    dev = [_dev(*h) for h in host]
+    outs = [torch.zeros((m, n), dtype=torch.bfloat16, device="cuda") for m in ms]
+    _say(f"[gpu case] grouped on the grid, process-wide workspace ms={ms} n={n} k={k}")
+    pkg.gemm_grouped(*[[d[i] for d in dev] for i in range(4)], outs, ms, n, k, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    name = pkg.last_kernel()
+    assert name.endswith(f"_grouped{len(ms)}") and "f_" not in name, name
+    for g, (h, m) in enumerate(zip(host, ms)):
+        _assert_every_element(outs[g].view(torch.int16).cpu().numpy().view(np.uint16), *h, m, n, k, f"{name} group {g}")
