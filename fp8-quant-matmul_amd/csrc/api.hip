@@ -1211,8 +1211,15 @@ int run_grouped_each(GroupTable tab, int n, int k, hipStream_t s, const Config& 
         p = grouped_each_plan(tab, n, k, cfg, can_split, ragged);
         if (p.variant < 0 || p.cost >= other || (one_by_one && !can_split))
             return GROUPED_NOT_APPLICABLE;
-        if (p.ksplit == 1 || (placement_ok(s) && workspace_for(with_header(0, true), s, explicit_ws, &w) == FP8GEMM_OK))
+        if (p.ksplit == 1)
             break;
+        if (!placement_ok(s))
+            continue;
+        const int rc = workspace_for(with_header(0, true), s, explicit_ws, &w);
+        if (rc == FP8GEMM_OK)
+            break;
+        if (rc != FP8GEMM_E_WORKSPACE)  // an error of the runtime's, as from a single problem
+            return rc;
     }
     const hipError_t e = launch_tile_each(tab, n, k, p.variant, p.ksplit, p.ksplit > 1 ? ws_mailbox(w) : nullptr, s);
     if (e == hipSuccess) {

@@ -3,7 +3,9 @@
  * "kernels K raised R again A missing M" -- kernels launched with more than 64 KiB of dynamic LDS, kernels whose limit was
  * raised, times it was raised again for one, launches above their kernel's limit.
  * With arguments "rows n k split groups [tile]" (split 0 = automatic; groups 0 = a single problem, by the decode kernels if
- * split; tile = a tile variant) only that call, and the mangled names of the kernels that it launches. */
+ * split; tile = a tile variant) only that call, and the mangled names of the kernels that it launches.
+ * With arguments "no-memory groups rows n k" only a grouped call in the process-wide workspace, which cannot be allocated: the
+ * names of the kernels that it launches and "code C". */
 #include <stddef.h>
 #include <stdint.h>
 #include <stdio.h>
@@ -75,7 +77,18 @@ int __hipPopCallConfiguration(dim3 *grid, dim3 *block, size_t *lds, void **strea
     return 0;
 }
 int hipGetDevice(int *device) { *device = 0; return 0; }
-int hipGetLastError(void) { return 0; }
+static int last_error;
+int hipGetLastError(void)
+{
+    const int e = last_error;
+    last_error = 0;
+    return e;
+}
+int hipMalloc(void **out, size_t bytes)
+{
+    (void)out, (void)bytes;
+    return last_error = 2; /* out of memory */
+}
 int hipStreamIsCapturing(void *stream, int *status) { (void)stream; *status = 0; return 0; }
 int hipGetSymbolAddress(void **address, const void *symbol) { (void)symbol; *address = (void *)4096; return 0; }
 /* what the look at the placement of workgroups reads back: eight XCDs in turn */
@@ -120,8 +133,25 @@ static int one_call(int words, char **word)
                   : fp8_block_gemm_ex(p, p, p, p, p, m, n, k, &opt, p, (size_t)1 << 32, 0);
 }
 
+static int no_memory(char **word)
+{
+    const int groups = atoi(word[2]), m = atoi(word[3]), n = atoi(word[4]), k = atoi(word[5]);
+    const void *ptr[64];
+    int rows[64];
+    grouped(2, 16, 0, 7168, 2048, 2, 0); /* looks at the placement of workgroups */
+    for (int g = 0; g < groups; ++g)
+        ptr[g] = p, rows[g] = m;
+    say_names = 1;
+    const int rc = fp8_block_gemm_grouped(groups, ptr, ptr, (const float *const *)ptr, (const float *const *)ptr, (void *const *)ptr,
+                                          rows, n, k, 0);
+    printf("code %d\n", rc);
+    return 0;
+}
+
 int main(int argc, char **argv)
 {
+    if (argc == 6 && !strcmp(argv[1], "no-memory"))
+        return no_memory(argv);
     if (argc >= 6)
         return one_call(argc, argv);
     const int rows[] = {1, 8, 15, 16, 24, 31, 32, 40, 47, 48, 56, 63, 64};

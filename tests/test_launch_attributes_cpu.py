@@ -88,3 +88,8 @@ def test_tall_groups_in_one_round(program, groups, m, n, k, columns):
 def test_tall_groups_with_a_tile_per_workgroup(program, groups, m, n, k, kernel):
     names = subprocess.run(["c++filt"], input="\n".join(program(m, n, k, 0, groups)), check=True, capture_output=True, text=True).stdout
     assert kernel in names, names
+
+
+def test_a_grouped_call_reports_that_no_workspace_can_be_allocated(program):
+    """rows off the grid, K to be split in the process-wide workspace: the runtime's error, before anything is launched"""
+    assert program("no-memory", 9, 87, 576, 7168) == ["code", "2"]
