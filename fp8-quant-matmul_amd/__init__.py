@@ -4,7 +4,7 @@ The directory name contains a hyphen, so the package is loaded by path: the repo
 __graft_entry__.load_package() registers it as module ``fp8_quant_matmul_amd``.
 Everything numerical happens in the HIP library behind the C ABI declared in
 include/fp8_block_gemm.h; this module only declares the ctypes prototypes, calls the hot entry
-points natively (_pycall.so) and offers pointer-level helpers for torch tensors.  There is no CPU fallback: a missing library or
+points natively where the extension module _pycall is built for the interpreter, and offers pointer-level helpers for torch tensors.  There is no CPU fallback: a missing library or
 a failing call raises.
 """
 from .capi import (  # noqa: F401

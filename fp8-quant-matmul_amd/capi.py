@@ -8,6 +8,7 @@ import ctypes as C
 import os
 import re
 import subprocess
+import sys
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 _LIB = None
@@ -40,7 +41,7 @@ def lib_path():
 
 def build(force=True):
     """Compile the HIP library for gfx950 (hipcc cross-compiles without a GPU)."""
-    cmd = ["make", "-C", _HERE, "-j8"] + (["-B"] if force else [])
+    cmd = ["make", "-C", _HERE, "-j8", f"PYTHON={sys.executable}"] + (["-B"] if force else [])
     subprocess.run(cmd, check=True, stdout=subprocess.DEVNULL)
 
 
@@ -122,16 +123,21 @@ def lib():
 
 def _load_call():
     """The native entry points of gemm, gemm_ex and the quantisers.  They answer None to arguments that are not tensors,
-    plain integers or None; those calls go through ctypes."""
+    plain integers or None; those calls go through ctypes, and so do all where the module was not built for this
+    interpreter."""
     global _CALL
     lib()
-    path = os.path.join(_HERE, "_pycall.so")
-    if not os.path.exists(path):
-        raise FileNotFoundError(f"{path} is missing: build it with __graft_entry__.build() or `make -C {_HERE}`")
-    from . import _pycall
-    _pycall.setup(Options)
+    try:
+        from . import _pycall
+        _pycall.setup(Options)
+    except ImportError:
+        _pycall = _ThroughCtypes
     _CALL = _pycall
     return _CALL
+
+
+class _ThroughCtypes:
+    gemm = gemm_ex = quantize_a = quantize_b = staticmethod(lambda *args: None)
 
 
 def error_string(code):

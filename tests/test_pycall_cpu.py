@@ -2,6 +2,9 @@
 its sizes or pointers)."""
 import ctypes as C
 import os
+import subprocess
+import sys
+import sysconfig
 
 import pytest
 
@@ -76,3 +79,33 @@ def test_the_library_is_loaded_once(pkg):
     outcome(pkg.gemm, 0, 0, 0, 0, 0, 1, 1, 128)
     paths = {line.split()[-1] for line in open("/proc/self/maps") if "libfp8gemm" in line}
     assert paths == {os.path.realpath(pkg.lib_path())}
+
+
+@pytest.mark.parametrize("name,args", [("gemm", [4096] * 5 + [16, 16, 100]), ("gemm_ex", [4096] * 5 + [16, 16, 100]),
+                                       ("quantize_a_1x128", [4096] * 3 + [16, 100]), ("quantize_b_128x128", [4096] * 3 + [16, 100])])
+def test_without_the_module(pkg, monkeypatch, name, args):
+    """not built, or for another interpreter: the library's answers all the same"""
+    f = getattr(pkg, name)
+    expected = outcome(f, *args)
+    assert expected[:2] == (pkg.Fp8GemmError, -2), expected
+    monkeypatch.setitem(f.__globals__, "_CALL", None)
+    monkeypatch.delattr(pkg, "_pycall", raising=False)
+    monkeypatch.setitem(sys.modules, pkg.__name__ + "._pycall", None)   # the import fails
+    assert outcome(f, *args) == expected
+
+
+HEADERS = pytest.mark.skipif(not os.path.exists(os.path.join(sysconfig.get_paths()["include"], "Python.h")), reason="no Python headers")
+
+
+@HEADERS
+def test_the_module_is_for_one_interpreter(pkg):
+    outcome(pkg.gemm, 0, 0, 0, 0, 0, 1, 1, 128)
+    assert pkg._pycall.__file__.endswith(sysconfig.get_config_var("EXT_SUFFIX"))
+
+
+@HEADERS
+def test_the_library_builds_without_pythons_headers(pkg):
+    make = ["make", "-n", "-B", "-C", os.path.dirname(pkg.lib_path()), "all"]
+    assert "pycall.cpp" in subprocess.run(make + [f"PYTHON={sys.executable}"], check=True, capture_output=True, text=True).stdout
+    without = subprocess.run(make + ["PYTHON=/bin/false"], check=True, capture_output=True, text=True).stdout
+    assert "pycall.cpp" not in without and "api.hip" in without
