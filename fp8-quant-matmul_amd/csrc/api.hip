@@ -38,6 +38,7 @@ struct Config {
     bool fused_ok = true;
     int fused_mode = -1;  // -1 = by cost, 0 = never, 1 = whenever fused_ok and the plan allows
     bool strips_for_tiles = true;  // 64-column strips may take the place of 64x64 tiles (strips_for_tiles below)
+    bool ragged = false;  // the problem is one with its rows rounded up to 16, which tiles take as they are (off_grid_plan)
     size_t partial_room = SIZE_MAX;  // automatic plans keep no more bytes of partial sums in the workspace (fitting_plan)
 };
 Config global_config()
@@ -181,7 +182,7 @@ double large_tile_cost(long tiles, int k, double per_kb)
 // least-squares fit to a sweep of every tile variant x ksplit over the 18 shapes of the
 // reference's table (/root/reference/README.md:15-25) and the five benchmark shapes (rms
 // error 10 %, the chosen plan within 6 % of the best measured one on all of them).
-double tile_cost(const GemmArgs& g, int variant, int ksplit, bool fused = false)
+double tile_cost(const GemmArgs& g, int variant, int ksplit, bool fused, bool ragged)
 {
     int bm, bn;
     tile_variant_dims(variant, &bm, &bn);
@@ -205,14 +206,21 @@ double tile_cost(const GemmArgs& g, int variant, int ksplit, bool fused = false)
     const long items = (ksplit > 1 && fused ? (tiles + 7) / 8 * 8 : tiles) * ksplit;
     // (64x64 tiles: the fit knows the kernel before four waves read ahead and all eight hand splits over.  Fill and store
     // take 0.72 us less, and with 64 tiles or fewer a K block takes 0.285 us for 32 of them and 0.015 more for every 32
-    // beyond, the hand-over starts 0.3 us earlier; with more tiles a block takes 9 % longer than the fit says.  649 random
+    // beyond, the hand-over starts 0.3 us earlier; with more tiles a block takes 9 % longer than the fit says, and 3.5 % with no more of
+    // them over a B that streams in.  649 random
     // problems of 48 ... 4096 rows, every plan measured: the one chosen was 1.4 / 1.7 % behind the best one from the Infinity
     // Cache / HBM and is 0.7 / 0.9 %; the 110 that change are 6 and 8 % faster on average (149 x 7168 x 256 as 128x128 5.07 us,
     // now 4.32; 224 x 2336 x 4096 as 128x128 in four 14.7 / 17.0, now in three 12.1 / 15.1; 256 x 336 x 1536 unsplit 4.69 / 6.60,
-    // now in three 4.49 / 5.30), at worst 800 x 576 x 7168 as 128x128 in seven 15.6 / 15.4, now in two 13.6 / 17.9.)
+    // now in three 4.49 / 5.30), at worst 368 x 1008 x 6144 as 128x128 in eight 14.7 / 16.0, now in two 14.0 / 19.4.)
     const bool small = variant == TILE_64x64;
     const bool light = small && !streams_b && tiles <= 64;
     const double of_small = !small ? 1.0 : light ? 0.838 : tiles > 64 ? 1.087 : 1.035;
+    // (128x128 tiles with ragged rows, whose A comes through registers: 0.06 us more to fill than the fit says, which decides where two
+    // plans are level.  Without it / with it, from the Infinity Cache and from HBM: 17 problems of 629 ... 637 x 4608 x 7168, 1891 ... 1915 x
+    // 1536 x 7168 and such, unsplit / as 128x192 in two splits, 0.96 and 1.12; 11 over K = 640 and 768, unsplit / as 64x64, 1.01 and 1.10; six in
+    // two splits / as 128x192 in four 0.96 and 1.07; three of 804 ... 815 x 576 x 7168 in seven splits / as 64x64 in two 1.10 and 0.88.
+    // On the grid it would be wrong: 51 unsplit ones / as 128x192 in two 0.88 and 1.06 (1920 x 1536 x 7168 26.8 us / 34.4 and 36.8 / 36.9),
+    // 46 / as 64x64 0.96 and 1.02.)
     // (256x192 in the persistent form: the fit knows the kernel before its barrier moved, 5 % slower)
     // (unsplit 128x128 tiles in one round: the fit knows the kernel before four waves read ahead of themselves, 10 - 15 %
     // slower from the caches, and level from HBM, where the copies bound it: they do also where a row of B starts
@@ -229,7 +237,7 @@ double tile_cost(const GemmArgs& g, int variant, int ksplit, bool fused = false)
     // tiles -- 36 random shapes of 512 ... 8192 rows where that margin decides, before / after: the 256x256 or
     // 256x128 plan +5.6 % with B cached, +10.3 % with B from HBM on average, worst -2.3 %)
     const double in_rounds = variant == TILE_128x192 && ksplit == 1 && tiles > NUM_CU ? 1.08 : 1.0;
-    double per_item = (small ? 0.23 : variant == TILE_128x128 ? 1.01 : 0.95) + 4.38 * area + kbs * per_kb * in_rounds;
+    double per_item = (small ? 0.23 : variant == TILE_128x128 && ragged ? 1.01 : 0.95) + 4.38 * area + kbs * per_kb * in_rounds;
     // (two 64x64 workgroups share a CU, but a single row of tiles with B from HBM is fastest with at most one
     // workgroup per CU: M = 48, 64 on 12 shapes, the split that keeps tiles x splits within 256 is the best
     // measured or within 2 % of it)
@@ -346,7 +354,7 @@ struct PlanKey {
     int m, n, k, lda;
     uint32_t low_bits;  // 6 low address bits of a, b, a_scale, b_scale and c
     int selected, force_variant, force_ksplit, persistent, fused_mode;
-    int allowed;  // bit 0: fused_ok, bit 1: strips_for_tiles
+    int allowed;  // bit 0: fused_ok, bit 1: strips_for_tiles, bit 2: ragged
     size_t partial_room;
     bool operator==(const PlanKey& o) const
     {
@@ -367,9 +375,9 @@ Plan make_plan(const GemmArgs& g, const Config& cfg)
     const PlanKey key{g.m, g.n, g.k, g.lda,
                       low6(g.a) | low6(g.b) << 6 | low6(g.a_scale) << 12 | low6(g.b_scale) << 18 | low6(g.c) << 24,
                       cfg.selected, cfg.force_variant, cfg.force_ksplit, cfg.persistent, cfg.fused_mode,
-                      (cfg.fused_ok ? 1 : 0) | (cfg.strips_for_tiles ? 2 : 0), cfg.partial_room};
+                      (cfg.fused_ok ? 1 : 0) | (cfg.strips_for_tiles ? 2 : 0) | (cfg.ragged ? 4 : 0), cfg.partial_room};
     const uint32_t h = ((uint32_t)g.m * 2654435761u) ^ ((uint32_t)g.n * 40503u) ^ ((uint32_t)g.k * 2246822519u) ^
-                       (cfg.fused_ok ? 0x9E3779B9u : 0u) ^ (cfg.partial_room != SIZE_MAX ? 0x85EBCA6Bu : 0u);
+                       (cfg.fused_ok ? 0x9E3779B9u : 0u) ^ (cfg.partial_room != SIZE_MAX ? 0x85EBCA6Bu : 0u) ^ (cfg.ragged ? 0xC2B2AE35u : 0u);
     PlanSlot& slot = slots[(h >> 16 ^ h) & 63];
     if (slot.used && slot.key == key)
         return slot.plan;
@@ -383,7 +391,7 @@ Plan make_plan(const GemmArgs& g, const Config& cfg)
 // operands that need one (their one or two extra launches cost about 5 us; the scalar kernel, one dependent load after the
 // other, takes 30 us for K = 128 already) or, where only m is off the grid, without any if the plan's tiles take that.  The
 // scalar kernel if padding pushes an operand past the size limit.
-Plan off_grid_plan(const GemmArgs& g, const Config& cfg)
+Plan off_grid_plan(const GemmArgs& g, Config cfg)
 {
     const long long m16 = (g.m + 15) & ~15, n16 = (g.n + 15) & ~15, lim = 0x7FFFFFFFll;
     if (m16 * g.k > lim || n16 * g.k > lim || m16 * n16 > lim)
@@ -391,6 +399,7 @@ Plan off_grid_plan(const GemmArgs& g, const Config& cfg)
     const uint8_t* const al8 = reinterpret_cast<const uint8_t*>(uintptr_t(4096));
     GemmArgs gp{al8, al8, reinterpret_cast<const float*>(uintptr_t(4096)), g.b_scale,
                 reinterpret_cast<uint16_t*>(uintptr_t(4096)), (int)m16, (int)n16, g.k};
+    cfg.ragged = tile_ragged_supports(g, TILE_128x128);
     Plan p = make_plan(gp, cfg);
     const bool tiles = p.family == FP8GEMM_KERNEL_LARGE || p.family == FP8GEMM_KERNEL_SPLITK;
     if (tiles && !p.persistent && tile_ragged_supports(g, p.variant) && tile_ragged_pays(g, p.variant, p.ksplit))
@@ -569,7 +578,7 @@ Plan compute_plan(const GemmArgs& g, const Config& cfg)
                 p.ksplit = t.ksplit;
                 decide_persistent(g, p, cfg);
                 decide_fused(g, p, cfg);
-                p.us = tile_cost(g, p.variant, p.ksplit, p.fused);
+                p.us = tile_cost(g, p.variant, p.ksplit, p.fused, cfg.ragged);
                 if (!p.fused && !has_room(p.ksplit))
                     break;
                 return p;
@@ -618,7 +627,7 @@ Plan compute_plan(const GemmArgs& g, const Config& cfg)
             const bool fused = tile_plan_fused(g, v, ks, cfg);
             if (!fused && !has_room(ks))
                 continue;
-            const double cst = tile_cost(g, v, ks, fused);
+            const double cst = tile_cost(g, v, ks, fused, cfg.ragged);
             if (cst < best) {
                 best = cst;
                 p.family = ks > 1 ? FP8GEMM_KERNEL_SPLITK : FP8GEMM_KERNEL_LARGE;
@@ -1037,7 +1046,7 @@ double grouped_tile_cost(const GroupTable& tab, int n, int k, int variant)
     if (variant == TILE_256x256)
         return large_tile_cost(grouped_tiles(tab, n, variant), k, 1.2);
     const long tiles = grouped_tiles(tab, n, variant);
-    // 128x256 tiles where they are no more than tiles of 256x256 would be, every group's last 256 rows being 128 at most: half
+    // 128x256 tiles where they are no more than tiles of 256x256 would be, which is where no group has more than 128 rows: half
     // of A's slots go to a third stage, more of B is on its way (19 launches of up to 128 rows a group 0.2 - 15 % ahead of 256x256,
     // 10 % on average).  Where they are more it is open, 15 of 25 with 1.08 to 1.65 times as many behind by up to 50 %.
     if (variant == TILE_128x256) {

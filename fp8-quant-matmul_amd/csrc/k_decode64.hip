@@ -18,7 +18,7 @@
 // 576 x 5888 7.26 -> 5.27 / 8.20 -> 6.22, 1 x 1536 x 7168 6.99 -> 5.63 / 7.27 -> 6.62, 24 x 1536 x 7168 7.90 -> 6.55, 24 x 1536 x
 // 1664 4.82 -> 3.90 / 5.66 -> 4.70, 1 x 4096 x 512 3.61 -> 2.99 / 3.77 -> 4.10, 24 x 3072 x 1536 4.58 -> 4.31, 48 x 576 x 4096 6.71 ->
 // 5.91 / 7.57 -> 6.75.  Where B is large the memory system decides, and 64 bytes of every k-row come slower than 128: 24 x
-// 7168 x 2048 6.61 -> 6.85 / 6.89 -> 8.32, 5 x 4608 x 7168 9.42 -> 11.45 / 9.62 -> 11.81 (decode64_cost).  The same pairs of
+// 7168 x 2048 6.61 -> 6.85 / 6.89 -> 8.32, 5 x 4608 x 7168 9.42 -> 11.45 / 9.62 -> 11.81 (decode64_us).  The same pairs of
 // blocks with 128-column strips, two columns to a wave: 24 x 7168 x 2048 6.69 -> 6.90, 16 x 7168 x 2048 5.69 -> 6.03; not kept.
 #include "tile_common.h"
 
@@ -390,7 +390,9 @@ inline bool neighbours_paired(int strips) { return strips > 16; }
 // us of a launch of one round, the mean of operands from the Infinity Cache and from HBM, as sums of the launch, the K blocks and
 // turns one behind the other, the hand-over (its trips, eight splits each or four, and its bytes) and B's bytes.  Fitted to
 // 340 random problems of 1 ... 64 rows, N = 256 ... 8192, K = 256 ... 8192, B up to 33 MB (strips of 64 columns in up to seven
-// splits each, 4 % rms; of 128 in the split that decode_strip_cost picks, 5 % rms).
+// splits each, 4 % rms; of 128 in the split that decode_strip_cost picks, 5 % rms).  They are asked for larger B too: of 64 random
+// problems of 33 ... 57 MB, K = 6912 ... 25216, that go to strips of 64, all are ahead from the Infinity Cache, by 22 %, and 61 from
+// HBM, by 16 % on average (1 x 1488 x 24704 16.6 -> 14.6 / 16.6 -> 15.2, 55 x 4096 x 9088 16.1 -> 15.5 / 17.0 -> 17.2).
 namespace {
 
 struct Chain {

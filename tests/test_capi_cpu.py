@@ -363,3 +363,10 @@ def test_plans_over_a_single_k_block(pkg, m, n, k, plan):
 def test_strips_of_64_columns_in_place_of_tiles(pkg, m, n, k, plan):
     """up to 20 MB of B"""
     assert pkg.plan(m, n, k) == plan
+
+
+@pytest.mark.parametrize("m,n,k,plan", [(640, 4608, 7168, "tile128x128_k1"), (1920, 1536, 7168, "tile128x128_k1"), (848, 1536, 7168, "tile128x128_k2f"),
+                                        (633, 4608, 7168, "tile128x192_k2"), (1913, 1536, 7168, "tile128x192_k2"), (842, 1536, 7168, "tile128x192_k4")])
+def test_plans_level_but_for_ragged_rows(pkg, m, n, k, plan):
+    """128x128 tiles take a little longer to fill where A comes through registers, and only there"""
+    assert pkg.plan(m, n, k) == plan

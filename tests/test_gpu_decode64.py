@@ -58,8 +58,19 @@ def test_automatic_dispatch(pkg, m, n, k):
     assert (dc[m:].cpu().numpy().view(np.uint16) == 0x7FC1).all(), "rows beyond m written"
 
 
-def test_a_split_that_does_not_exist_is_refused(pkg):
-    a, b, sa, sb = oracle.make_inputs(16, 512, 4096, 2300)
+# more splits than any plan has; splits that may not meet in the mailbox; 256 strips x 7 sending splits x 16 KiB of patches, which do
+# not fit it
+@pytest.mark.parametrize("m,n,k,ksplit,fused", [(16, 512, 4096, 17, -1), (16, 512, 4096, 4, 0), (64, 16384, 2048, 8, -1)])
+def test_a_split_that_does_not_exist_is_refused(pkg, m, n, k, ksplit, fused):
+    a, b, sa, sb = oracle.make_inputs(m, n, k, 2300)
     with pytest.raises(pkg.Fp8GemmError) as info:
-        _run(pkg, a, b, sa, sb, 16, 512, 4096, kernel=pkg.KERNEL_SKINNY, variant=3, ksplit=17)
+        _run(pkg, a, b, sa, sb, m, n, k, kernel=pkg.KERNEL_SKINNY, variant=3, ksplit=ksplit, fused=fused)
     assert info.value.code == -3
+
+
+def test_the_most_that_fits_the_mailbox(pkg):
+    m, n, k = 64, 16384, 2560
+    a, b, sa, sb = oracle.make_inputs(m, n, k, 2301, 0.5, 30.0)
+    got, name = _run(pkg, a, b, sa, sb, m, n, k, kernel=pkg.KERNEL_SKINNY, variant=3, ksplit=5)
+    assert name == "decode64_k5", name
+    _assert_every_element(got, a, b, sa, sb, m, n, k, f"{name} {m}x{n}x{k}")
