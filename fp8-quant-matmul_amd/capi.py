@@ -220,7 +220,7 @@ def force_config(tile_variant=-1, ksplit=0):
 
 def gemm_grouped(a, b, a_scale, b_scale, c, m, n, k, stream=None):
     """Grouped GEMM: lists of per-group tensors (or raw device pointers) and a list of per-group m;
-    all groups share n and k.  One persistent launch when every m is a multiple of 16."""
+    all groups share n and k.  One launch for up to 64 groups of a kind (at most 64 rows, or more)."""
     groups = len(m)
     if not (len(a) == len(b) == len(a_scale) == len(b_scale) == len(c) == groups):
         raise ValueError("one entry per group in every list")

@@ -244,7 +244,8 @@ const char* fp8_block_gemm_last_kernel(void);
  * is kept until fp8_block_gemm_release, so kernels in flight and graphs captured earlier stay valid --
  * but a graph replays into the buffer it was captured with, which later calls no longer share: give
  * captured work a workspace of its own.  A call that would have to allocate while its stream is being
- * captured returns FP8GEMM_E_WORKSPACE and leaves the capture valid.
+ * captured runs a plan next to as fast that fits what is there (as for fp8_block_gemm_ex), or returns FP8GEMM_E_WORKSPACE
+ * and leaves the capture valid.
  * fp8_block_gemm_set_workspace supplies a caller-owned buffer instead (256-byte aligned; NULL returns
  * to the library-owned one); it must hold fp8_block_gemm_workspace_bytes(m, n, k) for every shape
  * passed: what the plan needs under the switches in force when asked, for 16-byte aligned operands
